@@ -1,6 +1,7 @@
 // Tall-skinny block kernels (see block.hpp).
 #include "block.hpp"
 #include "omx_errors.hpp"
+#include "rng.hpp"
 
 namespace omx {
 
@@ -392,14 +393,6 @@ __global__ __launch_bounds__(BLK) void k_combine(ColList<T> Y, ColList<T> Y2, Co
   }
 }
 
-// splitmix64-based counter RNG -> standard normal via Box-Muller
-__device__ __forceinline__ uint64_t mix64(uint64_t z) {
-  z += 0x9e3779b97f4a7c15ull;
-  z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
-  z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
-  return z ^ (z >> 31);
-}
-
 template <typename T>
 __global__ __launch_bounds__(BLK) void k_randn(cplx<T>* base, long ld, long istride, int ncol, long K, uint64_t seed) {
   const int inst = blockIdx.y;
@@ -407,14 +400,8 @@ __global__ __launch_bounds__(BLK) void k_randn(cplx<T>* base, long ld, long istr
   for (long e = long(blockIdx.x) * BLK + threadIdx.x; e < total; e += long(gridDim.x) * BLK) {
     const int c = int(e / K);
     const long row = e - long(c) * K;
-    const uint64_t key = mix64(seed ^ mix64(uint64_t(inst) * 0x100000001b3ull + uint64_t(c))) + uint64_t(row) * 2;
-    const uint64_t h1 = mix64(key), h2 = mix64(key + 1);
-    const double u1 = (double(h1 >> 11) + 0.5) * (1.0 / 9007199254740992.0);
-    const double u2 = double(h2 >> 11) * (1.0 / 9007199254740992.0);
-    const double rad = sqrt(-2.0 * log(u1)) * 0.70710678118654752;
-    double s, co;
-    sincospi(2.0 * u2, &s, &co);
-    base[inst * istride + long(c) * ld + row] = cplx<T>{T(rad * co), T(rad * s)};
+    const c64 v = randn_at(seed, inst, c, row);
+    base[inst * istride + long(c) * ld + row] = cplx<T>{T(v.x), T(v.y)};
   }
 }
 

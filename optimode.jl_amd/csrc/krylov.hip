@@ -4,12 +4,14 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 namespace omx {
 
 namespace {
 
 constexpr int AB = 256;
+constexpr int RCQ = 16;  // Schur-complement coefficients per instance
 
 // out[(i*nb + b)] = Re sum_rows conj(a_i) b_i over block b's rows (vector i at base + i*ld),
 // accumulated in FP64
@@ -166,11 +168,16 @@ struct MinresState;
 // With WX the previous iteration's direction and solution updates come first, row by row:
 // w_new = c0 v' + c1 w1' + c2 w2' (into wout) and x += c3 w_new with v' the previous
 // iteration's u, which the output buffer y still holds until this row is written.
-template <typename T, bool WX>
+//
+// QM > 0: A u also takes -sum_c rc_c R_c (the Schur complement of VecOpsT::set_schur), the
+// coefficients rc_c = g_c <R_c, u> from k_minres_scalars; all columns' loads of a row are in
+// flight together, as in the block projection.
+template <typename T, bool WX, int QM>
 __global__ __launch_bounds__(AB) void k_minres_y1(const MinresState* ms, const cplx<T>* au, const cplx<T>* u,
                                                   const cplx<T>* r1, cplx<T>* y, long ld, long K, const int* act,
                                                   double* part, const cplx<T>* w1p, const cplx<T>* w2p,
-                                                  cplx<T>* wout, cplx<T>* x, const c64* wcoef);
+                                                  cplx<T>* wout, cplx<T>* x, const c64* wcoef, const cplx<T>* R,
+                                                  long ris, const int* nr, const c64* rc);
 
 // Stage-2 update fused with its scalar step: alfa = sum of the <v, y> partials (every block
 // the same, block 0 stores it), y <- y - (alfa/beta) r2
@@ -257,42 +264,76 @@ struct MinresState {
 // step of the iteration they follow.  Coefficients for the next lincomb go to coef.
 // one block per instance: the block sums the instance's partials (tree), then its first
 // thread runs the recurrence
-template <typename T, bool WX>
+template <typename T, bool WX, int NR>
+__device__ __forceinline__ double minres_y1_rows(const MinresState& m, const cplx<T>* au, const cplx<T>* u,
+                                                 const cplx<T>* r1, cplx<T>* y, long K, const cplx<T>* w1p,
+                                                 const cplx<T>* w2p, cplx<T>* wout, cplx<T>* x, const c64* wcoef,
+                                                 const cplx<T>* R, long ld, const c64* rc) {
+  // beta = 0 ends the instance (its v is zero): the zero scale keeps its updates finite
+  const double ib = m.beta > 0 ? 1.0 / m.beta : 0.0;
+  const double c0 = ib, c1 = -m.shift * ib, c2 = m.itn >= 1 && m.oldb > 0 ? -m.beta / m.oldb : 0.0;
+  double d0 = 0, d1 = 0, d2 = 0, d3 = 0, acc = 0;
+  if (WX) {
+    d0 = wcoef[0].x;
+    d1 = wcoef[1].x;
+    d2 = wcoef[2].x;
+    d3 = wcoef[3].x;
+  }
+  c64 cf[NR > 0 ? NR : 1];
+#pragma unroll
+  for (int c = 0; c < NR; ++c) cf[c] = rc[c];
+  for (long r = long(blockIdx.x) * AB + threadIdx.x; r < K; r += long(gridDim.x) * AB) {
+    cplx<T> e[NR > 0 ? NR : 1];
+#pragma unroll
+    for (int c = 0; c < NR; ++c) e[c] = R[c * ld + r];
+    if (WX) {
+      const cplx<T> pv = y[r], pb = w1p[r], pc = w2p[r], xr = x[r];
+      const double wx = d0 * double(pv.x) + d1 * double(pb.x) + d2 * double(pc.x);
+      const double wy = d0 * double(pv.y) + d1 * double(pb.y) + d2 * double(pc.y);
+      wout[r] = cplx<T>{T(wx), T(wy)};
+      x[r] = cplx<T>{T(double(xr.x) + d3 * wx), T(double(xr.y) + d3 * wy)};
+    }
+    const cplx<T> a = au[r], b = u[r], c = r1[r];
+    double ax = a.x, ay = a.y;
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      ax -= cf[q].x * double(e[q].x) - cf[q].y * double(e[q].y);
+      ay -= cf[q].x * double(e[q].y) + cf[q].y * double(e[q].x);
+    }
+    const cplx<T> yn{T(c0 * ax + c1 * double(b.x) + c2 * double(c.x)),
+                     T(c0 * ay + c1 * double(b.y) + c2 * double(c.y))};
+    y[r] = yn;
+    acc += double(b.x) * double(yn.x) + double(b.y) * double(yn.y);
+  }
+  return acc * ib;
+}
+
+template <typename T, bool WX, int QM, int NR = 1>
+__device__ __forceinline__ double minres_y1_cols(int n, const MinresState& m, const cplx<T>* au, const cplx<T>* u,
+                                                 const cplx<T>* r1, cplx<T>* y, long K, const cplx<T>* w1p,
+                                                 const cplx<T>* w2p, cplx<T>* wout, cplx<T>* x, const c64* wcoef,
+                                                 const cplx<T>* R, long ld, const c64* rc) {
+  if constexpr (NR <= QM) {
+    if (n == NR) return minres_y1_rows<T, WX, NR>(m, au, u, r1, y, K, w1p, w2p, wout, x, wcoef, R, ld, rc);
+    return minres_y1_cols<T, WX, QM, NR + 1>(n, m, au, u, r1, y, K, w1p, w2p, wout, x, wcoef, R, ld, rc);
+  }
+  return minres_y1_rows<T, WX, 0>(m, au, u, r1, y, K, w1p, w2p, wout, x, wcoef, R, ld, rc);
+}
+
+template <typename T, bool WX, int QM>
 __global__ __launch_bounds__(AB) void k_minres_y1(const MinresState* ms, const cplx<T>* au, const cplx<T>* u,
                                                   const cplx<T>* r1, cplx<T>* y, long ld, long K, const int* act,
                                                   double* part, const cplx<T>* w1p, const cplx<T>* w2p,
-                                                  cplx<T>* wout, cplx<T>* x, const c64* wcoef) {
+                                                  cplx<T>* wout, cplx<T>* x, const c64* wcoef, const cplx<T>* R,
+                                                  long ris, const int* nr, const c64* rc) {
   const int i = blockIdx.y;
   __shared__ double red[AB];
   double acc = 0;
   if (act[i]) {
-    const MinresState& m = ms[i];
-    // beta = 0 ends the instance (its v is zero): the zero scale keeps its updates finite
-    const double ib = m.beta > 0 ? 1.0 / m.beta : 0.0;
-    const double c0 = ib, c1 = -m.shift * ib, c2 = m.itn >= 1 ? -m.beta / m.oldb : 0.0;
-    double d0 = 0, d1 = 0, d2 = 0, d3 = 0;
-    if (WX) {
-      d0 = wcoef[4 * i].x;
-      d1 = wcoef[4 * i + 1].x;
-      d2 = wcoef[4 * i + 2].x;
-      d3 = wcoef[4 * i + 3].x;
-    }
     const long o = i * ld;
-    for (long r = long(blockIdx.x) * AB + threadIdx.x; r < K; r += long(gridDim.x) * AB) {
-      if (WX) {
-        const cplx<T> pv = y[o + r], pb = w1p[o + r], pc = w2p[o + r], xr = x[o + r];
-        const double wx = d0 * double(pv.x) + d1 * double(pb.x) + d2 * double(pc.x);
-        const double wy = d0 * double(pv.y) + d1 * double(pb.y) + d2 * double(pc.y);
-        wout[o + r] = cplx<T>{T(wx), T(wy)};
-        x[o + r] = cplx<T>{T(double(xr.x) + d3 * wx), T(double(xr.y) + d3 * wy)};
-      }
-      const cplx<T> a = au[o + r], b = u[o + r], c = r1[o + r];
-      const cplx<T> yn{T(c0 * double(a.x) + c1 * double(b.x) + c2 * double(c.x)),
-                       T(c0 * double(a.y) + c1 * double(b.y) + c2 * double(c.y))};
-      y[o + r] = yn;
-      acc += double(b.x) * double(yn.x) + double(b.y) * double(yn.y);
-    }
-    acc *= ib;
+    acc = minres_y1_cols<T, WX, QM>(QM > 0 ? nr[i] : 0, ms[i], au + o, u + o, r1 + o, y + o, K, WX ? w1p + o : nullptr,
+                                    WX ? w2p + o : nullptr, WX ? wout + o : nullptr, WX ? x + o : nullptr,
+                                    WX ? wcoef + 4 * i : nullptr, R + i * ris, ld, rc + i * RCQ);
   }
   red[threadIdx.x] = acc;
   __syncthreads();
@@ -323,10 +364,36 @@ __global__ __launch_bounds__(AB) void k_minres_y2(MinresState* ms, const double*
 // Coefficient slots (4 complex per instance each, slot s at coef + 4 ninst s): 0 for the
 // y updates of stages 1 and 2, 1 for the fused w/x update of stage 3, 2 for the next
 // v = y / beta (stages 0 and 3); slot 3 belongs to the projections.
+// With rpart (qm partial dots of the block residual columns per projection block), also the
+// Schur-complement coefficients rc_c = g_c <R_c, y> for the next operator application.
 __global__ __launch_bounds__(AB) void k_minres_scalars(MinresState* ms, const double* part, int nb, c64* coef,
-                                                       int stage, int ninst, const int* act) {
+                                                       int stage, int ninst, const int* act, const c64* rpart, int qm,
+                                                       const double* rg, c64* rc) {
   const int i = blockIdx.x;
   __shared__ double red[AB];
+  __shared__ double rr[AB], ri[AB];
+  if (rpart && act[i]) {
+    const int c = threadIdx.x % qm, j = threadIdx.x / qm, G = AB / qm;
+    double a = 0, b = 0;
+#pragma unroll 8
+    for (int q = j; q < nb; q += G) {
+      const c64 v = rpart[(long(i) * nb + q) * qm + c];
+      a += v.x;
+      b += v.y;
+    }
+    rr[threadIdx.x] = a;
+    ri[threadIdx.x] = b;
+    __syncthreads();
+    if (int(threadIdx.x) < qm) {
+      double sa = 0, sb = 0;
+      for (int q = 0; q < G; ++q) {
+        sa += rr[q * qm + threadIdx.x];
+        sb += ri[q * qm + threadIdx.x];
+      }
+      const double g = rg[RCQ * i + threadIdx.x];
+      rc[RCQ * i + threadIdx.x] = c64{g * sa, g * sb};
+    }
+  }
   double acc = 0;
   for (int b = threadIdx.x; b < nb; b += AB) acc += part[long(i) * nb + b];
   red[threadIdx.x] = acc;
@@ -369,6 +436,13 @@ __global__ __launch_bounds__(AB) void k_minres_scalars(MinresState* ms, const do
       c[0] = c64{1, 0};
       c[1] = c64{-m.alfa / m.beta, 0};
     } else if (stage == 3) {
+      // an instance whose beta is exactly zero has ended (<r, P r> rounds to or below zero once
+      // its residual is at the vectors' accuracy): the group's remaining iterations leave its x
+      // as it is (all coefficients zero) instead of dividing by that beta
+      if (m.beta == 0) {
+        m.done = 1;
+        return;
+      }
       // beta = sqrt(<r2, M r2>); rotations; w and x updates
       m.itn += 1;
       m.oldb = m.beta;
@@ -457,10 +531,12 @@ __device__ __forceinline__ void qdot_cols(int n, const cplx<T>* q, long qld, con
   }
 }
 
-// x <- x + sum_c cf_c Q_c over the rows, and sum of Re <d, x_new> when DOT
-template <typename T, int NQ, bool DOT>
+// x <- x + sum_c cf_c Q_c over the rows, and sum of Re <d, x_new> when DOT; with SCHUR also
+// the sums of conj(R_c) x_new (R laid out as Q) into sr, si
+template <typename T, int NQ, bool DOT, bool SCHUR>
 __device__ __forceinline__ double qproject_rows(const c64* cf, const cplx<T>* q, long qld, cplx<T>* x,
-                                                const cplx<T>* dv, long r0, long stride, long K) {
+                                                const cplx<T>* dv, long r0, long stride, long K, const cplx<T>* R,
+                                                double* rsr, double* rsi) {
   double acc = 0;
   for (long r = r0; r < K; r += stride) {
     const cplx<T> xv = x[r];
@@ -469,6 +545,11 @@ __device__ __forceinline__ double qproject_rows(const c64* cf, const cplx<T>* q,
     cplx<T> e[NQ];
 #pragma unroll
     for (int c = 0; c < NQ; ++c) e[c] = q[c * qld + r];
+    cplx<T> f[SCHUR ? NQ : 1];
+    if constexpr (SCHUR) {
+#pragma unroll
+      for (int c = 0; c < NQ; ++c) f[c] = R[c * qld + r];
+    }
     double nx = xv.x, ny = xv.y;
 #pragma unroll
     for (int c = 0; c < NQ; ++c) {
@@ -478,18 +559,30 @@ __device__ __forceinline__ double qproject_rows(const c64* cf, const cplx<T>* q,
     const cplx<T> xn{T(nx), T(ny)};
     x[r] = xn;
     if (DOT) acc += double(dr.x) * double(xn.x) + double(dr.y) * double(xn.y);
+    if constexpr (SCHUR) {
+#pragma unroll
+      for (int c = 0; c < NQ; ++c) {
+        rsr[c] += double(f[c].x) * double(xn.x) + double(f[c].y) * double(xn.y);
+        rsi[c] += double(f[c].x) * double(xn.y) - double(f[c].y) * double(xn.x);
+      }
+    }
   }
   return acc;
 }
 
-template <typename T, int QM, int NQ = 1>
+template <typename T, int QM, bool SCHUR, int NQ = 1>
 __device__ __forceinline__ double qproject_cols(int n, const c64* cf, const cplx<T>* q, long qld, cplx<T>* x,
-                                                const cplx<T>* dv, long r0, long stride, long K) {
+                                                const cplx<T>* dv, long r0, long stride, long K, const cplx<T>* R,
+                                                double* rsr, double* rsi) {
   if constexpr (NQ <= QM) {
-    if (n == NQ)
-      return dv ? qproject_rows<T, NQ, true>(cf, q, qld, x, dv, r0, stride, K)
-                : qproject_rows<T, NQ, false>(cf, q, qld, x, dv, r0, stride, K);
-    return qproject_cols<T, QM, NQ + 1>(n, cf, q, qld, x, dv, r0, stride, K);
+    if (n == NQ) {
+      if constexpr (SCHUR)
+        return qproject_rows<T, NQ, true, true>(cf, q, qld, x, dv, r0, stride, K, R, rsr, rsi);
+      else
+        return dv ? qproject_rows<T, NQ, true, false>(cf, q, qld, x, dv, r0, stride, K, R, rsr, rsi)
+                  : qproject_rows<T, NQ, false, false>(cf, q, qld, x, dv, r0, stride, K, R, rsr, rsi);
+    }
+    return qproject_cols<T, QM, SCHUR, NQ + 1>(n, cf, q, qld, x, dv, r0, stride, K, R, rsr, rsi);
   }
   return 0.0;
 }
@@ -535,11 +628,12 @@ __global__ __launch_bounds__(AB) void k_qdot(const cplx<T>* Q, long qld, long qi
 
 // x_i <- x_i - sum_c <Q_c, x_i> Q_c (the block projection), the coefficients summed by every
 // block from k_qdot's qnblk partials of its instance in one fixed order; with d, the
-// partials of Re <d_i, x_i new> into part[i gridDim.x + blockIdx.x]
-template <typename T, int QM>
+// partials of Re <d_i, x_i new> into part[i gridDim.x + blockIdx.x], and with SCHUR those of
+// <R_c, x_i new> into rpart[(i gridDim.x + blockIdx.x) QM + c] (zero past nq[i])
+template <typename T, int QM, bool SCHUR>
 __global__ __launch_bounds__(AB) void k_qproject(const c64* qpart, int qnblk, const cplx<T>* Q, long qld, long qis,
                                                  const int* nq, cplx<T>* X, const cplx<T>* d, long ld, long K,
-                                                 const int* act, double* part) {
+                                                 const int* act, double* part, const cplx<T>* R, c64* rpart) {
   constexpr int G = AB / QM;
   const int i = blockIdx.y;
   __shared__ double red[AB];
@@ -572,9 +666,40 @@ __global__ __launch_bounds__(AB) void k_qproject(const c64* qpart, int qnblk, co
     c64 cf[QM];
 #pragma unroll
     for (int c = 0; c < QM; ++c) cf[c] = c < n ? cfs[c] : c64{0, 0};
+    double rsr[SCHUR ? QM : 1], rsi[SCHUR ? QM : 1];
+    if constexpr (SCHUR) {
+#pragma unroll
+      for (int c = 0; c < QM; ++c) rsr[c] = rsi[c] = 0.0;
+    }
     if (n > 0)
-      acc = qproject_cols<T, QM>(n, cf, Q + i * qis, qld, X + i * ld, d ? d + i * ld : nullptr,
-                                 long(blockIdx.x) * AB + threadIdx.x, long(gridDim.x) * AB, K);
+      acc = qproject_cols<T, QM, SCHUR>(n, cf, Q + i * qis, qld, X + i * ld, d ? d + i * ld : nullptr,
+                                        long(blockIdx.x) * AB + threadIdx.x, long(gridDim.x) * AB, K,
+                                        SCHUR ? R + i * qis : nullptr, rsr, rsi);
+    if constexpr (SCHUR) {
+      // per column: a wavefront butterfly, then the wavefronts in order
+      const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
+      for (int c = 0; c < QM; ++c) {
+        double a = rsr[c], b = rsi[c];
+        for (int off = 32; off > 0; off >>= 1) {
+          a += __shfl_xor(a, off, 64);
+          b += __shfl_xor(b, off, 64);
+        }
+        if (lane == 0) {
+          gr[wv][c] = a;
+          gi[wv][c] = b;
+        }
+      }
+      __syncthreads();
+      if (threadIdx.x < QM) {
+        double a = 0, b = 0;
+        for (int w = 0; w < AB / 64; ++w) {
+          a += gr[w][threadIdx.x];
+          b += gi[w][threadIdx.x];
+        }
+        rpart[(long(i) * gridDim.x + blockIdx.x) * QM + threadIdx.x] = c64{a, b};
+      }
+    }
   }
   if (!part) return;
   red[threadIdx.x] = acc;
@@ -646,7 +771,7 @@ template <typename T> void VecOpsT<T>::set_block(const C* Qb, long qis, const in
   // the real dot partials (nb nblk, at the start, where the MINRES steps read them), then
   // the block partials (nb nblk QMAX complex): every block of k_qproject reads the latter
   // while others write the former, so the two never overlap
-  part.ensure(sizeof(c64) * size_t(nb) * (size_t(nblk) + size_t(nblk) * QMAX));
+  part.ensure(sizeof(c64) * size_t(nb) * (size_t(nblk) + 2 * size_t(nblk) * QMAX + RCQ));
   Q = Qb;
   qistride = qis;
   qn = nq;
@@ -656,20 +781,33 @@ template <typename T> void VecOpsT<T>::set_block(const C* Qb, long qis, const in
   qblk = std::max(1, std::min(nblk, 64));
 }
 
+template <typename T> void VecOpsT<T>::set_schur(const C* Rb, const double* weights) {
+  if (!Q) throw Error(OMX_ERR_INTERNAL, "the Schur complement needs the block projection");
+  R = Rb;
+  rg = weights;
+}
+
 template <typename T> void VecOpsT<T>::project_dot_to(C* x, const int* act, const C* dot_with, double* out) {
   const dim3 g(nblk, nb);
   if (Q) {
     c64* qp = part.template as<c64>() + size_t(nb) * nblk;
     const dim3 gq(qblk, nb);
-    if (qmax <= 8) {
-      hipLaunchKernelGGL((k_qdot<T, 8>), gq, dim3(AB), 0, s, Q, ld, qistride, qn, x, ld, K, act, qp);
-      hipLaunchKernelGGL((k_qproject<T, 8>), g, dim3(AB), 0, s, qp, qblk, Q, ld, qistride, qn, x, dot_with, ld, K,
-                         act, out);
-    } else {
-      hipLaunchKernelGGL((k_qdot<T, QMAX>), gq, dim3(AB), 0, s, Q, ld, qistride, qn, x, ld, K, act, qp);
-      hipLaunchKernelGGL((k_qproject<T, QMAX>), g, dim3(AB), 0, s, qp, qblk, Q, ld, qistride, qn, x, dot_with, ld, K,
-                         act, out);
-    }
+    // past the block partials: the residual columns' partials, and the coefficients from them
+    c64* rp = qp + size_t(nb) * nblk * QMAX;
+    auto launch = [&](auto QMc) {
+      constexpr int QMv = decltype(QMc)::value;
+      hipLaunchKernelGGL((k_qdot<T, QMv>), gq, dim3(AB), 0, s, Q, ld, qistride, qn, x, ld, K, act, qp);
+      if (R && dot_with)
+        hipLaunchKernelGGL((k_qproject<T, QMv, true>), g, dim3(AB), 0, s, qp, qblk, Q, ld, qistride, qn, x, dot_with, ld,
+                           K, act, out, R, rp);
+      else
+        hipLaunchKernelGGL((k_qproject<T, QMv, false>), g, dim3(AB), 0, s, qp, qblk, Q, ld, qistride, qn, x, dot_with,
+                           ld, K, act, out, R, rp);
+    };
+    if (qmax <= 8)
+      launch(std::integral_constant<int, 8>{});
+    else
+      launch(std::integral_constant<int, QMAX>{});
     return;
   }
   hipLaunchKernelGGL(k_cdot<T>, g, dim3(AB), 0, s, EV, x, ld, K, act, part.template as<c64>());
@@ -741,7 +879,10 @@ int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shi
   // y = P r1 (projected)
   launch_operator<T>(OP_P, plan, R1v, Yv, dm, sel, dk, nullptr, 0, s);
   V.project(y, act, r1);  // and the partials of <r1, y>
-  hipLaunchKernelGGL(k_minres_scalars, dim3(nb), dim3(AB), 0, s, ms, part, nblk, coef, 0, nb, act);
+  const int qm = V.qmax <= 8 ? 8 : VecOpsT<T>::QMAX;
+  const c64* rpart = V.R ? V.part.template as<c64>() + size_t(nb) * nblk * (1 + VecOpsT<T>::QMAX) : nullptr;
+  c64* rc = V.R ? V.part.template as<c64>() + size_t(nb) * nblk * (1 + 2 * VecOpsT<T>::QMAX) : nullptr;
+  hipLaunchKernelGGL(k_minres_scalars, dim3(nb), dim3(AB), 0, s, ms, part, nblk, coef, 0, nb, act, rpart, qm, V.rg, rc);
   OMX_HIP_CHECK(hipMemcpyAsync(r2, r1, vb, hipMemcpyDeviceToDevice, s));
   std::vector<int> live(want);
   int it = 0;
@@ -760,12 +901,24 @@ int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shi
     BView<T> Uv{y, ld, ld};
     launch_operator<T>(OP_M, plan, Uv, AVv, dm, sel, dk, nullptr, 0, s);
     // v-buffer <- (A u - shift u) / beta - (beta/oldb) r1 with the partials of <v, .>
+    auto y1 = [&](auto WXc, auto QMc) {
+      constexpr bool wx = decltype(WXc)::value;
+      hipLaunchKernelGGL((k_minres_y1<T, wx, decltype(QMc)::value>), vg, dim3(AB), 0, s, ms, avp, y, r1, v, ld, V.K, la,
+                         part, wx ? pw1 : nullptr, wx ? pw2 : nullptr, wx ? pwo : nullptr, wx ? x : nullptr,
+                         wx ? coef + 4 * nb : nullptr, V.R, V.qistride, V.qn, rc);
+    };
+    auto y1q = [&](auto WXc) {
+      if (!V.R)
+        y1(WXc, std::integral_constant<int, 0>{});
+      else if (V.qmax <= 8)
+        y1(WXc, std::integral_constant<int, 8>{});
+      else
+        y1(WXc, std::integral_constant<int, VecOpsT<T>::QMAX>{});
+    };
     if (fuse)
-      hipLaunchKernelGGL((k_minres_y1<T, true>), vg, dim3(AB), 0, s, ms, avp, y, r1, v, ld, V.K, la, part, pw1, pw2,
-                         pwo, x, coef + 4 * nb);
+      y1q(std::true_type{});
     else
-      hipLaunchKernelGGL((k_minres_y1<T, false>), vg, dim3(AB), 0, s, ms, avp, y, r1, v, ld, V.K, la, part, nullptr,
-                         nullptr, nullptr, nullptr, nullptr);
+      y1q(std::false_type{});
     // alfa = <v, .>; v-buffer -= (alfa/beta) r2 (stage 2 fused)
     hipLaunchKernelGGL((k_minres_y2<T>), vg, dim3(AB), 0, s, ms, part, nblk, r2, v, ld, V.K, la);
     C* u = y;   // the next iteration's v-buffer, read first by this iteration's w/x update
@@ -776,7 +929,8 @@ int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shi
     launch_operator<T>(OP_P, plan, R2b, Yb, dm, sel, dk, nullptr, 0, s);
     // yn <- yn - ev <ev, yn> (or the block projection) with the partials of <r2, yn>
     V.project_dot_to(yn, la, r2, cpart2);
-    hipLaunchKernelGGL(k_minres_scalars, dim3(nb), dim3(AB), 0, s, ms, cpart2, nblk, coef, 3, nb, la);
+    hipLaunchKernelGGL(k_minres_scalars, dim3(nb), dim3(AB), 0, s, ms, cpart2, nblk, coef, 3, nb, la, rpart, qm,
+                       V.rg, rc);
     // this iteration's w/x update, pending (its v is u, the next iteration's v-buffer)
     pw1 = w2;
     pw2 = w;

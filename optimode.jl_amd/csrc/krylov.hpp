@@ -42,6 +42,13 @@ template <typename T> struct VecOpsT {
   // most QMAX columns; nq on the device) instead of along ev_i.
   static constexpr int QMAX = 16;
   void set_block(const C* Qb, long qis, const int* nq, int nq_max);
+  // With a block whose columns are Ritz vectors but not yet eigenvectors, the system on its
+  // complement is the Schur complement (M - shift) - sum_c g_c R_c R_c^H, R_c = M Q_c - theta_c
+  // Q_c (laid out as the block), g_c = 1 / (theta_c - shift) (weights: 16 per instance, 0
+  // leaves a column out).  minres_complement_t then applies it in place of M - shift.
+  void set_schur(const C* Rb, const double* weights);
+  const C* R = nullptr;
+  const double* rg = nullptr;
   const C* Q = nullptr;
   long qistride = 0;
   const int* qn = nullptr;

@@ -1,0 +1,1346 @@
+// Shared-subspace eigensolve of all bands at once (see multik.hpp).
+//
+// Storage per problem, FP32: column slots of 7 planes of cs complex values (cs = N rounded up
+// to 64, the pads stay zero): planes 0-2 F0, 3-4 F1 (x, y), pixels column-major (iy fastest,
+// the order of eps6c); planes 5-6 g1, g2, plane waves row-major (ix fastest).  Slots: X and P
+// in two buffers each (an iteration reads one and writes the other), W in one.
+//
+// One iteration t (launches over all problems; a problem that is done returns at once):
+//   gram    three eps^-1-weighted Gram matrices of [F0 F1] and the norm's at its nodes (MFMA)
+//   reduce  sum of the chunk partials
+//   dense   per band: its pencil at k_j, Ritz pair j, Newton step of k_j
+//   combine X <- S C, P <- [W P] C, one pass over all planes (F0 and F1 stay consistent with g)
+//   colE    eps^-1 (F0 + k F1), inverse FFT along y
+//   rowR    inverse FFT along x, residual r = M x - lam x and its norm, P-map, FFT along x
+//   control norms, convergence, the columns that still iterate, k
+//   colP    FFT along y, eps_ave, FFT back
+//   rowW    FFT along x, w = P r -> g, D0 and D1, FFT along x
+//   colF    FFT along y of the five planes
+#include "multik.hpp"
+
+#include <algorithm>
+#include <chrono>
+#include <cmath>
+#include <cstdio>
+#include <cstring>
+
+#include "fft_lds.hpp"
+#include "omx_errors.hpp"
+#include "rng.hpp"
+#include "solver.hpp"
+
+namespace omx {
+
+namespace {
+
+constexpr int PLANES = 7;
+constexpr int FT = 512;   // threads of the transform kernels
+constexpr int NGRAM = 3 + MK_NODES + 1;  // G00, G01, G11, the nodes, the k-independent part
+
+struct MkState {
+  int m, nev;              // columns, bands
+  int na, np;              // W columns and P columns of the current search space
+  int iter, done, par;     // done: 1 converged, 2 failed; par: X / P buffer of the last space
+  int moves;               // iterations whose Newton step moved a band's k by more than ftol
+  int wcol[MK_MAXM];       // column of W slot s
+  int pslot[MK_MAXM];      // P slots in use
+  int its[MK_MAXM];        // iteration a band first met its thresholds (0: not yet)
+  double omega2, tol, ftol;
+  double k[MK_MAXM];       // current k per column
+  double keval[MK_MAXM];   // k the column's Ritz pair was taken at
+  double knew[MK_MAXM];    // after the Newton step
+  double lam[MK_MAXM], slope[MK_MAXM], rnorm[MK_MAXM];
+};
+
+struct MkGeo {
+  int nx, ny, mmax;
+  long N, cs, slots;       // slots: complex values per problem in the column store
+  double invdx, invdy;
+  FFTFactors fx, fy;
+  const c32 *twx, *twy;
+  const float* eps6c;
+  long eps_stride;
+};
+
+__device__ __forceinline__ long col_off(const MkGeo& g, int slot) { return long(slot) * PLANES * g.cs; }
+// slots: X buffer b, P buffer b, W
+__device__ __forceinline__ int slot_x(const MkGeo& g, int b, int c) { return b * g.mmax + c; }
+__device__ __forceinline__ int slot_p(const MkGeo& g, int b, int c) { return (2 + b) * g.mmax + c; }
+__device__ __forceinline__ int slot_w(const MkGeo& g, int c) { return 4 * g.mmax + c; }
+
+// slot of search-space column q = [X (m) | W (na) | P (np)] with X, P in buffer b
+__device__ __forceinline__ int space_slot(const MkGeo& g, const MkState& s, int b, int q) {
+  if (q < s.m) return slot_x(g, b, q);
+  if (q < s.m + s.na) return slot_w(g, q - s.m);
+  return slot_p(g, b, s.pslot[q - s.m - s.na]);
+}
+
+// Chebyshev nodes over the columns' k range (widened to 2% where it is narrower)
+__device__ __forceinline__ void mk_nodes(const MkState& s, double* node) {
+  double lo = s.k[0], hi = s.k[0];
+  for (int j = 1; j < s.m; ++j) {
+    lo = fmin(lo, s.k[j]);
+    hi = fmax(hi, s.k[j]);
+  }
+  const double c = 0.5 * (lo + hi), h = fmax(0.5 * (hi - lo), 0.01 * fabs(c));
+#pragma unroll
+  for (int t = 0; t < MK_NODES; ++t) node[t] = c + h * cospi((t + 0.5) / MK_NODES);
+}
+
+// in-plane part of a plane wave: n = z x w / rho (y at rho = 0)
+struct Wave {
+  float n0, n1, rho2, rho;
+};
+__device__ __forceinline__ Wave wave_at(int ix, int iy, const MkGeo& g) {
+  const float wx = -float(double(fft_index(ix, g.nx)) * g.invdx), wy = -float(double(fft_index(iy, g.ny)) * g.invdy);
+  Wave v;
+  v.rho2 = wx * wx + wy * wy;
+  v.rho = sqrtf(v.rho2);
+  const float ir = v.rho2 > 0.f ? 1.f / v.rho : 0.f;
+  v.n0 = -wy * ir;
+  v.n1 = v.rho2 > 0.f ? wx * ir : 1.f;
+  return v;
+}
+
+// ---------------------------------------------------------------------------------------
+// Start block: g of the X columns (buffer 0)
+// ---------------------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_mk_start(MkGeo geo, c32* cols, const MkState* st, int p, const c64* src,
+                                                  long lds, int nsrc, int hw, uint64_t seed) {
+  const int c = blockIdx.y;
+  const MkState& s = st[p];
+  c32* g1 = cols + p * geo.slots + col_off(geo, slot_x(geo, 0, c)) + 5 * geo.cs;
+  const double k = s.k[c];
+  for (long e = long(blockIdx.x) * 256 + threadIdx.x; e < geo.N; e += long(gridDim.x) * 256) {
+    const int iy = int(e / geo.nx), ix = int(e - long(iy) * geo.nx);
+    const double wx = double(fft_index(ix, geo.nx)) * geo.invdx, wy = double(fft_index(iy, geo.ny)) * geo.invdy;
+    const double w2 = wx * wx + wy * wy + k * k;
+    c64 h1, h2;
+    if (c >= nsrc) {
+      // random, weighted like the operator's inverse so that the low plane waves lead
+      const double f = 1.0 / w2;
+      h1 = randn_at(seed, p, c, 2 * e);
+      h2 = randn_at(seed, p, c, 2 * e + 1);
+      h1 = c64{h1.x * f, h1.y * f};
+      h2 = c64{h2.x * f, h2.y * f};
+    } else if (hw > 0) {
+      const int gx = ix < hw / 2 ? ix : ix - (geo.nx - hw), gy = iy < hw / 2 ? iy : iy - (geo.ny - hw);
+      const bool in = (ix < hw / 2 || ix >= geo.nx - hw / 2) && (iy < hw / 2 || iy >= geo.ny - hw / 2);
+      h1 = h2 = c64{0, 0};
+      if (in) {
+        const c64* v = src + long(c) * lds + 2 * (gx + long(hw) * gy);
+        h1 = v[0];
+        h2 = v[1];
+      }
+    } else {
+      const c64* v = src + long(c) * lds + 2 * e;
+      h1 = v[0];
+      h2 = v[1];
+    }
+    const double w = sqrt(w2);
+    g1[e] = c32{float(w * h1.x), float(w * h1.y)};
+    g1[geo.cs + e] = c32{float(h2.x), float(h2.y)};
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// Gram matrices on the matrix cores.  As in block.hip: the four k slots of one
+// v_mfma_f32_16x16x4 are four rows, lane (i = l % 16, g = l / 16) holds S consecutive rows of
+// column i of each 16-column tile, loaded straight from HBM with 16-byte loads, and the four
+// waves of a block take interleaved stages.  KIND 0: F0^H e F0, 1: F0^H e F1, 2: F1^H e F1
+// (e = eps^-1 per pixel, three components contracted per row), 3: the norm's matrices
+// g^H psi g for NB of the nodes (psi = 1 / (rho^2 + kappa^2) on g1; the last one g2^H g2).
+// Hermitian kinds compute the tiles on and above the diagonal only.
+// ---------------------------------------------------------------------------------------
+typedef float fx4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ fx4 mfma(float a, float b, fx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+template <int S> __device__ __forceinline__ void load_col(const c32* col, long row, c32 (&v)[S]) {
+  if (col != nullptr) {
+    const fx4* q = reinterpret_cast<const fx4*>(col + row);
+#pragma unroll
+    for (int j = 0; j < S / 2; ++j) {
+      const fx4 w = q[j];
+      v[2 * j] = c32{w.x, w.y};
+      v[2 * j + 1] = c32{w.z, w.w};
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < S; ++j) v[j] = c32{0.f, 0.f};
+  }
+}
+
+template <int NT, int KIND, int NB, int S>
+__global__ __launch_bounds__(256) void k_mk_gram(MkGeo geo, const c32* cols, const MkState* st, int buf, long rpc,
+                                                 c32* part) {
+  constexpr int PM = 16 * NT, NQ = KIND == 3 ? NB : 1;
+  __shared__ const c32* cp[PM];
+  __shared__ float kap2[MK_NODES];
+  __shared__ float red[4][8][64];
+  const int p = blockIdx.y, chunk = blockIdx.x, q0 = KIND == 3 ? blockIdx.z * NB : 0;
+  const MkState& s = st[p];
+  if (s.done) return;
+  const int n = s.m + s.na + s.np;
+  if (threadIdx.x < PM)
+    cp[threadIdx.x] =
+        int(threadIdx.x) < n ? cols + p * geo.slots + col_off(geo, space_slot(geo, s, buf, threadIdx.x)) : nullptr;
+  if (KIND == 3 && threadIdx.x == 0) {
+    double node[MK_NODES];
+    mk_nodes(s, node);
+    for (int t = 0; t < MK_NODES; ++t) kap2[t] = float(node[t] * node[t]);
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, g = lane >> 4;
+  const c32* col[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) col[t] = cp[t * 16 + i16];
+  fx4 ar[NQ][NT][NT], ai[NQ][NT][NT];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q)
+#pragma unroll
+    for (int a = 0; a < NT; ++a)
+#pragma unroll
+      for (int b = 0; b < NT; ++b) ar[q][a][b] = ai[q][a][b] = fx4{0.f, 0.f, 0.f, 0.f};
+  // += conj(x) y over the rows of a stage, every tile pair
+  auto product = [&](int q, const c32(&x)[NT][S], const c32(&y)[NT][S]) {
+#pragma unroll
+    for (int r = 0; r < S; ++r)
+#pragma unroll
+      for (int a = 0; a < NT; ++a)
+#pragma unroll
+        for (int b = 0; b < NT; ++b) {
+          if (KIND != 1 && a > b) continue;
+          ar[q][a][b] = mfma(x[a][r].x, y[b][r].x, ar[q][a][b]);
+          ai[q][a][b] = mfma(x[a][r].x, y[b][r].y, ai[q][a][b]);
+          ar[q][a][b] = mfma(x[a][r].y, y[b][r].y, ar[q][a][b]);
+          ai[q][a][b] = mfma(x[a][r].y, -y[b][r].x, ai[q][a][b]);
+        }
+  };
+  const long r0 = chunk * rpc, r1 = r0 + rpc < geo.N ? r0 + rpc : geo.N;
+  const float* eps = geo.eps6c + p * geo.eps_stride;
+  for (long row = r0 + (wave * 4 + g) * S; row - g * S < r1; row += 16 * S) {
+    const bool in = row < r1;  // rows past r1 belong to the next chunk (or are pads)
+    const c32* no = nullptr;
+    if (KIND < 3) {
+      float e[S][6];
+#pragma unroll
+      for (int r = 0; r < S; ++r)
+#pragma unroll
+        for (int c = 0; c < 6; ++c) e[r][c] = 0.f;
+      if (in && row + S <= geo.N) {
+        const fx4* q = reinterpret_cast<const fx4*>(eps + 6 * row);
+#pragma unroll
+        for (int j = 0; j < 6 * S / 4; ++j) {
+          const fx4 w = q[j];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) e[(4 * j + u) / 6][(4 * j + u) % 6] = w[u];
+        }
+      } else if (in) {
+#pragma unroll
+        for (int r = 0; r < S; ++r)
+          if (row + r < geo.N)
+#pragma unroll
+            for (int c = 0; c < 6; ++c) e[r][c] = eps[6 * (row + r) + c];
+      }
+      c32 x[3][NT][S], y[3][NT][S];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const c32* c = in ? col[t] : no;
+        if (KIND != 2)
+#pragma unroll
+          for (int a = 0; a < 3; ++a) load_col<S>(c ? c + a * geo.cs : no, row, x[a][t]);
+        if (KIND != 0) {
+          c32 f[2][S];
+#pragma unroll
+          for (int a = 0; a < 2; ++a) load_col<S>(c ? c + (3 + a) * geo.cs : no, row, f[a]);
+#pragma unroll
+          for (int r = 0; r < S; ++r) {
+            y[0][t][r] = f[0][r] * e[r][0] + f[1][r] * e[r][3];
+            y[1][t][r] = f[0][r] * e[r][3] + f[1][r] * e[r][1];
+            if (KIND == 1) y[2][t][r] = f[0][r] * e[r][4] + f[1][r] * e[r][5];
+            if (KIND == 2) {
+              x[0][t][r] = f[0][r];
+              x[1][t][r] = f[1][r];
+            }
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < S; ++r) {
+            const c32 f0 = x[0][t][r], f1 = x[1][t][r], f2 = x[2][t][r];
+            y[0][t][r] = f0 * e[r][0] + f1 * e[r][3] + f2 * e[r][4];
+            y[1][t][r] = f0 * e[r][3] + f1 * e[r][1] + f2 * e[r][5];
+            y[2][t][r] = f0 * e[r][4] + f1 * e[r][5] + f2 * e[r][2];
+          }
+        }
+      }
+#pragma unroll
+      for (int a = 0; a < (KIND == 2 ? 2 : 3); ++a) product(0, x[a], y[a]);
+    } else {
+      c32 x[NT][S], x2[NT][S], y[NT][S];
+      float rho2[S];
+#pragma unroll
+      for (int r = 0; r < S; ++r) {
+        const long e = row + r;
+        const int iy = int(e / geo.nx), ix = int(e - long(iy) * geo.nx);
+        const float wx = float(double(fft_index(ix, geo.nx)) * geo.invdx);
+        const float wy = float(double(fft_index(iy, geo.ny)) * geo.invdy);
+        rho2[r] = wx * wx + wy * wy;
+      }
+      const bool last = q0 + NB > MK_NODES;  // this group holds the k-independent matrix
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const c32* c = in ? col[t] : no;
+        if (q0 < MK_NODES) load_col<S>(c ? c + 5 * geo.cs : no, row, x[t]);
+        if (last) load_col<S>(c ? c + 6 * geo.cs : no, row, x2[t]);
+      }
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        if (q0 + q < MK_NODES) {
+          const float kk = kap2[q0 + q];
+          float ps[S];
+#pragma unroll
+          for (int r = 0; r < S; ++r) ps[r] = 1.f / (rho2[r] + kk);
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < S; ++r) y[t][r] = x[t][r] * ps[r];
+          product(q, x, y);
+        } else if (q0 + q == MK_NODES) {
+          product(q, x2, x2);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int gram = KIND == 3 ? 3 + q0 + q : KIND;
+    if (gram >= NGRAM) break;
+    c32* out = part + ((long(p) * gridDim.x + chunk) * NGRAM + gram) * PM * PM;
+#pragma unroll
+    for (int a = 0; a < NT; ++a)
+#pragma unroll
+      for (int b = 0; b < NT; ++b) {
+        if (KIND != 1 && a > b) continue;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          red[wave][r][lane] = ar[q][a][b][r];
+          red[wave][4 + r][lane] = ai[q][a][b][r];
+        }
+        __syncthreads();
+        // wave w finishes accumulator register w: rows 4 g + w
+        const float sr = (red[0][wave][lane] + red[1][wave][lane]) + (red[2][wave][lane] + red[3][wave][lane]);
+        const float si = (red[0][4 + wave][lane] + red[1][4 + wave][lane]) +
+                         (red[2][4 + wave][lane] + red[3][4 + wave][lane]);
+        out[(a * 16 + 4 * g + wave) * PM + b * 16 + i16] = c32{sr, si};
+      }
+  }
+}
+
+// red[p][gram][e] = sum over the chunks, FP64, fixed order (16 elements x 16 chunk groups)
+__global__ __launch_bounds__(256) void k_mk_reduce(const c32* part, int nchunk, int pm, const MkState* st, c64* red) {
+  __shared__ double sx[16][17], sy[16][17];
+  const int p = blockIdx.z, gram = blockIdx.y;
+  const MkState& s = st[p];
+  if (s.done) return;
+  const int e = blockIdx.x * 16 + (threadIdx.x & 15), grp = threadIdx.x >> 4, el = threadIdx.x & 15;
+  const int a = e / pm, b0 = (blockIdx.x * 16) % pm, n = s.m + s.na + s.np;
+  // a block covers one row's 16-column tile: skip those not computed or not used
+  if (a >= n || b0 >= n || (gram != 1 && (a >> 4) > (b0 >> 4))) return;
+  const long esz = long(pm) * pm;
+  const c32* q = part + (long(p) * nchunk * NGRAM + gram) * esz + e;
+  double ax = 0, ay = 0;
+#pragma unroll 8
+  for (int c = grp; c < nchunk; c += 16) {
+    const c32 v = q[long(c) * NGRAM * esz];
+    ax += v.x;
+    ay += v.y;
+  }
+  sx[grp][el] = ax;
+  sy[grp][el] = ay;
+  __syncthreads();
+  if (grp == 0) {
+    double tx = 0, ty = 0;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      tx += sx[u][el];
+      ty += sy[u][el];
+    }
+    red[(long(p) * NGRAM + gram) * esz + e] = c64{tx, ty};
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// Dense step: one workgroup per band.
+// ---------------------------------------------------------------------------------------
+constexpr int DT = 512;
+
+__device__ __forceinline__ c64 operator_conj_mul(c64 a, c64 b) {  // conj(a) b
+  return c64{a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x};
+}
+
+// Parallel cyclic Jacobi (dense.hip's round-robin ordering and rotations) for Hermitian A
+// (n x n, leading dimension ld) using A's symmetry: of the 2 x 2 blocks only those on and above
+// the diagonal are computed and their mirrors stored.  Stops after a sweep whose rotations
+// all have |sin| <= stop.  Returns the buffer holding the final matrix; V the eigenvectors.
+__device__ __forceinline__ void mk_pair(int t, int r, int m, int& p, int& q) {
+  const int ia = (t == 0) ? 0 : 1 + (t - 1 + r) % (m - 1);
+  const int ib = 1 + (m - 2 - t + r) % (m - 1);
+  p = ia < ib ? ia : ib;
+  q = ia < ib ? ib : ia;
+}
+
+__device__ c64* mk_jacobi(c64* A0, c64* A1, c64* V, int ld, int n, double stop) {
+  __shared__ int big[3];
+  __shared__ int rp[MK_MAXN / 2], rq[MK_MAXN / 2];
+  __shared__ double rc[MK_MAXN / 2];
+  __shared__ c64 rs[MK_MAXN / 2];
+  __shared__ unsigned short tri[(MK_MAXN / 2) * (MK_MAXN / 2 + 1) / 2];
+  const int m = n + (n & 1), npair = m / 2, nblk = npair * (npair + 1) / 2;
+  for (int e = threadIdx.x; e < m * m; e += blockDim.x) {
+    const int i = e / m, j = e - i * m;
+    V[i * ld + j] = c64{i == j ? 1.0 : 0.0, 0.0};
+    if (i == n || j == n) A0[i * ld + j] = c64{0.0, 0.0};
+  }
+  for (int e = threadIdx.x; e < npair * npair; e += blockDim.x) {
+    const int a = e / npair, b = e - a * npair;
+    if (a <= b) tri[a * npair - a * (a - 1) / 2 + (b - a)] = (unsigned short)(a * 64 + b);
+  }
+  if (threadIdx.x < 3) big[threadIdx.x] = 0;
+  __syncthreads();
+  c64 *Ac = A0, *An = A1;
+  const int nitem = nblk + m * npair;
+  for (int sweep = 0; sweep < 30; ++sweep) {
+    const int sl = sweep % 3;
+    if (threadIdx.x == 0) big[(sweep + 1) % 3] = 0;
+    for (int r = 0; r < m - 1; ++r) {
+      if (threadIdx.x < npair) {
+        int p, q;
+        mk_pair(threadIdx.x, r, m, p, q);
+        const double app = Ac[p * ld + p].x, aqq = Ac[q * ld + q].x;
+        const c64 apq = Ac[p * ld + q];
+        const double a2 = apq.x * apq.x + apq.y * apq.y;
+        double c = 1.0;
+        c64 sv{0.0, 0.0};
+        if (a2 > 1e-300 && a2 > 1e-32 * fabs(app * aqq)) {
+          const double ia = rsqrt(a2), z = 0.5 * (aqq - app) * ia, az = fabs(z);
+          double sn;
+          if (az > 1e150) {
+            sn = 0.5 / az;
+          } else {
+            const double h = rsqrt(1.0 + z * z), x = 0.5 * (1.0 + az * h), rx = rsqrt(x);
+            c = x * rx;
+            sn = 0.5 * h * rx;
+          }
+          const double f = (z >= 0 ? sn : -sn) * ia;
+          sv = c64{f * apq.x, f * apq.y};
+          if (sn > stop) big[sl] = 1;
+        }
+        rp[threadIdx.x] = p;
+        rq[threadIdx.x] = q;
+        rc[threadIdx.x] = c;
+        rs[threadIdx.x] = sv;
+      }
+      __syncthreads();
+      for (int idx = threadIdx.x; idx < nitem; idx += blockDim.x) {
+        if (idx < nblk) {
+          const int t1 = tri[idx] >> 6, t2 = tri[idx] & 63;
+          const int p1 = rp[t1], q1 = rq[t1], p2 = rp[t2], q2 = rq[t2];
+          const double c1 = rc[t1], c2 = rc[t2];
+          const c64 s1 = rs[t1], s2 = rs[t2];
+          const c64 x00 = Ac[p1 * ld + p2], x01 = Ac[p1 * ld + q2], x10 = Ac[q1 * ld + p2], x11 = Ac[q1 * ld + q2];
+          const c64 y00 = x00 * c1 - s1 * x10, y01 = x01 * c1 - s1 * x11;
+          const c64 y10 = operator_conj_mul(s1, x00) + x10 * c1, y11 = operator_conj_mul(s1, x01) + x11 * c1;
+          const c64 z00 = y00 * c2 - operator_conj_mul(s2, y01), z01 = s2 * y00 + y01 * c2;
+          const c64 z10 = y10 * c2 - operator_conj_mul(s2, y11), z11 = s2 * y10 + y11 * c2;
+          An[p1 * ld + p2] = z00;
+          An[p1 * ld + q2] = z01;
+          An[q1 * ld + p2] = z10;
+          An[q1 * ld + q2] = z11;
+          if (t1 != t2) {
+            An[p2 * ld + p1] = conj(z00);
+            An[q2 * ld + p1] = conj(z01);
+            An[p2 * ld + q1] = conj(z10);
+            An[q2 * ld + q1] = conj(z11);
+          }
+        } else {
+          const int e = idx - nblk, j = e / npair, t = e - j * npair;
+          const int p = rp[t], q = rq[t];
+          const double c = rc[t];
+          const c64 sv = rs[t];
+          const c64 vp = V[j * ld + p], vq = V[j * ld + q];
+          V[j * ld + p] = vp * c - operator_conj_mul(sv, vq);
+          V[j * ld + q] = sv * vp + vq * c;
+        }
+      }
+      __syncthreads();
+      c64* tmp = Ac;
+      Ac = An;
+      An = tmp;
+    }
+    if (big[sl] == 0) break;
+  }
+  return Ac;
+}
+
+// Ritz pair j of the pencil (A(k), B(k)) of the search space at column j's k.  The pencil is
+// scaled to unit B diagonal and reduced by the congruence that turns B into the identity
+// (one elimination step per column, applied to A as well); columns whose pivot falls below
+// 1e-5 (dependent to FP32 accuracy) are taken out of the space.  Bands whose k agree to 3e-5
+// share one k, so that near-degenerate bands take different vectors of one decomposition.
+// C: per problem and band, coefficients [column][vector] of the lowest msz Ritz vectors.
+__global__ __launch_bounds__(DT) void k_mk_dense(MkGeo geo, MkState* st, const c64* red, int pm, int ld, double stop,
+                                                 const int* msz, c32* Cx, c64* Cblk) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int j = blockIdx.x, p = blockIdx.y;
+  MkState& s = st[p];
+  if (s.done || j >= s.m) return;
+  const int n = s.m + s.na + s.np;
+  c64* A = reinterpret_cast<c64*>(smem_raw);
+  c64* B = A + (n + 1) * ld;  // Jacobi's second buffer afterwards
+  c64* V = B + (n + 1) * ld;
+  __shared__ double node[MK_NODES], lw[MK_NODES], dlw[MK_NODES], dsc[MK_MAXN], diagv[MK_MAXN];
+  __shared__ double kk_s, red_s[DT / 64][2];
+  __shared__ int drop[MK_MAXN], rank[MK_MAXN];
+  __shared__ c64 y[MK_MAXN];
+  if (threadIdx.x == 0) {
+    int a = j, b = j;
+    while (a > 0 && fabs(s.k[a - 1] - s.k[a]) < 3e-5 * fabs(s.k[a])) --a;
+    while (b + 1 < s.m && fabs(s.k[b + 1] - s.k[b]) < 3e-5 * fabs(s.k[b])) ++b;
+    double kk = 0;
+    for (int i = a; i <= b; ++i) kk += s.k[i];
+    kk /= double(b - a + 1);
+    kk_s = kk;
+    mk_nodes(s, node);
+    for (int t = 0; t < MK_NODES; ++t) {  // Lagrange weights at kk and their k-derivatives
+      double w = 1, dw = 0;
+      for (int u = 0; u < MK_NODES; ++u) {
+        if (u == t) continue;
+        const double q = 1.0 / (node[t] - node[u]);
+        dw = dw * (kk - node[u]) * q + w * q;
+        w *= (kk - node[u]) * q;
+      }
+      lw[t] = w;
+      dlw[t] = dw;
+    }
+  }
+  __syncthreads();
+  const double kk = kk_s;
+  const long esz = long(pm) * pm;
+  const c64* G = red + long(p) * NGRAM * esz;
+  for (int e = threadIdx.x; e < n * n; e += DT) {
+    const int a = e / n, b = e - a * n;
+    if (a > b) continue;
+    const long o = long(a) * pm + b;
+    const c64 g00 = G[o], g01 = G[esz + o], g10 = G[esz + long(b) * pm + a], g11 = G[2 * esz + o];
+    c64 va{g00.x + kk * (g01.x + g10.x) + kk * kk * g11.x, g00.y + kk * (g01.y - g10.y) + kk * kk * g11.y};
+    c64 vb = G[(NGRAM - 1) * esz + o];
+#pragma unroll
+    for (int t = 0; t < MK_NODES; ++t) {
+      const c64 w = G[(3 + t) * esz + o];
+      vb.x += lw[t] * w.x;
+      vb.y += lw[t] * w.y;
+    }
+    if (a == b) va.y = vb.y = 0;
+    A[a * ld + b] = va;
+    A[b * ld + a] = conj(va);
+    B[a * ld + b] = vb;
+    B[b * ld + a] = conj(vb);
+  }
+  __syncthreads();
+  for (int a = threadIdx.x; a < n; a += DT) {
+    const double d = B[a * ld + a].x;
+    dsc[a] = d > 0 ? 1.0 / sqrt(d) : 0.0;
+    drop[a] = 0;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < n * n; e += DT) {
+    const int a = e / n, b = e - a * n;
+    const double f = dsc[a] * dsc[b];
+    A[a * ld + b] = A[a * ld + b] * (f / double(geo.N));  // the transforms are unnormalised
+    B[a * ld + b] = B[a * ld + b] * f;
+  }
+  __syncthreads();
+  // congruence: after step k, rows and columns <= k of B are the identity's.  Row k of A takes
+  // its own column operation only once the other rows have used it, at the start of step k + 1.
+  for (int k = 0; k < n; ++k) {
+    const double d = B[k * ld + k].x;
+    const bool bad = !(d > 1e-5);
+    const double f = bad ? 0.0 : rsqrt(d);
+    if (k > 0 && !drop[k - 1]) {
+      const int r = k - 1;
+      const double arr = A[r * ld + r].x;
+      for (int b = k + threadIdx.x; b < n; b += DT) {
+        const c64 v = A[r * ld + b] - B[r * ld + b] * arr;
+        A[r * ld + b] = v;
+        A[b * ld + r] = conj(v);
+      }
+    }
+    __syncthreads();
+    // scale row and column k of A and row k of B (column k of B is its mirror, not kept)
+    for (int b = threadIdx.x; b < n; b += DT) {
+      if (b > k) B[k * ld + b] = B[k * ld + b] * f;
+      if (b != k) {
+        const c64 v = A[k * ld + b] * f;
+        A[k * ld + b] = v;
+        A[b * ld + k] = conj(v);
+      } else {
+        A[k * ld + k] = c64{A[k * ld + k].x * f * f, 0.0};
+        B[k * ld + k] = c64{bad ? 0.0 : 1.0 / f, 0.0};  // U[k][k]
+        if (bad) drop[k] = 1;
+      }
+    }
+    __syncthreads();
+    if (!bad) {
+      const double akk = A[k * ld + k].x;
+      const int w = n - 1 - k;
+      for (int e = threadIdx.x; e < n * w; e += DT) {
+        const int a = e / w, b = k + 1 + (e - a * w);
+        if (a == k) continue;
+        const c64 ub = B[k * ld + b];  // U[k][b]
+        if (a < k) {
+          // finished row: A[a][b] -= A[a][k] U[k][b]; its mirror is written too
+          const c64 v = A[a * ld + b] - A[a * ld + k] * ub;
+          A[a * ld + b] = v;
+          A[b * ld + a] = conj(v);
+        } else if (a <= b) {
+          const c64 ua = B[k * ld + a];
+          const c64 v = A[a * ld + b] - operator_conj_mul(ua, A[k * ld + b]) - A[a * ld + k] * ub +
+                        operator_conj_mul(ua, ub) * akk;
+          A[a * ld + b] = a == b ? c64{v.x, 0.0} : v;
+          A[b * ld + a] = conj(v);
+          B[a * ld + b] = B[a * ld + b] - operator_conj_mul(ua, ub);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  // dropped columns: decoupled, at the end of the spectrum
+  {
+    double mx = 0;
+    for (int a = 0; a < n; ++a) mx = fmax(mx, fabs(A[a * ld + a].x));
+    __syncthreads();
+    for (int e = threadIdx.x; e < n * n; e += DT) {
+      const int a = e / n, b = e - a * n;
+      if (drop[a] || drop[b]) A[a * ld + b] = a == b ? c64{16.0 * mx + 1.0, 0.0} : c64{0.0, 0.0};
+    }
+  }
+  __syncthreads();
+  // U (upper, in B) is needed after the Jacobi, which uses B's storage: keep it in global memory
+  c64* Ug = Cblk + ((long(p) * geo.mmax + j) * 2 + 1) * MK_MAXN * MK_MAXN;
+  for (int e = threadIdx.x; e < n * n; e += DT) {
+    const int a = e / n, b = e - a * n;
+    if (a <= b) Ug[a * MK_MAXN + b] = B[a * ld + b];
+  }
+  __syncthreads();
+  const c64* Ad = mk_jacobi(A, B, V, ld, n, stop);
+  for (int a = threadIdx.x; a < n; a += DT) diagv[a] = Ad[a * ld + a].x;
+  __syncthreads();
+  for (int a = threadIdx.x; a < n; a += DT) {
+    int r = 0;
+    for (int l = 0; l < n; ++l)
+      if (diagv[l] < diagv[a] || (diagv[l] == diagv[a] && l < a)) ++r;
+    rank[r] = a;
+  }
+  __syncthreads();
+  // back substitution c = D U^-1 v for the lowest vectors: band j's own, and the block's
+  const int nv = j < s.nev ? max(msz[p * MK_MAXM + j], j + 1) : j + 1;
+  // every matrix buffer but V is free now: U back into LDS
+  c64* U = A;
+  for (int e = threadIdx.x; e < n * n; e += DT) {
+    const int a = e / n, b = e - a * n;
+    if (a <= b) U[a * ld + b] = Ug[a * MK_MAXN + b];
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < nv; q += DT) {  // one thread per vector, in place in V's column
+    const int c = rank[q];
+    for (int a = n - 1; a >= 0; --a) {
+      if (drop[a]) {
+        V[a * ld + c] = c64{0.0, 0.0};
+        continue;
+      }
+      c64 v = V[a * ld + c];
+      for (int b = a + 1; b < n; ++b) v = v - U[a * ld + b] * V[b * ld + c];
+      V[a * ld + c] = v * (1.0 / U[a * ld + a].x);
+    }
+  }
+  __syncthreads();
+  c64* Cb = Cblk + ((long(p) * geo.mmax + j) * 2) * MK_MAXN * MK_MAXN;
+  for (int e = threadIdx.x; e < n * nv; e += DT) {
+    const int a = e / nv, q = e - a * nv;
+    const c64 v = V[a * ld + rank[q]] * dsc[a];
+    Cb[a * MK_MAXM + q] = v;
+    if (q == j) {
+      y[a] = v;
+      Cx[(long(p) * MK_MAXN + a) * MK_MAXM + j] = c32{float(v.x), float(v.y)};
+    }
+  }
+  __syncthreads();
+  // slope = y^H (dA/dk - lam dB/dk) y (y^H B y = 1)
+  const double lam = diagv[rank[j]];
+  double acc = 0;
+  for (int e = threadIdx.x; e < n * n; e += DT) {
+    const int a = e / n, b = e - a * n;
+    if (a > b) continue;
+    const long o = long(a) * pm + b;
+    const c64 g01 = G[esz + o], g10 = G[esz + long(b) * pm + a], g11 = G[2 * esz + o];
+    c64 d{(g01.x + g10.x + 2 * kk * g11.x) / geo.N, (g01.y - g10.y + 2 * kk * g11.y) / geo.N};
+#pragma unroll
+    for (int t = 0; t < MK_NODES; ++t) {
+      const c64 w = G[(3 + t) * esz + o];
+      d.x -= lam * dlw[t] * w.x;
+      d.y -= lam * dlw[t] * w.y;
+    }
+    if (a == b) d.y = 0;
+    const c64 z = d * y[b];
+    acc += (a == b ? 1.0 : 2.0) * (y[a].x * z.x + y[a].y * z.y);
+  }
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if ((threadIdx.x & 63) == 0) red_s[threadIdx.x >> 6][0] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double slope = 0;
+    for (int w = 0; w < DT / 64; ++w) slope += red_s[w][0];
+    // early Ritz values are far above the band's: the first steps move k by at most a tenth
+    const double lim = (s.iter < 4 ? 0.1 : 0.25) * fabs(kk);
+    double dk = -(lam - s.omega2) / slope;
+    if (!isfinite(dk)) dk = 0;
+    dk = fmin(fmax(dk, -lim), lim);
+    s.keval[j] = kk;
+    s.lam[j] = lam;
+    s.slope[j] = slope;
+    s.knew[j] = kk + dk;
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// Block update: X' = S Cx, P' = the W and P part of it, over the flat 7-plane columns.
+// ---------------------------------------------------------------------------------------
+template <int QM>
+__global__ __launch_bounds__(256) void k_mk_combine(MkGeo geo, c32* cols, const MkState* st, const c32* Cx, int buf) {
+  __shared__ const c32* in[MK_MAXN];
+  __shared__ c32* outx[QM];
+  __shared__ c32* outp[QM];
+  __shared__ c32 Cs[MK_MAXN][QM];
+  const int p = blockIdx.y;
+  const MkState& s = st[p];
+  if (s.done) return;
+  const int m = s.m, n = m + s.na + s.np;
+  c32* base = cols + p * geo.slots;
+  // W and P first: their sum is P', then X's part completes X'
+  for (int a = threadIdx.x; a < n; a += 256) {
+    const int q = a < n - m ? a + m : a - (n - m);
+    in[a] = base + col_off(geo, space_slot(geo, s, buf, q));
+  }
+  for (int e = threadIdx.x; e < n * QM; e += 256) {
+    const int a = e / QM, j = e - a * QM, q = a < n - m ? a + m : a - (n - m);
+    Cs[a][j] = j < m ? Cx[(long(p) * MK_MAXN + q) * MK_MAXM + j] : c32{0.f, 0.f};
+  }
+  if (threadIdx.x < QM) {
+    const int j = threadIdx.x;
+    outx[j] = j < m ? base + col_off(geo, slot_x(geo, buf ^ 1, j)) : nullptr;
+    c32* q = nullptr;
+    for (int w = 0; w < s.na; ++w)
+      if (s.wcol[w] == j) q = base + col_off(geo, slot_p(geo, buf ^ 1, w));
+    outp[j] = q;
+  }
+  __syncthreads();
+  const int nwp = n - m;
+  const long L = PLANES * geo.cs / 2;  // pairs of values
+  for (long e = long(blockIdx.x) * 256 + threadIdx.x; e < L; e += long(gridDim.x) * 256) {
+    c32 a0[QM], a1[QM];
+#pragma unroll
+    for (int j = 0; j < QM; ++j) a0[j] = a1[j] = c32{0.f, 0.f};
+    auto add = [&](int from, int to) {
+      int a = from;
+      for (; a + 4 <= to; a += 4) {  // four columns' loads in flight together
+        fx4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = reinterpret_cast<const fx4*>(in[a + u])[e];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int j = 0; j < QM; ++j) {
+            const c32 c = Cs[a + u][j];
+            a0[j] = a0[j] + c32{v[u].x, v[u].y} * c;
+            a1[j] = a1[j] + c32{v[u].z, v[u].w} * c;
+          }
+      }
+      for (; a < to; ++a) {
+        const fx4 v = reinterpret_cast<const fx4*>(in[a])[e];
+#pragma unroll
+        for (int j = 0; j < QM; ++j) {
+          const c32 c = Cs[a][j];
+          a0[j] = a0[j] + c32{v.x, v.y} * c;
+          a1[j] = a1[j] + c32{v.z, v.w} * c;
+        }
+      }
+    };
+    add(0, nwp);
+#pragma unroll
+    for (int j = 0; j < QM; ++j)
+      if (outp[j]) reinterpret_cast<fx4*>(outp[j])[e] = fx4{a0[j].x, a0[j].y, a1[j].x, a1[j].y};
+    add(nwp, n);
+#pragma unroll
+    for (int j = 0; j < QM; ++j)
+      if (outx[j]) reinterpret_cast<fx4*>(outx[j])[e] = fx4{a0[j].x, a0[j].y, a1[j].x, a1[j].y};
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// Transforms.  Column kernels hold TX columns (fixed ix, all iy) of each plane in LDS, row
+// kernels RB rows; the intermediate field Dm is [problem column][plane][ix][iy].
+// ---------------------------------------------------------------------------------------
+// eps^-1 (F0 + k F1) of X (buffer buf), inverse FFT along y
+template <int VPT>
+__global__ __launch_bounds__(FT) void k_mk_colE(MkGeo geo, const c32* cols, const MkState* st, int buf, c32* Dm,
+                                                int TX) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int p = blockIdx.y / geo.mmax, c = blockIdx.y - p * geo.mmax;
+  const MkState& s = st[p];
+  if (s.done || c >= s.m) return;
+  const int ny = geo.ny;
+  c32* tw = reinterpret_cast<c32*>(smem_raw);
+  c32* sm = tw + ny;
+  for (int t = threadIdx.x; t < ny; t += FT) tw[t] = geo.twy[t];
+  const int ix0 = blockIdx.x * TX, tx = min(TX, geo.nx - ix0), nv = tx * ny;
+  const float k = float(s.keval[c]);
+  const c32* x = cols + p * geo.slots + col_off(geo, slot_x(geo, buf, c)) + long(ix0) * ny;
+  const float* ep = geo.eps6c + p * geo.eps_stride + 6L * ix0 * ny;
+  for (int e = threadIdx.x; e < TX * ny; e += FT) {
+    c32 y0{0.f, 0.f}, y1 = y0, y2 = y0;
+    if (e < nv) {
+      const c32 d0 = x[e] + x[3 * geo.cs + e] * k, d1 = x[geo.cs + e] + x[4 * geo.cs + e] * k, d2 = x[2 * geo.cs + e];
+      const float2* q = reinterpret_cast<const float2*>(ep + 6L * e);
+      const float2 ea = q[0], eb = q[1], ec = q[2];  // xx yy, zz xy, xz yz
+      y0 = d0 * ea.x + d1 * eb.y + d2 * ec.x;
+      y1 = d0 * eb.y + d1 * ea.y + d2 * ec.y;
+      y2 = d0 * ec.x + d1 * ec.y + d2 * eb.x;
+    }
+    sm[e] = y0;
+    sm[TX * ny + e] = y1;
+    sm[2 * TX * ny + e] = y2;
+  }
+  __syncthreads();
+  fft_lds<float, +1, VPT>(sm, 3 * TX, ny, 1, geo.fy, tw);
+  c32* d = Dm + long(blockIdx.y) * 3 * geo.cs + long(ix0) * ny;
+  for (int e = threadIdx.x; e < nv; e += FT) {
+    d[e] = sm[e];
+    d[geo.cs + e] = sm[TX * ny + e];
+    d[2 * geo.cs + e] = sm[2 * TX * ny + e];
+  }
+}
+
+// rows of Dm into LDS, [plane][row][ix] with row stride nx + 1
+__device__ __forceinline__ void rows_in(const MkGeo& geo, const c32* d, int iy0, int rb, int RB, int nplane, c32* sm) {
+  const int nx = geo.nx, ny = geo.ny, sb = nx + 1;
+  for (int e = threadIdx.x; e < nplane * RB * nx; e += FT) {
+    const int q = e / RB, r = e - q * RB, a = q / nx, ix = q - a * nx;
+    sm[(a * RB + r) * sb + ix] = r < rb ? d[a * geo.cs + long(ix) * ny + iy0 + r] : c32{0.f, 0.f};
+  }
+}
+__device__ __forceinline__ void rows_out(const MkGeo& geo, c32* d, int iy0, int rb, int RB, int nplane, const c32* sm) {
+  const int nx = geo.nx, ny = geo.ny, sb = nx + 1;
+  for (int e = threadIdx.x; e < nplane * RB * nx; e += FT) {
+    const int q = e / RB, r = e - q * RB, a = q / nx, ix = q - a * nx;
+    if (r < rb) d[a * geo.cs + long(ix) * ny + iy0 + r] = sm[(a * RB + r) * sb + ix];
+  }
+}
+
+// inverse FFT along x, M x, residual and its norm, the preconditioner's map, FFT along x
+template <int VPT>
+__global__ __launch_bounds__(FT) void k_mk_rowR(MkGeo geo, const c32* cols, const MkState* st, int buf, c32* Dm,
+                                                int RB, double* normp) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int p = blockIdx.y / geo.mmax, c = blockIdx.y - p * geo.mmax;
+  const MkState& s = st[p];
+  if (s.done || c >= s.m) return;
+  const int nx = geo.nx, sb = nx + 1;
+  c32* tw = reinterpret_cast<c32*>(smem_raw);
+  c32* sm = tw + nx;
+  for (int t = threadIdx.x; t < nx; t += FT) tw[t] = geo.twx[t];
+  const int iy0 = blockIdx.x * RB, rb = min(RB, geo.ny - iy0);
+  c32* d = Dm + long(blockIdx.y) * 3 * geo.cs;
+  rows_in(geo, d, iy0, rb, RB, 3, sm);
+  __syncthreads();
+  fft_lds<float, +1, VPT>(sm, 3 * RB, sb, 1, geo.fx, tw);
+  const c32* g1 = cols + p * geo.slots + col_off(geo, slot_x(geo, buf, c)) + 5 * geo.cs + long(iy0) * nx;
+  const float k = float(s.keval[c]), lam = float(s.lam[c]), scale = 1.f / float(geo.N);
+  double acc = 0;
+  for (int e = threadIdx.x; e < rb * nx; e += FT) {
+    const int r = e / nx, ix = e - r * nx;
+    const Wave w = wave_at(ix, iy0 + r, geo);
+    const float mag2 = w.rho2 + k * k, mag = sqrtf(mag2), im = 1.f / mag;
+    c32 *s0 = sm + r * sb + ix, *s1 = s0 + RB * sb, *s2 = s1 + RB * sb;
+    const c32 e0 = *s0, e1 = *s1, e2 = *s2, x1 = g1[e], x2 = g1[geo.cs + e];
+    const c32 en = e0 * w.n0 + e1 * w.n1, em = (e0 * w.n1 - e1 * w.n0) * k - e2 * w.rho;
+    const c32 r1 = en * (-mag * scale) - x1 * (lam * im), r2 = em * scale - x2 * lam;
+    acc += double(r1.x) * r1.x + double(r1.y) * r1.y + double(r2.x) * r2.x + double(r2.y) * r2.y;
+    const c32 t = r2 * (k * im);
+    *s0 = (r1 * w.n0 - t * w.n1) * im;
+    *s1 = (r1 * w.n1 + t * w.n0) * im;
+    *s2 = r2 * (w.rho * im * im);
+  }
+  __syncthreads();
+  fft_lds<float, +1, VPT>(sm, 3 * RB, sb, 1, geo.fx, tw);
+  rows_out(geo, d, iy0, rb, RB, 3, sm);
+  __shared__ double red[FT / 64];
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0;
+    for (int q = 0; q < FT / 64; ++q) t += red[q];
+    normp[long(blockIdx.y) * gridDim.x + blockIdx.x] = t;
+  }
+}
+
+// Residual norms, convergence, the next search space.  One block per problem.
+__global__ __launch_bounds__(256) void k_mk_control(MkGeo geo, MkState* st, const double* normp, int nrb, int cur) {
+  const int p = blockIdx.x;
+  MkState& s = st[p];
+  if (s.done) return;
+  __shared__ double nr[MK_MAXM];
+  const int lane = threadIdx.x & 63;
+  for (int c = threadIdx.x >> 6; c < s.m; c += 4) {
+    double a = 0;
+    for (int b = lane; b < nrb; b += 64) a += normp[(long(p) * geo.mmax + c) * nrb + b];
+    for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
+    if (lane == 0) nr[c] = sqrt(a);
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  bool all = true, bad = false, moved = false;
+  int act[MK_MAXM];
+  for (int c = 0; c < s.m; ++c) {
+    const double rn = nr[c], dk = s.knew[c] - s.k[c];
+    bad = bad || !isfinite(rn) || !isfinite(s.lam[c]);
+    act[c] = rn > s.tol;
+    const bool still = fabs(dk * s.slope[c]) <= s.ftol, conv = !act[c] && still;
+    if (c < s.nev) {
+      moved = moved || !still;
+      if (conv && !s.its[c]) s.its[c] = s.iter + 1;
+      if (!conv) s.its[c] = 0;
+      all = all && conv;
+    }
+    s.rnorm[c] = rn;
+    s.k[c] = s.knew[c];
+  }
+  s.iter += 1;
+  s.moves += moved;
+  s.par = cur;
+  if (bad) {
+    s.done = 2;
+    return;
+  }
+  if (all) {  // the current space and its coefficients are the result
+    s.done = 1;
+    return;
+  }
+  int np = 0;
+  for (int w = 0; w < s.na; ++w)
+    if (act[s.wcol[w]]) s.pslot[np++] = w;
+  s.np = np;
+  int na = 0;
+  for (int c = 0; c < s.m; ++c)
+    if (act[c]) s.wcol[na++] = c;
+  s.na = na;
+}
+
+// FFT along y, eps_ave, FFT back, for the columns that go on
+template <int VPT>
+__global__ __launch_bounds__(FT) void k_mk_colP(MkGeo geo, const MkState* st, c32* Dm, int TX) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int p = blockIdx.y / geo.mmax, w = blockIdx.y - p * geo.mmax;
+  const MkState& s = st[p];
+  if (s.done || w >= s.na) return;
+  const int ny = geo.ny;
+  c32* tw = reinterpret_cast<c32*>(smem_raw);
+  c32* sm = tw + ny;
+  for (int t = threadIdx.x; t < ny; t += FT) tw[t] = geo.twy[t];
+  const int ix0 = blockIdx.x * TX, tx = min(TX, geo.nx - ix0), nv = tx * ny;
+  c32* d = Dm + (long(p) * geo.mmax + s.wcol[w]) * 3 * geo.cs + long(ix0) * ny;
+  for (int e = threadIdx.x; e < TX * ny; e += FT)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) sm[a * TX * ny + e] = e < nv ? d[a * geo.cs + e] : c32{0.f, 0.f};
+  __syncthreads();
+  fft_lds<float, +1, VPT>(sm, 3 * TX, ny, 1, geo.fy, tw);
+  const float* ep = geo.eps6c + p * geo.eps_stride + 6L * ix0 * ny;
+  for (int e = threadIdx.x; e < nv; e += FT) {
+    const float ea = 3.f / (ep[6L * e] + ep[6L * e + 1] + ep[6L * e + 2]);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) sm[a * TX * ny + e] = sm[a * TX * ny + e] * ea;
+  }
+  __syncthreads();
+  fft_lds<float, -1, VPT>(sm, 3 * TX, ny, 1, geo.fy, tw);
+  for (int e = threadIdx.x; e < nv; e += FT)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) d[a * geo.cs + e] = sm[a * TX * ny + e];
+}
+
+// START false: FFT along x, w = P r, its g into W.  START true: g of X (buffer 0) as it is.
+// Then D0 and D1 of g, FFT along x (three planes, then two).
+template <int VPT, bool START>
+__global__ __launch_bounds__(FT) void k_mk_rowW(MkGeo geo, c32* cols, const MkState* st, const c32* Dm, int RB) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int p = blockIdx.y / geo.mmax, w = blockIdx.y - p * geo.mmax;
+  const MkState& s = st[p];
+  if (s.done || w >= (START ? s.m : s.na)) return;
+  const int nx = geo.nx, sb = nx + 1, c = START ? w : s.wcol[w];
+  c32* tw = reinterpret_cast<c32*>(smem_raw);
+  c32* sm = tw + nx;
+  for (int t = threadIdx.x; t < nx; t += FT) tw[t] = geo.twx[t];
+  const int iy0 = blockIdx.x * RB, rb = min(RB, geo.ny - iy0);
+  c32* out = cols + p * geo.slots + col_off(geo, START ? slot_x(geo, 0, w) : slot_w(geo, w));
+  c32* g1 = out + 5 * geo.cs + long(iy0) * nx;
+  if (!START) {
+    rows_in(geo, Dm + (long(p) * geo.mmax + c) * 3 * geo.cs, iy0, rb, RB, 3, sm);
+    __syncthreads();
+    fft_lds<float, -1, VPT>(sm, 3 * RB, sb, 1, geo.fx, tw);
+  } else {
+    __syncthreads();
+  }
+  const float k = START ? 0.f : float(s.keval[c]), scale = 1.f / float(geo.N);
+  for (int e = threadIdx.x; e < RB * nx; e += FT) {
+    const int r = e / nx, ix = e - r * nx;
+    c32 *s0 = sm + r * sb + ix, *s1 = s0 + RB * sb, *s2 = s1 + RB * sb;
+    c32 a1{0.f, 0.f}, a2{0.f, 0.f};
+    Wave v{0.f, 0.f, 0.f, 0.f};
+    if (r < rb) {
+      v = wave_at(ix, iy0 + r, geo);
+      if (START) {
+        a1 = g1[e];
+        a2 = g1[geo.cs + e];
+      } else {
+        const c32 e0 = *s0, e1 = *s1, e2 = *s2;
+        a1 = (e0 * v.n0 + e1 * v.n1) * scale;
+        a2 = ((e0 * v.n1 - e1 * v.n0) * k - e2 * v.rho) * (-scale / (v.rho2 + k * k));
+        g1[e] = a1;
+        g1[geo.cs + e] = a2;
+      }
+    }
+    *s0 = a1 * -v.n0;
+    *s1 = a1 * -v.n1;
+    *s2 = a2 * -v.rho;
+  }
+  __syncthreads();
+  fft_lds<float, -1, VPT>(sm, 3 * RB, sb, 1, geo.fx, tw);
+  rows_out(geo, out, iy0, rb, RB, 3, sm);
+  __syncthreads();
+  for (int e = threadIdx.x; e < RB * nx; e += FT) {  // this thread's own g2 of the loop above
+    const int r = e / nx, ix = e - r * nx;
+    c32 *s0 = sm + r * sb + ix, *s1 = s0 + RB * sb;
+    c32 a2{0.f, 0.f};
+    Wave v{0.f, 0.f, 0.f, 0.f};
+    if (r < rb) {
+      v = wave_at(ix, iy0 + r, geo);
+      a2 = g1[geo.cs + e];
+    }
+    *s0 = a2 * v.n1;
+    *s1 = a2 * -v.n0;
+  }
+  __syncthreads();
+  fft_lds<float, -1, VPT>(sm, 2 * RB, sb, 1, geo.fx, tw);
+  rows_out(geo, out + 3 * geo.cs, iy0, rb, RB, 2, sm);
+}
+
+// FFT along y of the five planes of W (START: of X, buffer 0); blockIdx.z: planes 0-2 or 3-4
+template <int VPT, bool START>
+__global__ __launch_bounds__(FT) void k_mk_colF(MkGeo geo, c32* cols, const MkState* st, int TX) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int p = blockIdx.y / geo.mmax, w = blockIdx.y - p * geo.mmax;
+  const MkState& s = st[p];
+  if (s.done || w >= (START ? s.m : s.na)) return;
+  const int ny = geo.ny, a0 = blockIdx.z ? 3 : 0, na = blockIdx.z ? 2 : 3;
+  c32* tw = reinterpret_cast<c32*>(smem_raw);
+  c32* sm = tw + ny;
+  for (int t = threadIdx.x; t < ny; t += FT) tw[t] = geo.twy[t];
+  const int ix0 = blockIdx.x * TX, tx = min(TX, geo.nx - ix0), nv = tx * ny;
+  c32* d = cols + p * geo.slots + col_off(geo, START ? slot_x(geo, 0, w) : slot_w(geo, w)) + a0 * geo.cs +
+           long(ix0) * ny;
+  for (int e = threadIdx.x; e < TX * ny; e += FT)
+    for (int a = 0; a < na; ++a) sm[a * TX * ny + e] = e < nv ? d[a * geo.cs + e] : c32{0.f, 0.f};
+  __syncthreads();
+  fft_lds<float, -1, VPT>(sm, na * TX, ny, 1, geo.fy, tw);
+  for (int e = threadIdx.x; e < nv; e += FT)
+    for (int a = 0; a < na; ++a) d[a * geo.cs + e] = sm[a * TX * ny + e];
+}
+
+// Each band's block for the FP64 refinement: its lowest Ritz vectors at its k as transverse
+// coefficients (h1 = g1 / |w|, h2 = g2), sums in FP64.  The space's G planes are read once per
+// instance; blockIdx.z: groups of HQ vectors.
+constexpr int HQ = 4;
+__global__ __launch_bounds__(256) void k_mk_handover(MkGeo geo, const c32* cols, const MkState* st, const int2* inst,
+                                                     const int* msz, const c64* Cblk, c64* X64, long ld, long istride) {
+  __shared__ const c32* in[MK_MAXN];
+  __shared__ c64 Cs[MK_MAXN][HQ];
+  const int i = blockIdx.y, p = inst[i].x, j = inst[i].y, q0 = blockIdx.z * HQ;
+  const MkState& s = st[p];
+  const int nq = min(HQ, msz[p * MK_MAXM + j] - q0);
+  if (nq <= 0) return;
+  const int n = s.m + s.na + s.np;
+  const c64* Cb = Cblk + (long(p) * geo.mmax + j) * 2 * MK_MAXN * MK_MAXN;
+  for (int a = threadIdx.x; a < n; a += 256)
+    in[a] = cols + p * geo.slots + col_off(geo, space_slot(geo, s, s.par, a)) + 5 * geo.cs;
+  for (int e = threadIdx.x; e < n * HQ; e += 256) {
+    const int a = e / HQ, q = e - a * HQ;
+    Cs[a][q] = q < nq ? Cb[a * MK_MAXM + q0 + q] : c64{0.0, 0.0};
+  }
+  __syncthreads();
+  const double k = s.k[j];
+  for (long e = long(blockIdx.x) * 256 + threadIdx.x; e < geo.N; e += long(gridDim.x) * 256) {
+    const int iy = int(e / geo.nx), ix = int(e - long(iy) * geo.nx);
+    const double wx = double(fft_index(ix, geo.nx)) * geo.invdx, wy = double(fft_index(iy, geo.ny)) * geo.invdy;
+    const double im = 1.0 / sqrt(wx * wx + wy * wy + k * k);
+    c64 a1[HQ], a2[HQ];
+#pragma unroll
+    for (int q = 0; q < HQ; ++q) a1[q] = a2[q] = c64{0.0, 0.0};
+    for (int a = 0; a < n; ++a) {
+      const c32 f1 = in[a][e], f2 = in[a][geo.cs + e];
+      const c64 v1{f1.x, f1.y}, v2{f2.x, f2.y};
+#pragma unroll
+      for (int q = 0; q < HQ; ++q) {
+        a1[q] = a1[q] + v1 * Cs[a][q];
+        a2[q] = a2[q] + v2 * Cs[a][q];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < HQ; ++q)
+      if (q < nq) {
+        c64* o = X64 + i * istride + long(q0 + q) * ld + 2 * e;
+        o[0] = a1[q] * im;
+        o[1] = a2[q];
+      }
+  }
+}
+
+// every radix pass of nb sequences fits FT threads of vpt values
+bool fits(int nb, const FFTFactors& f, int vpt) {
+  for (int p = 0; p < f.n; ++p) {
+    const int R = f.r[p];
+    if ((long(nb) * (f.L / R) + FT - 1) / FT > (vpt + R - 1) / R) return false;
+  }
+  return true;
+}
+
+constexpr size_t MK_LDS = 64 * 1024;
+
+// sequences of length L per block for three planes: at most 16, within MK_LDS and the bound of
+// 16 values per thread; fewer while the launch would leave CUs idle
+int pick_rows(int L, int other, long vecs, const FFTFactors& f) {
+  int r = 16;
+  while (r > 1 && (sizeof(c32) * (L + 3 * size_t(r) * (L + 1)) > MK_LDS || !fits(3 * r, f, 16))) r /= 2;
+  if (sizeof(c32) * (L + 3 * size_t(r) * (L + 1)) > 160 * 1024 || !fits(3 * r, f, 16)) return 0;
+  while (r > 4 && long((other + r - 1) / r) * vecs < 512) r /= 2;
+  return r;
+}
+
+}  // namespace
+
+bool multik_fits(const Solver& S) {
+  return S.nz == 1 && pick_rows(S.nx, S.ny, 1 << 20, S.p32.plan.fx) > 0 &&
+         pick_rows(S.ny, S.nx, 1 << 20, S.p32.plan.fy) > 0;
+}
+
+bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* eps6c, long eps_stride, int maxit,
+                  const std::vector<int>& msize, c64* X64, long ld, long istride, std::vector<double>& kout,
+                  std::vector<int>& iters, std::vector<int>& moves, SolveStats& stats) {
+  const int P = int(probs.size());
+  hipStream_t sm = S.stream;
+  MkGeo g{};
+  g.nx = S.nx;
+  g.ny = S.ny;
+  g.N = S.N;
+  g.cs = (S.N + 63) / 64 * 64;
+  g.invdx = 1.0 / S.Dx;
+  g.invdy = 1.0 / S.Dy;
+  g.fx = S.p32.plan.fx;
+  g.fy = S.p32.plan.fy;
+  g.twx = S.p32.plan.twx;
+  g.twy = S.p32.plan.twy;
+  g.eps6c = eps6c;
+  g.eps_stride = eps_stride;
+  g.mmax = 1;
+  int ninst = 0;
+  const int most = int(std::min<long>(MK_MAXM, S.K / 3));
+  std::vector<MkState> hs(P);
+  for (int p = 0; p < P; ++p) {
+    const MkProblem& q = probs[p];
+    MkState& s = hs[p];
+    std::memset(&s, 0, sizeof(s));
+    s.nev = q.nev;
+    s.m = std::max(q.nev, std::min(q.nev + MK_GUARD, most));
+    s.omega2 = q.omega * q.omega;
+    s.tol = q.tol;
+    s.ftol = q.ftol;
+    for (int j = 0; j < s.m; ++j) s.k[j] = s.knew[j] = s.keval[j] = q.k[std::min<size_t>(j, q.k.size() - 1)];
+    g.mmax = std::max(g.mmax, s.m);
+    ninst += q.nev;
+  }
+  g.slots = 5L * g.mmax * PLANES * g.cs;
+  const int nmax = 3 * g.mmax, NT = (nmax + 15) / 16, pm = 16 * NT;
+  const long vecs = long(P) * g.mmax;
+  const int RB = pick_rows(S.nx, S.ny, vecs, g.fx), TX = pick_rows(S.ny, S.nx, vecs, g.fy);
+  if (RB == 0 || TX == 0) return false;
+  const int nrb = (S.ny + RB - 1) / RB, ncb = (S.nx + TX - 1) / TX;
+  // Gram chunks: about 128 over the problems, whole stages of 64 rows, at least four of them
+  const int nchunk = int(std::max<long>(1, std::min<long>((S.N + 255) / 256, std::max(8, 128 / P))));
+  const long rpc = ((S.N + nchunk - 1) / nchunk + 63) / 64 * 64;
+  const int nch = int((S.N + rpc - 1) / rpc);
+  MultiKWorkspace& W = S.multik_ws;
+  const size_t colb = sizeof(c32) * size_t(P) * g.slots;
+  if (W.cols.size() < colb || W.geom != g.cs * 64 + g.mmax) {
+    W.cols.ensure(colb);
+    // the pads past N of every plane are read as zeros
+    OMX_HIP_CHECK(hipMemsetAsync(W.cols.as<void>(), 0, W.cols.size(), sm));
+    W.geom = g.cs * 64 + g.mmax;
+  }
+  W.dm.ensure(sizeof(c32) * size_t(vecs) * 3 * g.cs);
+  W.part.ensure(sizeof(c32) * size_t(P) * nch * NGRAM * pm * pm);
+  W.red.ensure(sizeof(c64) * size_t(P) * NGRAM * pm * pm);
+  W.cx.ensure(sizeof(c32) * size_t(P) * MK_MAXN * MK_MAXM);
+  W.cblk.ensure(sizeof(c64) * size_t(vecs) * 2 * MK_MAXN * MK_MAXN);
+  W.normp.ensure(sizeof(double) * size_t(vecs) * nrb);
+  W.state.ensure(sizeof(MkState) * P);
+  W.ints.ensure(sizeof(int) * size_t(P) * MK_MAXM + sizeof(int2) * ninst);
+  if (W.snap_bytes < sizeof(MkState) * P) {
+    for (int b = 0; b < 2; ++b) W.snap[b].alloc(sizeof(MkState) * P);
+    W.snap_bytes = sizeof(MkState) * P;
+  }
+  for (int b = 0; b < 2; ++b)
+    if (!W.ev[b]) OMX_HIP_CHECK(hipEventCreateWithFlags(&W.ev[b], hipEventDisableTiming));
+  c32* cols = W.cols.as<c32>();
+  c32* dm = W.dm.as<c32>();
+  c32* part = W.part.as<c32>();
+  c64* red = W.red.as<c64>();
+  c32* cx = W.cx.as<c32>();
+  c64* cblk = W.cblk.as<c64>();
+  double* normp = W.normp.as<double>();
+  MkState* st = W.state.as<MkState>();
+  int2* instd = W.ints.as<int2>();
+  int* mszd = reinterpret_cast<int*>(instd + ninst);
+  std::vector<int> hmsz(size_t(P) * MK_MAXM, 0);
+  std::vector<int2> hinst;
+  for (int p = 0; p < P; ++p)
+    for (int j = 0; j < probs[p].nev; ++j) {
+      hmsz[size_t(p) * MK_MAXM + j] = msize[hinst.size()];
+      hinst.push_back(int2{p, j});
+    }
+  OMX_HIP_CHECK(hipMemcpyAsync(st, hs.data(), sizeof(MkState) * P, hipMemcpyHostToDevice, sm));
+  OMX_HIP_CHECK(hipMemcpyAsync(instd, hinst.data(), sizeof(int2) * ninst, hipMemcpyHostToDevice, sm));
+  OMX_HIP_CHECK(hipMemcpyAsync(mszd, hmsz.data(), sizeof(int) * hmsz.size(), hipMemcpyHostToDevice, sm));
+  const size_t ldsr = sizeof(c32) * (S.nx + 3 * size_t(RB) * (S.nx + 1));
+  const size_t ldsc = sizeof(c32) * (S.ny + 3 * size_t(TX) * S.ny);
+  const dim3 gr(nrb, unsigned(vecs)), gc(ncb, unsigned(vecs)), gc2(ncb, unsigned(vecs), 2);
+  const int vpt = fits(3 * RB, g.fx, 8) && fits(3 * TX, g.fy, 8) ? 8 : 16;
+  for (int p = 0; p < P; ++p)
+    hipLaunchKernelGGL(k_mk_start, dim3(unsigned(std::min<long>((S.N + 255) / 256, 256)), hs[p].m), dim3(256), 0, sm, g,
+                       cols, st, p, probs[p].src, probs[p].lds, probs[p].src ? probs[p].nsrc : 0, probs[p].lowres,
+                       S.opt.seed);
+  auto transforms = [&](auto V, auto START) {
+    constexpr int v = decltype(V)::value;
+    constexpr bool start = decltype(START)::value;
+    hipLaunchKernelGGL((k_mk_rowW<v, start>), gr, dim3(FT), ldsr, sm, g, cols, st, dm, RB);
+    hipLaunchKernelGGL((k_mk_colF<v, start>), gc2, dim3(FT), ldsc, sm, g, cols, st, TX);
+  };
+  using v8 = std::integral_constant<int, 8>;
+  using v16 = std::integral_constant<int, 16>;
+  if (vpt == 8)
+    transforms(v8{}, std::true_type{});
+  else
+    transforms(v16{}, std::true_type{});
+  auto gram = [&](auto T, int buf) {
+    constexpr int nt = decltype(T)::value;
+    constexpr int S_ = nt <= 2 ? 4 : 2, NB = nt <= 2 ? 3 : (nt == 3 ? 2 : 1);
+    const dim3 gg(nch, P), gb(nch, P, (MK_NODES + NB) / NB);
+    hipLaunchKernelGGL((k_mk_gram<nt, 0, 1, S_>), gg, dim3(256), 0, sm, g, cols, st, buf, rpc, part);
+    hipLaunchKernelGGL((k_mk_gram<nt, 1, 1, S_>), gg, dim3(256), 0, sm, g, cols, st, buf, rpc, part);
+    hipLaunchKernelGGL((k_mk_gram<nt, 2, 1, S_>), gg, dim3(256), 0, sm, g, cols, st, buf, rpc, part);
+    hipLaunchKernelGGL((k_mk_gram<nt, 3, NB, S_>), gb, dim3(256), 0, sm, g, cols, st, buf, rpc, part);
+  };
+  const int ldd = (nmax + 1) | 1;  // odd sizes are padded to even ones in the Jacobi
+  const size_t ldsd = sizeof(c64) * 3 * size_t(nmax + 1) * ldd;
+  const dim3 gcomb(unsigned(std::min<long>((PLANES * g.cs / 2 + 255) / 256, std::max(1, 2048 / P))), P);
+  const bool prof = S.prof.enabled;
+  int cur = 0, it = 0;
+  bool fin = false, ok = true;
+  for (; it < maxit && !fin; ++it) {
+    switch (NT) {
+      case 1: gram(std::integral_constant<int, 1>{}, cur); break;
+      case 2: gram(std::integral_constant<int, 2>{}, cur); break;
+      case 3: gram(std::integral_constant<int, 3>{}, cur); break;
+      default: gram(std::integral_constant<int, 4>{}, cur); break;
+    }
+    hipLaunchKernelGGL(k_mk_reduce, dim3(pm * pm / 16, NGRAM, P), dim3(256), 0, sm, part, nch, pm, st, red);
+    hipLaunchKernelGGL(k_mk_dense, dim3(g.mmax, P), dim3(DT), ldsd, sm, g, st, red, pm, ldd, S.opt.jac_stop32, mszd, cx,
+                       cblk);
+    if (g.mmax <= 4)
+      hipLaunchKernelGGL((k_mk_combine<4>), gcomb, dim3(256), 0, sm, g, cols, st, cx, cur);
+    else if (g.mmax <= 8)
+      hipLaunchKernelGGL((k_mk_combine<8>), gcomb, dim3(256), 0, sm, g, cols, st, cx, cur);
+    else if (g.mmax <= 12)
+      hipLaunchKernelGGL((k_mk_combine<12>), gcomb, dim3(256), 0, sm, g, cols, st, cx, cur);
+    else
+      hipLaunchKernelGGL((k_mk_combine<MK_MAXM>), gcomb, dim3(256), 0, sm, g, cols, st, cx, cur);
+    const hipEvent_t ea = prof ? S.prof.begin(sm) : nullptr;
+    auto chain = [&](auto V) {
+      constexpr int v = decltype(V)::value;
+      hipLaunchKernelGGL((k_mk_colE<v>), gc, dim3(FT), ldsc, sm, g, cols, st, cur ^ 1, dm, TX);
+      hipLaunchKernelGGL((k_mk_rowR<v>), gr, dim3(FT), ldsr, sm, g, cols, st, cur ^ 1, dm, RB, normp);
+      hipLaunchKernelGGL(k_mk_control, dim3(P), dim3(256), 0, sm, g, st, normp, nrb, cur);
+      hipLaunchKernelGGL((k_mk_colP<v>), gc, dim3(FT), ldsc, sm, g, st, dm, TX);
+      transforms(V, std::false_type{});
+    };
+    if (vpt == 8)
+      chain(v8{});
+    else
+      chain(v16{});
+    OMX_HIP_CHECK(hipGetLastError());
+    if (prof) S.prof.commit(ea, S.prof.begin(sm), &S.prof.op32, 2.0 * (32.0 * S.N * vecs + 24.0 * S.N * P));
+    OMX_HIP_CHECK(hipMemcpyAsync(W.snap[it & 1].as<void>(), st, sizeof(MkState) * P, hipMemcpyDeviceToHost, sm));
+    OMX_HIP_CHECK(hipEventRecord(W.ev[it & 1], sm));
+    cur ^= 1;
+    if (it == 0) continue;
+    // the state after the iteration before (an iteration enqueued after the end does nothing)
+    OMX_HIP_CHECK(hipEventSynchronize(W.ev[(it - 1) & 1]));
+    const MkState* h = W.snap[(it - 1) & 1].as<MkState>();
+    fin = true;
+    for (int p = 0; p < P; ++p) fin = fin && h[p].done;
+    if (S.trace) {
+      std::fprintf(stderr, "[omx] multik it %d:", it - 1);
+      for (int p = 0; p < P; ++p) {
+        double rm = 0;
+        for (int j = 0; j < h[p].nev; ++j) rm = std::max(rm, h[p].rnorm[j]);
+        std::fprintf(stderr, " [na %d np %d res %.1e k1 %.6f%s]", h[p].na, h[p].np, rm / h[p].omega2, h[p].k[0],
+                     h[p].done == 1 ? " done" : (h[p].done ? " FAILED" : ""));
+      }
+      std::fprintf(stderr, "\n");
+    }
+  }
+  OMX_HIP_CHECK(hipStreamSynchronize(sm));
+  OMX_HIP_CHECK(hipMemcpy(hs.data(), st, sizeof(MkState) * P, hipMemcpyDeviceToHost));
+  for (int p = 0; p < P; ++p) ok = ok && hs[p].done == 1;
+  if (!ok) return false;
+  kout.clear();
+  iters.clear();
+  moves.clear();
+  for (const MkState& h : hs) moves.push_back(h.moves);
+  int mmax = 1;
+  for (int p = 0, i = 0; p < P; ++p)
+    for (int j = 0; j < probs[p].nev; ++j, ++i) {
+      kout.push_back(hs[p].k[j]);
+      iters.push_back(hs[p].its[j]);
+      mmax = std::max(mmax, msize[i]);
+      stats.matvec += hs[p].its[j];
+      stats.precon += hs[p].its[j];
+    }
+  hipLaunchKernelGGL(k_mk_handover, dim3(unsigned(std::min<long>((S.N + 255) / 256, 512)), ninst, (mmax + HQ - 1) / HQ),
+                     dim3(256), 0, sm, g, cols, st, instd, mszd, cblk, X64, ld, istride);
+  OMX_HIP_CHECK(hipGetLastError());
+  return true;
+}
+
+}  // namespace omx

@@ -189,6 +189,18 @@ __global__ __launch_bounds__(RB) void k_band_resid(const c64* X, const c64* AX, 
   if (threadIdx.x == 0) part[long(i) * gridDim.x + blockIdx.x] = red[0];
 }
 
+__global__ __launch_bounds__(RB) void k_block_resid(const c64* X, const c64* AX, long ld, long istride,
+                                                    const double* lam, const int* n1, long K, cplx<float>* R) {
+  const int i = blockIdx.y, c = blockIdx.z;
+  if (c >= n1[i]) return;
+  const long o = i * istride + c * ld;
+  const double l = lam[RF_MAXC * i + c];
+  for (long r = long(blockIdx.x) * RB + threadIdx.x; r < K; r += long(gridDim.x) * RB) {
+    const c64 a = X[o + r], b = AX[o + r];
+    R[o + r] = cplx<float>{float(b.x - l * a.x), float(b.y - l * a.y)};
+  }
+}
+
 __global__ __launch_bounds__(RB) void k_scale_cols(c64* x, long ld, const double* scale, const int* n1, long K) {
   const int i = blockIdx.y;
   if (n1[i] == 0) return;
@@ -224,6 +236,13 @@ void launch_band_resid(const c64* X, const c64* AX, long ld, long istride, const
                        const int* n1, int ninst, long K, int nblk, c64* xb, c64* rb, double* part, hipStream_t s) {
   hipLaunchKernelGGL(k_band_resid, dim3(nblk, ninst), dim3(RB), 0, s, X, AX, ld, istride, col, lam, n1, K, xb, rb,
                      part);
+  OMX_HIP_CHECK(hipGetLastError());
+}
+
+void launch_block_resid(const c64* X, const c64* AX, long ld, long istride, const double* lam, const int* n1,
+                        int ncol, int ninst, long K, cplx<float>* R, hipStream_t s) {
+  hipLaunchKernelGGL(k_block_resid, dim3(std::min(64, rows_grid(K)), ninst, ncol), dim3(RB), 0, s, X, AX, ld, istride,
+                     lam, n1, K, R);
   OMX_HIP_CHECK(hipGetLastError());
 }
 

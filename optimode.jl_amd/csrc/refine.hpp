@@ -36,6 +36,11 @@ void launch_bcombine(const RCols& U, const c64* C, const int* n1, int omode, c64
 void launch_band_resid(const c64* X, const c64* AX, long ld, long istride, const int* col, const double* lam,
                        const int* n1, int ninst, long K, int nblk, c64* xb, c64* rb, double* part, hipStream_t s);
 
+// R_c = AX_c - lam[RF_MAXC i + c] X_c in FP32 (same layout as X) for the n1[i] columns of
+// every instance with n1[i] > 0
+void launch_block_resid(const c64* X, const c64* AX, long ld, long istride, const double* lam, const int* n1,
+                        int ncol, int ninst, long K, cplx<float>* R, hipStream_t s);
+
 // x_i *= scale[i] (compact vectors)
 void launch_scale_cols(c64* x, long ld, const double* scale, const int* n1, int ninst, long K, hipStream_t s);
 

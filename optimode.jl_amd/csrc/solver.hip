@@ -3,6 +3,7 @@
 // solvers/gpu.jl:213-242) in an FP32 phase followed by an FP64 refinement phase.
 #include "solver.hpp"
 #include "krylov.hpp"
+#include "multik.hpp"
 #include "refine.hpp"
 
 #include <algorithm>
@@ -777,6 +778,8 @@ void Solver::set_option(const std::string& key, double v) {
     opt.jd_first_tol = std::max(0.0, v);
   else if (key == "streams2")
     opt.streams2 = v != 0 ? 1 : 0;
+  else if (key == "multik")
+    opt.multik = v != 0 ? 1 : 0;
   else if (key == "graphs")
     opt.graphs = v != 0 ? 1 : 0;
   else if (key == "jac_stop32")
@@ -1300,6 +1303,14 @@ void Solver::solve_omega2(double k, int nev, double tol, int maxiter, double* H_
 
 namespace {
 
+// Shared-subspace FP32 phase: |change of w^2| / w^2 by which a band's k must have settled
+// (the refinement's first Newton step takes it from there), and its iteration cap, the
+// total a caller's limits allow one band of the per-band form, at most 200.
+constexpr double MK_FTOL = 1e-5;
+int multik_maxit(int maxiter, int max_eigsolves) {
+  return int(std::min<long>(200, long(maxiter) * std::min(max_eigsolves, 8)));
+}
+
 // Newton driver over a batch of band instances (instance i follows band i).
 template <typename T>
 int newton_phase(Solver& S, Batch<T>& b, std::vector<NewtonState>& hns, const std::vector<int>& bands,
@@ -1601,6 +1612,7 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
   const OpPlan<double>& plan = S.p64.plan;
   std::vector<int> n1h(ninst, 0), jdh(ninst, 0);
   std::vector<double> lam_band(ninst, 0.0), rn(ninst, 0.0);
+  std::vector<double> theta(size_t(ninst) * RF_MAXC, 0.0), schur(size_t(ninst) * 16, 0.0);  // block Ritz values
   std::vector<c64> hG(size_t(ninst) * RF_PAIRS), hB(size_t(ninst) * RF_PAIRS), hC(size_t(ninst) * RF_PAIRS);
   auto up_n1 = [&](const std::vector<int>& v) {
     OMX_HIP_CHECK(hipMemcpyAsync(n1d.as<void>(), v.data(), sizeof(int) * ninst, hipMemcpyHostToDevice, s));
@@ -1633,10 +1645,19 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
       c64* Ci = hC.data() + size_t(i) * RF_PAIRS;
       const int n = m + ((any_t && with_t[i]) ? 1 : 0);
       if (!dense_geig(n, hG.data() + size_t(i) * RF_PAIRS, hB.data() + size_t(i) * RF_PAIRS, lam, C))
+      {
+        if (S.trace) {
+          const c64* Bi = hB.data() + size_t(i) * RF_PAIRS;
+          std::fprintf(stderr, "[omx] refinement: instance %d of %d columns lost rank, diagonal of U^H U:", i, n);
+          for (int l = 0; l < n; ++l) std::fprintf(stderr, " %.3e", Bi[l + RF_MAXC * l].x);
+          std::fprintf(stderr, "\n");
+        }
         throw Error(OMX_ERR_CHOLESKY, "refinement: the Rayleigh-Ritz basis lost rank");
+      }
       for (int j = 0; j < m; ++j)
         for (int l = 0; l < n; ++l) Ci[l + RF_MAXC * j] = c64{C[l + size_t(n) * j].real(), C[l + size_t(n) * j].imag()};
       lam_band[i] = lam[bands[i]];
+      std::copy(lam.begin(), lam.begin() + m, theta.begin() + size_t(i) * RF_MAXC);
     }
     OMX_HIP_CHECK(hipMemcpyAsync(Cd.as<void>(), hC.data(), sizeof(c64) * hC.size(), hipMemcpyHostToDevice, s));
     // in place: each row's inputs are read before its outputs are written (one thread per
@@ -1714,7 +1735,29 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
           W.nqd.ensure(sizeof(int) * size_t(ninst));
           launch_convert<double, float>(b.p(b.X[b.cur]), ld, istride, W.Xf.as<cf>(), ld, qis, ninst, b.M, K, s);
           OMX_HIP_CHECK(hipMemcpyAsync(W.nqd.as<void>(), msize.data(), sizeof(int) * ninst, hipMemcpyHostToDevice, s));
-          V32.set_block(W.Xf.as<cf>(), qis, W.nqd.as<int>(), *std::max_element(msize.begin(), msize.end()));
+          const int mmax = *std::max_element(msize.begin(), msize.end());
+          V32.set_block(W.Xf.as<cf>(), qis, W.nqd.as<int>(), mmax);
+          // The block's other vectors are Ritz vectors, not eigenvectors (their residuals at
+          // this band's k can be several percent of w^2 after the shared-subspace phase):
+          // the exact system on the block's complement takes them into account.  Ritz values
+          // within 1e-3 of the band's stay out (their own residuals are small: bands that
+          // close converged at nearly the same k).
+          W.Rf.ensure(sizeof(cf) * size_t(ninst) * qis);
+          W.rgd.ensure(sizeof(double) * schur.size());
+          W.thd.ensure(sizeof(double) * theta.size());
+          for (int i = 0; i < ninst; ++i)
+            for (int l = 0; l < 16; ++l) {
+              const double d = l < msize[i] ? theta[size_t(i) * RF_MAXC + l] - lam_band[i] : 0.0;
+              schur[size_t(i) * 16 + l] =
+                  l != bands[i] && std::fabs(d) > 1e-3 * std::fabs(lam_band[i]) ? 1.0 / d : 0.0;
+            }
+          OMX_HIP_CHECK(hipMemcpyAsync(W.rgd.as<void>(), schur.data(), sizeof(double) * schur.size(),
+                                       hipMemcpyHostToDevice, s));
+          OMX_HIP_CHECK(hipMemcpyAsync(W.thd.as<void>(), theta.data(), sizeof(double) * theta.size(),
+                                       hipMemcpyHostToDevice, s));
+          launch_block_resid(b.p(b.X[b.cur]), b.p(b.AX[b.cur]), ld, istride, W.thd.as<double>(), W.nqd.as<int>(), mmax,
+                             ninst, K, W.Rf.as<cf>(), s);
+          V32.set_schur(W.Rf.as<cf>(), W.rgd.as<double>());
         }
         its = minres_complement_t<float>(S, V32, lam_band, b.kd.as<double>(), W.RBf.as<cf>(), W.Tf.as<cf>(), jdh,
                                          S.opt.jd_rtol, S.opt.jd_maxit, false);
@@ -1885,9 +1928,14 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
     msize[i] = (opt.guard < 0 || opt.plain) ? M : std::min(M, i + 1 + opt.guard);
   }
   const int maxit64 = std::max(maxiter, opt.maxiter_fp64);
-  const auto b64p = workspace<double>(*this, ninst, M, maxit64);
+  // FP32 phase in one search space (multik.hip): its blocks carry columns past the last band
+  // too, which take the next modes out of the top bands' correction solves
+  const bool use_multik =
+      opt.multik && opt.refine && opt.fp32_newton && !opt.fp64_only && !opt.plain && multik_fits(*this);
+  const int M64 = use_multik ? multik_block(nev, K) : M;
+  const auto b64p = workspace<double>(*this, ninst, M64, maxit64);
   Batch<double>& b64 = *b64p;
-  int newton_total = 0;
+  int newton_total = 0, mk_moves = 0;  // mk_moves: Newton steps inside the shared-subspace phase
   const int nguess_used = (Hguess && nguess > 0) ? std::min(nguess, M) : 0;
   const int ghw = opt.guess_lowres;
   if (nguess_used && ghw > 0 && (nz > 1 || ghw % 2 != 0 || ghw > nx || ghw > ny))
@@ -1982,6 +2030,58 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
     OMX_HIP_CHECK(hipStreamSynchronize(stream));
   };
 
+  // the FP32 phase in one search space; false if this solve does not take it or a band did not
+  // converge there
+  auto multik_phase = [&]() {
+    if (!use_multik) return false;
+    std::vector<int> msize_mk(ninst);
+    for (int i = 0; i < ninst; ++i) msize_mk[i] = opt.guard < 0 ? M64 : std::min(M64, i + 1 + opt.guard);
+    MkProblem q;
+    q.omega = omega;
+    q.nev = nev;
+    q.tol = tol32;
+    q.ftol = std::max(k_tol, MK_FTOL * w2);
+    q.k.assign(1, k0);
+    DevMem up;
+    if (warm) {
+      q.src = last_evecs.as<c64>();
+      q.lds = ld;
+      q.nsrc = std::min(last_nev, nev);
+      q.k.assign(last_kmags.begin(), last_kmags.begin() + q.nsrc);
+    } else if (nguess_used) {
+      const size_t per = ghw > 0 ? 2 * size_t(ghw) * ghw : size_t(K);
+      q.src = ghw > 0 ? guess_dev : nullptr;
+      if (!q.src) {
+        up.alloc(sizeof(c64) * nguess_used * per);
+        OMX_HIP_CHECK(hipMemcpyAsync(up.as<void>(), Hguess, sizeof(c64) * nguess_used * per, hipMemcpyHostToDevice,
+                                     stream));
+        q.src = up.as<c64>();
+      }
+      q.lds = long(per);
+      q.nsrc = nguess_used;
+      q.lowres = ghw;
+      if (banded) q.k.assign(kguess, kguess + nev);
+    }
+    std::vector<double> kk;
+    std::vector<int> its, moves;
+    if (!multik_solve(*this, {q}, p32.plan.eps6c, 0, multik_maxit(maxiter, max_eigsolves), msize_mk, b64.p(b64.X[0]), ld,
+                      b64.istride, kk, its, moves, stats))
+      return false;
+    msize = msize_mk;
+    mk_moves = moves[0];
+    for (int i = 0; i < ninst; ++i) {
+      hns[i].k = kk[i];
+      hns[i].nsolves = 1;
+      hns[i].k_tol = k_tol;
+      stats.it32 += its[i];
+    }
+    OMX_HIP_CHECK(hipMemcpyAsync(b64.kd.as<void>(), kk.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, stream));
+    ++newton_total;
+    OMX_HIP_CHECK(hipStreamSynchronize(stream));  // kk and the uploaded guess go out of scope
+    t_fp32_end = std::chrono::steady_clock::now();
+    return true;
+  };
+
   if (opt.plain) {
     // the reference's algorithm (solve.jl:89-113 with the DFTK backend): each band runs
     // Newton from k_guess with its own random nev-column start, every eigensolve to eig_tol
@@ -2004,6 +2104,9 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
       for (int i = 0; i < ninst; ++i)
         if (i != b) hns[i] = keep[i];
     }
+  } else if (!opt.fp64_only && multik_phase()) {
+    // all bands in one search space (multik.hip); below, one LOBPCG block per band: 3D cells,
+    // FP64 LOBPCG after the FP32 phase, and what the shared space left unconverged
   } else if (!opt.fp64_only) {
     // two half-batches of bands on two streams (the seed eigensolve runs in the first)
     const int na = (ninst + 1) / 2, nb = ninst - na;
@@ -2138,7 +2241,7 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
   (void)hipEventDestroy(e1);
   if (info) {
     info->converged = ok ? 1 : 0;
-    info->n_newton = newton_total;
+    info->n_newton = newton_total + mk_moves;
     info->lobpcg_iters_fp32 = stats.it32;
     info->lobpcg_iters_fp64 = stats.it64;
     info->n_matvec = stats.matvec;
@@ -2218,7 +2321,7 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
   OMX_HIP_CHECK(hipEventCreate(&e1));
   OMX_HIP_CHECK(hipEventRecord(e0, s));
   // the problems' eps^-1, and which one each instance reads
-  const size_t n6 = size_t(6) * N;
+  const size_t n6 = (size_t(6) * N + 63) / 64 * 64;  // fields start on whole lines
   multi_e32r.ensure(sizeof(float) * n6 * P);
   multi_e32c.ensure(sizeof(float) * n6 * P);
   multi_e64r.ensure(sizeof(double) * n6 * P);
@@ -2289,7 +2392,8 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
       kinit[i] = k0[p];
     }
   const int maxit64 = std::max(maxiter, opt.maxiter_fp64);
-  const auto b64p = workspace<double>(*this, ninst, M, maxit64);
+  const bool use_multik = opt.multik && opt.refine && opt.fp32_newton && !opt.fp64_only && multik_fits(*this);
+  const auto b64p = workspace<double>(*this, ninst, use_multik ? multik_block(M, K) : M, maxit64);
   Batch<double>& b64 = *b64p;
   std::vector<int> it32_inst(ninst, 0);
 
@@ -2337,7 +2441,41 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
     return it;
   };
 
-  if (!opt.fp64_only) {
+  // the FP32 phase of every problem in its own shared search space (multik.hip)
+  auto multik_phase = [&]() {
+    if (!use_multik) return false;
+    std::vector<MkProblem> mk(P);
+    std::vector<int> msize_mk(ninst);
+    for (int p = 0; p < P; ++p) {
+      const int most = multik_block(probs[p].nev, K);
+      for (int j = 0; j < probs[p].nev; ++j)
+        msize_mk[off[p] + j] = opt.guard < 0 ? most : std::min(most, j + 1 + opt.guard);
+      mk[p].omega = probs[p].omega;
+      mk[p].nev = probs[p].nev;
+      mk[p].tol = tol32[off[p]];
+      mk[p].ftol = std::max(probs[p].k_tol, MK_FTOL * w2[off[p]]);
+      mk[p].k.assign(1, k0[p]);
+    }
+    std::vector<double> kk;
+    std::vector<int> its, moves;
+    if (!multik_solve(*this, mk, p32.plan.eps6c, p32.plan.eps_stride, multik_maxit(maxiter, max_eigsolves), msize_mk,
+                      b64.p(b64.X[0]), ld, b64.istride, kk, its, moves, stats))
+      return false;
+    msize = msize_mk;
+    for (int i = 0; i < ninst; ++i) {
+      hns[i].k = kk[i];
+      hns[i].nsolves = 1;
+      hns[i].k_tol = probs[prob_of[i]].k_tol;
+      it32_inst[i] += its[i];
+      stats.it32 += its[i];
+    }
+    OMX_HIP_CHECK(hipMemcpyAsync(b64.kd.as<void>(), kk.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, s));
+    ++newton_total;
+    OMX_HIP_CHECK(hipStreamSynchronize(s));
+    return true;
+  };
+  if (!opt.fp64_only && multik_phase()) {
+  } else if (!opt.fp64_only) {
     const auto b32p = workspace<float>(*this, ninst, M, maxiter);
     Batch<float>& b32 = *b32p;
     for (int i = 0; i < ninst; ++i) hns[i].k_tol = std::max(probs[prob_of[i]].k_tol, opt.fp32_switch * w2[i]);

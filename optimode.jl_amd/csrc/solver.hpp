@@ -191,6 +191,8 @@ struct Options {
   int streams2 = 1;             // FP32 Newton phase of solve_k as two half-batches of bands on two
                                 // streams in lockstep (one half's latency-bound dense steps overlap
                                 // the other half's memory-bound kernels)
+  int multik = 1;               // FP32 phase of solve_k on 2D cells in one search space shared by all
+                                // bands (multik.hip); 0: one LOBPCG block per band
   int graphs = 0;               // MINRES iterations replayed from a captured HIP graph (groups of 12;
                                 // same results, no measured gain: the gaps are GPU-side)
 };
@@ -219,6 +221,20 @@ struct RefineWorkspace {
   DevMem n1d, zero, cold, lamd, Tm, T2, ATm, XB, RBm, part, Gd, Bd, Cd, normp, scl, dots;
   DevMem XBf, RBf, Tf;  // FP32 copies for the correction solves (option jd_fp32)
   DevMem Xf, nqd;       // FP32 copy of the block and its column counts (option jd_deflate)
+  DevMem Rf, rgd, thd;  // FP32 residual block, Schur weights and Ritz values of the block
+};
+
+// Buffers of the shared-subspace FP32 phase (multik.hip), kept on the handle between solves.
+struct MultiKWorkspace {
+  DevMem cols, dm, part, red, cx, cblk, normp, state, ints;
+  long geom = 0;          // plane size and column count the zeroed pads belong to
+  PinnedMem snap[2];
+  size_t snap_bytes = 0;
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  ~MultiKWorkspace() {
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+  }
 };
 
 // One problem of a batched solve on a handle's grid (Solver::solve_k_multi).
@@ -309,6 +325,7 @@ class Solver {
   DevMem krylov_ws;                  // MINRES vectors and scratch (grown on demand)
   DevMem vec_part, vec_coef;          // partial sums and coefficients of the vector helpers
   RefineWorkspace refine_ws;          // buffers of the FP64 refinement phase
+  MultiKWorkspace multik_ws;          // buffers of the shared-subspace FP32 phase
   DevMem field_scratch, argmax_v, argmax_i;  // canonicalize_phase
   // solve_k_multi: the problems' eps^-1 stacked per precision and layout, the instance ->
   // field map, and the band eigenvectors of all instances

@@ -1,0 +1,102 @@
+"""The shared-subspace FP32 phase of solve_k against the per-band form on the same problems:
+grids at the edges of its tiles (odd sizes, odd pixel counts, sizes that leave partial row and
+column blocks), the smallest and the widest blocks, every kind of start, and batches.
+
+Both forms end in the same FP64 refinement with |change of w^2| <= k_tol = 1e-11, so k agrees
+to k_tol / (slope k) <= 1e-11 / (2 * 0.3 * 0.3) < 6e-11; 2e-10 allows for both sides."""
+import numpy as np
+import pytest
+
+import omx
+from omx import geometry as G
+
+pytestmark = pytest.mark.gpu
+W0 = 1 / 1.55
+KW = dict(k_tol=1e-11, eig_tol=1e-9, max_eigsolves=60, maxiter=300, return_info=True)
+
+
+def _eps(nx, ny, seed=0):
+    """A ridge whose core has every tensor entry, averaged linearly at the interface."""
+    r = np.random.default_rng(seed)
+    a = r.uniform(-0.3, 0.3, 3)
+    Q, _ = np.linalg.qr(np.eye(3) + np.array([[0, a[0], a[1]], [-a[0], 0, a[2]], [-a[1], -a[2], 0]]))
+    core = Q @ np.diag([4.2, 4.0, 4.2]) @ Q.T
+    g = omx.Grid(6.0, 4.0, nx, ny)
+    return g, G.ridge_waveguide(g, 1.5 + 0.1 * seed, 0.6, 75.0, core, backend="gpu")
+
+
+def _solve(g, ei, nev, multik, **kw):
+    s = omx.HIPSolver()
+    s.options["multik"] = float(multik)
+    return omx.solve_k(W0, ei, g, s, nev=nev, **{**KW, **kw})
+
+
+@pytest.mark.parametrize("nx,ny,nev", [(16, 12, 1), (12, 18, 2), (27, 25, 3), (40, 30, 6), (64, 64, 13), (135, 81, 4),
+                                       (100, 48, 7), (128, 96, 16), (50, 250, 5), (256, 128, 15)])
+def test_matches_the_per_band_form(nx, ny, nev):
+    print(f"multik {nx}x{ny} nev {nev}", flush=True)
+    g, ei = _eps(nx, ny)
+    k0, ev0, i0 = _solve(g, ei, nev, 0)
+    k1, ev1, i1 = _solve(g, ei, nev, 1)
+    assert i0["converged"] == i1["converged"] == 1
+    assert np.max(np.abs(k1 / k0 - 1)) < 2e-10
+    for j in range(nev):
+        # bands closer than 1e-4 share a subspace; the others match one by one
+        near = [i for i in range(nev) if abs(k0[i] - k0[j]) < 1e-4]
+        w = sum(abs(np.vdot(ev0[i], ev1[j])) ** 2 for i in near)
+        assert w > 1 - 1e-9
+
+
+def test_degenerate_bands():
+    """A square core: the two lowest bands are degenerate by symmetry."""
+    print("multik degenerate", flush=True)
+    g = omx.Grid(4.0, 4.0, 48, 48)
+    ei = G.rect_waveguide(g, w=1.0, h=1.0)
+    k0, _, _ = _solve(g, ei, 4, 0)
+    k1, ev, _ = _solve(g, ei, 4, 1)
+    assert abs(k0[0] - k0[1]) < 1e-9
+    assert np.max(np.abs(k1 / k0 - 1)) < 2e-10
+    assert abs(np.vdot(ev[0], ev[1])) < 1e-6
+
+
+def test_every_start_reaches_the_same_bands():
+    print("multik starts", flush=True)
+    g, ei = _eps(90, 64)
+    nev = 4
+    k0, ev, _ = _solve(g, ei, nev, 0)
+    n2 = 2 * g.N
+    full = np.stack(ev)
+    r = np.random.default_rng(1)
+    noisy = full + 0.05 * r.standard_normal((nev, 2 * n2)).view(np.complex128) / np.sqrt(n2)
+    for kw in (dict(kguess=1.01 * k0[0], Hguess=noisy), dict(kguess=0.99 * k0, Hguess=noisy, band_guess=True),
+               dict(Hguess=noisy[:2]), dict(kguess=k0[:1])):
+        k1, _, info = _solve(g, ei, nev, 1, **kw)
+        assert info["converged"] == 1
+        assert np.max(np.abs(k1 / k0 - 1)) < 2e-10
+    low = np.zeros((nev, 2, 16, 16), dtype=np.complex128)
+    sx, sy = np.r_[0:8, 90 - 8:90], np.r_[0:8, 64 - 8:64]
+    for j in range(nev):
+        low[j] = full[j].reshape((2, 90, 64), order="F")[:, sx][:, :, sy]
+    rows = low.transpose(0, 3, 2, 1).reshape(nev, -1)
+    k1, _, _ = _solve(g, ei, nev, 1, kguess=k0[:1], Hguess=rows, guess_hw=16)
+    assert np.max(np.abs(k1 / k0 - 1)) < 2e-10
+    s = omx.HIPSolver(warm_start=True)
+    omx.solve_k(0.99 * W0, ei, g, s, nev=nev, **KW)
+    k1, _, _ = omx.solve_k(W0, ei, g, s, nev=nev, **KW)
+    assert np.max(np.abs(k1 / k0 - 1)) < 2e-10
+
+
+def test_batch_on_an_odd_grid():
+    """Problems of one launch group with their own eps^-1, omega and mode count, on a grid whose
+    pixel count is odd (the fields' strides)."""
+    print("multik batch", flush=True)
+    probs, refs = [], []
+    for i, nev in enumerate((3, 6, 1)):
+        g, ei = _eps(45, 75, seed=i)
+        probs.append(dict(grid=g, epsinv=ei, omega=W0 * (1 + 0.02 * i), nev=nev, k_tol=1e-11, eig_tol=1e-9, maxiter=300))
+        s = omx.HIPSolver()
+        s.options["multik"] = 0.0
+        refs.append(omx.solve_k(probs[-1]["omega"], ei, g, s, nev=nev, **KW)[0])
+    for q, k0 in zip(omx.solve_k_batch(probs), refs):
+        assert q["status"] == 0
+        assert np.max(np.abs(q["kmags"] / k0 - 1)) < 2e-10
