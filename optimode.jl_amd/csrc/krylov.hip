@@ -11,7 +11,7 @@ namespace omx {
 namespace {
 
 constexpr int AB = 256;
-constexpr int RCQ = 16;  // Schur-complement coefficients per instance
+constexpr int RCQ = 18;  // Schur-complement coefficients per instance
 
 // out[(i*nb + b)] = Re sum_rows conj(a_i) b_i over block b's rows (vector i at base + i*ld),
 // accumulated in FP64
@@ -157,6 +157,44 @@ __device__ __forceinline__ double block_sum(const double* p, int n, double* red)
   const double r = red[0];
   __syncthreads();
   return r;
+}
+
+// Sums V values over a wavefront: halves of the values are exchanged between halves of the
+// lanes, so V values take about V + 6 shuffles instead of 6 V.  V rounds up to a power of two
+// (at most 64); lane l returns with the sum of value wave_sums_index<V>(l) (fixed order).
+template <int V> __host__ __device__ constexpr int pow2_ceil() {
+  int p = 1;
+  while (p < V) p *= 2;
+  return p;
+}
+template <int V> __device__ __forceinline__ int wave_sums_index(int lane) {
+  constexpr int P = pow2_ceil<V>();
+  int idx = 0;
+#pragma unroll
+  for (int w = P / 2, off = 32; w >= 1; w /= 2, off /= 2) idx += (lane & off) ? w : 0;
+  return idx;
+}
+template <int W, int OFF> __device__ __forceinline__ void wave_sums_step(double* x, int lane) {
+  if constexpr (W >= 1) {
+    const bool hi = (lane & OFF) != 0;
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      const double keep = hi ? x[i + W] : x[i], send = hi ? x[i] : x[i + W];
+      x[i] = keep + __shfl_xor(send, OFF, 64);
+    }
+    wave_sums_step<W / 2, OFF / 2>(x, lane);
+  } else if constexpr (OFF >= 1) {
+    x[0] += __shfl_xor(x[0], OFF, 64);
+    wave_sums_step<0, OFF / 2>(x, lane);
+  }
+}
+template <int V> __device__ __forceinline__ double wave_sums(const double (&v)[V], int lane) {
+  constexpr int P = pow2_ceil<V>();
+  double x[P];
+#pragma unroll
+  for (int i = 0; i < P; ++i) x[i] = i < V ? v[i] : 0.0;
+  wave_sums_step<P / 2, 32>(x, lane);
+  return x[0];
 }
 
 struct MinresState;
@@ -376,7 +414,7 @@ __global__ __launch_bounds__(AB) void k_minres_scalars(MinresState* ms, const do
     const int c = threadIdx.x % qm, j = threadIdx.x / qm, G = AB / qm;
     double a = 0, b = 0;
 #pragma unroll 8
-    for (int q = j; q < nb; q += G) {
+    for (int q = j < G ? j : nb; q < nb; q += G) {
       const c64 v = rpart[(long(i) * nb + q) * qm + c];
       a += v.x;
       b += v.y;
@@ -602,17 +640,11 @@ __global__ __launch_bounds__(AB) void k_qdot(const cplx<T>* Q, long qld, long qi
     qdot_cols<T, QM>(n, Q + i * qis, qld, X + i * ld, long(blockIdx.x) * AB + threadIdx.x, long(gridDim.x) * AB, K,
                      sr, si);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-  for (int c = 0; c < QM; ++c) {
-    double a = sr[c], b = si[c];
-    for (int off = 32; off > 0; off >>= 1) {
-      a += __shfl_down(a, off, 64);
-      b += __shfl_down(b, off, 64);
-    }
-    if (lane == 0) {
-      wr[wv][c] = a;
-      wi[wv][c] = b;
-    }
+  const double a1 = wave_sums<QM>(sr, lane), b1 = wave_sums<QM>(si, lane);
+  const int ix = wave_sums_index<QM>(lane);
+  if (ix < QM) {  // lanes that hold the same sum store the same value
+    wr[wv][ix] = a1;
+    wi[wv][ix] = b1;
   }
   __syncthreads();
   if (threadIdx.x < QM) {
@@ -645,13 +677,15 @@ __global__ __launch_bounds__(AB) void k_qproject(const c64* qpart, int qnblk, co
     {
       const int c = threadIdx.x % QM, j = threadIdx.x / QM;
       double a = 0, b = 0;
-      for (int q = j; q < qnblk; q += G) {
+      for (int q = j < G ? j : qnblk; q < qnblk; q += G) {
         const c64 v = qpart[(long(i) * qnblk + q) * QM + c];
         a += v.x;
         b += v.y;
       }
-      gr[j][c] = a;
-      gi[j][c] = b;
+      if (j < G) {
+        gr[j][c] = a;
+        gi[j][c] = b;
+      }
       __syncthreads();
       if (threadIdx.x < QM) {
         double sa = 0, sb = 0;
@@ -666,7 +700,7 @@ __global__ __launch_bounds__(AB) void k_qproject(const c64* qpart, int qnblk, co
     c64 cf[QM];
 #pragma unroll
     for (int c = 0; c < QM; ++c) cf[c] = c < n ? cfs[c] : c64{0, 0};
-    double rsr[SCHUR ? QM : 1], rsi[SCHUR ? QM : 1];
+    double rsr[QM], rsi[QM];
     if constexpr (SCHUR) {
 #pragma unroll
       for (int c = 0; c < QM; ++c) rsr[c] = rsi[c] = 0.0;
@@ -676,19 +710,13 @@ __global__ __launch_bounds__(AB) void k_qproject(const c64* qpart, int qnblk, co
                                         long(blockIdx.x) * AB + threadIdx.x, long(gridDim.x) * AB, K,
                                         SCHUR ? R + i * qis : nullptr, rsr, rsi);
     if constexpr (SCHUR) {
-      // per column: a wavefront butterfly, then the wavefronts in order
+      // per column: each wavefront's sum, then the wavefronts in order
       const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-      for (int c = 0; c < QM; ++c) {
-        double a = rsr[c], b = rsi[c];
-        for (int off = 32; off > 0; off >>= 1) {
-          a += __shfl_xor(a, off, 64);
-          b += __shfl_xor(b, off, 64);
-        }
-        if (lane == 0) {
-          gr[wv][c] = a;
-          gi[wv][c] = b;
-        }
+      const double a1 = wave_sums<QM>(rsr, lane), b1 = wave_sums<QM>(rsi, lane);
+      const int ix = wave_sums_index<QM>(lane);
+      if (ix < QM) {
+        gr[wv][ix] = a1;
+        gi[wv][ix] = b1;
       }
       __syncthreads();
       if (threadIdx.x < QM) {
@@ -767,7 +795,7 @@ void VecOpsT<T>::lincomb(std::initializer_list<const C*> ins, C* outp, const int
 }
 
 template <typename T> void VecOpsT<T>::set_block(const C* Qb, long qis, const int* nq, int nq_max) {
-  if (nq_max < 1 || nq_max > QMAX) throw Error(OMX_ERR_INTERNAL, "block projection: 1..16 columns");
+  if (nq_max < 1 || nq_max > QMAX) throw Error(OMX_ERR_INTERNAL, "block projection: 1..18 columns");
   // the real dot partials (nb nblk, at the start, where the MINRES steps read them), then
   // the block partials (nb nblk QMAX complex): every block of k_qproject reads the latter
   // while others write the former, so the two never overlap
@@ -778,7 +806,18 @@ template <typename T> void VecOpsT<T>::set_block(const C* Qb, long qis, const in
   qmax = nq_max;
   // a few thousand rows per block: the per-block reduction of the column dots stays small
   // beside the rows' loads
-  qblk = std::max(1, std::min(nblk, 64));
+  qblk = std::max(1, std::min(nblk, std::max(64, 1024 / nb)));
+}
+
+// the compiled column bounds of the block kernels
+int qm_of(int n) { return n <= 4 ? 4 : (n <= 8 ? 8 : (n <= 12 ? 12 : 18)); }
+template <typename F> void with_qm(int n, const F& f) {
+  switch (qm_of(n)) {
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 12: f(std::integral_constant<int, 12>{}); break;
+    default: f(std::integral_constant<int, 18>{}); break;
+  }
 }
 
 template <typename T> void VecOpsT<T>::set_schur(const C* Rb, const double* weights) {
@@ -791,23 +830,20 @@ template <typename T> void VecOpsT<T>::project_dot_to(C* x, const int* act, cons
   const dim3 g(nblk, nb);
   if (Q) {
     c64* qp = part.template as<c64>() + size_t(nb) * nblk;
-    const dim3 gq(qblk, nb);
+    const dim3 gq(qblk, nb);  // the projection's partials: qblk per instance too
     // past the block partials: the residual columns' partials, and the coefficients from them
     c64* rp = qp + size_t(nb) * nblk * QMAX;
     auto launch = [&](auto QMc) {
       constexpr int QMv = decltype(QMc)::value;
       hipLaunchKernelGGL((k_qdot<T, QMv>), gq, dim3(AB), 0, s, Q, ld, qistride, qn, x, ld, K, act, qp);
       if (R && dot_with)
-        hipLaunchKernelGGL((k_qproject<T, QMv, true>), g, dim3(AB), 0, s, qp, qblk, Q, ld, qistride, qn, x, dot_with, ld,
+        hipLaunchKernelGGL((k_qproject<T, QMv, true>), gq, dim3(AB), 0, s, qp, qblk, Q, ld, qistride, qn, x, dot_with, ld,
                            K, act, out, R, rp);
       else
-        hipLaunchKernelGGL((k_qproject<T, QMv, false>), g, dim3(AB), 0, s, qp, qblk, Q, ld, qistride, qn, x, dot_with,
+        hipLaunchKernelGGL((k_qproject<T, QMv, false>), gq, dim3(AB), 0, s, qp, qblk, Q, ld, qistride, qn, x, dot_with,
                            ld, K, act, out, R, rp);
     };
-    if (qmax <= 8)
-      launch(std::integral_constant<int, 8>{});
-    else
-      launch(std::integral_constant<int, QMAX>{});
+    with_qm(qmax, launch);
     return;
   }
   hipLaunchKernelGGL(k_cdot<T>, g, dim3(AB), 0, s, EV, x, ld, K, act, part.template as<c64>());
@@ -879,10 +915,11 @@ int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shi
   // y = P r1 (projected)
   launch_operator<T>(OP_P, plan, R1v, Yv, dm, sel, dk, nullptr, 0, s);
   V.project(y, act, r1);  // and the partials of <r1, y>
-  const int qm = V.qmax <= 8 ? 8 : VecOpsT<T>::QMAX;
+  const int qm = qm_of(V.qmax);
   const c64* rpart = V.R ? V.part.template as<c64>() + size_t(nb) * nblk * (1 + VecOpsT<T>::QMAX) : nullptr;
   c64* rc = V.R ? V.part.template as<c64>() + size_t(nb) * nblk * (1 + 2 * VecOpsT<T>::QMAX) : nullptr;
-  hipLaunchKernelGGL(k_minres_scalars, dim3(nb), dim3(AB), 0, s, ms, part, nblk, coef, 0, nb, act, rpart, qm, V.rg, rc);
+  const int pblk = V.Q ? V.qblk : nblk;  // partials per instance a projection leaves
+  hipLaunchKernelGGL(k_minres_scalars, dim3(nb), dim3(AB), 0, s, ms, part, pblk, coef, 0, nb, act, rpart, qm, V.rg, rc);
   OMX_HIP_CHECK(hipMemcpyAsync(r2, r1, vb, hipMemcpyDeviceToDevice, s));
   std::vector<int> live(want);
   int it = 0;
@@ -910,10 +947,8 @@ int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shi
     auto y1q = [&](auto WXc) {
       if (!V.R)
         y1(WXc, std::integral_constant<int, 0>{});
-      else if (V.qmax <= 8)
-        y1(WXc, std::integral_constant<int, 8>{});
       else
-        y1(WXc, std::integral_constant<int, VecOpsT<T>::QMAX>{});
+        with_qm(V.qmax, [&](auto q) { y1(WXc, q); });
     };
     if (fuse)
       y1q(std::true_type{});
@@ -929,7 +964,7 @@ int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shi
     launch_operator<T>(OP_P, plan, R2b, Yb, dm, sel, dk, nullptr, 0, s);
     // yn <- yn - ev <ev, yn> (or the block projection) with the partials of <r2, yn>
     V.project_dot_to(yn, la, r2, cpart2);
-    hipLaunchKernelGGL(k_minres_scalars, dim3(nb), dim3(AB), 0, s, ms, cpart2, nblk, coef, 3, nb, la, rpart, qm,
+    hipLaunchKernelGGL(k_minres_scalars, dim3(nb), dim3(AB), 0, s, ms, cpart2, pblk, coef, 3, nb, la, rpart, qm,
                        V.rg, rc);
     // this iteration's w/x update, pending (its v is u, the next iteration's v-buffer)
     pw1 = w2;

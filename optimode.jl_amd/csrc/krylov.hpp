@@ -40,11 +40,11 @@ template <typename T> struct VecOpsT {
   // Block deflation: from here on the projections remove the components of x_i along the
   // nq[i] orthonormal columns of instance i's block Qb (column c at Qb + i qis + c ld, at
   // most QMAX columns; nq on the device) instead of along ev_i.
-  static constexpr int QMAX = 16;
+  static constexpr int QMAX = 18;
   void set_block(const C* Qb, long qis, const int* nq, int nq_max);
   // With a block whose columns are Ritz vectors but not yet eigenvectors, the system on its
   // complement is the Schur complement (M - shift) - sum_c g_c R_c R_c^H, R_c = M Q_c - theta_c
-  // Q_c (laid out as the block), g_c = 1 / (theta_c - shift) (weights: 16 per instance, 0
+  // Q_c (laid out as the block), g_c = 1 / (theta_c - shift) (weights: QMAX per instance, 0
   // leaves a column out).  minres_complement_t then applies it in place of M - shift.
   void set_schur(const C* Rb, const double* weights);
   const C* R = nullptr;
@@ -53,7 +53,7 @@ template <typename T> struct VecOpsT {
   long qistride = 0;
   const int* qn = nullptr;
   int qmax = 0;   // the largest nq[i] (host): columns the block kernels are compiled for
-  int qblk = 0;   // row blocks per instance of the block dots
+  int qblk = 0;   // row blocks per instance of the block dots and of the block projection
 };
 using VecOps = VecOpsT<double>;
 

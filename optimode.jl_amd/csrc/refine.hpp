@@ -6,7 +6,7 @@
 
 namespace omx {
 
-constexpr int RF_MAXC = 17;                 // block columns (<= 16) + one correction
+constexpr int RF_MAXC = 19;                 // block columns (<= 18) + one correction
 constexpr int RF_PAIRS = RF_MAXC * RF_MAXC;
 
 // Columns of instance i: block columns c < n1[i] at blk + i*istride + c*ld, then (when

@@ -1564,7 +1564,8 @@ bool dense_geig(int n, const c64* Gp, const c64* Bp, std::vector<double>& lam, s
 // band's Ritz value is the bands[i]-th of the block, as LOBPCG's locking order gives it.
 int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, const std::vector<int>& bands,
                  const std::vector<int>& msize, const std::vector<double>& tols, int max_steps, SolveStats& stats,
-                 int& newton_total, double& max_resid, std::vector<double>* resid_inst = nullptr) {
+                 int& newton_total, double& max_resid, std::vector<double>* resid_inst = nullptr,
+                 bool loose_blocks = false) {
   const int ninst = b.ninst;
   const long K = S.K, ld = S.ld, istride = b.istride;
   hipStream_t s = S.stream;
@@ -1612,7 +1613,7 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
   const OpPlan<double>& plan = S.p64.plan;
   std::vector<int> n1h(ninst, 0), jdh(ninst, 0);
   std::vector<double> lam_band(ninst, 0.0), rn(ninst, 0.0);
-  std::vector<double> theta(size_t(ninst) * RF_MAXC, 0.0), schur(size_t(ninst) * 16, 0.0);  // block Ritz values
+  std::vector<double> theta(size_t(ninst) * RF_MAXC, 0.0), schur(size_t(ninst) * VecOpsT<float>::QMAX, 0.0);
   std::vector<c64> hG(size_t(ninst) * RF_PAIRS), hB(size_t(ninst) * RF_PAIRS), hC(size_t(ninst) * RF_PAIRS);
   auto up_n1 = [&](const std::vector<int>& v) {
     OMX_HIP_CHECK(hipMemcpyAsync(n1d.as<void>(), v.data(), sizeof(int) * ninst, hipMemcpyHostToDevice, s));
@@ -1737,27 +1738,31 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
           OMX_HIP_CHECK(hipMemcpyAsync(W.nqd.as<void>(), msize.data(), sizeof(int) * ninst, hipMemcpyHostToDevice, s));
           const int mmax = *std::max_element(msize.begin(), msize.end());
           V32.set_block(W.Xf.as<cf>(), qis, W.nqd.as<int>(), mmax);
-          // The block's other vectors are Ritz vectors, not eigenvectors (their residuals at
-          // this band's k can be several percent of w^2 after the shared-subspace phase):
-          // the exact system on the block's complement takes them into account.  Ritz values
-          // within 1e-3 of the band's stay out (their own residuals are small: bands that
-          // close converged at nearly the same k).
-          W.Rf.ensure(sizeof(cf) * size_t(ninst) * qis);
-          W.rgd.ensure(sizeof(double) * schur.size());
-          W.thd.ensure(sizeof(double) * theta.size());
-          for (int i = 0; i < ninst; ++i)
-            for (int l = 0; l < 16; ++l) {
-              const double d = l < msize[i] ? theta[size_t(i) * RF_MAXC + l] - lam_band[i] : 0.0;
-              schur[size_t(i) * 16 + l] =
-                  l != bands[i] && std::fabs(d) > 1e-3 * std::fabs(lam_band[i]) ? 1.0 / d : 0.0;
-            }
-          OMX_HIP_CHECK(hipMemcpyAsync(W.rgd.as<void>(), schur.data(), sizeof(double) * schur.size(),
-                                       hipMemcpyHostToDevice, s));
-          OMX_HIP_CHECK(hipMemcpyAsync(W.thd.as<void>(), theta.data(), sizeof(double) * theta.size(),
-                                       hipMemcpyHostToDevice, s));
-          launch_block_resid(b.p(b.X[b.cur]), b.p(b.AX[b.cur]), ld, istride, W.thd.as<double>(), W.nqd.as<int>(), mmax,
-                             ninst, K, W.Rf.as<cf>(), s);
-          V32.set_schur(W.Rf.as<cf>(), W.rgd.as<double>());
+          // The block's other vectors are Ritz vectors, not eigenvectors (loose_blocks: their
+          // residuals at this band's k can be several percent of w^2 after the shared-subspace
+          // phase): the exact system on the block's complement takes them into account.  After
+          // the per-band form, which locks every column, the extra term changes no iteration
+          // count and costs 2% (128x96x24, 4 bands: 37.7 against 36.3 ms).  Ritz values within
+          // 1e-3 of the band's stay out (their own residuals are small: bands that close
+          // converged at nearly the same k).
+          if (loose_blocks) {
+            W.Rf.ensure(sizeof(cf) * size_t(ninst) * qis);
+            W.rgd.ensure(sizeof(double) * schur.size());
+            W.thd.ensure(sizeof(double) * theta.size());
+            for (int i = 0; i < ninst; ++i)
+              for (int l = 0; l < VecOpsT<float>::QMAX; ++l) {
+                const double d = l < msize[i] ? theta[size_t(i) * RF_MAXC + l] - lam_band[i] : 0.0;
+                schur[size_t(i) * VecOpsT<float>::QMAX + l] =
+                    l != bands[i] && std::fabs(d) > 1e-3 * std::fabs(lam_band[i]) ? 1.0 / d : 0.0;
+              }
+            OMX_HIP_CHECK(hipMemcpyAsync(W.rgd.as<void>(), schur.data(), sizeof(double) * schur.size(),
+                                         hipMemcpyHostToDevice, s));
+            OMX_HIP_CHECK(hipMemcpyAsync(W.thd.as<void>(), theta.data(), sizeof(double) * theta.size(),
+                                         hipMemcpyHostToDevice, s));
+            launch_block_resid(b.p(b.X[b.cur]), b.p(b.AX[b.cur]), ld, istride, W.thd.as<double>(), W.nqd.as<int>(), mmax,
+                               ninst, K, W.Rf.as<cf>(), s);
+            V32.set_schur(W.Rf.as<cf>(), W.rgd.as<double>());
+          }
         }
         its = minres_complement_t<float>(S, V32, lam_band, b.kd.as<double>(), W.RBf.as<cf>(), W.Tf.as<cf>(), jdh,
                                          S.opt.jd_rtol, S.opt.jd_maxit, false);
@@ -1936,6 +1941,7 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
   const auto b64p = workspace<double>(*this, ninst, M64, maxit64);
   Batch<double>& b64 = *b64p;
   int newton_total = 0, mk_moves = 0;  // mk_moves: Newton steps inside the shared-subspace phase
+  bool mk_done = false;                // the shared-subspace phase made the blocks
   const int nguess_used = (Hguess && nguess > 0) ? std::min(nguess, M) : 0;
   const int ghw = opt.guess_lowres;
   if (nguess_used && ghw > 0 && (nz > 1 || ghw % 2 != 0 || ghw > nx || ghw > ny))
@@ -2068,6 +2074,7 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
                       b64.istride, kk, its, moves, stats))
       return false;
     msize = msize_mk;
+    mk_done = true;
     mk_moves = moves[0];
     for (int i = 0; i < ninst; ++i) {
       hns[i].k = kk[i];
@@ -2207,7 +2214,7 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
     const int left = std::max(1, max_eigsolves - newton_total);
     if (opt.refine && !opt.fp64_only)
       stats.it64 += refine_phase(*this, b64, hns, bands, msize, std::vector<double>(size_t(ninst), eig_tol), left,
-                                 stats, newton_total, max_resid);
+                                 stats, newton_total, max_resid, nullptr, mk_done);
     else
       stats.it64 +=
           newton_phase(*this, b64, hns, bands, nchk, msize, eig_tol, maxit64, left, stats, newton_total, true);
@@ -2442,6 +2449,7 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
   };
 
   // the FP32 phase of every problem in its own shared search space (multik.hip)
+  bool mk_done = false;
   auto multik_phase = [&]() {
     if (!use_multik) return false;
     std::vector<MkProblem> mk(P);
@@ -2462,6 +2470,7 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
                       b64.p(b64.X[0]), ld, b64.istride, kk, its, moves, stats))
       return false;
     msize = msize_mk;
+    mk_done = true;
     for (int i = 0; i < ninst; ++i) {
       hns[i].k = kk[i];
       hns[i].nsolves = 1;
@@ -2501,7 +2510,8 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
   std::vector<double> resid(ninst, 0.0);
   const int left = std::max(1, max_eigsolves - newton_total);
   if (opt.refine && !opt.fp64_only)
-    stats.it64 += refine_phase(*this, b64, hns, bands, msize, eig_tol, left, stats, newton_total, max_resid, &resid);
+    stats.it64 += refine_phase(*this, b64, hns, bands, msize, eig_tol, left, stats, newton_total, max_resid, &resid,
+                               mk_done);
   else
     stats.it64 += newton_phase(*this, b64, hns, bands, nchk, msize, eig_tol, maxit64, left, stats, newton_total, true);
   // band eigenvectors of every instance, phase-canonicalised together (fields.jl:258-260)
