@@ -34,6 +34,7 @@ namespace omx {
 namespace {
 
 constexpr int PLANES = 7;
+constexpr double MK_CLUSTER = 3e-5;  // bands whose k agree to this take their vectors at one k
 constexpr int FT = 512;   // threads of the transform kernels
 constexpr int NGRAM = 3 + MK_NODES + 1;  // G00, G01, G11, the nodes, the k-independent part
 
@@ -47,6 +48,7 @@ struct MkState {
   int its[MK_MAXM];        // iteration a band first met its thresholds (0: not yet)
   double omega2, tol, ftol;
   double k[MK_MAXM];       // current k per column
+  double kold[MK_MAXM];    // k per column in the last iteration made
   double keval[MK_MAXM];   // k the column's Ritz pair was taken at
   double knew[MK_MAXM];    // after the Newton step
   double lam[MK_MAXM], slope[MK_MAXM], rnorm[MK_MAXM];
@@ -75,16 +77,15 @@ __device__ __forceinline__ int space_slot(const MkGeo& g, const MkState& s, int 
   return slot_p(g, b, s.pslot[q - s.m - s.na]);
 }
 
-// Chebyshev nodes over the columns' k range (widened to 2% where it is narrower)
-__device__ __forceinline__ void mk_nodes(const MkState& s, double* node) {
-  double lo = s.k[0], hi = s.k[0];
-  for (int j = 1; j < s.m; ++j) {
-    lo = fmin(lo, s.k[j]);
-    hi = fmax(hi, s.k[j]);
+// Chebyshev node t over the columns' k range (widened to 2% where it is narrower)
+__device__ __forceinline__ double mk_node(const double* k, int m, int t) {
+  double lo = k[0], hi = k[0];
+  for (int j = 1; j < m; ++j) {
+    lo = fmin(lo, k[j]);
+    hi = fmax(hi, k[j]);
   }
   const double c = 0.5 * (lo + hi), h = fmax(0.5 * (hi - lo), 0.01 * fabs(c));
-#pragma unroll
-  for (int t = 0; t < MK_NODES; ++t) node[t] = c + h * cospi((t + 0.5) / MK_NODES);
+  return c + h * cospi((t + 0.5) / MK_NODES);
 }
 
 // in-plane part of a plane wave: n = z x w / rho (y at rho = 0)
@@ -146,13 +147,14 @@ __global__ __launch_bounds__(256) void k_mk_start(MkGeo geo, c32* cols, const Mk
 // ---------------------------------------------------------------------------------------
 // Gram matrices on the matrix cores.  As in block.hip: the four k slots of one
 // v_mfma_f32_16x16x4 are four rows, lane (i = l % 16, g = l / 16) holds S consecutive rows of
-// column i of each 16-column tile, loaded straight from HBM with 16-byte loads, and the four
+// column i of each 16-column tile, loaded straight from HBM with 16-byte loads, and the
 // waves of a block take interleaved stages.  KIND 0: F0^H e F0, 1: F0^H e F1, 2: F1^H e F1
 // (e = eps^-1 per pixel, three components contracted per row), 3: the norm's matrices
 // g^H psi g for NB of the nodes (psi = 1 / (rho^2 + kappa^2) on g1; the last one g2^H g2).
 // Hermitian kinds compute the tiles on and above the diagonal only.
 // ---------------------------------------------------------------------------------------
 typedef float fx4 __attribute__((ext_vector_type(4)));
+constexpr int GW = 8;  // waves per Gram block
 
 __device__ __forceinline__ fx4 mfma(float a, float b, fx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -174,25 +176,10 @@ template <int S> __device__ __forceinline__ void load_col(const c32* col, long r
 }
 
 template <int NT, int KIND, int NB, int S>
-__global__ __launch_bounds__(256) void k_mk_gram(MkGeo geo, const c32* cols, const MkState* st, int buf, long rpc,
-                                                 c32* part) {
+__device__ __forceinline__ void gram_body(const MkGeo& geo, const c32* const* cp, const float* kap2,
+                                          float (*red)[8][64], int p, int q0, int nt, long rpc, c32* part) {
   constexpr int PM = 16 * NT, NQ = KIND == 3 ? NB : 1;
-  __shared__ const c32* cp[PM];
-  __shared__ float kap2[MK_NODES];
-  __shared__ float red[4][8][64];
-  const int p = blockIdx.y, chunk = blockIdx.x, q0 = KIND == 3 ? blockIdx.z * NB : 0;
-  const MkState& s = st[p];
-  if (s.done) return;
-  const int n = s.m + s.na + s.np;
-  if (threadIdx.x < PM)
-    cp[threadIdx.x] =
-        int(threadIdx.x) < n ? cols + p * geo.slots + col_off(geo, space_slot(geo, s, buf, threadIdx.x)) : nullptr;
-  if (KIND == 3 && threadIdx.x == 0) {
-    double node[MK_NODES];
-    mk_nodes(s, node);
-    for (int t = 0; t < MK_NODES; ++t) kap2[t] = float(node[t] * node[t]);
-  }
-  __syncthreads();
+  const int chunk = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, g = lane >> 4;
   const c32* col[NT];
 #pragma unroll
@@ -212,7 +199,7 @@ __global__ __launch_bounds__(256) void k_mk_gram(MkGeo geo, const c32* cols, con
       for (int a = 0; a < NT; ++a)
 #pragma unroll
         for (int b = 0; b < NT; ++b) {
-          if (KIND != 1 && a > b) continue;
+          if ((KIND != 1 && a > b) || a >= nt || b >= nt) continue;
           ar[q][a][b] = mfma(x[a][r].x, y[b][r].x, ar[q][a][b]);
           ai[q][a][b] = mfma(x[a][r].x, y[b][r].y, ai[q][a][b]);
           ar[q][a][b] = mfma(x[a][r].y, y[b][r].y, ar[q][a][b]);
@@ -221,7 +208,7 @@ __global__ __launch_bounds__(256) void k_mk_gram(MkGeo geo, const c32* cols, con
   };
   const long r0 = chunk * rpc, r1 = r0 + rpc < geo.N ? r0 + rpc : geo.N;
   const float* eps = geo.eps6c + p * geo.eps_stride;
-  for (long row = r0 + (wave * 4 + g) * S; row - g * S < r1; row += 16 * S) {
+  for (long row = r0 + (wave * 4 + g) * S; row - g * S < r1; row += 4 * GW * S) {
     const bool in = row < r1;  // rows past r1 belong to the next chunk (or are pads)
     const c32* no = nullptr;
     if (KIND < 3) {
@@ -323,7 +310,7 @@ __global__ __launch_bounds__(256) void k_mk_gram(MkGeo geo, const c32* cols, con
     for (int a = 0; a < NT; ++a)
 #pragma unroll
       for (int b = 0; b < NT; ++b) {
-        if (KIND != 1 && a > b) continue;
+        if ((KIND != 1 && a > b) || a >= nt || b >= nt) continue;
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -331,13 +318,49 @@ __global__ __launch_bounds__(256) void k_mk_gram(MkGeo geo, const c32* cols, con
           red[wave][4 + r][lane] = ai[q][a][b][r];
         }
         __syncthreads();
-        // wave w finishes accumulator register w: rows 4 g + w
-        const float sr = (red[0][wave][lane] + red[1][wave][lane]) + (red[2][wave][lane] + red[3][wave][lane]);
-        const float si = (red[0][4 + wave][lane] + red[1][4 + wave][lane]) +
-                         (red[2][4 + wave][lane] + red[3][4 + wave][lane]);
-        out[(a * 16 + 4 * g + wave) * PM + b * 16 + i16] = c32{sr, si};
+        // wave w < 4 finishes accumulator register w: rows 4 g + w
+        if (wave < 4) {
+          float sr = 0.f, si = 0.f;
+#pragma unroll
+          for (int u = 0; u < GW; ++u) {
+            sr += red[u][wave][lane];
+            si += red[u][4 + wave][lane];
+          }
+          out[(a * 16 + 4 * g + wave) * PM + b * 16 + i16] = c32{sr, si};
+        }
       }
   }
+}
+
+// One launch: blockIdx.z 0-2 the three eps^-1 kinds, then the node groups.  Eight waves per
+// block: 128 chunks of four waves in a launch per kind left half the SIMDs without a wave
+// (256^2, 30 columns: 155 us in four launches).
+template <int NT, int NB, int S>
+__global__ __launch_bounds__(64 * GW) void k_mk_gram(MkGeo geo, const c32* cols, const MkState* st, int buf, long rpc,
+                                                     c32* part) {
+  __shared__ const c32* cp[16 * NT];
+  __shared__ float kap2[MK_NODES];
+  __shared__ float red[GW][8][64];
+  const int p = blockIdx.y, kind = blockIdx.z;
+  const MkState& s = st[p];
+  if (s.done) return;
+  const int n = s.m + s.na + s.np, nt = (n + 15) / 16;
+  if (threadIdx.x < 16 * NT)
+    cp[threadIdx.x] =
+        int(threadIdx.x) < n ? cols + p * geo.slots + col_off(geo, space_slot(geo, s, buf, threadIdx.x)) : nullptr;
+  if (threadIdx.x < MK_NODES) {
+    const double node = mk_node(s.k, s.m, threadIdx.x);
+    kap2[threadIdx.x] = float(node * node);
+  }
+  __syncthreads();
+  if (kind == 0)
+    gram_body<NT, 0, 1, S>(geo, cp, kap2, red, p, 0, nt, rpc, part);
+  else if (kind == 1)
+    gram_body<NT, 1, 1, S>(geo, cp, kap2, red, p, 0, nt, rpc, part);
+  else if (kind == 2)
+    gram_body<NT, 2, 1, S>(geo, cp, kap2, red, p, 0, nt, rpc, part);
+  else
+    gram_body<NT, 3, NB, S>(geo, cp, kap2, red, p, (kind - 3) * NB, nt, rpc, part);
 }
 
 // red[p][gram][e] = sum over the chunks, FP64, fixed order (16 elements x 16 chunk groups)
@@ -376,35 +399,55 @@ __global__ __launch_bounds__(256) void k_mk_reduce(const c32* part, int nchunk, 
 // ---------------------------------------------------------------------------------------
 // Dense step: one workgroup per band.
 // ---------------------------------------------------------------------------------------
-constexpr int DT = 512;
+constexpr int MK_SWEEPS = 10;  // Jacobi sweeps whose rotations are kept (4 to 7 are made)
 
-__device__ __forceinline__ c64 operator_conj_mul(c64 a, c64 b) {  // conj(a) b
-  return c64{a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x};
+struct MkRot {
+  double c;
+  c64 s;
+};
+
+__device__ __forceinline__ void mk_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// 1 / sqrt(x) for x in FP32's range: the FP32 estimate and two Newton steps (about 1e-15)
+__device__ __forceinline__ double rsqrt_fast(double x) {
+  double r = double(__builtin_amdgcn_rsqf(float(x)));
+  const double h = 0.5 * x;
+  r = r * (1.5 - h * r * r);
+  r = r * (1.5 - h * r * r);
+  return r;
+}
+
+// a value of lane l + 1 (UP false) or l - 1 (UP true) of the wavefront, lanes past the ends 0
+template <bool UP> __device__ __forceinline__ double lane_shift(double v) {
+  union {
+    double d;
+    int i[2];
+  } u{v};
+  u.i[0] = __builtin_amdgcn_update_dpp(0, u.i[0], UP ? 0x138 : 0x130, 0xf, 0xf, true);
+  u.i[1] = __builtin_amdgcn_update_dpp(0, u.i[1], UP ? 0x138 : 0x130, 0xf, 0xf, true);
+  return u.d;
 }
 
 // Parallel cyclic Jacobi (dense.hip's round-robin ordering and rotations) for Hermitian A
 // (n x n, leading dimension ld) using A's symmetry: of the 2 x 2 blocks only those on and above
 // the diagonal are computed and their mirrors stored.  Stops after a sweep whose rotations
-// all have |sin| <= stop.  Returns the buffer holding the final matrix; V the eigenvectors.
-__device__ __forceinline__ void mk_pair(int t, int r, int m, int& p, int& q) {
-  const int ia = (t == 0) ? 0 : 1 + (t - 1 + r) % (m - 1);
-  const int ib = 1 + (m - 2 - t + r) % (m - 1);
-  p = ia < ib ? ia : ib;
-  q = ia < ib ? ib : ia;
-}
-
-__device__ c64* mk_jacobi(c64* A0, c64* A1, c64* V, int ld, int n, double stop) {
+// all have |sin| <= stop.  The eigenvectors are not accumulated (two thirds of a round's
+// arithmetic): the rotations of round q go to rot[q npair + t], and a caller applies them in
+// reverse to the few unit vectors it wants.  Returns the rounds made; A0 / A1 by parity hold
+// the final matrix (rounds even: A0).
+__device__ int mk_jacobi(c64* A0, c64* A1, int ld, int n, double stop, MkRot* rot) {
   __shared__ int big[3];
   __shared__ int rp[MK_MAXN / 2], rq[MK_MAXN / 2];
   __shared__ double rc[MK_MAXN / 2];
   __shared__ c64 rs[MK_MAXN / 2];
   __shared__ unsigned short tri[(MK_MAXN / 2) * (MK_MAXN / 2 + 1) / 2];
   const int m = n + (n & 1), npair = m / 2, nblk = npair * (npair + 1) / 2;
-  for (int e = threadIdx.x; e < m * m; e += blockDim.x) {
-    const int i = e / m, j = e - i * m;
-    V[i * ld + j] = c64{i == j ? 1.0 : 0.0, 0.0};
-    if (i == n || j == n) A0[i * ld + j] = c64{0.0, 0.0};
-  }
+  if (n & 1)  // an odd size is padded by a zero row and column, which never rotate
+    for (int e = threadIdx.x; e < m; e += blockDim.x) A0[n * ld + e] = A0[e * ld + n] = c64{0.0, 0.0};
   for (int e = threadIdx.x; e < npair * npair; e += blockDim.x) {
     const int a = e / npair, b = e - a * npair;
     if (a <= b) tri[a * npair - a * (a - 1) / 2 + (b - a)] = (unsigned short)(a * 64 + b);
@@ -412,78 +455,270 @@ __device__ c64* mk_jacobi(c64* A0, c64* A1, c64* V, int ld, int n, double stop) 
   if (threadIdx.x < 3) big[threadIdx.x] = 0;
   __syncthreads();
   c64 *Ac = A0, *An = A1;
-  const int nitem = nblk + m * npair;
-  for (int sweep = 0; sweep < 30; ++sweep) {
+  int rounds = 0, ua = (int(threadIdx.x) + m - 2) % (m - 1), ub = max(0, m - 2 - int(threadIdx.x));  // (t - 1), (m - 2 - t)
+  for (int sweep = 0; sweep < MK_SWEEPS; ++sweep) {
     const int sl = sweep % 3;
     if (threadIdx.x == 0) big[(sweep + 1) % 3] = 0;
     for (int r = 0; r < m - 1; ++r) {
-      if (threadIdx.x < npair) {
-        int p, q;
-        mk_pair(threadIdx.x, r, m, p, q);
+      if (int(threadIdx.x) < npair) {
+        const int t = threadIdx.x;
+        const int ia = t == 0 ? 0 : 1 + ua, ib = 1 + ub;
+        ua = ua + 1 == m - 1 ? 0 : ua + 1;
+        ub = ub + 1 == m - 1 ? 0 : ub + 1;
+        const bool fwd = ia < ib;
+        const int p = fwd ? ia : ib, q = fwd ? ib : ia;
         const double app = Ac[p * ld + p].x, aqq = Ac[q * ld + q].x;
         const c64 apq = Ac[p * ld + q];
         const double a2 = apq.x * apq.x + apq.y * apq.y;
         double c = 1.0;
         c64 sv{0.0, 0.0};
-        if (a2 > 1e-300 && a2 > 1e-32 * fabs(app * aqq)) {
-          const double ia = rsqrt(a2), z = 0.5 * (aqq - app) * ia, az = fabs(z);
-          double sn;
-          if (az > 1e150) {
-            sn = 0.5 / az;
-          } else {
-            const double h = rsqrt(1.0 + z * z), x = 0.5 * (1.0 + az * h), rx = rsqrt(x);
-            c = x * rx;
-            sn = 0.5 * h * rx;
-          }
-          const double f = (z >= 0 ? sn : -sn) * ia;
+        // The angle is taken to FP32 accuracy (what is left of A_pq falls by 1e-7, a sweep's
+        // other fill is larger), the rotation itself is unitary to FP64: three FP64 square
+        // roots in a chain were half of a round's latency.
+        if (a2 > 1e-30) {
+          const double ia2 = rsqrt_fast(a2), z = 0.5 * (aqq - app) * ia2;
+          const float az = fabsf(float(z));
+          const float tf = az > 1e15f ? 0.f : 1.f / (az + sqrtf(1.f + az * az));
+          c = rsqrt_fast(1.0 + double(tf) * tf);
+          const double sn = double(tf) * c, f = (z >= 0 ? sn : -sn) * ia2;
           sv = c64{f * apq.x, f * apq.y};
           if (sn > stop) big[sl] = 1;
         }
-        rp[threadIdx.x] = p;
-        rq[threadIdx.x] = q;
-        rc[threadIdx.x] = c;
-        rs[threadIdx.x] = sv;
+        rp[t] = p;
+        rq[t] = q;
+        rc[t] = c;
+        rs[t] = sv;
+        // kept relative to (ia, ib), the order the reverse pass meets the pair in
+        rot[long(rounds) * npair + t] = MkRot{c, fwd ? sv : c64{-sv.x, sv.y}};
       }
       __syncthreads();
-      for (int idx = threadIdx.x; idx < nitem; idx += blockDim.x) {
-        if (idx < nblk) {
-          const int t1 = tri[idx] >> 6, t2 = tri[idx] & 63;
-          const int p1 = rp[t1], q1 = rq[t1], p2 = rp[t2], q2 = rq[t2];
-          const double c1 = rc[t1], c2 = rc[t2];
-          const c64 s1 = rs[t1], s2 = rs[t2];
-          const c64 x00 = Ac[p1 * ld + p2], x01 = Ac[p1 * ld + q2], x10 = Ac[q1 * ld + p2], x11 = Ac[q1 * ld + q2];
-          const c64 y00 = x00 * c1 - s1 * x10, y01 = x01 * c1 - s1 * x11;
-          const c64 y10 = operator_conj_mul(s1, x00) + x10 * c1, y11 = operator_conj_mul(s1, x01) + x11 * c1;
-          const c64 z00 = y00 * c2 - operator_conj_mul(s2, y01), z01 = s2 * y00 + y01 * c2;
-          const c64 z10 = y10 * c2 - operator_conj_mul(s2, y11), z11 = s2 * y10 + y11 * c2;
-          An[p1 * ld + p2] = z00;
-          An[p1 * ld + q2] = z01;
-          An[q1 * ld + p2] = z10;
-          An[q1 * ld + q2] = z11;
-          if (t1 != t2) {
-            An[p2 * ld + p1] = conj(z00);
-            An[q2 * ld + p1] = conj(z01);
-            An[p2 * ld + q1] = conj(z10);
-            An[q2 * ld + q1] = conj(z11);
-          }
-        } else {
-          const int e = idx - nblk, j = e / npair, t = e - j * npair;
-          const int p = rp[t], q = rq[t];
-          const double c = rc[t];
-          const c64 sv = rs[t];
-          const c64 vp = V[j * ld + p], vq = V[j * ld + q];
-          V[j * ld + p] = vp * c - operator_conj_mul(sv, vq);
-          V[j * ld + q] = sv * vp + vq * c;
+      for (int idx = threadIdx.x; idx < nblk; idx += blockDim.x) {
+        const int t1 = tri[idx] >> 6, t2 = tri[idx] & 63;
+        const int p1 = rp[t1], q1 = rq[t1], p2 = rp[t2], q2 = rq[t2];
+        const double c1 = rc[t1], c2 = rc[t2];
+        const c64 s1 = rs[t1], s2 = rs[t2];
+        const c64 x00 = Ac[p1 * ld + p2], x01 = Ac[p1 * ld + q2], x10 = Ac[q1 * ld + p2], x11 = Ac[q1 * ld + q2];
+        const c64 y00 = x00 * c1 - s1 * x10, y01 = x01 * c1 - s1 * x11;
+        const c64 y10 = cmulc(s1, x00) + x10 * c1, y11 = cmulc(s1, x01) + x11 * c1;
+        const c64 z00 = y00 * c2 - cmulc(s2, y01), z01 = s2 * y00 + y01 * c2;
+        const c64 z10 = y10 * c2 - cmulc(s2, y11), z11 = s2 * y10 + y11 * c2;
+        An[p1 * ld + p2] = z00;
+        An[p1 * ld + q2] = z01;
+        An[q1 * ld + p2] = z10;
+        An[q1 * ld + q2] = z11;
+        if (t1 != t2) {
+          An[p2 * ld + p1] = conj(z00);
+          An[q2 * ld + p1] = conj(z01);
+          An[p2 * ld + q1] = conj(z10);
+          An[q2 * ld + q1] = conj(z11);
         }
       }
       __syncthreads();
       c64* tmp = Ac;
       Ac = An;
       An = tmp;
+      ++rounds;
     }
     if (big[sl] == 0) break;
   }
-  return Ac;
+  return rounds;
+}
+
+__device__ __forceinline__ double read_lane(double v, int l) {  // l uniform
+  union {
+    double d;
+    int i[2];
+  } u{v};
+  u.i[0] = __builtin_amdgcn_readlane(u.i[0], l);
+  u.i[1] = __builtin_amdgcn_readlane(u.i[1], l);
+  return u.d;
+}
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+// 1 / x for normal x (estimate and two Newton steps)
+__device__ __forceinline__ double rcp_fast(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = r * (2.0 - x * r);
+  return r * (2.0 - x * r);
+}
+
+// c = D U^-1 v for a wavefront's vector (lane a holds entry a); dropped columns get 0
+__device__ __forceinline__ c64 mk_backsub(c64 v, const c64* U, int ld, int n, const int* drop, const double* dsc,
+                                          int lane) {
+  for (int a = n - 1; a >= 0; --a) {
+    const double ua = drop[a] ? 0.0 : rcp_fast(U[a * ld + a].x);
+    const c64 ca{read_lane(v.x, a) * ua, read_lane(v.y, a) * ua};
+    if (lane == a) v = ca;
+    if (lane < a) v = v - U[lane * ld + a] * ca;
+  }
+  return lane < n ? v * dsc[lane] : c64{0.0, 0.0};
+}
+
+// Eigenpair j (0-based, ascending) of Hermitian A (n x n, all in LDS, destroyed): Householder
+// tridiagonalisation with the congruence's layout (lane = column, rows dealt to the
+// wavefronts; two barriers per step), then on the first wavefront multisection for the
+// eigenvalue (64 Sturm counts per pass), the eigenvector of the tridiagonal matrix by its
+// twisted factorisation, and the reflectors back.  Returns false, leaving the pair to the
+// Jacobi, when another eigenvalue lies within 1e-4 of it: vectors of a cluster have to come
+// from one decomposition.  lam and c = D U^-1 vector (into out) for every wavefront's use after
+// the next barrier.  A full Jacobi (5 to 8 sweeps of n - 1 rounds at 0.8 us) finds n pairs
+// where a band takes one.
+template <int NW>
+__device__ bool tridiag_pair(c64* A, int ld, int n, int j, c64 (*pr)[64], c64* part, double* lam, c64* out,
+                             const c64* U, const int* drop, const double* dsc) {
+  __shared__ double d[MK_MAXN], e[MK_MAXN], e2[MK_MAXN], dp[MK_MAXN], dm[MK_MAXN];
+  __shared__ c64 tau[MK_MAXN];
+  __shared__ int single;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const c64 zero{0.0, 0.0};
+  if (wv == 0) pr[0][lane] = lane < n ? A[lane] : zero;
+  __syncthreads();
+  for (int k = 0; k < n; ++k) {
+    const c64 rowk = pr[k & 1][lane];
+    if (k == n - 1) {
+      if (threadIdx.x == 0) d[k] = pr[k & 1][k].x;
+      break;
+    }
+    const c64 x = lane > k && lane < n ? conj(rowk) : zero;  // column k below the diagonal
+    const double sg = wave_sum(lane > k + 1 ? abs2(x) : 0.0);
+    const double ar = read_lane(x.x, k + 1), ai = read_lane(x.y, k + 1);
+    c64 t = zero, v = lane == k + 1 ? c64{1.0, 0.0} : zero;
+    double ek = ar;
+    if (sg > 0.0 || ai != 0.0) {
+      const double nrm = sqrt(ar * ar + ai * ai + sg);
+      ek = ar >= 0 ? -nrm : nrm;
+      const double ib = 1.0 / ek, dr = ar - ek, q = 1.0 / (dr * dr + ai * ai);
+      t = c64{(ek - ar) * ib, -ai * ib};
+      if (lane > k + 1) v = x * c64{dr * q, -ai * q};
+    }
+    // p = tau A v from the owned rows (A[a][b] v_b = conj(A[b][a]) v_b)
+    c64 acc = zero;
+    for (int b = wv; b < n; b += NW) {
+      if (b <= k) continue;
+      const c64 vb{read_lane(v.x, b), read_lane(v.y, b)};
+      if (lane > k && lane < n) acc = acc + cmulc(A[b * ld + lane], vb);
+    }
+    part[wv * 64 + lane] = acc;
+    if (wv == k % NW) {
+      if (lane < n) A[k * ld + lane] = v;  // the reflector, for the way back
+      if (lane == 0) {
+        d[k] = pr[k & 1][k].x;
+        e[k] = ek;
+        e2[k] = ek * ek;
+        tau[k] = t;
+      }
+    }
+    __syncthreads();
+    c64 pv = zero;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) pv = pv + part[q * 64 + lane];
+    pv = t * pv;
+    const c64 pd = cmulc(pv, v);  // p^H v
+    const c64 al = t * c64{-0.5 * wave_sum(pd.x), -0.5 * wave_sum(pd.y)};
+    const c64 w = pv + al * v;
+    for (int a = wv; a < n; a += NW) {
+      if (a <= k) continue;
+      const c64 va{read_lane(v.x, a), read_lane(v.y, a)}, wa{read_lane(w.x, a), read_lane(w.y, a)};
+      if (lane > k && lane < n) {
+        // v_a conj(w) + w_a conj(v)
+        c64 u = A[a * ld + lane] - cmulc(w, va) - cmulc(v, wa);
+        if (lane == a) u.y = 0.0;
+        A[a * ld + lane] = u;
+        if (a == k + 1) pr[(k + 1) & 1][lane] = u;
+      }
+    }
+    __syncthreads();
+  }
+  __syncthreads();
+  if (wv == 0) {
+    const double di = lane < n ? d[lane] : 0.0;
+    const double rad = (lane < n && lane > 0 ? fabs(e[lane - 1]) : 0.0) + (lane < n - 1 ? fabs(e[lane]) : 0.0);
+    double lo = lane < n ? di - rad : 1e300, hi = lane < n ? di + rad : -1e300;
+    for (int off = 32; off > 0; off >>= 1) {
+      lo = fmin(lo, __shfl_xor(lo, off, 64));
+      hi = fmax(hi, __shfl_xor(hi, off, 64));
+    }
+    const double scale = fmax(fabs(lo), fabs(hi)), tiny = 1e-30 * scale + 1e-300;
+    lo -= 1e-12 * scale;
+    hi += 1e-12 * scale;
+    auto count = [&](double sig) {  // eigenvalues below sig
+      double q = d[0] - sig;
+      int c = q < 0;
+      for (int i = 1; i < n; ++i) {
+        if (fabs(q) < tiny) q = -tiny;
+        q = (d[i] - sig) - e2[i - 1] * rcp_fast(q);
+        c += q < 0;
+      }
+      return c;
+    };
+    for (int pass = 0; pass < 10 && hi - lo > 1e-13 * scale; ++pass) {
+      const double sig = lo + (hi - lo) * ((lane + 1) * (1.0 / 65.0));
+      const unsigned long long above = __ballot(count(sig) > j);
+      const int f = above ? __ffsll((long long)above) - 1 : 64;
+      const double nh = f < 64 ? __shfl(sig, f & 63, 64) : hi, nl = f > 0 ? __shfl(sig, (f - 1) & 63, 64) : lo;
+      hi = nh;
+      lo = nl;
+    }
+    const double l = 0.5 * (lo + hi), del = fmax(1e-4 * fabs(l), 1e-9 * scale);
+    const int cc = count(lane == 0 ? l - del : l + del);
+    const bool one = __shfl(cc, 1, 64) - __shfl(cc, 0, 64) == 1;
+    if (lane == 0) {
+      single = one ? 1 : 0;
+      *lam = l;
+    }
+    if (one) {
+      // LDL^H from the top (lane 0) and UDU^H from the bottom (lane 1), met at the index where
+      // the twisted pivot is smallest
+      if (lane < 2) {
+        double q = 0;
+        for (int i = 0; i < n; ++i) {
+          const int r = lane == 0 ? i : n - 1 - i;
+          q = (d[r] - l) - (i > 0 ? e2[lane == 0 ? r - 1 : r] * rcp_fast(q) : 0.0);
+          if (fabs(q) < tiny) q = q < 0 ? -tiny : tiny;
+          (lane == 0 ? dp : dm)[r] = q;
+        }
+      }
+      mk_wave_sync();
+      double g = lane < n ? fabs(dp[lane] + dm[lane] - (di - l)) : 1e300;
+      int r = lane;
+      for (int off = 32; off > 0; off >>= 1) {
+        const double og = __shfl_xor(g, off, 64);
+        const int orr = __shfl_xor(r, off, 64);
+        if (og < g || (og == g && orr < r)) {
+          g = og;
+          r = orr;
+        }
+      }
+      const double up = lane < n - 1 ? -e[lane] * rcp_fast(dp[lane]) : 0.0;
+      const double dn = lane > 0 && lane < n ? -e[lane - 1] * rcp_fast(dm[lane]) : 0.0;
+      // z_i = up_i z_{i+1} above the twist, dn_i z_{i-1} below it
+      double z = lane == r ? 1.0 : 0.0, zc = 1.0;
+      for (int i = r - 1; i >= 0; --i) {
+        zc *= read_lane(up, i);
+        if (lane == i) z = zc;
+      }
+      zc = 1.0;
+      for (int i = r + 1; i < n; ++i) {
+        zc *= read_lane(dn, i);
+        if (lane == i) z = zc;
+      }
+      const double iz = 1.0 / sqrt(wave_sum(z * z));
+      c64 yv{z * iz, 0.0};
+      for (int k = n - 2; k >= 0; --k) {  // reflectors: y -= tau v (v^H y)
+        const c64 v = lane > k && lane < n ? A[k * ld + lane] : zero;
+        const c64 dt = cmulc(v, yv);
+        const c64 sm = tau[k] * c64{wave_sum(dt.x), wave_sum(dt.y)};
+        yv = yv - v * sm;
+      }
+      yv = mk_backsub(yv, U, ld, n, drop, dsc, lane);
+      if (lane < n) out[lane] = yv;
+    }
+  }
+  __syncthreads();
+  return single != 0;
 }
 
 // Ritz pair j of the pencil (A(k), B(k)) of the search space at column j's k.  The pencil is
@@ -491,44 +726,55 @@ __device__ c64* mk_jacobi(c64* A0, c64* A1, c64* V, int ld, int n, double stop) 
 // (one elimination step per column, applied to A as well); columns whose pivot falls below
 // 1e-5 (dependent to FP32 accuracy) are taken out of the space.  Bands whose k agree to 3e-5
 // share one k, so that near-degenerate bands take different vectors of one decomposition.
-// C: per problem and band, coefficients [column][vector] of the lowest msz Ritz vectors.
+// Latency-bound on one CU per band.
+// FINAL false: Cx column j, lam, slope and the Newton step.  FINAL true (after the last
+// iteration, at the k and on the Gram matrices of that iteration): the coefficients Cblk
+// [column][vector] of the lowest msz vectors of each band's block.
+template <int DT, bool FINAL>
 __global__ __launch_bounds__(DT) void k_mk_dense(MkGeo geo, MkState* st, const c64* red, int pm, int ld, double stop,
-                                                 const int* msz, c32* Cx, c64* Cblk) {
+                                                 const int* msz, c32* Cx, c64* Cblk, MkRot* rotg, long rotn) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int j = blockIdx.x, p = blockIdx.y;
   MkState& s = st[p];
-  if (s.done || j >= s.m) return;
+  if (FINAL ? s.done != 1 || j >= s.nev : s.done || j >= s.m) return;
   const int n = s.m + s.na + s.np;
   c64* A = reinterpret_cast<c64*>(smem_raw);
-  c64* B = A + (n + 1) * ld;  // Jacobi's second buffer afterwards
-  c64* V = B + (n + 1) * ld;
+  const int rows = (n + 1) & ~1;  // an odd size is padded to an even one in the Jacobi
+  c64* A1 = A + rows * ld;
+  c64* B = A1 + rows * ld;  // U of B = U^H U after the congruence
   __shared__ double node[MK_NODES], lw[MK_NODES], dlw[MK_NODES], dsc[MK_MAXN], diagv[MK_MAXN];
-  __shared__ double kk_s, red_s[DT / 64][2];
+  __shared__ double kk_s, red_s[DT / 64];
   __shared__ int drop[MK_MAXN], rank[MK_MAXN];
   __shared__ c64 y[MK_MAXN];
+  __shared__ c64 xs[DT / 64][64];
+  __shared__ c64 prA[2][64], prB[2][64];
+  __shared__ double lam_s;
   if (threadIdx.x == 0) {
+    const double* kv = FINAL ? s.kold : s.k;
     int a = j, b = j;
-    while (a > 0 && fabs(s.k[a - 1] - s.k[a]) < 3e-5 * fabs(s.k[a])) --a;
-    while (b + 1 < s.m && fabs(s.k[b + 1] - s.k[b]) < 3e-5 * fabs(s.k[b])) ++b;
+    while (a > 0 && fabs(kv[a - 1] - kv[a]) < MK_CLUSTER * fabs(kv[a])) --a;
+    while (b + 1 < s.m && fabs(kv[b + 1] - kv[b]) < MK_CLUSTER * fabs(kv[b])) ++b;
     double kk = 0;
-    for (int i = a; i <= b; ++i) kk += s.k[i];
+    for (int i = a; i <= b; ++i) kk += kv[i];
     kk /= double(b - a + 1);
     kk_s = kk;
-    mk_nodes(s, node);
-    for (int t = 0; t < MK_NODES; ++t) {  // Lagrange weights at kk and their k-derivatives
-      double w = 1, dw = 0;
-      for (int u = 0; u < MK_NODES; ++u) {
-        if (u == t) continue;
-        const double q = 1.0 / (node[t] - node[u]);
-        dw = dw * (kk - node[u]) * q + w * q;
-        w *= (kk - node[u]) * q;
-      }
-      lw[t] = w;
-      dlw[t] = dw;
-    }
   }
+  if (threadIdx.x < MK_NODES) node[threadIdx.x] = mk_node(FINAL ? s.kold : s.k, s.m, threadIdx.x);
   __syncthreads();
   const double kk = kk_s;
+  if (threadIdx.x < MK_NODES) {  // Lagrange weights at kk and their k-derivatives
+    const int t = threadIdx.x;
+    double w = 1, dw = 0;
+    for (int u = 0; u < MK_NODES; ++u) {
+      if (u == t) continue;
+      const double q = 1.0 / (node[t] - node[u]);
+      dw = dw * (kk - node[u]) * q + w * q;
+      w *= (kk - node[u]) * q;
+    }
+    lw[t] = w;
+    dlw[t] = dw;
+  }
+  __syncthreads();
   const long esz = long(pm) * pm;
   const c64* G = red + long(p) * NGRAM * esz;
   for (int e = threadIdx.x; e < n * n; e += DT) {
@@ -548,7 +794,6 @@ __global__ __launch_bounds__(DT) void k_mk_dense(MkGeo geo, MkState* st, const c
     A[a * ld + b] = va;
     A[b * ld + a] = conj(va);
     B[a * ld + b] = vb;
-    B[b * ld + a] = conj(vb);
   }
   __syncthreads();
   for (int a = threadIdx.x; a < n; a += DT) {
@@ -557,62 +802,61 @@ __global__ __launch_bounds__(DT) void k_mk_dense(MkGeo geo, MkState* st, const c
     drop[a] = 0;
   }
   __syncthreads();
+  const double iN = 1.0 / double(geo.N);  // the transforms are unnormalised
   for (int e = threadIdx.x; e < n * n; e += DT) {
     const int a = e / n, b = e - a * n;
     const double f = dsc[a] * dsc[b];
-    A[a * ld + b] = A[a * ld + b] * (f / double(geo.N));  // the transforms are unnormalised
-    B[a * ld + b] = B[a * ld + b] * f;
+    A[a * ld + b] = A[a * ld + b] * (f * iN);
+    if (a <= b) B[a * ld + b] = B[a * ld + b] * f;
   }
   __syncthreads();
-  // congruence: after step k, rows and columns <= k of B are the identity's.  Row k of A takes
-  // its own column operation only once the other rows have used it, at the start of step k + 1.
+  // Congruence: after step k, rows and columns <= k of B are the identity's.  Lane b holds
+  // column b, each wavefront the rows congruent to its number, and the pivot row comes from a
+  // double buffer its owner filled one step earlier: one barrier per step (in three phases
+  // with three barriers a step took 1.8 us).
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  constexpr int NW = DT / 64;
+  const c64 zero{0.0, 0.0};
+  if (wv == 0) {
+    prA[0][lane] = lane < n ? A[lane] : zero;
+    prB[0][lane] = lane < n ? B[lane] : zero;
+  }
+  __syncthreads();
   for (int k = 0; k < n; ++k) {
-    const double d = B[k * ld + k].x;
+    const c64(*pa) = prA[k & 1];
+    const c64(*pb) = prB[k & 1];
+    const double d = pb[k].x;
     const bool bad = !(d > 1e-5);
-    const double f = bad ? 0.0 : rsqrt(d);
-    if (k > 0 && !drop[k - 1]) {
-      const int r = k - 1;
-      const double arr = A[r * ld + r].x;
-      for (int b = k + threadIdx.x; b < n; b += DT) {
-        const c64 v = A[r * ld + b] - B[r * ld + b] * arr;
-        A[r * ld + b] = v;
-        A[b * ld + r] = conj(v);
+    const double f = bad ? 0.0 : rsqrt_fast(d);
+    const c64 ub = lane > k ? pb[lane] * f : zero;
+    const c64 ak = lane != k ? pa[lane] * f : zero;
+    const double akk = pa[k].x * f * f;
+    const c64 fin = ak - ub * akk;  // row k after its own column operation
+    for (int a = wv; a < n; a += NW) {
+      if (a == k) {
+        if (lane < n) A[k * ld + lane] = lane == k ? c64{akk, 0.0} : fin;
+        if (lane > k && lane < n) B[k * ld + lane] = ub;
+        if (lane == k) {
+          B[k * ld + k] = c64{bad ? 0.0 : d * f, 0.0};  // U[k][k]
+          drop[k] = bad ? 1 : 0;
+        }
+        continue;
       }
-    }
-    __syncthreads();
-    // scale row and column k of A and row k of B (column k of B is its mirror, not kept)
-    for (int b = threadIdx.x; b < n; b += DT) {
-      if (b > k) B[k * ld + b] = B[k * ld + b] * f;
-      if (b != k) {
-        const c64 v = A[k * ld + b] * f;
-        A[k * ld + b] = v;
-        A[b * ld + k] = conj(v);
-      } else {
-        A[k * ld + k] = c64{A[k * ld + k].x * f * f, 0.0};
-        B[k * ld + k] = c64{bad ? 0.0 : 1.0 / f, 0.0};  // U[k][k]
-        if (bad) drop[k] = 1;
-      }
-    }
-    __syncthreads();
-    if (!bad) {
-      const double akk = A[k * ld + k].x;
-      const int w = n - 1 - k;
-      for (int e = threadIdx.x; e < n * w; e += DT) {
-        const int a = e / w, b = k + 1 + (e - a * w);
-        if (a == k) continue;
-        const c64 ub = B[k * ld + b];  // U[k][b]
-        if (a < k) {
-          // finished row: A[a][b] -= A[a][k] U[k][b]; its mirror is written too
-          const c64 v = A[a * ld + b] - A[a * ld + k] * ub;
-          A[a * ld + b] = v;
-          A[b * ld + a] = conj(v);
-        } else if (a <= b) {
-          const c64 ua = B[k * ld + a];
-          const c64 v = A[a * ld + b] - operator_conj_mul(ua, A[k * ld + b]) - A[a * ld + k] * ub +
-                        operator_conj_mul(ua, ub) * akk;
-          A[a * ld + b] = a == b ? c64{v.x, 0.0} : v;
-          A[b * ld + a] = conj(v);
-          B[a * ld + b] = B[a * ld + b] - operator_conj_mul(ua, ub);
+      const c64 ua{read_lane(ub.x, a), read_lane(ub.y, a)}, aka{read_lane(ak.x, a), read_lane(ak.y, a)};
+      const c64 fa{read_lane(fin.x, a), read_lane(fin.y, a)};
+      if (lane < n) {
+        c64 v = A[a * ld + lane] - cmulc(ua, ak) - cmulc(aka, ub) + cmulc(ua, ub) * akk;
+        if (lane == k) v = conj(fa);
+        if (lane == a) v.y = 0.0;
+        A[a * ld + lane] = v;
+        c64 vb = zero;
+        if (a > k && lane >= a) {
+          vb = B[a * ld + lane] - cmulc(ua, ub);
+          B[a * ld + lane] = vb;
+        }
+        if (a == k + 1) {
+          prA[(k + 1) & 1][lane] = v;
+          prB[(k + 1) & 1][lane] = vb;
         }
       }
     }
@@ -621,22 +865,30 @@ __global__ __launch_bounds__(DT) void k_mk_dense(MkGeo geo, MkState* st, const c
   // dropped columns: decoupled, at the end of the spectrum
   {
     double mx = 0;
-    for (int a = 0; a < n; ++a) mx = fmax(mx, fabs(A[a * ld + a].x));
-    __syncthreads();
-    for (int e = threadIdx.x; e < n * n; e += DT) {
-      const int a = e / n, b = e - a * n;
-      if (drop[a] || drop[b]) A[a * ld + b] = a == b ? c64{16.0 * mx + 1.0, 0.0} : c64{0.0, 0.0};
+    int any = 0;
+    for (int a = 0; a < n; ++a) {
+      mx = fmax(mx, fabs(A[a * ld + a].x));
+      any |= drop[a];
     }
+    __syncthreads();
+    if (any)
+      for (int e = threadIdx.x; e < n * n; e += DT) {
+        const int a = e / n, b = e - a * n;
+        if (drop[a] || drop[b]) A[a * ld + b] = a == b ? c64{16.0 * mx + 1.0, 0.0} : c64{0.0, 0.0};
+      }
   }
   __syncthreads();
-  // U (upper, in B) is needed after the Jacobi, which uses B's storage: keep it in global memory
-  c64* Ug = Cblk + ((long(p) * geo.mmax + j) * 2 + 1) * MK_MAXN * MK_MAXN;
-  for (int e = threadIdx.x; e < n * n; e += DT) {
-    const int a = e / n, b = e - a * n;
-    if (a <= b) Ug[a * MK_MAXN + b] = B[a * ld + b];
+  bool jac = FINAL;
+  if (!FINAL) {
+    // keep the reduced matrix: the tridiagonal form overwrites it
+    for (int a = wv; a < n; a += NW)
+      if (lane < n) A1[a * ld + lane] = A[a * ld + lane];
+    jac = !tridiag_pair<NW>(A, ld, n, j, prA, &xs[0][0], &lam_s, y, B, drop, dsc);
   }
-  __syncthreads();
-  const c64* Ad = mk_jacobi(A, B, V, ld, n, stop);
+  MkRot* rot = rotg + (long(p) * geo.mmax + j) * rotn;
+  if (jac) {  // block-uniform
+  const int rounds = mk_jacobi(FINAL ? A : A1, FINAL ? A1 : A, ld, n, stop, rot);
+  const c64* Ad = ((rounds & 1) != 0) == FINAL ? A1 : A;
   for (int a = threadIdx.x; a < n; a += DT) diagv[a] = Ad[a * ld + a].x;
   __syncthreads();
   for (int a = threadIdx.x; a < n; a += DT) {
@@ -645,49 +897,81 @@ __global__ __launch_bounds__(DT) void k_mk_dense(MkGeo geo, MkState* st, const c
       if (diagv[l] < diagv[a] || (diagv[l] == diagv[a] && l < a)) ++r;
     rank[r] = a;
   }
+  __threadfence_block();  // the block's rotations, read back below
   __syncthreads();
-  // back substitution c = D U^-1 v for the lowest vectors: band j's own, and the block's
-  const int nv = j < s.nev ? max(msz[p * MK_MAXM + j], j + 1) : j + 1;
-  // every matrix buffer but V is free now: U back into LDS
-  c64* U = A;
-  for (int e = threadIdx.x; e < n * n; e += DT) {
-    const int a = e / n, b = e - a * n;
-    if (a <= b) U[a * ld + b] = Ug[a * MK_MAXN + b];
-  }
-  __syncthreads();
-  for (int q = threadIdx.x; q < nv; q += DT) {  // one thread per vector, in place in V's column
-    const int c = rank[q];
-    for (int a = n - 1; a >= 0; --a) {
-      if (drop[a]) {
-        V[a * ld + c] = c64{0.0, 0.0};
-        continue;
+  if (!FINAL && threadIdx.x == 0) lam_s = diagv[rank[j]];
+  // the wanted vectors: V e = (rotations in reverse) e, then c = D U^-1 V e; one wavefront per
+  // vector, lane t the pair t of a round, the rotations staged in LDS
+  const int m = n + (n & 1), npair = m / 2;
+  const int v0 = FINAL ? 0 : j, nv = FINAL ? msz[p * MK_MAXM + j] : 1;
+  // The vector stays in registers: lane t holds the pair's elements (xl, xr), and from a round to
+  // the one before it all elements but the first move one place round the ring of pairs, i.e.
+  // xl comes from lane t - 1 and xr from lane t + 1.
+  MkRot* rl = reinterpret_cast<MkRot*>(A);  // both matrix buffers are free
+  const int chunk = max(1, int(2L * rows * ld * sizeof(c64) / (sizeof(MkRot) * npair)));
+  c64* Cb = Cblk + (long(p) * geo.mmax + j) * MK_MAXN * MK_MAXM;
+  for (int base = 0; base < nv; base += DT / 64) {
+    const bool mine = base + wv < nv;
+    const int q = v0 + base + wv;
+    // the pairs of the last round (rounds is a multiple of m - 1: its index within a sweep is m - 2)
+    const int el = lane == 0 ? 0 : 1 + (lane - 1 + m - 2) % (m - 1), er = 1 + (m - 2 - min(lane, m - 2) + m - 2) % (m - 1);
+    const int hot = mine ? rank[q] : -1;
+    c64 xl{lane < npair && el == hot ? 1.0 : 0.0, 0.0}, xr{lane < npair && er == hot ? 1.0 : 0.0, 0.0};
+    for (int r1 = rounds; r1 > 0; r1 -= chunk) {
+      const int r0 = max(0, r1 - chunk), cnt = (r1 - r0) * npair;
+      __syncthreads();
+      for (int e = threadIdx.x; e < cnt; e += DT) rl[e] = rot[long(r0) * npair + e];
+      __syncthreads();
+      if (mine) {
+        const int t = min(lane, npair - 1);
+        MkRot R = rl[(r1 - 1 - r0) * npair + t];
+        for (int r = r1 - 1; r >= r0; --r) {
+          const MkRot Rn = rl[(max(r - 1, r0) - r0) * npair + t];
+          const c64 yl = xl * R.c + R.s * xr, yr = xr * R.c - cmulc(R.s, xl);
+          if (r == 0) {
+            xl = yl;
+            xr = yr;
+          } else {
+            // to round r - 1: L_t <- L_{t-1} (t >= 2), L_1 <- R_0, R_t <- R_{t+1}, R_last <- L_last
+            const c64 sl{lane_shift<true>(lane == 0 ? yr.x : yl.x), lane_shift<true>(lane == 0 ? yr.y : yl.y)};
+            const c64 sr{lane_shift<false>(yr.x), lane_shift<false>(yr.y)};
+            xl = lane == 0 ? yl : sl;
+            xr = lane == npair - 1 ? (npair == 1 ? yr : yl) : sr;
+          }
+          R = Rn;
+        }
       }
-      c64 v = V[a * ld + c];
-      for (int b = a + 1; b < n; ++b) v = v - U[a * ld + b] * V[b * ld + c];
-      V[a * ld + c] = v * (1.0 / U[a * ld + a].x);
+    }
+    if (mine && lane < npair) {  // pairs of round 0
+      xs[wv][lane == 0 ? 0 : lane] = xl;
+      xs[wv][1 + (m - 2 - lane)] = xr;
+    }
+    if (mine) {
+      mk_wave_sync();
+      c64 v = lane < n ? xs[wv][lane] : c64{0.0, 0.0};
+      v = mk_backsub(v, B, ld, n, drop, dsc, lane);
+      if (lane < n) {
+        if (FINAL)
+          Cb[lane * MK_MAXM + q] = v;
+        else
+          y[lane] = v;
+      }
     }
   }
-  __syncthreads();
-  c64* Cb = Cblk + ((long(p) * geo.mmax + j) * 2) * MK_MAXN * MK_MAXN;
-  for (int e = threadIdx.x; e < n * nv; e += DT) {
-    const int a = e / nv, q = e - a * nv;
-    const c64 v = V[a * ld + rank[q]] * dsc[a];
-    Cb[a * MK_MAXM + q] = v;
-    if (q == j) {
-      y[a] = v;
-      Cx[(long(p) * MK_MAXN + a) * MK_MAXM + j] = c32{float(v.x), float(v.y)};
-    }
   }
+  if (FINAL) return;
   __syncthreads();
+  if (int(threadIdx.x) < n)
+    Cx[(long(p) * MK_MAXN + threadIdx.x) * MK_MAXM + j] = c32{float(y[threadIdx.x].x), float(y[threadIdx.x].y)};
   // slope = y^H (dA/dk - lam dB/dk) y (y^H B y = 1)
-  const double lam = diagv[rank[j]];
+  const double lam = lam_s;
   double acc = 0;
   for (int e = threadIdx.x; e < n * n; e += DT) {
     const int a = e / n, b = e - a * n;
     if (a > b) continue;
     const long o = long(a) * pm + b;
     const c64 g01 = G[esz + o], g10 = G[esz + long(b) * pm + a], g11 = G[2 * esz + o];
-    c64 d{(g01.x + g10.x + 2 * kk * g11.x) / geo.N, (g01.y - g10.y + 2 * kk * g11.y) / geo.N};
+    c64 d{(g01.x + g10.x + 2 * kk * g11.x) * iN, (g01.y - g10.y + 2 * kk * g11.y) * iN};
 #pragma unroll
     for (int t = 0; t < MK_NODES; ++t) {
       const c64 w = G[(3 + t) * esz + o];
@@ -699,11 +983,11 @@ __global__ __launch_bounds__(DT) void k_mk_dense(MkGeo geo, MkState* st, const c
     acc += (a == b ? 1.0 : 2.0) * (y[a].x * z.x + y[a].y * z.y);
   }
   for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-  if ((threadIdx.x & 63) == 0) red_s[threadIdx.x >> 6][0] = acc;
+  if (lane == 0) red_s[wv] = acc;
   __syncthreads();
   if (threadIdx.x == 0) {
     double slope = 0;
-    for (int w = 0; w < DT / 64; ++w) slope += red_s[w][0];
+    for (int w = 0; w < DT / 64; ++w) slope += red_s[w];
     // early Ritz values are far above the band's: the first steps move k by at most a tenth
     const double lim = (s.iter < 4 ? 0.1 : 0.25) * fabs(kk);
     double dk = -(lam - s.omega2) / slope;
@@ -927,6 +1211,7 @@ __global__ __launch_bounds__(256) void k_mk_control(MkGeo geo, MkState* st, cons
       all = all && conv;
     }
     s.rnorm[c] = rn;
+    s.kold[c] = s.k[c];
     s.k[c] = s.knew[c];
   }
   s.iter += 1;
@@ -937,6 +1222,16 @@ __global__ __launch_bounds__(256) void k_mk_control(MkGeo geo, MkState* st, cons
     return;
   }
   if (all) {  // the current space and its coefficients are the result
+    // bands close enough to have shared a k (k_mk_dense) are handed over at one k too: their
+    // vectors are orthogonal there
+    for (int a = 0; a < s.nev;) {
+      int b = a;
+      double sum = s.k[a];
+      while (b + 1 < s.nev && fabs(s.k[b + 1] - s.k[b]) < MK_CLUSTER * fabs(s.k[b])) sum += s.k[++b];
+      for (int i = a; i <= b; ++i) s.knew[i] = sum / (b - a + 1);
+      a = b + 1;
+    }
+    for (int i = 0; i < s.nev; ++i) s.k[i] = s.knew[i];
     s.done = 1;
     return;
   }
@@ -1082,7 +1377,7 @@ __global__ __launch_bounds__(256) void k_mk_handover(MkGeo geo, const c32* cols,
   const int nq = min(HQ, msz[p * MK_MAXM + j] - q0);
   if (nq <= 0) return;
   const int n = s.m + s.na + s.np;
-  const c64* Cb = Cblk + (long(p) * geo.mmax + j) * 2 * MK_MAXN * MK_MAXN;
+  const c64* Cb = Cblk + (long(p) * geo.mmax + j) * MK_MAXN * MK_MAXM;
   for (int a = threadIdx.x; a < n; a += 256)
     in[a] = cols + p * geo.slots + col_off(geo, space_slot(geo, s, s.par, a)) + 5 * geo.cs;
   for (int e = threadIdx.x; e < n * HQ; e += 256) {
@@ -1186,10 +1481,18 @@ bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* e
   const int RB = pick_rows(S.nx, S.ny, vecs, g.fx), TX = pick_rows(S.ny, S.nx, vecs, g.fy);
   if (RB == 0 || TX == 0) return false;
   const int nrb = (S.ny + RB - 1) / RB, ncb = (S.nx + TX - 1) / TX;
-  // Gram chunks: about 128 over the problems, whole stages of 64 rows, at least four of them
+  // Gram chunks: about 128 over the problems, of whole 64-row steps, a stage of every wave or more
   const int nchunk = int(std::max<long>(1, std::min<long>((S.N + 255) / 256, std::max(8, 128 / P))));
   const long rpc = ((S.N + nchunk - 1) / nchunk + 63) / 64 * 64;
   const int nch = int((S.N + rpc - 1) / rpc);
+  // the widest space's three matrices and the kernel's own arrays share a CU's 160 KB
+  {
+    hipFuncAttributes fa{}, fb{};
+    OMX_HIP_CHECK(hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(&k_mk_dense<512, false>)));
+    OMX_HIP_CHECK(hipFuncGetAttributes(&fb, reinterpret_cast<const void*>(&k_mk_dense<512, true>)));
+    const size_t dyn = sizeof(c64) * 3 * size_t((nmax + 1) & ~1) * ((nmax + 1) | 1);
+    if (std::max(fa.sharedSizeBytes, fb.sharedSizeBytes) + dyn > 160 * 1024) return false;
+  }
   MultiKWorkspace& W = S.multik_ws;
   const size_t colb = sizeof(c32) * size_t(P) * g.slots;
   if (W.cols.size() < colb || W.geom != g.cs * 64 + g.mmax) {
@@ -1202,7 +1505,9 @@ bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* e
   W.part.ensure(sizeof(c32) * size_t(P) * nch * NGRAM * pm * pm);
   W.red.ensure(sizeof(c64) * size_t(P) * NGRAM * pm * pm);
   W.cx.ensure(sizeof(c32) * size_t(P) * MK_MAXN * MK_MAXM);
-  W.cblk.ensure(sizeof(c64) * size_t(vecs) * 2 * MK_MAXN * MK_MAXN);
+  W.cblk.ensure(sizeof(c64) * size_t(vecs) * MK_MAXN * MK_MAXM);
+  const long rotn = long(MK_SWEEPS) * nmax * ((nmax + 1) / 2);
+  W.rot.ensure(sizeof(MkRot) * size_t(vecs) * rotn);
   W.normp.ensure(sizeof(double) * size_t(vecs) * nrb);
   W.state.ensure(sizeof(MkState) * P);
   W.ints.ensure(sizeof(int) * size_t(P) * MK_MAXM + sizeof(int2) * ninst);
@@ -1255,14 +1560,15 @@ bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* e
   auto gram = [&](auto T, int buf) {
     constexpr int nt = decltype(T)::value;
     constexpr int S_ = nt <= 2 ? 4 : 2, NB = nt <= 2 ? 3 : (nt == 3 ? 2 : 1);
-    const dim3 gg(nch, P), gb(nch, P, (MK_NODES + NB) / NB);
-    hipLaunchKernelGGL((k_mk_gram<nt, 0, 1, S_>), gg, dim3(256), 0, sm, g, cols, st, buf, rpc, part);
-    hipLaunchKernelGGL((k_mk_gram<nt, 1, 1, S_>), gg, dim3(256), 0, sm, g, cols, st, buf, rpc, part);
-    hipLaunchKernelGGL((k_mk_gram<nt, 2, 1, S_>), gg, dim3(256), 0, sm, g, cols, st, buf, rpc, part);
-    hipLaunchKernelGGL((k_mk_gram<nt, 3, NB, S_>), gb, dim3(256), 0, sm, g, cols, st, buf, rpc, part);
+    hipLaunchKernelGGL((k_mk_gram<nt, NB, S_>), dim3(nch, P, 3 + (MK_NODES + NB) / NB), dim3(64 * GW), 0, sm, g, cols,
+                       st, buf, rpc, part);
   };
-  const int ldd = (nmax + 1) | 1;  // odd sizes are padded to even ones in the Jacobi
-  const size_t ldsd = sizeof(c64) * 3 * size_t(nmax + 1) * ldd;
+  const int ldd = (nmax + 1) | 1;
+  const size_t ldsd = sizeof(c64) * 3 * size_t((nmax + 1) & ~1) * ldd;
+  auto dense = [&](auto F) {
+    hipLaunchKernelGGL((k_mk_dense<512, decltype(F)::value>), dim3(g.mmax, P), dim3(512), ldsd, sm, g, st, red, pm, ldd,
+                       S.opt.jac_stop32, mszd, cx, cblk, W.rot.as<MkRot>(), rotn);
+  };
   const dim3 gcomb(unsigned(std::min<long>((PLANES * g.cs / 2 + 255) / 256, std::max(1, 2048 / P))), P);
   const bool prof = S.prof.enabled;
   int cur = 0, it = 0;
@@ -1275,8 +1581,7 @@ bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* e
       default: gram(std::integral_constant<int, 4>{}, cur); break;
     }
     hipLaunchKernelGGL(k_mk_reduce, dim3(pm * pm / 16, NGRAM, P), dim3(256), 0, sm, part, nch, pm, st, red);
-    hipLaunchKernelGGL(k_mk_dense, dim3(g.mmax, P), dim3(DT), ldsd, sm, g, st, red, pm, ldd, S.opt.jac_stop32, mszd, cx,
-                       cblk);
+    dense(std::false_type{});
     if (g.mmax <= 4)
       hipLaunchKernelGGL((k_mk_combine<4>), gcomb, dim3(256), 0, sm, g, cols, st, cx, cur);
     else if (g.mmax <= 8)
@@ -1337,6 +1642,7 @@ bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* e
       stats.matvec += hs[p].its[j];
       stats.precon += hs[p].its[j];
     }
+  dense(std::true_type{});
   hipLaunchKernelGGL(k_mk_handover, dim3(unsigned(std::min<long>((S.N + 255) / 256, 512)), ninst, (mmax + HQ - 1) / HQ),
                      dim3(256), 0, sm, g, cols, st, instd, mszd, cblk, X64, ld, istride);
   OMX_HIP_CHECK(hipGetLastError());

@@ -56,9 +56,9 @@ bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* e
                   std::vector<int>& iters, std::vector<int>& moves, SolveStats& stats);
 
 // columns of the widest block handed over for nev bands on a grid of K unknowns: the space's
-// columns past the bands too, at most the refinement's 16
+// columns past the bands too
 inline int multik_block(int nev, long K) {
-  return int(std::max<long>(nev, std::min<long>(std::min<long>(nev + MK_GUARD, 16), K / 3)));
+  return int(std::max<long>(nev, std::min<long>(nev + MK_GUARD, K / 3)));
 }
 
 // whether the grid fits the phase's transforms

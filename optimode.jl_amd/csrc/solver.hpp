@@ -226,7 +226,7 @@ struct RefineWorkspace {
 
 // Buffers of the shared-subspace FP32 phase (multik.hip), kept on the handle between solves.
 struct MultiKWorkspace {
-  DevMem cols, dm, part, red, cx, cblk, normp, state, ints;
+  DevMem cols, dm, part, red, cx, cblk, rot, normp, state, ints;
   long geom = 0;          // plane size and column count the zeroed pads belong to
   PinnedMem snap[2];
   size_t snap_bytes = 0;
