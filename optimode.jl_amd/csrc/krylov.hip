@@ -207,15 +207,20 @@ struct MinresState;
 // w_new = c0 v' + c1 w1' + c2 w2' (into wout) and x += c3 w_new with v' the previous
 // iteration's u, which the output buffer y still holds until this row is written.
 //
-// QM > 0: A u also takes -sum_c rc_c R_c (the Schur complement of VecOpsT::set_schur), the
-// coefficients rc_c = g_c <R_c, u> from k_minres_scalars; all columns' loads of a row are in
-// flight together, as in the block projection.
+// QM > 0 (the Schur complement of VecOpsT::set_schur): u holds z = P y before its projection
+// and au M z.  With c = Q^H z, d = R^H z (= R^H u, since R^H Q = 0) and M Q = Q Theta + R,
+//   u                       = z - Q c                                 (stored over z)
+//   M u - shift u - R g d   = M z - shift z - Q (Theta - shift) c - R (c + g d)
+// and Q d is the part of that along the block, which the projected operator drops: one pass
+// over Q and R makes the projection of z, the operator's Schur term and the projection of y
+// (left in, that last part makes the preconditioned operator non-symmetric).  The column
+// coefficients come from k_minres_scalars; all columns' loads of a row are in flight together.
 template <typename T, bool WX, int QM>
-__global__ __launch_bounds__(AB) void k_minres_y1(const MinresState* ms, const cplx<T>* au, const cplx<T>* u,
+__global__ __launch_bounds__(AB) void k_minres_y1(const MinresState* ms, const cplx<T>* au, cplx<T>* u,
                                                   const cplx<T>* r1, cplx<T>* y, long ld, long K, const int* act,
                                                   double* part, const cplx<T>* w1p, const cplx<T>* w2p,
-                                                  cplx<T>* wout, cplx<T>* x, const c64* wcoef, const cplx<T>* R,
-                                                  long ris, const int* nr, const c64* rc);
+                                                  cplx<T>* wout, cplx<T>* x, const c64* wcoef, const cplx<T>* Q,
+                                                  const cplx<T>* R, long qis, const int* nq, const c64* qrc);
 
 // Stage-2 update fused with its scalar step: alfa = sum of the <v, y> partials (every block
 // the same, block 0 stores it), y <- y - (alfa/beta) r2
@@ -303,13 +308,13 @@ struct MinresState {
 // one block per instance: the block sums the instance's partials (tree), then its first
 // thread runs the recurrence
 template <typename T, bool WX, int NR>
-__device__ __forceinline__ double minres_y1_rows(const MinresState& m, const cplx<T>* au, const cplx<T>* u,
+__device__ __forceinline__ double minres_y1_rows(const MinresState& m, const cplx<T>* au, cplx<T>* u,
                                                  const cplx<T>* r1, cplx<T>* y, long K, const cplx<T>* w1p,
                                                  const cplx<T>* w2p, cplx<T>* wout, cplx<T>* x, const c64* wcoef,
-                                                 const cplx<T>* R, long ld, const c64* rc) {
+                                                 const cplx<T>* Q, const cplx<T>* R, long ld, const c64 (*cf)[3]) {
   // beta = 0 ends the instance (its v is zero): the zero scale keeps its updates finite
   const double ib = m.beta > 0 ? 1.0 / m.beta : 0.0;
-  const double c0 = ib, c1 = -m.shift * ib, c2 = m.itn >= 1 && m.oldb > 0 ? -m.beta / m.oldb : 0.0;
+  const double c0 = ib, c1 = -m.shift, c2 = m.itn >= 1 && m.oldb > 0 ? -m.beta / m.oldb : 0.0;
   double d0 = 0, d1 = 0, d2 = 0, d3 = 0, acc = 0;
   if (WX) {
     d0 = wcoef[0].x;
@@ -317,13 +322,13 @@ __device__ __forceinline__ double minres_y1_rows(const MinresState& m, const cpl
     d2 = wcoef[2].x;
     d3 = wcoef[3].x;
   }
-  c64 cf[NR > 0 ? NR : 1];
-#pragma unroll
-  for (int c = 0; c < NR; ++c) cf[c] = rc[c];
   for (long r = long(blockIdx.x) * AB + threadIdx.x; r < K; r += long(gridDim.x) * AB) {
-    cplx<T> e[NR > 0 ? NR : 1];
+    cplx<T> e[NR > 0 ? NR : 1], f[NR > 0 ? NR : 1];
 #pragma unroll
-    for (int c = 0; c < NR; ++c) e[c] = R[c * ld + r];
+    for (int c = 0; c < NR; ++c) {
+      e[c] = Q[c * ld + r];
+      f[c] = R[c * ld + r];
+    }
     if (WX) {
       const cplx<T> pv = y[r], pb = w1p[r], pc = w2p[r], xr = x[r];
       const double wx = d0 * double(pv.x) + d1 * double(pb.x) + d2 * double(pc.x);
@@ -331,15 +336,25 @@ __device__ __forceinline__ double minres_y1_rows(const MinresState& m, const cpl
       wout[r] = cplx<T>{T(wx), T(wy)};
       x[r] = cplx<T>{T(double(xr.x) + d3 * wx), T(double(xr.y) + d3 * wy)};
     }
-    const cplx<T> a = au[r], b = u[r], c = r1[r];
-    double ax = a.x, ay = a.y;
+    const cplx<T> a = au[r], c = r1[r];
+    cplx<T> b = u[r];
+    double ax = double(a.x) + c1 * double(b.x), ay = double(a.y) + c1 * double(b.y);
+    if constexpr (NR > 0) {
+      asm volatile("" ::: "memory");  // the coefficients stay in LDS (in registers they cost the occupancy)
+      double ux = b.x, uy = b.y;
 #pragma unroll
-    for (int q = 0; q < NR; ++q) {
-      ax -= cf[q].x * double(e[q].x) - cf[q].y * double(e[q].y);
-      ay -= cf[q].x * double(e[q].y) + cf[q].y * double(e[q].x);
+      for (int q = 0; q < NR; ++q) {
+        const c64 u0 = cf[q][0], q0 = cf[q][1], r0 = cf[q][2];
+        const double ex = e[q].x, ey = e[q].y, fx = f[q].x, fy = f[q].y;
+        ux += u0.x * ex - u0.y * ey;
+        uy += u0.x * ey + u0.y * ex;
+        ax += q0.x * ex - q0.y * ey + r0.x * fx - r0.y * fy;
+        ay += q0.x * ey + q0.y * ex + r0.x * fy + r0.y * fx;
+      }
+      b = cplx<T>{T(ux), T(uy)};
+      u[r] = b;
     }
-    const cplx<T> yn{T(c0 * ax + c1 * double(b.x) + c2 * double(c.x)),
-                     T(c0 * ay + c1 * double(b.y) + c2 * double(c.y))};
+    const cplx<T> yn{T(c0 * ax + c2 * double(c.x)), T(c0 * ay + c2 * double(c.y))};
     y[r] = yn;
     acc += double(b.x) * double(yn.x) + double(b.y) * double(yn.y);
   }
@@ -347,31 +362,36 @@ __device__ __forceinline__ double minres_y1_rows(const MinresState& m, const cpl
 }
 
 template <typename T, bool WX, int QM, int NR = 1>
-__device__ __forceinline__ double minres_y1_cols(int n, const MinresState& m, const cplx<T>* au, const cplx<T>* u,
+__device__ __forceinline__ double minres_y1_cols(int n, const MinresState& m, const cplx<T>* au, cplx<T>* u,
                                                  const cplx<T>* r1, cplx<T>* y, long K, const cplx<T>* w1p,
                                                  const cplx<T>* w2p, cplx<T>* wout, cplx<T>* x, const c64* wcoef,
-                                                 const cplx<T>* R, long ld, const c64* rc) {
+                                                 const cplx<T>* Q, const cplx<T>* R, long ld, const c64 (*cf)[3]) {
   if constexpr (NR <= QM) {
-    if (n == NR) return minres_y1_rows<T, WX, NR>(m, au, u, r1, y, K, w1p, w2p, wout, x, wcoef, R, ld, rc);
-    return minres_y1_cols<T, WX, QM, NR + 1>(n, m, au, u, r1, y, K, w1p, w2p, wout, x, wcoef, R, ld, rc);
+    if (n == NR) return minres_y1_rows<T, WX, NR>(m, au, u, r1, y, K, w1p, w2p, wout, x, wcoef, Q, R, ld, cf);
+    return minres_y1_cols<T, WX, QM, NR + 1>(n, m, au, u, r1, y, K, w1p, w2p, wout, x, wcoef, Q, R, ld, cf);
   }
-  return minres_y1_rows<T, WX, 0>(m, au, u, r1, y, K, w1p, w2p, wout, x, wcoef, R, ld, rc);
+  return minres_y1_rows<T, WX, 0>(m, au, u, r1, y, K, w1p, w2p, wout, x, wcoef, Q, R, ld, cf);
 }
 
 template <typename T, bool WX, int QM>
-__global__ __launch_bounds__(AB) void k_minres_y1(const MinresState* ms, const cplx<T>* au, const cplx<T>* u,
+__global__ __launch_bounds__(AB) void k_minres_y1(const MinresState* ms, const cplx<T>* au, cplx<T>* u,
                                                   const cplx<T>* r1, cplx<T>* y, long ld, long K, const int* act,
                                                   double* part, const cplx<T>* w1p, const cplx<T>* w2p,
-                                                  cplx<T>* wout, cplx<T>* x, const c64* wcoef, const cplx<T>* R,
-                                                  long ris, const int* nr, const c64* rc) {
+                                                  cplx<T>* wout, cplx<T>* x, const c64* wcoef, const cplx<T>* Q,
+                                                  const cplx<T>* R, long qis, const int* nq, const c64* qrc) {
   const int i = blockIdx.y;
   __shared__ double red[AB];
+  __shared__ c64 cf[QM > 0 ? QM : 1][3];
   double acc = 0;
   if (act[i]) {
+    if constexpr (QM > 0) {
+      if (threadIdx.x < 3 * QM) cf[threadIdx.x / 3][threadIdx.x % 3] = qrc[i * 3 * RCQ + threadIdx.x];
+      __syncthreads();
+    }
     const long o = i * ld;
-    acc = minres_y1_cols<T, WX, QM>(QM > 0 ? nr[i] : 0, ms[i], au + o, u + o, r1 + o, y + o, K, WX ? w1p + o : nullptr,
+    acc = minres_y1_cols<T, WX, QM>(QM > 0 ? nq[i] : 0, ms[i], au + o, u + o, r1 + o, y + o, K, WX ? w1p + o : nullptr,
                                     WX ? w2p + o : nullptr, WX ? wout + o : nullptr, WX ? x + o : nullptr,
-                                    WX ? wcoef + 4 * i : nullptr, R + i * ris, ld, rc + i * RCQ);
+                                    WX ? wcoef + 4 * i : nullptr, Q + i * qis, R + i * qis, ld, cf);
   }
   red[threadIdx.x] = acc;
   __syncthreads();
@@ -402,34 +422,49 @@ __global__ __launch_bounds__(AB) void k_minres_y2(MinresState* ms, const double*
 // Coefficient slots (4 complex per instance each, slot s at coef + 4 ninst s): 0 for the
 // y updates of stages 1 and 2, 1 for the fused w/x update of stage 3, 2 for the next
 // v = y / beta (stages 0 and 3); slot 3 belongs to the projections.
-// With rpart (qm partial dots of the block residual columns per projection block), also the
-// Schur-complement coefficients rc_c = g_c <R_c, y> for the next operator application.
+// With qpart (k_qrdot's partials: qm columns per block, those of Q of every instance, then
+// those of R), also the column coefficients of the next k_minres_y1: for column c at qrc +
+// 3 (RCQ i + c) those of u along Q_c, of y along Q_c and of y along R_c.
 __global__ __launch_bounds__(AB) void k_minres_scalars(MinresState* ms, const double* part, int nb, c64* coef,
-                                                       int stage, int ninst, const int* act, const c64* rpart, int qm,
-                                                       const double* rg, c64* rc) {
+                                                       int stage, int ninst, const int* act, const c64* qpart, int qm,
+                                                       const double* rg, c64* qrc) {
   const int i = blockIdx.x;
   __shared__ double red[AB];
   __shared__ double rr[AB], ri[AB];
-  if (rpart && act[i]) {
-    const int c = threadIdx.x % qm, j = threadIdx.x / qm, G = AB / qm;
+  if (qpart && act[i]) {
+    // 2 qm <= 36 sums over nb partials, AB / (2 qm) threads each
+    const int n = 2 * qm, v = threadIdx.x % n, j = threadIdx.x / n, G = AB / n;
+    const c64* src = qpart + (v < qm ? long(i) : long(ninst) + i) * nb * qm + (v < qm ? v : v - qm);
     double a = 0, b = 0;
 #pragma unroll 8
     for (int q = j < G ? j : nb; q < nb; q += G) {
-      const c64 v = rpart[(long(i) * nb + q) * qm + c];
-      a += v.x;
-      b += v.y;
+      const c64 t = src[long(q) * qm];
+      a += t.x;
+      b += t.y;
     }
     rr[threadIdx.x] = a;
     ri[threadIdx.x] = b;
     __syncthreads();
-    if (int(threadIdx.x) < qm) {
-      double sa = 0, sb = 0;
-      for (int q = 0; q < G; ++q) {
-        sa += rr[q * qm + threadIdx.x];
-        sb += ri[q * qm + threadIdx.x];
+    if (int(threadIdx.x) < n) {
+      for (int q = 1; q < G; ++q) {
+        a += rr[q * n + threadIdx.x];
+        b += ri[q * n + threadIdx.x];
       }
-      const double g = rg[RCQ * i + threadIdx.x];
-      rc[RCQ * i + threadIdx.x] = c64{g * sa, g * sb};
+    }
+    __syncthreads();
+    if (int(threadIdx.x) < n) {
+      rr[threadIdx.x] = a;
+      ri[threadIdx.x] = b;
+    }
+    __syncthreads();
+    if (int(threadIdx.x) < qm) {
+      const int c = threadIdx.x;
+      const c64 qz{rr[c], ri[c]}, rz{rr[qm + c], ri[qm + c]};
+      const double g = rg[2 * RCQ * i + c], ts = rg[2 * RCQ * i + RCQ + c];
+      c64* o = qrc + 3 * (RCQ * i + c);
+      o[0] = c64{-qz.x, -qz.y};
+      o[1] = c64{-ts * qz.x - rz.x, -ts * qz.y - rz.y};
+      o[2] = c64{-qz.x - g * rz.x, -qz.y - g * rz.y};
     }
   }
   double acc = 0;
@@ -541,11 +576,15 @@ __global__ __launch_bounds__(AB) void k_proj_coef(const c64* part, int nblk, c64
 // Column loops of the block projection with the instance's column count NQ fixed at
 // compile time (qdot_cols / qproject_cols pick it from the runtime count): every load of a
 // row is issued before the first use, so a row costs one memory round trip, not one per column.
-template <typename T, int NQ>
-__device__ __forceinline__ void qdot_rows(const cplx<T>* q, long qld, const cplx<T>* x, long r0, long stride, long K,
-                                          double* sr, double* si) {
+// With dv also the sum of Re <dv, x>.
+template <typename T, int NQ, bool DOT>
+__device__ __forceinline__ double qdot_rows(const cplx<T>* q, long qld, const cplx<T>* x, const cplx<T>* dv, long r0,
+                                            long stride, long K, double* sr, double* si) {
+  double acc = 0;
   for (long r = r0; r < K; r += stride) {
     const cplx<T> xv = x[r];
+    cplx<T> dr{T(0), T(0)};
+    if (DOT) dr = dv[r];
     cplx<T> e[NQ];
 #pragma unroll
     for (int c = 0; c < NQ; ++c) e[c] = q[c * qld + r];
@@ -555,26 +594,25 @@ __device__ __forceinline__ void qdot_rows(const cplx<T>* q, long qld, const cplx
       sr[c] += double(e[c].x) * xx + double(e[c].y) * xy;
       si[c] += double(e[c].x) * xy - double(e[c].y) * xx;
     }
+    if (DOT) acc += double(dr.x) * xx + double(dr.y) * xy;
   }
+  return acc;
 }
 
-template <typename T, int QM, int NQ = 1>
-__device__ __forceinline__ void qdot_cols(int n, const cplx<T>* q, long qld, const cplx<T>* x, long r0, long stride,
-                                          long K, double* sr, double* si) {
+template <typename T, int QM, bool DOT, int NQ = 1>
+__device__ __forceinline__ double qdot_cols(int n, const cplx<T>* q, long qld, const cplx<T>* x, const cplx<T>* dv,
+                                            long r0, long stride, long K, double* sr, double* si) {
   if constexpr (NQ <= QM) {
-    if (n == NQ)
-      qdot_rows<T, NQ>(q, qld, x, r0, stride, K, sr, si);
-    else
-      qdot_cols<T, QM, NQ + 1>(n, q, qld, x, r0, stride, K, sr, si);
+    if (n == NQ) return qdot_rows<T, NQ, DOT>(q, qld, x, dv, r0, stride, K, sr, si);
+    return qdot_cols<T, QM, DOT, NQ + 1>(n, q, qld, x, dv, r0, stride, K, sr, si);
   }
+  return 0.0;
 }
 
-// x <- x + sum_c cf_c Q_c over the rows, and sum of Re <d, x_new> when DOT; with SCHUR also
-// the sums of conj(R_c) x_new (R laid out as Q) into sr, si
-template <typename T, int NQ, bool DOT, bool SCHUR>
+// x <- x + sum_c cf_c Q_c over the rows, and sum of Re <d, x_new> when DOT
+template <typename T, int NQ, bool DOT>
 __device__ __forceinline__ double qproject_rows(const c64* cf, const cplx<T>* q, long qld, cplx<T>* x,
-                                                const cplx<T>* dv, long r0, long stride, long K, const cplx<T>* R,
-                                                double* rsr, double* rsi) {
+                                                const cplx<T>* dv, long r0, long stride, long K) {
   double acc = 0;
   for (long r = r0; r < K; r += stride) {
     const cplx<T> xv = x[r];
@@ -583,11 +621,6 @@ __device__ __forceinline__ double qproject_rows(const c64* cf, const cplx<T>* q,
     cplx<T> e[NQ];
 #pragma unroll
     for (int c = 0; c < NQ; ++c) e[c] = q[c * qld + r];
-    cplx<T> f[SCHUR ? NQ : 1];
-    if constexpr (SCHUR) {
-#pragma unroll
-      for (int c = 0; c < NQ; ++c) f[c] = R[c * qld + r];
-    }
     double nx = xv.x, ny = xv.y;
 #pragma unroll
     for (int c = 0; c < NQ; ++c) {
@@ -597,54 +630,56 @@ __device__ __forceinline__ double qproject_rows(const c64* cf, const cplx<T>* q,
     const cplx<T> xn{T(nx), T(ny)};
     x[r] = xn;
     if (DOT) acc += double(dr.x) * double(xn.x) + double(dr.y) * double(xn.y);
-    if constexpr (SCHUR) {
-#pragma unroll
-      for (int c = 0; c < NQ; ++c) {
-        rsr[c] += double(f[c].x) * double(xn.x) + double(f[c].y) * double(xn.y);
-        rsi[c] += double(f[c].x) * double(xn.y) - double(f[c].y) * double(xn.x);
-      }
-    }
   }
   return acc;
 }
 
-template <typename T, int QM, bool SCHUR, int NQ = 1>
+template <typename T, int QM, int NQ = 1>
 __device__ __forceinline__ double qproject_cols(int n, const c64* cf, const cplx<T>* q, long qld, cplx<T>* x,
-                                                const cplx<T>* dv, long r0, long stride, long K, const cplx<T>* R,
-                                                double* rsr, double* rsi) {
+                                                const cplx<T>* dv, long r0, long stride, long K) {
   if constexpr (NQ <= QM) {
-    if (n == NQ) {
-      if constexpr (SCHUR)
-        return qproject_rows<T, NQ, true, true>(cf, q, qld, x, dv, r0, stride, K, R, rsr, rsi);
-      else
-        return dv ? qproject_rows<T, NQ, true, false>(cf, q, qld, x, dv, r0, stride, K, R, rsr, rsi)
-                  : qproject_rows<T, NQ, false, false>(cf, q, qld, x, dv, r0, stride, K, R, rsr, rsi);
-    }
-    return qproject_cols<T, QM, SCHUR, NQ + 1>(n, cf, q, qld, x, dv, r0, stride, K, R, rsr, rsi);
+    if (n == NQ)
+      return dv ? qproject_rows<T, NQ, true>(cf, q, qld, x, dv, r0, stride, K)
+                : qproject_rows<T, NQ, false>(cf, q, qld, x, dv, r0, stride, K);
+    return qproject_cols<T, QM, NQ + 1>(n, cf, q, qld, x, dv, r0, stride, K);
   }
   return 0.0;
 }
 
 // Block projection: partials of <Q_c, x> (c < nq[i], complex, FP64) over this block's
 // rows into part[(i gridDim.x + blockIdx.x) QM + c] (zero for c >= nq[i])
-template <typename T, int QM>
-__global__ __launch_bounds__(AB) void k_qdot(const cplx<T>* Q, long qld, long qis, const int* nq, const cplx<T>* X,
-                                             long ld, long K, const int* act, c64* part) {
+// With BOTH (k_minres_y1's Schur form) blockIdx.z = 1 takes the columns of R instead, into
+// part + gridDim.y gridDim.x QM, and blockIdx.z = 0 leaves the partials of Re <d_i, x_i> in
+// dpart[i gridDim.x + blockIdx.x].
+template <typename T, int QM, bool BOTH>
+__global__ __launch_bounds__(AB) void k_qdot(const cplx<T>* Q, const cplx<T>* R, long qld, long qis, const int* nq,
+                                             const cplx<T>* X, const cplx<T>* d, long ld, long K, const int* act,
+                                             c64* part, double* dpart) {
   const int i = blockIdx.y;
   const int n = act[i] ? nq[i] : 0;
-  __shared__ double wr[AB / 64][QM], wi[AB / 64][QM];
-  double sr[QM], si[QM];
+  const bool second = BOTH && blockIdx.z == 1;
+  __shared__ double wr[AB / 64][QM], wi[AB / 64][QM], wd[AB / 64];
+  double sr[QM], si[QM], acc = 0;
 #pragma unroll
   for (int c = 0; c < QM; ++c) sr[c] = si[c] = 0.0;
-  if (n > 0)
-    qdot_cols<T, QM>(n, Q + i * qis, qld, X + i * ld, long(blockIdx.x) * AB + threadIdx.x, long(gridDim.x) * AB, K,
-                     sr, si);
+  const long r0 = long(blockIdx.x) * AB + threadIdx.x, stride = long(gridDim.x) * AB;
+  if (n > 0) {
+    if (!BOTH)
+      qdot_cols<T, QM, false>(n, Q + i * qis, qld, X + i * ld, nullptr, r0, stride, K, sr, si);
+    else  // the second half's sum of <d, x> is not used
+      acc = qdot_cols<T, QM, true>(n, (second ? R : Q) + i * qis, qld, X + i * ld, d + i * ld, r0, stride, K, sr, si);
+  }
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const double a1 = wave_sums<QM>(sr, lane), b1 = wave_sums<QM>(si, lane);
   const int ix = wave_sums_index<QM>(lane);
   if (ix < QM) {  // lanes that hold the same sum store the same value
     wr[wv][ix] = a1;
     wi[wv][ix] = b1;
+  }
+  if (BOTH && !second) {
+    const double one[1] = {acc};
+    const double t = wave_sums<1>(one, lane);
+    if (lane == 0) wd[wv] = t;
   }
   __syncthreads();
   if (threadIdx.x < QM) {
@@ -654,18 +689,22 @@ __global__ __launch_bounds__(AB) void k_qdot(const cplx<T>* Q, long qld, long qi
       a += wr[w][c];
       b += wi[w][c];
     }
-    part[(long(i) * gridDim.x + blockIdx.x) * QM + c] = c64{a, b};
+    part[((second ? long(gridDim.y) : 0L) + i) * gridDim.x * QM + blockIdx.x * QM + c] = c64{a, b};
+  }
+  if (BOTH && !second && threadIdx.x == 0) {
+    double a = 0;
+    for (int w = 0; w < AB / 64; ++w) a += wd[w];
+    dpart[long(i) * gridDim.x + blockIdx.x] = a;
   }
 }
 
 // x_i <- x_i - sum_c <Q_c, x_i> Q_c (the block projection), the coefficients summed by every
 // block from k_qdot's qnblk partials of its instance in one fixed order; with d, the
-// partials of Re <d_i, x_i new> into part[i gridDim.x + blockIdx.x], and with SCHUR those of
-// <R_c, x_i new> into rpart[(i gridDim.x + blockIdx.x) QM + c] (zero past nq[i])
-template <typename T, int QM, bool SCHUR>
+// partials of Re <d_i, x_i new> into part[i gridDim.x + blockIdx.x]
+template <typename T, int QM>
 __global__ __launch_bounds__(AB) void k_qproject(const c64* qpart, int qnblk, const cplx<T>* Q, long qld, long qis,
                                                  const int* nq, cplx<T>* X, const cplx<T>* d, long ld, long K,
-                                                 const int* act, double* part, const cplx<T>* R, c64* rpart) {
+                                                 const int* act, double* part) {
   constexpr int G = AB / QM;
   const int i = blockIdx.y;
   __shared__ double red[AB];
@@ -700,34 +739,9 @@ __global__ __launch_bounds__(AB) void k_qproject(const c64* qpart, int qnblk, co
     c64 cf[QM];
 #pragma unroll
     for (int c = 0; c < QM; ++c) cf[c] = c < n ? cfs[c] : c64{0, 0};
-    double rsr[QM], rsi[QM];
-    if constexpr (SCHUR) {
-#pragma unroll
-      for (int c = 0; c < QM; ++c) rsr[c] = rsi[c] = 0.0;
-    }
     if (n > 0)
-      acc = qproject_cols<T, QM, SCHUR>(n, cf, Q + i * qis, qld, X + i * ld, d ? d + i * ld : nullptr,
-                                        long(blockIdx.x) * AB + threadIdx.x, long(gridDim.x) * AB, K,
-                                        SCHUR ? R + i * qis : nullptr, rsr, rsi);
-    if constexpr (SCHUR) {
-      // per column: each wavefront's sum, then the wavefronts in order
-      const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-      const double a1 = wave_sums<QM>(rsr, lane), b1 = wave_sums<QM>(rsi, lane);
-      const int ix = wave_sums_index<QM>(lane);
-      if (ix < QM) {
-        gr[wv][ix] = a1;
-        gi[wv][ix] = b1;
-      }
-      __syncthreads();
-      if (threadIdx.x < QM) {
-        double a = 0, b = 0;
-        for (int w = 0; w < AB / 64; ++w) {
-          a += gr[w][threadIdx.x];
-          b += gi[w][threadIdx.x];
-        }
-        rpart[(long(i) * gridDim.x + blockIdx.x) * QM + threadIdx.x] = c64{a, b};
-      }
-    }
+      acc = qproject_cols<T, QM>(n, cf, Q + i * qis, qld, X + i * ld, d ? d + i * ld : nullptr,
+                                 long(blockIdx.x) * AB + threadIdx.x, long(gridDim.x) * AB, K);
   }
   if (!part) return;
   red[threadIdx.x] = acc;
@@ -799,7 +813,7 @@ template <typename T> void VecOpsT<T>::set_block(const C* Qb, long qis, const in
   // the real dot partials (nb nblk, at the start, where the MINRES steps read them), then
   // the block partials (nb nblk QMAX complex): every block of k_qproject reads the latter
   // while others write the former, so the two never overlap
-  part.ensure(sizeof(c64) * size_t(nb) * (size_t(nblk) + 2 * size_t(nblk) * QMAX + RCQ));
+  part.ensure(sizeof(c64) * size_t(nb) * (size_t(nblk) + 2 * size_t(nblk) * QMAX + 3 * RCQ));
   Q = Qb;
   qistride = qis;
   qn = nq;
@@ -826,22 +840,25 @@ template <typename T> void VecOpsT<T>::set_schur(const C* Rb, const double* weig
   rg = weights;
 }
 
+// partials of Q^H x and R^H x (past the real partials) and of Re <d, x> (out)
+template <typename T> void VecOpsT<T>::dots_schur(const C* x, const int* act, const C* d, double* out) {
+  with_qm(qmax, [&](auto QMc) {
+    hipLaunchKernelGGL((k_qdot<T, decltype(QMc)::value, true>), dim3(qblk, nb, 2), dim3(AB), 0, s, Q, R, ld, qistride,
+                       qn, x, d, ld, K, act, part.template as<c64>() + size_t(nb) * nblk, out);
+  });
+}
+
 template <typename T> void VecOpsT<T>::project_dot_to(C* x, const int* act, const C* dot_with, double* out) {
   const dim3 g(nblk, nb);
   if (Q) {
     c64* qp = part.template as<c64>() + size_t(nb) * nblk;
     const dim3 gq(qblk, nb);  // the projection's partials: qblk per instance too
-    // past the block partials: the residual columns' partials, and the coefficients from them
-    c64* rp = qp + size_t(nb) * nblk * QMAX;
     auto launch = [&](auto QMc) {
       constexpr int QMv = decltype(QMc)::value;
-      hipLaunchKernelGGL((k_qdot<T, QMv>), gq, dim3(AB), 0, s, Q, ld, qistride, qn, x, ld, K, act, qp);
-      if (R && dot_with)
-        hipLaunchKernelGGL((k_qproject<T, QMv, true>), gq, dim3(AB), 0, s, qp, qblk, Q, ld, qistride, qn, x, dot_with, ld,
-                           K, act, out, R, rp);
-      else
-        hipLaunchKernelGGL((k_qproject<T, QMv, false>), gq, dim3(AB), 0, s, qp, qblk, Q, ld, qistride, qn, x, dot_with,
-                           ld, K, act, out, R, rp);
+      hipLaunchKernelGGL((k_qdot<T, QMv, false>), gq, dim3(AB), 0, s, Q, R, ld, qistride, qn, x, dot_with, ld, K, act,
+                         qp, out);
+      hipLaunchKernelGGL((k_qproject<T, QMv>), gq, dim3(AB), 0, s, qp, qblk, Q, ld, qistride, qn, x, dot_with, ld, K,
+                         act, out);
     };
     with_qm(qmax, launch);
     return;
@@ -914,12 +931,16 @@ int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shi
   const OpPlan<T>& plan = S.pd<T>().plan;
   // y = P r1 (projected)
   launch_operator<T>(OP_P, plan, R1v, Yv, dm, sel, dk, nullptr, 0, s);
-  V.project(y, act, r1);  // and the partials of <r1, y>
+  // and the partials of <r1, y>; with the Schur term y stays as it is, k_minres_y1 projects it
+  if (V.R)
+    V.dots_schur(y, act, r1, part);
+  else
+    V.project(y, act, r1);
   const int qm = qm_of(V.qmax);
-  const c64* rpart = V.R ? V.part.template as<c64>() + size_t(nb) * nblk * (1 + VecOpsT<T>::QMAX) : nullptr;
-  c64* rc = V.R ? V.part.template as<c64>() + size_t(nb) * nblk * (1 + 2 * VecOpsT<T>::QMAX) : nullptr;
+  const c64* qpart = V.R ? V.part.template as<c64>() + size_t(nb) * nblk : nullptr;
+  c64* qrc = V.R ? V.part.template as<c64>() + size_t(nb) * nblk * (1 + 2 * VecOpsT<T>::QMAX) : nullptr;
   const int pblk = V.Q ? V.qblk : nblk;  // partials per instance a projection leaves
-  hipLaunchKernelGGL(k_minres_scalars, dim3(nb), dim3(AB), 0, s, ms, part, pblk, coef, 0, nb, act, rpart, qm, V.rg, rc);
+  hipLaunchKernelGGL(k_minres_scalars, dim3(nb), dim3(AB), 0, s, ms, part, pblk, coef, 0, nb, act, qpart, qm, V.rg, qrc);
   OMX_HIP_CHECK(hipMemcpyAsync(r2, r1, vb, hipMemcpyDeviceToDevice, s));
   std::vector<int> live(want);
   int it = 0;
@@ -942,7 +963,7 @@ int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shi
       constexpr bool wx = decltype(WXc)::value;
       hipLaunchKernelGGL((k_minres_y1<T, wx, decltype(QMc)::value>), vg, dim3(AB), 0, s, ms, avp, y, r1, v, ld, V.K, la,
                          part, wx ? pw1 : nullptr, wx ? pw2 : nullptr, wx ? pwo : nullptr, wx ? x : nullptr,
-                         wx ? coef + 4 * nb : nullptr, V.R, V.qistride, V.qn, rc);
+                         wx ? coef + 4 * nb : nullptr, V.Q, V.R, V.qistride, V.qn, qrc);
     };
     auto y1q = [&](auto WXc) {
       if (!V.R)
@@ -963,9 +984,12 @@ int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shi
     BView<T> R2b{r2, ld, ld}, Yb{yn, ld, ld};
     launch_operator<T>(OP_P, plan, R2b, Yb, dm, sel, dk, nullptr, 0, s);
     // yn <- yn - ev <ev, yn> (or the block projection) with the partials of <r2, yn>
-    V.project_dot_to(yn, la, r2, cpart2);
-    hipLaunchKernelGGL(k_minres_scalars, dim3(nb), dim3(AB), 0, s, ms, cpart2, pblk, coef, 3, nb, la, rpart, qm,
-                       V.rg, rc);
+    if (V.R)
+      V.dots_schur(yn, la, r2, cpart2);
+    else
+      V.project_dot_to(yn, la, r2, cpart2);
+    hipLaunchKernelGGL(k_minres_scalars, dim3(nb), dim3(AB), 0, s, ms, cpart2, pblk, coef, 3, nb, la, qpart, qm,
+                       V.rg, qrc);
     // this iteration's w/x update, pending (its v is u, the next iteration's v-buffer)
     pw1 = w2;
     pw2 = w;

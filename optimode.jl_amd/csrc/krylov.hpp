@@ -45,8 +45,12 @@ template <typename T> struct VecOpsT {
   // With a block whose columns are Ritz vectors but not yet eigenvectors, the system on its
   // complement is the Schur complement (M - shift) - sum_c g_c R_c R_c^H, R_c = M Q_c - theta_c
   // Q_c (laid out as the block), g_c = 1 / (theta_c - shift) (weights: QMAX per instance, 0
-  // leaves a column out).  minres_complement_t then applies it in place of M - shift.
+  // leaves a column out; then theta_c - shift, QMAX per instance too, per instance after its
+  // weights).  minres_complement_t then applies it in place of M - shift, and the block's
+  // columns must satisfy Q^H R = 0 (Ritz vectors of the block).
   void set_schur(const C* Rb, const double* weights);
+  // partials of Q^H x and R^H x, for k_minres_scalars, and of Re <d_i, x_i> into out
+  void dots_schur(const C* x, const int* act, const C* d, double* out);
   const C* R = nullptr;
   const double* rg = nullptr;
   const C* Q = nullptr;

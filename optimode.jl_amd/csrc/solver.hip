@@ -1613,7 +1613,7 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
   const OpPlan<double>& plan = S.p64.plan;
   std::vector<int> n1h(ninst, 0), jdh(ninst, 0);
   std::vector<double> lam_band(ninst, 0.0), rn(ninst, 0.0);
-  std::vector<double> theta(size_t(ninst) * RF_MAXC, 0.0), schur(size_t(ninst) * VecOpsT<float>::QMAX, 0.0);
+  std::vector<double> theta(size_t(ninst) * RF_MAXC, 0.0), schur(size_t(ninst) * 2 * VecOpsT<float>::QMAX, 0.0);
   std::vector<c64> hG(size_t(ninst) * RF_PAIRS), hB(size_t(ninst) * RF_PAIRS), hC(size_t(ninst) * RF_PAIRS);
   auto up_n1 = [&](const std::vector<int>& v) {
     OMX_HIP_CHECK(hipMemcpyAsync(n1d.as<void>(), v.data(), sizeof(int) * ninst, hipMemcpyHostToDevice, s));
@@ -1752,8 +1752,9 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
             for (int i = 0; i < ninst; ++i)
               for (int l = 0; l < VecOpsT<float>::QMAX; ++l) {
                 const double d = l < msize[i] ? theta[size_t(i) * RF_MAXC + l] - lam_band[i] : 0.0;
-                schur[size_t(i) * VecOpsT<float>::QMAX + l] =
-                    l != bands[i] && std::fabs(d) > 1e-3 * std::fabs(lam_band[i]) ? 1.0 / d : 0.0;
+                double* w = schur.data() + size_t(i) * 2 * VecOpsT<float>::QMAX + l;
+                w[0] = l != bands[i] && std::fabs(d) > 1e-3 * std::fabs(lam_band[i]) ? 1.0 / d : 0.0;
+                w[VecOpsT<float>::QMAX] = d;
               }
             OMX_HIP_CHECK(hipMemcpyAsync(W.rgd.as<void>(), schur.data(), sizeof(double) * schur.size(),
                                          hipMemcpyHostToDevice, s));
