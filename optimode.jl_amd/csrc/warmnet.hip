@@ -15,7 +15,6 @@ namespace {
 constexpr int TB = 256;
 constexpr int TS = 16;   // output tile edge of a convolution block (TS x TS = TB threads)
 constexpr int COB = 8;   // output channels per convolution block
-constexpr int WG = 4;    // output channels per weight-gradient block
 constexpr int NBL = 256; // blocks of the field-loss reduction
 
 // 3x3 convolution, zero padding: out[b][o][y][x] = act(bias[o] + sum_i sum_t
@@ -73,17 +72,21 @@ __global__ __launch_bounds__(TB) void k_conv(const float* in, int cin, const flo
   }
 }
 
-// The same convolution on the matrix cores: an implicit GEMM, out (16 output channels x the
-// 256 pixels of a TS x TS tile) = W (16 x 9 cin) . im2col(in) (9 cin x 256), contracted in
-// steps of 16 with v_mfma_f32_16x16x16bf16_1k: bf16 operands (round to nearest even of the
-// FP32 weights and activations), FP32 accumulation.  The block stages the input halo of all
-// cin channels and its 16 output channels' weights in LDS (FP32); wave w computes tile rows
-// 4w .. 4w + 3, one 16 x 16 MFMA tile (16 channels x the 16 pixels of a row) each.  Operand
+// The same convolution on the matrix cores: an implicit GEMM, out (16 NM output channels x the
+// 256 pixels of a TS x TS tile) = W . im2col(in), contracted in steps of 16 with
+// v_mfma_f32_16x16x16bf16_1k: bf16 operands (round to nearest even of the FP32 weights and
+// activations), FP32 accumulation.  The contraction runs tap by tap over the channels (cp =
+// cin rounded up to 16), so that the 4 consecutive k of a lane are 4 channels of one pixel:
+// the block stages its input halo as [pixel][channel] and its weights as [output][tap][channel]
+// in LDS, already in bf16, and an operand is one 8-byte read.  Rows of both are padded to 16
+// mod 32 values, which spreads the 16 rows of a read over all banks.  Wave w computes tile
+// rows 4w .. 4w + 3, NM 16 x 16 MFMA tiles (16 channels x the 16 pixels of a row) each.  Operand
 // layout of the instruction: A lane l -> (row l%16, k 4(l/16) + j), B lane l -> (k 4(l/16)
 // + j, column l%16), accumulator register j of lane l -> (row 4(l/16) + j, column l%16).
+// Bound: the halo's loads and the conversion, once per value.  64 x 64 maps, 8 bands, 16
+// samples: 29 us a call against 53 with FP32 in LDS, converted at every read, 16 outputs a block.
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-constexpr int CMX_CO = 16;   // output channels per MFMA convolution block
 constexpr int HALO = (TS + 2) * (TS + 2);
 
 __device__ __forceinline__ short bf16_rne(float f) {
@@ -92,58 +95,65 @@ __device__ __forceinline__ short bf16_rne(float f) {
   return short(u >> 16);
 }
 
-template <bool BWD>
+__host__ __device__ constexpr int mfma_pad(int n) { return n % 32 == 0 ? n + 16 : n; }  // n: a multiple of 16
+__host__ __device__ constexpr int round16(int n) { return (n + 15) / 16 * 16; }
+
+template <bool BWD, int NM>
 __global__ __launch_bounds__(TB) void k_conv_mfma(const float* in, int cin, const float* w, const float* bias,
                                                   float* out, int cout, int res, int relu) {
-  extern __shared__ __align__(16) float smf[];
-  const int kin = cin * 9, kp = ((kin + 15) / 16) * 16;
-  float* tile = smf;                 // [cin][TS + 2][TS + 2]
-  float* ws = smf + long(cin) * HALO;  // [CMX_CO][kp]
+  extern __shared__ __align__(16) short smh[];
+  const int cp = round16(cin), cs = mfma_pad(cp), ks = mfma_pad(9 * cp);
+  short* tile = smh;             // [HALO][cs]
+  short* ws = smh + HALO * cs;   // [16 NM][ks]
   const int ntx = (res + TS - 1) / TS;
   const int ty0 = (int(blockIdx.x) / ntx) * TS, tx0 = (int(blockIdx.x) % ntx) * TS;
-  const int o0 = blockIdx.y * CMX_CO;
+  const int o0 = blockIdx.y * 16 * NM;
   const int b = blockIdx.z;
   const long plane = long(res) * res;
   const float* inb = in + long(b) * cin * plane;
-  for (int e = threadIdx.x; e < cin * HALO; e += TB) {
-    const int i = e / HALO, q = e - i * HALO, r = q / (TS + 2), c = q - r * (TS + 2);
+#pragma unroll 4
+  for (int e = threadIdx.x; e < cp / 4 * HALO; e += TB) {
+    const int i = e / HALO * 4, q = e % HALO, r = q / (TS + 2), c = q - r * (TS + 2);
     const int yy = ty0 + r - 1, xx = tx0 + c - 1;
-    tile[e] = (yy >= 0 && yy < res && xx >= 0 && xx < res) ? inb[long(i) * plane + long(yy) * res + xx] : 0.f;
+    const bool ok = yy >= 0 && yy < res && xx >= 0 && xx < res;
+    const float* ip = inb + long(i) * plane + long(yy) * res + xx;
+    bf16x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = ok && i + j < cin ? bf16_rne(ip[j * plane]) : short(0);
+    *reinterpret_cast<bf16x4*>(tile + q * cs + i) = v;
   }
-  for (int e = threadIdx.x; e < CMX_CO * kp; e += TB) {
-    const int j = e / kp, k = e - j * kp, o = o0 + j;
-    float v = 0.f;
-    if (o < cout && k < kin) {
-      const int i = k / 9, t = k - i * 9;
-      v = BWD ? w[(long(i) * cout + o) * 9 + 8 - t] : w[(long(o) * cin + i) * 9 + t];
-    }
-    ws[e] = v;
+  // one (output, input) pair per thread and round: its 9 taps
+#pragma unroll 2
+  for (int e = threadIdx.x; e < 16 * NM * cp; e += TB) {
+    const int j = BWD ? e % (16 * NM) : e / cp, i = BWD ? e / (16 * NM) : e % cp, o = o0 + j;
+    const bool ok = o < cout && i < cin;
+    const float* wp = w + (BWD ? long(i) * cout + o : long(o) * cin + i) * 9;
+#pragma unroll
+    for (int t = 0; t < 9; ++t) ws[j * ks + t * cp + i] = ok ? bf16_rne(wp[BWD ? 8 - t : t]) : short(0);
   }
   __syncthreads();
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int lr = lane & 15, lg = lane >> 4;
-  f32x4 acc[4];
+  f32x4 acc[4][NM];
 #pragma unroll
-  for (int rr = 0; rr < 4; ++rr) acc[rr] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < kp; k0 += 16) {
-    bf16x4 a;
-    int off[4];
-    bool ok[4];
+  for (int rr = 0; rr < 4; ++rr)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int k = k0 + 4 * lg + j;
-      a[j] = bf16_rne(ws[lr * kp + k]);
-      ok[j] = k < kin;
-      const int i = ok[j] ? k / 9 : 0, t = k - (k / 9) * 9;
-      off[j] = i * HALO + (t / 3) * (TS + 2) + lr + t % 3;  // tap t of pixel (row 0, column lr)
-    }
+    for (int m = 0; m < NM; ++m) acc[rr][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      const int ly = wv * 4 + rr;
-      bf16x4 bv;
+  for (int t = 0; t < 9; ++t) {
+    const short* tp = tile + ((wv * 4 + t / 3) * (TS + 2) + lr + t % 3) * cs + 4 * lg;
+    const short* wt = ws + lr * ks + t * cp + 4 * lg;
+    for (int c0 = 0; c0 < cp; c0 += 16) {
+      bf16x4 a[NM];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) bv[j] = ok[j] ? bf16_rne(tile[off[j] + ly * (TS + 2)]) : short(0);
-      acc[rr] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bv, acc[rr], 0, 0, 0);
+      for (int m = 0; m < NM; ++m) a[m] = *reinterpret_cast<const bf16x4*>(wt + m * 16 * ks + c0);
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        const bf16x4 bv = *reinterpret_cast<const bf16x4*>(tp + rr * (TS + 2) * cs + c0);
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+          acc[rr][m] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], bv, acc[rr][m], 0, 0, 0);
+      }
     }
   }
   const int x = tx0 + lr;
@@ -152,74 +162,123 @@ __global__ __launch_bounds__(TB) void k_conv_mfma(const float* in, int cin, cons
     const int y = ty0 + wv * 4 + rr;
     if (y >= res || x >= res) continue;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int o = o0 + 4 * lg + j;
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int o = o0 + 16 * m + 4 * lg + j;
+        if (o >= cout) continue;
+        float v = acc[rr][m][j] + (bias ? bias[o] : 0.f);
+        if (relu) v = fmaxf(v, 0.f);
+        out[(long(b) * cout + o) * plane + long(y) * res + x] = v;
+      }
+  }
+}
+
+// Weight gradient on the FP32 matrix cores: dw[(o cin + i) 9 + t] = sum_b sum_p dout[b][o][p]
+// in[b][i][p + off_t] and db[o] = sum_b sum_p dout[b][o][p], a GEMM of (32 outputs) x (9 taps of
+// 16 input channels) contracted over the pixels in steps of 4 (v_mfma_f32_16x16x4f32: A lane l ->
+// (row l%16, k l/16), B lane l -> (k l/16, column l%16), accumulators as above).
+// Block (split, group of 16 inputs, group of 32 outputs) takes its split's share of the tiles of
+// all samples: input halo and dout tile in LDS (FP32, row strides 4 mod 64: no bank conflicts),
+// wave w the 16-pixel rows 4w .. 4w + 3; a B operand serves 2 MFMAs, an A operand 9 (10 with the
+// ones column of db).  The waves' sums are added in order through LDS and the splits' by
+// k_wgrad_sum: every value in one fixed order.  One block per (input, 4 outputs) walking all
+// samples' pixels left most CUs idle and re-read dout per input (64 x 64 maps, 8 bands, 16
+// samples, all six layers: 1.26 ms; this form 0.22 and its sums 0.03).
+constexpr int WGI = 16, WGO = 32;            // input and output channels of a block
+constexpr int WG_TS = HALO, WG_DS = TS * TS + 4;  // LDS row strides: 324 = 260 = 4 mod 64
+constexpr int WG_VALS = 2 * 10 * 256;        // values a wave ends with: 2 row tiles, 9 taps and db
+constexpr size_t WG_LDS_TILES = sizeof(float) * (WGI * WG_TS + WGO * WG_DS);
+constexpr size_t WG_LDS = WG_LDS_TILES > sizeof(float) * 4 * WG_VALS / 2 ? WG_LDS_TILES : sizeof(float) * 4 * WG_VALS / 2;
+__global__ __launch_bounds__(TB) void k_conv_wgrad(const float* in, int cin, const float* dout, int cout, int res,
+                                                   int ntiles, float* part) {
+  extern __shared__ __align__(16) float smf[];
+  float* tin = smf;                  // [WGI][WG_TS]
+  float* td = smf + WGI * WG_TS;     // [WGO][WG_DS]
+  const int i0 = blockIdx.y * WGI, o0 = blockIdx.z * WGO;
+  const int ntx = (res + TS - 1) / TS;
+  const long plane = long(res) * res;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lr = lane & 15, lg = lane >> 4;
+  const bool bias = blockIdx.y == 0;
+  f32x4 acc[2][10];
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int t = 0; t < 10; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int tl = blockIdx.x; tl < ntiles; tl += gridDim.x) {
+    const int b = tl / (ntx * ntx), q = tl - b * ntx * ntx, ty0 = q / ntx * TS, tx0 = q % ntx * TS;
+    const float* ib = in + (long(b) * cin + i0) * plane;
+    const float* db = dout + (long(b) * cout + o0) * plane;
+    __syncthreads();  // the tile before is read
+#pragma unroll 7
+    for (int e = threadIdx.x; e < WGI * HALO; e += TB) {
+      const int i = e / HALO, h = e - i * HALO, r = h / (TS + 2), c = h - r * (TS + 2);
+      const int yy = ty0 + r - 1, xx = tx0 + c - 1;
+      tin[e] = i0 + i < cin && yy >= 0 && yy < res && xx >= 0 && xx < res ? ib[i * plane + long(yy) * res + xx] : 0.f;
+    }
+    const int y = ty0 + int(threadIdx.x) / TS, x = tx0 + int(threadIdx.x) % TS;
+    const bool ok = y < res && x < res;
+#pragma unroll 8
+    for (int o = 0; o < WGO; ++o)
+      td[o * WG_DS + threadIdx.x] = ok && o0 + o < cout ? db[o * plane + long(y) * res + x] : 0.f;
+    __syncthreads();
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr)
+#pragma unroll
+      for (int xc = 0; xc < TS; xc += 4) {
+        const int py = wv * 4 + rr, px = xc + lg;
+        const float a0 = td[lr * WG_DS + py * TS + px], a1 = td[(16 + lr) * WG_DS + py * TS + px];
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+          const float bv = tin[lr * WG_TS + (py + t / 3) * (TS + 2) + px + t % 3];
+          acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, bv, acc[0][t], 0, 0, 0);
+          acc[1][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, bv, acc[1][t], 0, 0, 0);
+        }
+        if (bias) {
+          acc[0][9] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, 1.f, acc[0][9], 0, 0, 0);
+          acc[1][9] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, 1.f, acc[1][9], 0, 0, 0);
+        }
+      }
+  }
+  // the waves' sums, one row tile at a time, value (t, j, lane) of wave w at w 2560 + (4t + j) 64 + lane
+  float* wsum = smf;
+  const int nw = cout * cin * 9;
+  float* pw = part + long(blockIdx.x) * (nw + cout);
+  for (int m = 0; m < 2; ++m) {
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 10; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) wsum[(wv * 40 + 4 * t + j) * 64 + lane] = m ? acc[1][t][j] : acc[0][t][j];
+    __syncthreads();
+    for (int e = threadIdx.x; e < 40 * 64; e += TB) {
+      const int l = e & 63, tj = e >> 6, t = tj >> 2, o = o0 + 16 * m + 4 * (l >> 4) + (tj & 3), i = i0 + (l & 15);
+      const float v = ((wsum[e] + wsum[40 * 64 + e]) + wsum[80 * 64 + e]) + wsum[120 * 64 + e];
       if (o >= cout) continue;
-      float v = acc[rr][j] + (bias ? bias[o] : 0.f);
-      if (relu) v = fmaxf(v, 0.f);
-      out[(long(b) * cout + o) * plane + long(y) * res + x] = v;
+      if (t < 9) {
+        if (i < cin) pw[(long(o) * cin + i) * 9 + t] = v;
+      } else if (bias && (l & 15) == 0) {
+        pw[nw + o] = v;
+      }
     }
   }
 }
 
-// Weight gradient: dw[(o cin + i) 9 + t] = sum_b sum_p dout[b][o][p] in[b][i][p + off_t] and
-// (blocks with i = 0) db[o] = sum_b sum_p dout[b][o][p]; block (i, group of WG outputs); each
-// value reduced per wavefront by a fixed butterfly, then over the wavefronts in order.
-__global__ __launch_bounds__(TB) void k_conv_wgrad(const float* in, int cin, const float* dout, int cout, int res,
-                                                   int B, float* dw, float* db) {
-  const int i = blockIdx.x, o0 = blockIdx.y * WG;
-  const long plane = long(res) * res;
-  float acc[WG][9], bacc[WG];
-#pragma unroll
-  for (int j = 0; j < WG; ++j) {
-    bacc[j] = 0.f;
-#pragma unroll
-    for (int t = 0; t < 9; ++t) acc[j][t] = 0.f;
-  }
-  for (long e = threadIdx.x; e < long(B) * plane; e += TB) {
-    const int b = int(e / plane);
-    const long p = e - long(b) * plane;
-    const int y = int(p / res), x = int(p - long(p / res) * res);
-    const float* ip = in + (long(b) * cin + i) * plane;
-    float v[9];
-#pragma unroll
-    for (int t = 0; t < 9; ++t) {
-      const int yy = y + t / 3 - 1, xx = x + t % 3 - 1;
-      v[t] = (yy >= 0 && yy < res && xx >= 0 && xx < res) ? ip[long(yy) * res + xx] : 0.f;
-    }
-#pragma unroll
-    for (int j = 0; j < WG; ++j) {
-      const int o = o0 + j;
-      const float d = o < cout ? dout[(long(b) * cout + o) * plane + p] : 0.f;
-      bacc[j] += d;
-#pragma unroll
-      for (int t = 0; t < 9; ++t) acc[j][t] += d * v[t];
-    }
-  }
-  constexpr int NV = WG * 10, NW = TB / 64;
-  __shared__ float red[NW][NV];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int q = 0; q < NV; ++q) {
-    float v = q < WG * 9 ? acc[q / 9][q % 9] : bacc[q - WG * 9];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (lane == 0) red[wave][q] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < NV) {
-    const int q = threadIdx.x;
-    float s = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) s += red[w][q];
-    if (q < WG * 9) {
-      const int o = o0 + q / 9;
-      if (o < cout) dw[(long(o) * cin + i) * 9 + q % 9] = s;
-    } else {
-      const int o = o0 + (q - WG * 9);
-      if (i == 0 && o < cout) db[o] = s;
-    }
-  }
+// dw (nw values) and db from the splits' partials, in order
+__global__ __launch_bounds__(64) void k_wgrad_sum(const float* part, int splits, int nw, int n, float* dw, float* db) {
+  const int e = blockIdx.x * 64 + threadIdx.x;
+  if (e >= n) return;
+  float s = 0.f;
+#pragma unroll 16
+  for (int q = 0; q < splits; ++q) s += part[long(q) * n + e];
+  (e < nw ? dw + e : db + (e - nw))[0] = s;
+}
+
+// splits of k_conv_wgrad: about a block per CU over all channel groups, each with at least a tile
+int wgrad_splits(int cin, int cout, int ntiles) {
+  const int groups = (cin + WGI - 1) / WGI * ((cout + WGO - 1) / WGO);
+  return std::max(1, std::min(ntiles, (256 + groups - 1) / groups));
 }
 
 // 2x2 average pooling: out (B C planes of h x h) from in (planes of 2h x 2h)
@@ -572,19 +631,34 @@ void WarmNet::ensure_batch(int B) {
   dk_.alloc(f * nev_);
   dg_.alloc(f * 32);
   part_.alloc(sizeof(double) * (NBL + 1));
+  size_t wn = 0;
+  for (const Conv& c : c_) {
+    const int nt = (c.res + TS - 1) / TS;
+    wn = std::max(wn, size_t(wgrad_splits(c.ci, c.co, nt * nt * B)) * (size_t(c.co) * c.ci * 9 + c.co));
+  }
+  wpart_.alloc(sizeof(float) * wn);
   B_ = B;
 }
 
-static size_t conv_mfma_lds(int cin) {
-  return sizeof(float) * (size_t(cin) * HALO + size_t(CMX_CO) * (((cin * 9 + 15) / 16) * 16));
+// One block for up to 32 output channels: the halo is staged once (16 channels: half the MFMAs
+// would work on padding)
+template <bool BWD>
+static void launch_conv_mfma(const float* in, int cin, const float* w, const float* bias, float* out, int cout, int res,
+                             int B, int relu, hipStream_t s) {
+  const int nt = (res + TS - 1) / TS, cp = round16(cin), nm = cout <= 16 ? 1 : 2;
+  const size_t lds = sizeof(short) * (size_t(HALO) * mfma_pad(cp) + size_t(16 * nm) * mfma_pad(9 * cp));
+  const dim3 g(nt * nt, (cout + 16 * nm - 1) / (16 * nm), B);
+  if (nm == 1)
+    hipLaunchKernelGGL((k_conv_mfma<BWD, 1>), g, dim3(TB), lds, s, in, cin, w, bias, out, cout, res, relu);
+  else
+    hipLaunchKernelGGL((k_conv_mfma<BWD, 2>), g, dim3(TB), lds, s, in, cin, w, bias, out, cout, res, relu);
 }
 
 void WarmNet::conv(const Conv& c, const float* in, float* out, int B, bool relu) {
   const int nt = (c.res + TS - 1) / TS;
   const float* P = P_.as<float>();
   if (bf16_)
-    hipLaunchKernelGGL(k_conv_mfma<false>, dim3(nt * nt, (c.co + CMX_CO - 1) / CMX_CO, B), dim3(TB),
-                       conv_mfma_lds(c.ci), s_, in, c.ci, P + c.w, P + c.b, out, c.co, c.res, relu ? 1 : 0);
+    launch_conv_mfma<false>(in, c.ci, P + c.w, P + c.b, out, c.co, c.res, B, relu ? 1 : 0, s_);
   else
     hipLaunchKernelGGL(k_conv<false>, dim3(nt * nt, (c.co + COB - 1) / COB, B), dim3(TB), 0, s_, in, c.ci, P + c.w,
                        P + c.b, out, c.co, c.res, relu ? 1 : 0);
@@ -592,13 +666,15 @@ void WarmNet::conv(const Conv& c, const float* in, float* out, int B, bool relu)
 
 void WarmNet::conv_bwd(const Conv& c, const float* in, const float* dout, float* din, int B) {
   float* G = G_.as<float>();
-  hipLaunchKernelGGL(k_conv_wgrad, dim3(c.ci, (c.co + WG - 1) / WG), dim3(TB), 0, s_, in, c.ci, dout, c.co, c.res, B,
-                     G + c.w, G + c.b);
+  const int nt = (c.res + TS - 1) / TS, nw = c.co * c.ci * 9, n = nw + c.co;
+  const int splits = wgrad_splits(c.ci, c.co, nt * nt * B);
+  hipLaunchKernelGGL(k_conv_wgrad, dim3(splits, (c.ci + WGI - 1) / WGI, (c.co + WGO - 1) / WGO), dim3(TB), WG_LDS, s_,
+                     in, c.ci, dout, c.co, c.res, nt * nt * B, wpart_.as<float>());
+  hipLaunchKernelGGL(k_wgrad_sum, dim3((n + 63) / 64), dim3(64), 0, s_, wpart_.as<float>(), splits, nw, n, G + c.w,
+                     G + c.b);
   if (din) {
-    const int nt = (c.res + TS - 1) / TS;
     if (bf16_)
-      hipLaunchKernelGGL(k_conv_mfma<true>, dim3(nt * nt, (c.ci + CMX_CO - 1) / CMX_CO, B), dim3(TB),
-                         conv_mfma_lds(c.co), s_, dout, c.co, P_.as<float>() + c.w, nullptr, din, c.ci, c.res, 0);
+      launch_conv_mfma<true>(dout, c.co, P_.as<float>() + c.w, nullptr, din, c.ci, c.res, B, 0, s_);
     else
       hipLaunchKernelGGL(k_conv<true>, dim3(nt * nt, (c.ci + COB - 1) / COB, B), dim3(TB), 0, s_, dout, c.co,
                          P_.as<float>() + c.w, nullptr, din, c.ci, c.res, 0);

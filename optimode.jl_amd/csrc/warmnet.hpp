@@ -81,7 +81,7 @@ class WarmNet {
   DevMem P_, G_, M1_, M2_;  // parameters, gradient, Adam moments
   int B_ = 0;               // batch capacity of the activation buffers
   DevMem x_, a1_, p1_, a2_, p2_, a3_, g_, k_, cat4_, a4_, cat5_, a5_, y_;
-  DevMem dy_, da5_, dcat5_, da4_, dcat4_, da3_, dp2_, da2_, dp1_, da1_, dk_, dg_, part_, lossd_;
+  DevMem dy_, da5_, dcat5_, da4_, dcat4_, da3_, dp2_, da2_, dp1_, da1_, dk_, dg_, part_, lossd_, wpart_;
   DevMem dft_, low_;  // inverse-DFT intermediate and result of guess_device
   long adam_t_ = 0;
 

@@ -70,6 +70,26 @@ def test_bf16_mfma_convolutions_match_oracle_to_bf16(hw, nev, B):
     assert np.max(np.abs(y32 - yr)) < 1e-5 * np.max(np.abs(yr))
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("hw,nev,B", [(4, 1, 1), (12, 16, 2), (20, 5, 3), (36, 9, 2)])
+def test_convolutions_at_tile_and_channel_remainders(hw, nev, B, bf16):
+    """Planes of 1 to 36 pixels an edge (tiles of 16: 20 and 36 leave 4, the smaller ones part
+    of a tile), 4 to 64 field channels (groups of 16 and 32), a weight gradient of one tile and
+    of several per split.  FP32: rounding of 1e-6 with a factor for six layers of sums; bf16
+    convolutions: 2^-9 per operand, twelve operands deep, times 4 for the largest of the values."""
+    print(f"warmnet remainders hw {hw} nev {nev} B {B} bf16 {bf16}", flush=True)
+    p, x, tf, tk = _rand_case(hw, nev, B, 3)
+    net = WS.WarmNet(hw, nev, bf16=bf16)
+    net.params = p
+    y, _ = net.forward(x)
+    yr, _ = W.forward(p.astype(np.float64), x, hw, nev)
+    _, g = net.loss_grad(x, tf, tk, 0.5)
+    _, gr = W.loss_grad(p.astype(np.float64), x, tf, tk, 0.5, hw, nev)
+    ty, tg = (3e-2, 5e-2) if bf16 else (1e-5, 1e-5)
+    assert np.max(np.abs(y - yr)) < ty * np.max(np.abs(yr))
+    assert np.linalg.norm(g - gr) < tg * np.linalg.norm(gr)
+
+
 def test_training_reduces_loss_and_is_deterministic():
     hw, nev = 16, 2
     rng = np.random.default_rng(4)
