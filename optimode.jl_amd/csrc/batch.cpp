@@ -50,8 +50,15 @@ void solve_k_batch(int device, int nprob, omx_problem* probs, int max_group, int
     }
     buckets[std::make_tuple(p.nx, p.ny, p.Dx, p.Dy)].push_back(j);
   }
-  for (auto& kv : buckets) {
-    std::vector<int>& ids = kv.second;
+  DevCache cache;  // the grids' handles come and go: the next one takes the memory of the one before
+  // largest grids first: their blocks hold what the smaller ones need
+  std::vector<std::vector<int>*> order;
+  for (auto& kv : buckets) order.push_back(&kv.second);
+  std::stable_sort(order.begin(), order.end(), [&](const std::vector<int>* a, const std::vector<int>* b) {
+    return long(probs[(*a)[0]].nx) * probs[(*a)[0]].ny > long(probs[(*b)[0]].nx) * probs[(*b)[0]].ny;
+  });
+  for (std::vector<int>* bucket : order) {
+    std::vector<int>& ids = *bucket;
     std::stable_sort(ids.begin(), ids.end(), [&](int a, int b) { return probs[a].nev > probs[b].nev; });
     const omx_problem& p0 = probs[ids[0]];
     std::unique_ptr<Solver> h;

@@ -67,38 +67,46 @@ template <> PrecisionData<double>& Solver::pd<double>() { return p64; }
 
 // A symmetric per-pixel 3x3 field (column-major (3,3,Nx,Ny) or (3,3,Nx,Ny,Nz), FP64 host) in
 // the two device layouts the operator reads: 6 unique entries xx, yy, zz, xy, xz, yz per
-// pixel, row-major (iz, iy, ix) and column-major per plane (iz, ix, iy).
+// pixel, row-major (iz, iy, ix) and column-major per plane (iz, ix, iy: pixel (ix, iy, iz) at
+// 6 (iy + ny (ix + nx iz))).  The field goes up as it is and the device makes the layouts: on
+// the host the transposed copies of both precisions took 10 ms of a 512 x 256 solve's start.
 template <typename T>
-void upload_tensor6(const Solver& S, const double* E, DevMem& rowm, DevMem& colm) {
-  const long N = S.N;
-  std::vector<T> e6(size_t(6) * N);
-  for (long p = 0; p < N; ++p) {
-    const double* e = E + 9 * p;
-    T* o = e6.data() + 6 * p;
-    o[0] = T(e[0]);  // xx
-    o[1] = T(e[4]);  // yy
-    o[2] = T(e[8]);  // zz
-    o[3] = T(e[3]);  // (0,1)
-    o[4] = T(e[6]);  // (0,2)
-    o[5] = T(e[7]);  // (1,2)
+__global__ __launch_bounds__(256) void k_pack6(const double* E, long N, int nx, int ny, T* row, T* col) {
+  const long p = long(blockIdx.x) * 256 + threadIdx.x;
+  if (p >= N) return;
+  const double* e = E + 9 * p;
+  const T o[6] = {T(e[0]), T(e[4]), T(e[8]), T(e[3]), T(e[6]), T(e[7])};
+  const long nxy = long(nx) * ny, iz = p / nxy, q = p - iz * nxy, iy = q / nx, ix = q - iy * nx;
+  T* r = row + 6 * p;
+  T* c = col + 6 * (iy + ny * ix + nxy * iz);
+#pragma unroll
+  for (int a = 0; a < 6; ++a) {
+    r[a] = o[a];
+    c[a] = o[a];
   }
-  rowm.ensure(sizeof(T) * 6 * N);
-  OMX_HIP_CHECK(hipMemcpy(rowm.as<void>(), e6.data(), sizeof(T) * 6 * N, hipMemcpyHostToDevice));
-  // column-major copy per plane: pixel (ix, iy, iz) at 6 (iy + ny (ix + nx iz)) (the
-  // register path reads it on 2D cells)
-  std::vector<T> e6c(size_t(6) * N);
-  const long nxy = long(S.nx) * S.ny;
-  for (int iz = 0; iz < S.nz; ++iz)
-    for (int ix = 0; ix < S.nx; ++ix)
-      for (int iy = 0; iy < S.ny; ++iy)
-        for (int a = 0; a < 6; ++a)
-          e6c[6 * (iy + size_t(S.ny) * ix + nxy * iz) + a] = e6[6 * (ix + size_t(S.nx) * iy + nxy * iz) + a];
-  colm.ensure(sizeof(T) * 6 * N);
-  OMX_HIP_CHECK(hipMemcpy(colm.as<void>(), e6c.data(), sizeof(T) * 6 * N, hipMemcpyHostToDevice));
 }
 
-template void upload_tensor6<float>(const Solver&, const double*, DevMem&, DevMem&);
-template void upload_tensor6<double>(const Solver&, const double*, DevMem&, DevMem&);
+// the field in the handle's staging buffer, and from there in the layouts of precision T
+void stage_tensor(Solver& S, const double* E) {
+  S.tensor_raw.ensure(sizeof(double) * 9 * S.N);
+  OMX_HIP_CHECK(hipMemcpyAsync(S.tensor_raw.as<void>(), E, sizeof(double) * 9 * S.N, hipMemcpyHostToDevice, S.stream));
+}
+template <typename T> void pack_tensor(Solver& S, T* rowm, T* colm) {
+  hipLaunchKernelGGL(k_pack6<T>, dim3((S.N + 255) / 256), dim3(256), 0, S.stream, S.tensor_raw.as<double>(), S.N, S.nx,
+                     S.ny, rowm, colm);
+  OMX_HIP_CHECK(hipGetLastError());
+}
+
+template <typename T>
+void upload_tensor6(Solver& S, const double* E, DevMem& rowm, DevMem& colm) {
+  rowm.ensure(sizeof(T) * 6 * S.N);
+  colm.ensure(sizeof(T) * 6 * S.N);
+  stage_tensor(S, E);
+  pack_tensor<T>(S, rowm.as<T>(), colm.as<T>());
+  OMX_HIP_CHECK(hipStreamSynchronize(S.stream));  // E is the caller's
+}
+
+template void upload_tensor6<double>(Solver&, const double*, DevMem&, DevMem&);
 
 // the symmetry test set_epsinv applies, for any per-pixel 3x3 field
 void check_symmetric(long N, const double* E, const char* what) {
@@ -276,8 +284,10 @@ template <typename T> void select_operator(Solver& S, PrecisionData<T>& P) {
   pl.dot_blocks = S.nz * (S.ny / (pl.reg ? reg_rows_of(pl) : pl.rows_per_block));
 }
 
-template <typename T> void upload_eps(Solver& S, PrecisionData<T>& P) {
-  upload_tensor6<T>(S, S.epsinv_host.data(), P.eps6, P.eps6c);
+template <typename T> void pack_eps(Solver& S, PrecisionData<T>& P) {
+  P.eps6.ensure(sizeof(T) * 6 * S.N);
+  P.eps6c.ensure(sizeof(T) * 6 * S.N);
+  pack_tensor<T>(S, P.eps6.template as<T>(), P.eps6c.template as<T>());
   P.plan.eps6 = P.eps6.template as<T>();
   P.plan.eps6c = P.eps6c.template as<T>();
 }
@@ -309,14 +319,8 @@ template <typename T> class Batch {
     ld = S.ld;
     istride = long(M) * ld;
     const size_t blk = sizeof(cplx<T>) * size_t(ninst) * istride;
-    for (int b = 0; b < 2; ++b) {
-      X[b].alloc(blk);
-      AX[b].alloc(blk);
-      R[b].alloc(blk);
-      P[b].alloc(blk);
-      AP[b].alloc(blk);
-    }
-    AR.alloc(blk);
+    X[0].alloc(blk);
+    AX[0].alloc(blk);
     D.alloc(sizeof(cplx<T>) * size_t(ninst) * M * 3 * S.N);
     pm = (3 * M <= 16) ? 16 : (3 * M <= 32 ? 32 : 48);
     qmax = M <= 4 ? 4 : (M <= 8 ? 8 : 16);
@@ -328,7 +332,6 @@ template <typename T> class Batch {
     st.alloc(sizeof(LState) * ninst);
     shape.alloc(sizeof(int) * F_NFIELDS * ninst);
     OMX_HIP_CHECK(hipMemset(shape.as<void>(), 0, sizeof(int) * F_NFIELDS * ninst));
-    gramp.alloc(sizeof(c64) * size_t(ninst) * nchunk_max * pm * pm);
     red.alloc(sizeof(c64) * size_t(ninst) * pm * pm);
     normp.alloc(sizeof(double) * size_t(ninst) * nblk_max * qmax);
     Cx.alloc(sizeof(c64) * size_t(ninst) * pm * pm);
@@ -353,6 +356,14 @@ template <typename T> class Batch {
       snap[b].alloc(sizeof(LState) * ninst);
       OMX_HIP_CHECK(hipEventCreateWithFlags(&snap_ev[b], hipEventDisableTiming));
     }
+  }
+  // The blocks that only LOBPCG's own iterations use (run_begin), 9 of the 11: the FP64 batch
+  // whose pairs come from the shared search space never needs them, and mapping them took
+  // longer than its refinement where a call makes its own handle (four grids up to 256 x 256,
+  // six problems: 127 -> 122 ms with the packing above).
+  void lobpcg_blocks() {
+    const size_t blk = sizeof(cplx<T>) * size_t(ninst) * istride;
+    for (DevMem* m : {&X[1], &AX[1], &R[0], &R[1], &P[0], &P[1], &AP[0], &AP[1], &AR}) m->ensure(blk);
   }
   ~Batch() {
     for (int b = 0; b < 2; ++b)
@@ -401,6 +412,7 @@ template <typename T> class Batch {
   void gram(const ColList<T>& A, const ColList<T>& B, int ca, int cb, int pmv = -1, bool bpre = false,
             bool herm = false) {
     const int pg = pmv < 0 ? pm : pmv;
+    gramp.ensure(sizeof(c64) * size_t(ninst) * nchunk_max * pm * pm);
     launch_gram<T>(A, B, ninst, K, nchunk, pg, gramp.as<c64>(), sm, ca, cb, bpre, herm);
     // instances whose A has no columns were skipped by the Gram: skip their reduction too
     launch_reduce(gramp.as<c64>(), ninst, nchunk, pg * pg, red.as<c64>(), sm, A.p[0].s.cnt);
@@ -456,6 +468,7 @@ template <typename T> class Batch {
                  const std::vector<int>& ncheck, const std::vector<int>& msize, const std::vector<double>& tols,
                  int maxiter, SolveStats& stats) {
     if (maxiter > maxiter_alloc) maxiter = maxiter_alloc;
+    lobpcg_blocks();
     r = RunState{};
     r.act = act;
     r.maxiter = maxiter;
@@ -693,7 +706,6 @@ Solver::Solver(int dev, int nx_, int ny_, int nz_, double Dx_, double Dy_, doubl
   OMX_HIP_CHECK(hipSetDevice(dev));
   noalloc_init(dev);
   OMX_HIP_CHECK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-  OMX_HIP_CHECK(hipStreamCreateWithFlags(&stream2, hipStreamNonBlocking));
   N = long(nx) * ny * nz;
   K = 2 * N;
   ld = (K + 63) / 64 * 64;
@@ -735,8 +747,10 @@ void Solver::set_epsinv(const double* epsinv) {
   }
   epsinv_host.assign(epsinv, epsinv + n9);
   OMX_HIP_CHECK(hipSetDevice(device));
-  upload_eps<float>(*this, p32);
-  upload_eps<double>(*this, p64);
+  stage_tensor(*this, epsinv_host.data());
+  pack_eps<float>(*this, p32);
+  pack_eps<double>(*this, p64);
+  OMX_HIP_CHECK(hipStreamSynchronize(stream));
 }
 
 void Solver::set_option(const std::string& key, double v) {
@@ -869,6 +883,7 @@ void Solver::autotune(int nev, int* choice_out, double* us_out) {
   } restore{*this, saved};
   const int M = nev, ninst = nev;
   Batch<float> b(*this, ninst, M, 2);  // not from the cache: freed when tuning ends
+  b.lobpcg_blocks();
   hipStream_t s = stream;
   for (int q = 0; q < 2; ++q) {
     launch_randn<float>(b.p(b.X[q]), ld, b.istride, ninst, M, K, 101 + q, s);
@@ -2118,7 +2133,8 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
   } else if (!opt.fp64_only) {
     // two half-batches of bands on two streams (the seed eigensolve runs in the first)
     const int na = (ninst + 1) / 2, nb = ninst - na;
-    const bool split = opt.streams2 && nb > 0 && !warm && !banded && opt.fp32_newton && stream2;
+    const bool split = opt.streams2 && nb > 0 && !warm && !banded && opt.fp32_newton;
+    if (split && !stream2) OMX_HIP_CHECK(hipStreamCreateWithFlags(&stream2, hipStreamNonBlocking));
     const auto b32p = workspace<float>(*this, split ? na : ninst, M, maxiter);
     Batch<float>& b32 = *b32p;
     const std::shared_ptr<Batch<float>> b32q = split ? workspace<float>(*this, nb, M, maxiter, 1) : nullptr;
@@ -2273,27 +2289,6 @@ namespace {
 
 // Host conversion of a (3,3,Nx,Ny) column-major field to the operator's two 6-entry layouts,
 // written to device memory at rowm / colm (2D cells).
-template <typename T> void put_tensor6(const Solver& S, const double* E, T* rowm, T* colm, hipStream_t s) {
-  const long N = S.N;
-  std::vector<T> e6(size_t(6) * N), e6c(size_t(6) * N);
-  for (long p = 0; p < N; ++p) {
-    const double* e = E + 9 * p;
-    T* o = e6.data() + 6 * p;
-    o[0] = T(e[0]);
-    o[1] = T(e[4]);
-    o[2] = T(e[8]);
-    o[3] = T(e[3]);
-    o[4] = T(e[6]);
-    o[5] = T(e[7]);
-  }
-  for (int ix = 0; ix < S.nx; ++ix)
-    for (int iy = 0; iy < S.ny; ++iy)
-      for (int a = 0; a < 6; ++a) e6c[6 * (iy + size_t(S.ny) * ix) + a] = e6[6 * (ix + size_t(S.nx) * iy) + a];
-  OMX_HIP_CHECK(hipMemcpyAsync(rowm, e6.data(), sizeof(T) * e6.size(), hipMemcpyHostToDevice, s));
-  OMX_HIP_CHECK(hipMemcpyAsync(colm, e6c.data(), sizeof(T) * e6c.size(), hipMemcpyHostToDevice, s));
-  OMX_HIP_CHECK(hipStreamSynchronize(s));  // the host arrays go out of scope
-}
-
 }  // namespace
 
 // Several solve_k problems on this grid in one batch (no reference counterpart as one call:
@@ -2341,8 +2336,9 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
     off[p] = o;
     for (int j = 0; j < probs[p].nev; ++j) slot[o + j] = p;
     o += probs[p].nev;
-    put_tensor6<float>(*this, probs[p].epsinv, multi_e32r.as<float>() + n6 * p, multi_e32c.as<float>() + n6 * p, s);
-    put_tensor6<double>(*this, probs[p].epsinv, multi_e64r.as<double>() + n6 * p, multi_e64c.as<double>() + n6 * p, s);
+    stage_tensor(*this, probs[p].epsinv);
+    pack_tensor<float>(*this, multi_e32r.as<float>() + n6 * p, multi_e32c.as<float>() + n6 * p);
+    pack_tensor<double>(*this, multi_e64r.as<double>() + n6 * p, multi_e64c.as<double>() + n6 * p);
     double mn = 1e300;  // k_guess (MaxwellEigenmodes.jl:63)
     for (long q = 0; q < N; ++q)
       for (int a = 0; a < 3; ++a) mn = std::min(mn, probs[p].epsinv[9 * q + 4 * a]);

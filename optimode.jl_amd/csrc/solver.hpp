@@ -5,6 +5,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "omx.h"
@@ -16,6 +17,54 @@
 
 namespace omx {
 
+// Device blocks that DevMem releases and takes while a scope of it is open on the thread: a call
+// that makes a handle per grid reuses the first one's memory in the next (four grids up to
+// 256 x 256, six problems: 225 hipMalloc and hipFree took 27 of 122 ms).  The blocks go back
+// to the device with the scope, or when an allocation fails.  A block is kept only after the
+// device is idle, as hipFree itself would wait, so whichever stream takes it next may use it.
+class DevCache {
+ public:
+  DevCache() : outer_(current()) { current() = this; }
+  ~DevCache() {
+    current() = outer_;
+    drop();
+  }
+  DevCache(const DevCache&) = delete;
+  DevCache& operator=(const DevCache&) = delete;
+  static DevCache*& current() {
+    static thread_local DevCache* c = nullptr;
+    return c;
+  }
+  // the smallest kept block of at least `bytes` (its size into cap), or nullptr
+  void* take(size_t bytes, size_t& cap) {
+    size_t best = blocks_.size();
+    for (size_t j = 0; j < blocks_.size(); ++j)
+      if (blocks_[j].second >= bytes && (best == blocks_.size() || blocks_[j].second < blocks_[best].second)) best = j;
+    if (best == blocks_.size()) return nullptr;
+    void* p = blocks_[best].first;
+    cap = blocks_[best].second;
+    blocks_.erase(blocks_.begin() + long(best));
+    return p;
+  }
+  bool put(void* p, size_t cap) noexcept {
+    if (hipDeviceSynchronize() != hipSuccess) return false;
+    try {
+      blocks_.emplace_back(p, cap);
+    } catch (...) {
+      return false;
+    }
+    return true;
+  }
+  void drop() noexcept {
+    for (auto& b : blocks_) (void)hipFree(b.first);
+    blocks_.clear();
+  }
+
+ private:
+  DevCache* outer_;
+  std::vector<std::pair<void*, size_t>> blocks_;
+};
+
 // Owning device allocation.
 class DevMem {
  public:
@@ -24,36 +73,52 @@ class DevMem {
   ~DevMem() { release(); }
   DevMem(const DevMem&) = delete;
   DevMem& operator=(const DevMem&) = delete;
-  DevMem(DevMem&& o) noexcept : p_(o.p_), n_(o.n_) { o.p_ = nullptr; o.n_ = 0; }
+  DevMem(DevMem&& o) noexcept : p_(o.p_), n_(o.n_), cap_(o.cap_) {
+    o.p_ = nullptr;
+    o.n_ = o.cap_ = 0;
+  }
   DevMem& operator=(DevMem&& o) noexcept {
     if (this != &o) {
       release();
       p_ = o.p_;
       n_ = o.n_;
+      cap_ = o.cap_;
       o.p_ = nullptr;
-      o.n_ = 0;
+      o.n_ = o.cap_ = 0;
     }
     return *this;
   }
   void alloc(size_t bytes) {
     release();
-    if (bytes) OMX_HIP_CHECK(hipMalloc(&p_, bytes));
+    if (bytes) {
+      DevCache* c = DevCache::current();
+      if (c) p_ = c->take(bytes, cap_);
+      if (!p_) {
+        cap_ = bytes;
+        if (c && hipMalloc(&p_, bytes) != hipSuccess) {
+          (void)hipGetLastError();
+          p_ = nullptr;
+          c->drop();
+        }
+        if (!p_) OMX_HIP_CHECK(hipMalloc(&p_, bytes));
+      }
+    }
     n_ = bytes;
   }
   void ensure(size_t bytes) {
     if (bytes > n_) alloc(bytes);
   }
   void release() {
-    if (p_) (void)hipFree(p_);
+    if (p_ && !(DevCache::current() && DevCache::current()->put(p_, cap_))) (void)hipFree(p_);
     p_ = nullptr;
-    n_ = 0;
+    n_ = cap_ = 0;
   }
   template <typename U> U* as() const { return static_cast<U*>(p_); }
   size_t size() const { return n_; }
 
  private:
   void* p_ = nullptr;
-  size_t n_ = 0;
+  size_t n_ = 0, cap_ = 0;  // bytes asked for; of the block
 };
 
 template <typename T> struct PrecisionData {
@@ -302,7 +367,7 @@ class Solver {
   // shared state, public for the templated engine
   int device;
   hipStream_t stream = nullptr;
-  hipStream_t stream2 = nullptr;  // second stream of the two-stream FP32 Newton phase
+  hipStream_t stream2 = nullptr;  // second stream of the two-stream FP32 Newton phase (made when one runs)
   int nx, ny;
   double Dx, Dy;
   int nz = 1;       // planes along z (1: a 2D cell)
@@ -322,6 +387,7 @@ class Solver {
   ModeSlot modes[MODE_SLOTS];
   bool trace = false;               // OMX_TRACE=1: per-Newton-step iteration log on stderr
   DevMem scratch_a, scratch_b, scratch_c;
+  DevMem tensor_raw;  // a per-pixel 3x3 field as the host holds it, on its way to the operator's layouts
   DevMem krylov_ws;                  // MINRES vectors and scratch (grown on demand)
   DevMem vec_part, vec_coef;          // partial sums and coefficients of the vector helpers
   RefineWorkspace refine_ws;          // buffers of the FP64 refinement phase
@@ -352,7 +418,7 @@ class Solver {
 
 // A symmetric per-pixel 3x3 field (column-major (3,3,Nx,Ny), FP64 host) uploaded in the two
 // device layouts the operator reads (row-major and column-major pixel order, 6 entries each).
-template <typename T> void upload_tensor6(const Solver& S, const double* E, DevMem& rowm, DevMem& colm);
+template <typename T> void upload_tensor6(Solver& S, const double* E, DevMem& rowm, DevMem& colm);
 // throws unless every pixel of E is finite and symmetric
 void check_symmetric(long N, const double* E, const char* what);
 // per pixel, out = sym(L M R) for column-major 3x3 fields
