@@ -885,7 +885,8 @@ template <typename T> void VecOpsT<T>::project(C* x, const int* act, const C* do
 
 template <typename T>
 int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shifts, const double* dk, cplx<T>* r,
-                        cplx<T>* xout, const std::vector<int>& want, double rtol, int maxit, bool throw_on_cap) {
+                        cplx<T>* xout, const std::vector<int>& want, const std::vector<double>& rtol, int maxit,
+                        bool throw_on_cap) {
   using C = cplx<T>;
   hipStream_t s = S.stream;
   const int nb = V.nb;
@@ -917,7 +918,7 @@ int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shi
   std::vector<MinresState> hm(nb);
   for (int i = 0; i < nb; ++i) {
     std::memset(&hm[i], 0, sizeof(MinresState));
-    hm[i].rtol = rtol;
+    hm[i].rtol = rtol[i];
     hm[i].shift = shifts[i];
     hm[i].active = want[i];
   }
@@ -1055,9 +1056,9 @@ int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shi
 template struct VecOpsT<double>;
 template struct VecOpsT<float>;
 template int minres_complement_t<double>(Solver&, VecOpsT<double>&, const std::vector<double>&, const double*, c64*,
-                                         c64*, const std::vector<int>&, double, int, bool);
+                                         c64*, const std::vector<int>&, const std::vector<double>&, int, bool);
 template int minres_complement_t<float>(Solver&, VecOpsT<float>&, const std::vector<double>&, const double*,
-                                        cplx<float>*, cplx<float>*, const std::vector<int>&, double, int, bool);
+                                        cplx<float>*, cplx<float>*, const std::vector<int>&, const std::vector<double>&, int, bool);
 
 
 }  // namespace omx

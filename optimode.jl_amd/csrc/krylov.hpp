@@ -67,17 +67,18 @@ using VecOps = VecOpsT<double>;
 // indefinite above the lowest band), with vectors and operator applications in T and the
 // recurrences in FP64.  r is projected on entry and overwritten; xout receives the
 // solution orthogonalised against ev twice.  Stops when the preconditioned residual
-// estimate falls below rtol times its start, or after maxit iterations (an error only when
+// estimate falls below rtol_i times its start, or after maxit iterations (an error only when
 // throw_on_cap).  Returns the iteration count.
 template <typename T>
 int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shifts, const double* dk, cplx<T>* r,
-                        cplx<T>* xout, const std::vector<int>& want, double rtol, int maxit = 1000,
+                        cplx<T>* xout, const std::vector<int>& want, const std::vector<double>& rtol, int maxit = 1000,
                         bool throw_on_cap = true);
 
 inline int minres_complement(Solver& S, VecOps& V, const std::vector<double>& shifts, const double* dk, c64* r,
                              c64* xout, const std::vector<int>& want, double rtol, int maxit = 1000,
                              bool throw_on_cap = true) {
-  return minres_complement_t<double>(S, V, shifts, dk, r, xout, want, rtol, maxit, throw_on_cap);
+  return minres_complement_t<double>(S, V, shifts, dk, r, xout, want, std::vector<double>(want.size(), rtol), maxit,
+                                     throw_on_cap);
 }
 
 }  // namespace omx

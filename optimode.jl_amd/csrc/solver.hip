@@ -1734,6 +1734,14 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
       if (!need || jd >= jd_max) break;
       // t: (M - rho) t = r on the complement of x (the sign of t is immaterial)
       VecOps V(S, s, ninst, ld, K, XB.as<c64>());
+      // A correction reduces the residual by about its tolerance or better.  One that can be
+      // the last after the shared-subspace phase (at jd_rtol / 10) aims at a tenth of the target:
+      // a few iterations more than at jd_rtol, for a pair that is not merely just converged and
+      // often one correction less; looser where the residual is nearly there.
+      std::vector<double> rtols(ninst, S.opt.jd_rtol);
+      for (int i = 0; i < ninst && loose_blocks; ++i)
+        if (jdh[i] && step_tol[i] == tols[i] && 0.1 * S.opt.jd_rtol * rn[i] <= tols[i])
+          rtols[i] = std::min(std::max(0.1 * tols[i] / rn[i], 0.1 * S.opt.jd_rtol), std::max(0.05, S.opt.jd_rtol));
       int its;
       const auto t_mr0 = tnow();
       if (S.opt.jd_fp32) {
@@ -1781,11 +1789,11 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
           }
         }
         its = minres_complement_t<float>(S, V32, lam_band, b.kd.as<double>(), W.RBf.as<cf>(), W.Tf.as<cf>(), jdh,
-                                         S.opt.jd_rtol, S.opt.jd_maxit, false);
+                                         rtols, S.opt.jd_maxit, false);
         launch_convert<float, double>(W.Tf.as<cf>(), ld, ld, Tm.as<c64>(), ld, ld, ninst, 1, K, s);
       } else {
-        its = minres_complement(S, V, lam_band, b.kd.as<double>(), RBm.as<c64>(), Tm.as<c64>(), jdh, S.opt.jd_rtol,
-                                S.opt.jd_maxit, false);
+        its = minres_complement_t<double>(S, V, lam_band, b.kd.as<double>(), RBm.as<c64>(), Tm.as<c64>(), jdh, rtols,
+                                          S.opt.jd_maxit, false);
       }
       for (int i = 0; i < ninst; ++i) {
         stats.matvec += long(its) * jdh[i];
