@@ -705,7 +705,11 @@ Solver::Solver(int dev, int nx_, int ny_, int nz_, double Dx_, double Dy_, doubl
   if (nz > 1 && !(Dz > 0 && std::isfinite(Dz))) throw Error(OMX_ERR_INVALID_ARG, "the period Dz must be positive");
   OMX_HIP_CHECK(hipSetDevice(dev));
   noalloc_init(dev);
+  // one after the other: streams share the few hardware queues in the order of their creation,
+  // and a second stream made later can land on the first one's (no overlap: 38.7 against 36.2 ms
+  // at 128x96x24, 4 bands)
   OMX_HIP_CHECK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+  OMX_HIP_CHECK(hipStreamCreateWithFlags(&stream2, hipStreamNonBlocking));
   N = long(nx) * ny * nz;
   K = 2 * N;
   ld = (K + 63) / 64 * 64;
@@ -1907,6 +1911,25 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
   return outer;
 }
 
+// A solve whose refinement fails from the shared search space's blocks is done again with one
+// LOBPCG block per band, so that nothing the per-band form solves is lost to the shared one.
+struct WithoutMultiK {
+  Solver& S;
+  const int was;
+  explicit WithoutMultiK(Solver& s) : S(s), was(s.opt.multik) { S.opt.multik = 0; }
+  ~WithoutMultiK() { S.opt.multik = was; }
+};
+// the refinement's steps; an error of its own (a block that lost rank) leaves the bands not
+// done where the shared search space made the blocks
+template <typename F> int refine_after(bool mk_done, const F& refine) {
+  try {
+    return refine();
+  } catch (const Error&) {
+    if (!mk_done) throw;
+    return 0;
+  }
+}
+
 }  // namespace
 
 void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int max_eigsolves, int maxiter,
@@ -2141,8 +2164,7 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
   } else if (!opt.fp64_only) {
     // two half-batches of bands on two streams (the seed eigensolve runs in the first)
     const int na = (ninst + 1) / 2, nb = ninst - na;
-    const bool split = opt.streams2 && nb > 0 && !warm && !banded && opt.fp32_newton;
-    if (split && !stream2) OMX_HIP_CHECK(hipStreamCreateWithFlags(&stream2, hipStreamNonBlocking));
+    const bool split = opt.streams2 && nb > 0 && !warm && !banded && opt.fp32_newton && stream2;
     const auto b32p = workspace<float>(*this, split ? na : ninst, M, maxiter);
     Batch<float>& b32 = *b32p;
     const std::shared_ptr<Batch<float>> b32q = split ? workspace<float>(*this, nb, M, maxiter, 1) : nullptr;
@@ -2238,8 +2260,10 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
   if (!opt.plain) {
     const int left = std::max(1, max_eigsolves - newton_total);
     if (opt.refine && !opt.fp64_only)
-      stats.it64 += refine_phase(*this, b64, hns, bands, msize, std::vector<double>(size_t(ninst), eig_tol), left,
-                                 stats, newton_total, max_resid, nullptr, mk_done);
+      stats.it64 += refine_after(mk_done, [&] {
+        return refine_phase(*this, b64, hns, bands, msize, std::vector<double>(size_t(ninst), eig_tol), left, stats,
+                            newton_total, max_resid, nullptr, mk_done);
+      });
     else
       stats.it64 +=
           newton_phase(*this, b64, hns, bands, nchk, msize, eig_tol, maxit64, left, stats, newton_total, true);
@@ -2255,6 +2279,12 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
   for (int i = 0; i < ninst; ++i) {
     kmags[i] = hns[i].k;
     if (hns[i].done != 1) ok = false;
+  }
+  if (!ok && mk_done) {
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    WithoutMultiK off(*this);
+    return solve_k(omega, nev, k_tol, eig_tol, max_eigsolves, maxiter, kguess, Hguess, nguess, kmags, evecs, info);
   }
   // eigenvector of band i = column i of instance i; canonicalise phase (fields.jl:258-260)
   last_evecs.ensure(sizeof(c64) * size_t(nev) * ld);
@@ -2515,10 +2545,17 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
   std::vector<double> resid(ninst, 0.0);
   const int left = std::max(1, max_eigsolves - newton_total);
   if (opt.refine && !opt.fp64_only)
-    stats.it64 += refine_phase(*this, b64, hns, bands, msize, eig_tol, left, stats, newton_total, max_resid, &resid,
-                               mk_done);
+    stats.it64 += refine_after(mk_done, [&] {
+      return refine_phase(*this, b64, hns, bands, msize, eig_tol, left, stats, newton_total, max_resid, &resid, mk_done);
+    });
   else
     stats.it64 += newton_phase(*this, b64, hns, bands, nchk, msize, eig_tol, maxit64, left, stats, newton_total, true);
+  if (mk_done && std::any_of(hns.begin(), hns.end(), [](const NewtonState& h) { return h.done != 1; })) {
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    WithoutMultiK off(*this);
+    return solve_k_multi(probs);
+  }
   // band eigenvectors of every instance, phase-canonicalised together (fields.jl:258-260)
   multi_evecs.ensure(sizeof(c64) * size_t(ninst) * ld);
   for (int i = 0; i < ninst; ++i)

@@ -367,7 +367,7 @@ class Solver {
   // shared state, public for the templated engine
   int device;
   hipStream_t stream = nullptr;
-  hipStream_t stream2 = nullptr;  // second stream of the two-stream FP32 Newton phase (made when one runs)
+  hipStream_t stream2 = nullptr;  // second stream of the two-stream FP32 Newton phase
   int nx, ny;
   double Dx, Dy;
   int nz = 1;       // planes along z (1: a 2D cell)
