@@ -25,6 +25,7 @@
 #include <cstring>
 
 #include "fft_lds.hpp"
+#include "multik_math.hpp"
 #include "omx_errors.hpp"
 #include "rng.hpp"
 #include "solver.hpp"
@@ -891,12 +892,7 @@ __global__ __launch_bounds__(DT) void k_mk_dense(MkGeo geo, MkState* st, const c
   const c64* Ad = ((rounds & 1) != 0) == FINAL ? A1 : A;
   for (int a = threadIdx.x; a < n; a += DT) diagv[a] = Ad[a * ld + a].x;
   __syncthreads();
-  for (int a = threadIdx.x; a < n; a += DT) {
-    int r = 0;
-    for (int l = 0; l < n; ++l)
-      if (diagv[l] < diagv[a] || (diagv[l] == diagv[a] && l < a)) ++r;
-    rank[r] = a;
-  }
+  for (int a = threadIdx.x; a < n; a += DT) rank[mk_position(diagv, n, a)] = a;
   __threadfence_block();  // the block's rotations, read back below
   __syncthreads();
   if (!FINAL && threadIdx.x == 0) lam_s = diagv[rank[j]];
