@@ -98,7 +98,9 @@ const char* omx_last_error(const omx_solver* h);
    (solve_omega2's, 1e-5), "fp32_switch", "jd_rtol", "jd_first_tol" (residual / omega^2 at which
    the FP64 refinement's first Newton step moves k, 3e-5), "maxiter_fp64", "guard", "seed"; start modes
    "warm_start" and "band_guess" (omx_solve_k); "multik" (1: the FP32 phase of omx_solve_k and
-   omx_solve_k_batch on 2D cells in one search space for all bands, 0: one LOBPCG block per band); "guess_lowres" = hw > 0 (even, <= Nx, Ny):
+   omx_solve_k_batch on 2D cells in one search space for all bands, 0: one LOBPCG block per
+   band) with its iteration cap "multik_maxit" (200; a solve that reaches it is done per band;
+   the batch has the default); "guess_lowres" = hw > 0 (even, <= Nx, Ny):
    omx_solve_k's Hguess vectors hold only their hw x hw lowest plane waves, 2 hw^2 complex
    each at c + 2(gx + hw gy) in FFT order, and are scattered into the start block on the GPU */
 int omx_set_option(omx_solver* h, const char* key, double value);
@@ -333,6 +335,12 @@ int omx_solve_k_learned(omx_solver* h, omx_warmnet* net, double omega, int nev, 
    "op_fp64".  Returns total milliseconds, launches and algorithmic bytes
    (32 N m + 24 N per FP32 application of m vectors, twice that in FP64). */
 int omx_get_kernel_stats(omx_solver* h, const char* family, double* total_ms, int64_t* launches, double* bytes);
+
+/* Which form the FP32 phases of the calling thread's last omx_solve_k, omx_solve_k_learned or
+   omx_solve_k_batch took (no counterpart in the reference), in problems: solved from the
+   blocks of the search space all bands share (option "multik"), or per band; redone counts
+   those of per_band that the shared search space was tried on first.  Each pointer may be NULL. */
+int omx_solve_phases(int64_t* shared, int64_t* per_band, int64_t* redone);
 
 #ifdef __cplusplus
 }

@@ -181,6 +181,7 @@ int omx_sliceinv_3x3_pullback(int device, int64_t npix, const double* Y, const d
 
 int omx_solve_k_batch(int device, int nprob, omx_problem* probs, int max_group, int fp64_only) {
   try {
+    omx::solve_phases() = {};
     omx::solve_k_batch(device, nprob, probs, max_group, fp64_only);
     return OMX_OK;
   } catch (const omx::Error& e) {
@@ -273,6 +274,7 @@ int omx_solve_k(omx_solver* h, double omega, int nev, double k_tol, double eig_t
                 const double* kguess, const double* Hguess, int nguess, double* kmags_out, double* evecs_out,
                 omx_info* info) {
   return guarded(h, [&](omx::Solver& s) {
+    omx::solve_phases() = {};
     s.solve_k(omega, nev, k_tol, eig_tol, max_eigsolves, maxiter, kguess, Hguess, nguess, kmags_out, evecs_out, info);
   });
 }
@@ -375,6 +377,7 @@ int omx_solve_k_learned(omx_solver* h, omx_warmnet* net, double omega, int nev, 
   if (!net || !net->n) return OMX_ERR_INVALID_ARG;
   return guarded(h, [&](omx::Solver& s) {
     std::lock_guard<std::mutex> lk(net->mu);
+    omx::solve_phases() = {};
     omx::solve_k_learned(s, *net->n, omega, nev, k0_scale, k_tol, eig_tol, max_eigsolves, maxiter, kmags_out,
                          evecs_out, info);
   });
@@ -395,6 +398,14 @@ int omx_get_kernel_stats(omx_solver* h, const char* family, double* total_ms, in
     *launches = st->launches;
     *bytes = st->bytes;
   });
+}
+
+int omx_solve_phases(int64_t* shared, int64_t* per_band, int64_t* redone) {
+  const omx::SolvePhases& p = omx::solve_phases();
+  if (shared) *shared = p.shared;
+  if (per_band) *per_band = p.per_band;
+  if (redone) *redone = p.redone;
+  return OMX_OK;
 }
 
 }  // extern "C"

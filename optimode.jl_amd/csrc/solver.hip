@@ -65,6 +65,11 @@ Profiler::~Profiler() {
 template <> PrecisionData<float>& Solver::pd<float>() { return p32; }
 template <> PrecisionData<double>& Solver::pd<double>() { return p64; }
 
+SolvePhases& solve_phases() {
+  static thread_local SolvePhases p;
+  return p;
+}
+
 // A symmetric per-pixel 3x3 field (column-major (3,3,Nx,Ny) or (3,3,Nx,Ny,Nz), FP64 host) in
 // the two device layouts the operator reads: 6 unique entries xx, yy, zz, xy, xz, yz per
 // pixel, row-major (iz, iy, ix) and column-major per plane (iz, ix, iy: pixel (ix, iy, iz) at
@@ -798,6 +803,8 @@ void Solver::set_option(const std::string& key, double v) {
     opt.streams2 = v != 0 ? 1 : 0;
   else if (key == "multik")
     opt.multik = v != 0 ? 1 : 0;
+  else if (key == "multik_maxit")
+    opt.multik_maxit = std::max(1, int(v));
   else if (key == "graphs")
     opt.graphs = v != 0 ? 1 : 0;
   else if (key == "jac_stop32")
@@ -1324,10 +1331,10 @@ namespace {
 
 // Shared-subspace FP32 phase: |change of w^2| / w^2 by which a band's k must have settled
 // (the refinement's first Newton step takes it from there), and its iteration cap, the
-// total a caller's limits allow one band of the per-band form, at most 200.
+// total a caller's limits allow one band of the per-band form, at most option multik_maxit.
 constexpr double MK_FTOL = 1e-5;
-int multik_maxit(int maxiter, int max_eigsolves) {
-  return int(std::min<long>(200, long(maxiter) * std::min(max_eigsolves, 8)));
+int multik_cap(const Solver& S, int maxiter, int max_eigsolves) {
+  return int(std::min<long>(S.opt.multik_maxit, long(maxiter) * std::min(max_eigsolves, 8)));
 }
 
 // Newton driver over a batch of band instances (instance i follows band i).
@@ -2117,9 +2124,11 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
     }
     std::vector<double> kk;
     std::vector<int> its, moves;
-    if (!multik_solve(*this, {q}, p32.plan.eps6c, 0, multik_maxit(maxiter, max_eigsolves), msize_mk, b64.p(b64.X[0]), ld,
-                      b64.istride, kk, its, moves, stats))
+    if (!multik_solve(*this, {q}, p32.plan.eps6c, 0, multik_cap(*this, maxiter, max_eigsolves), msize_mk, b64.p(b64.X[0]), ld,
+                      b64.istride, kk, its, moves, stats)) {
+      ++solve_phases().redone;
       return false;
+    }
     msize = msize_mk;
     mk_done = true;
     mk_moves = moves[0];
@@ -2281,11 +2290,13 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
     if (hns[i].done != 1) ok = false;
   }
   if (!ok && mk_done) {
+    ++solve_phases().redone;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     WithoutMultiK off(*this);
     return solve_k(omega, nev, k_tol, eig_tol, max_eigsolves, maxiter, kguess, Hguess, nguess, kmags, evecs, info);
   }
+  ++(mk_done ? solve_phases().shared : solve_phases().per_band);
   // eigenvector of band i = column i of instance i; canonicalise phase (fields.jl:258-260)
   last_evecs.ensure(sizeof(c64) * size_t(nev) * ld);
   for (int i = 0; i < ninst; ++i)
@@ -2501,9 +2512,11 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
     }
     std::vector<double> kk;
     std::vector<int> its, moves;
-    if (!multik_solve(*this, mk, p32.plan.eps6c, p32.plan.eps_stride, multik_maxit(maxiter, max_eigsolves), msize_mk,
-                      b64.p(b64.X[0]), ld, b64.istride, kk, its, moves, stats))
+    if (!multik_solve(*this, mk, p32.plan.eps6c, p32.plan.eps_stride, multik_cap(*this, maxiter, max_eigsolves), msize_mk,
+                      b64.p(b64.X[0]), ld, b64.istride, kk, its, moves, stats)) {
+      solve_phases().redone += P;
       return false;
+    }
     msize = msize_mk;
     mk_done = true;
     for (int i = 0; i < ninst; ++i) {
@@ -2551,11 +2564,13 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
   else
     stats.it64 += newton_phase(*this, b64, hns, bands, nchk, msize, eig_tol, maxit64, left, stats, newton_total, true);
   if (mk_done && std::any_of(hns.begin(), hns.end(), [](const NewtonState& h) { return h.done != 1; })) {
+    solve_phases().redone += P;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     WithoutMultiK off(*this);
     return solve_k_multi(probs);
   }
+  (mk_done ? solve_phases().shared : solve_phases().per_band) += P;
   // band eigenvectors of every instance, phase-canonicalised together (fields.jl:258-260)
   multi_evecs.ensure(sizeof(c64) * size_t(ninst) * ld);
   for (int i = 0; i < ninst; ++i)

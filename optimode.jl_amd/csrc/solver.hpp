@@ -258,6 +258,7 @@ struct Options {
                                 // the other half's memory-bound kernels)
   int multik = 1;               // FP32 phase of solve_k on 2D cells in one search space shared by all
                                 // bands (multik.hip); 0: one LOBPCG block per band
+  int multik_maxit = 200;       // its iteration cap (10 to 60 are made)
   int graphs = 0;               // MINRES iterations replayed from a captured HIP graph (groups of 12;
                                 // same results, no measured gain: the gaps are GPU-side)
 };
@@ -301,6 +302,15 @@ struct MultiKWorkspace {
       if (e) (void)hipEventDestroy(e);
   }
 };
+
+// Which form the FP32 phases of the calling thread's last solve_k or batch took, in problems
+// (omx_solve_phases).
+struct SolvePhases {
+  long shared = 0;    // solved from the shared search space's blocks
+  long per_band = 0;  // solved from one LOBPCG block per band, or in FP64 throughout
+  long redone = 0;    // of those, the ones the shared search space was tried on first
+};
+SolvePhases& solve_phases();
 
 // One problem of a batched solve on a handle's grid (Solver::solve_k_multi).
 struct MultiProblem {

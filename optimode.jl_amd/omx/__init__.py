@@ -27,7 +27,8 @@ from ._lib import OmxError, OmxInfo, OMX_PREC_FP32, OMX_PREC_FP64  # noqa: F401
 
 __all__ = ["Grid", "Grid3", "HIPSolver", "HelmholtzMap", "solve_omega2", "solve_k", "solve_k_batch", "rrule_solve_k",
            "group_index", "ng_gvd", "k_guess", "solve_k_periodic", "period_derivatives", "rrule_solve_k_periodic",
-           "sliceinv_3x3", "rrule_sliceinv_3x3", "OmxError", "library_path", "exported_symbols", "kernel_stats"]
+           "sliceinv_3x3", "rrule_sliceinv_3x3", "OmxError", "library_path", "exported_symbols", "kernel_stats",
+           "solve_phases"]
 
 
 def library_path():
@@ -197,6 +198,16 @@ def kernel_stats(solver, family):
     _lib.check(_lib.lib().omx_get_kernel_stats(h.h, family.encode(), ctypes.byref(ms), ctypes.byref(n),
                                                ctypes.byref(b)), h.h)
     return ms.value, n.value, b.value
+
+
+def solve_phases():
+    """Which form the FP32 phases of this thread's last ``solve_k``, ``solve_k_learned`` or
+    ``solve_k_batch`` took, in problems: ``shared`` (blocks from the search space all bands
+    share), ``per_band``, and ``redone``, those of ``per_band`` the shared search space was
+    tried on first."""
+    n = [ctypes.c_int64() for _ in range(3)]
+    _lib.check(_lib.lib().omx_solve_phases(*(ctypes.byref(v) for v in n)), None)
+    return dict(zip(("shared", "per_band", "redone"), (v.value for v in n)))
 
 
 def _cols(H, n2):

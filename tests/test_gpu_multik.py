@@ -25,10 +25,19 @@ def _eps(nx, ny, seed=0):
     return g, G.ridge_waveguide(g, 1.5 + 0.1 * seed, 0.6, 75.0, core, backend="gpu")
 
 
-def _solve(g, ei, nev, multik, **kw):
-    s = omx.HIPSolver()
+SHARED = dict(shared=1, per_band=0, redone=0)
+PER_BAND = dict(shared=0, per_band=1, redone=0)
+REDONE = dict(shared=0, per_band=1, redone=1)
+
+
+def _solve(g, ei, nev, multik, took=None, solver=None, **kw):
+    """solve_k with the option ``multik``; a solve that the shared search space does not finish
+    ends in the per-band form, so what is compared with that form has to say which one it took."""
+    s = omx.HIPSolver() if solver is None else solver
     s.options["multik"] = float(multik)
-    return omx.solve_k(W0, ei, g, s, nev=nev, **{**KW, **kw})
+    res = omx.solve_k(W0, ei, g, s, nev=nev, **{**KW, **kw})
+    assert omx.solve_phases() == ((SHARED if multik else PER_BAND) if took is None else took)
+    return res
 
 
 @pytest.mark.parametrize("nx,ny,nev", [(16, 12, 1), (12, 18, 2), (27, 25, 3), (40, 30, 6), (64, 64, 13), (135, 81, 4),
@@ -61,6 +70,18 @@ def test_degenerate_bands():
     assert np.linalg.svd(np.stack(ev[:2]), compute_uv=False)[-1] > 0.5
 
 
+def test_a_solve_the_shared_space_gives_up_is_done_per_band():
+    """Two iterations never converge: the per-band form then has to give what it gives alone."""
+    print("multik give-up", flush=True)
+    g, ei = _eps(64, 48)
+    s = omx.HIPSolver()
+    s.options["multik_maxit"] = 2.0
+    k1, _, i1 = _solve(g, ei, 4, 1, took=REDONE, solver=s)
+    k0, _, i0 = _solve(g, ei, 4, 0)
+    assert i0["converged"] == i1["converged"] == 1
+    assert np.max(np.abs(k1 / k0 - 1)) < 2e-10
+
+
 def test_every_start_reaches_the_same_bands():
     print("multik starts", flush=True)
     g, ei = _eps(90, 64)
@@ -84,7 +105,9 @@ def test_every_start_reaches_the_same_bands():
     assert np.max(np.abs(k1 / k0 - 1)) < 2e-10
     s = omx.HIPSolver(warm_start=True)
     omx.solve_k(0.99 * W0, ei, g, s, nev=nev, **KW)
+    assert omx.solve_phases() == SHARED
     k1, _, _ = omx.solve_k(W0, ei, g, s, nev=nev, **KW)
+    assert omx.solve_phases() == SHARED
     assert np.max(np.abs(k1 / k0 - 1)) < 2e-10
 
 
@@ -99,6 +122,8 @@ def test_batch_on_an_odd_grid():
         s = omx.HIPSolver()
         s.options["multik"] = 0.0
         refs.append(omx.solve_k(probs[-1]["omega"], ei, g, s, nev=nev, **KW)[0])
-    for q, k0 in zip(omx.solve_k_batch(probs), refs):
+    res = omx.solve_k_batch(probs)
+    assert omx.solve_phases() == dict(shared=3, per_band=0, redone=0)
+    for q, k0 in zip(res, refs):
         assert q["status"] == 0
         assert np.max(np.abs(q["kmags"] / k0 - 1)) < 2e-10
