@@ -1588,6 +1588,9 @@ bool dense_geig(int n, const c64* Gp, const c64* Bp, std::vector<double>& lam, s
 // tolerance jd_rtol, at most jd_maxit iterations), t orthogonalised against the block and Rayleigh-Ritz on [block, t],
 // until |M x - rho x| <= tol; then the Newton update of k from rho and HMkH(x).  The
 // band's Ritz value is the bands[i]-th of the block, as LOBPCG's locking order gives it.
+// loose_blocks: the blocks are the shared search space's.  An instance whose block loses rank
+// then ends as not done, and the others go on (its solve is done again per band); an error
+// of the device or of an allocation is the caller's, here as everywhere.
 int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, const std::vector<int>& bands,
                  const std::vector<int>& msize, const std::vector<double>& tols, int max_steps, SolveStats& stats,
                  int& newton_total, double& max_resid, std::vector<double>* resid_inst = nullptr,
@@ -1666,26 +1669,31 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
     std::fill(hC.begin(), hC.end(), c64{0, 0});
     std::vector<double> lam;
     std::vector<cd> C;
+    bool lost = false;
     for (int i = 0; i < ninst; ++i) {
       const int m = n1h[i];
       if (m == 0) continue;
       c64* Ci = hC.data() + size_t(i) * RF_PAIRS;
       const int n = m + ((any_t && with_t[i]) ? 1 : 0);
-      if (!dense_geig(n, hG.data() + size_t(i) * RF_PAIRS, hB.data() + size_t(i) * RF_PAIRS, lam, C))
-      {
+      if (!dense_geig(n, hG.data() + size_t(i) * RF_PAIRS, hB.data() + size_t(i) * RF_PAIRS, lam, C)) {
         if (S.trace) {
           const c64* Bi = hB.data() + size_t(i) * RF_PAIRS;
           std::fprintf(stderr, "[omx] refinement: instance %d of %d columns lost rank, diagonal of U^H U:", i, n);
           for (int l = 0; l < n; ++l) std::fprintf(stderr, " %.3e", Bi[l + RF_MAXC * l].x);
           std::fprintf(stderr, "\n");
         }
-        throw Error(OMX_ERR_CHOLESKY, "refinement: the Rayleigh-Ritz basis lost rank");
+        if (!loose_blocks) throw Error(OMX_ERR_CHOLESKY, "refinement: the Rayleigh-Ritz basis lost rank");
+        n1h[i] = 0;
+        hns[i].done = 2;
+        lost = true;
+        continue;
       }
       for (int j = 0; j < m; ++j)
         for (int l = 0; l < n; ++l) Ci[l + RF_MAXC * j] = c64{C[l + size_t(n) * j].real(), C[l + size_t(n) * j].imag()};
       lam_band[i] = lam[bands[i]];
       std::copy(lam.begin(), lam.begin() + m, theta.begin() + size_t(i) * RF_MAXC);
     }
+    if (lost) up_n1(n1h);
     OMX_HIP_CHECK(hipMemcpyAsync(Cd.as<void>(), hC.data(), sizeof(c64) * hC.size(), hipMemcpyHostToDevice, s));
     // in place: each row's inputs are read before its outputs are written (one thread per
     // row); instances outside this Rayleigh-Ritz are left as they are
@@ -1926,17 +1934,6 @@ struct WithoutMultiK {
   explicit WithoutMultiK(Solver& s) : S(s), was(s.opt.multik) { S.opt.multik = 0; }
   ~WithoutMultiK() { S.opt.multik = was; }
 };
-// the refinement's steps; an error of its own (a block that lost rank) leaves the bands not
-// done where the shared search space made the blocks
-template <typename F> int refine_after(bool mk_done, const F& refine) {
-  try {
-    return refine();
-  } catch (const Error&) {
-    if (!mk_done) throw;
-    return 0;
-  }
-}
-
 }  // namespace
 
 void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int max_eigsolves, int maxiter,
@@ -2269,10 +2266,8 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
   if (!opt.plain) {
     const int left = std::max(1, max_eigsolves - newton_total);
     if (opt.refine && !opt.fp64_only)
-      stats.it64 += refine_after(mk_done, [&] {
-        return refine_phase(*this, b64, hns, bands, msize, std::vector<double>(size_t(ninst), eig_tol), left, stats,
-                            newton_total, max_resid, nullptr, mk_done);
-      });
+      stats.it64 += refine_phase(*this, b64, hns, bands, msize, std::vector<double>(size_t(ninst), eig_tol), left,
+                                 stats, newton_total, max_resid, nullptr, mk_done);
     else
       stats.it64 +=
           newton_phase(*this, b64, hns, bands, nchk, msize, eig_tol, maxit64, left, stats, newton_total, true);
@@ -2558,9 +2553,8 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
   std::vector<double> resid(ninst, 0.0);
   const int left = std::max(1, max_eigsolves - newton_total);
   if (opt.refine && !opt.fp64_only)
-    stats.it64 += refine_after(mk_done, [&] {
-      return refine_phase(*this, b64, hns, bands, msize, eig_tol, left, stats, newton_total, max_resid, &resid, mk_done);
-    });
+    stats.it64 +=
+        refine_phase(*this, b64, hns, bands, msize, eig_tol, left, stats, newton_total, max_resid, &resid, mk_done);
   else
     stats.it64 += newton_phase(*this, b64, hns, bands, nchk, msize, eig_tol, maxit64, left, stats, newton_total, true);
   if (mk_done && std::any_of(hns.begin(), hns.end(), [](const NewtonState& h) { return h.done != 1; })) {

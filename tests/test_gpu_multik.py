@@ -82,6 +82,32 @@ def test_a_solve_the_shared_space_gives_up_is_done_per_band():
     assert np.max(np.abs(k1 / k0 - 1)) < 2e-10
 
 
+def test_a_block_that_loses_rank_ends_its_solve_only():
+    """A start block of zeros on a grid too small for guard columns leaves the shared search
+    space empty: its blocks have no rank.  That is not an error of the call, which then does
+    what the per-band form does with such a start, and the handle goes on."""
+    print("multik lost rank", flush=True)
+    g, ei = _eps(5, 5)
+    nev = 16  # 3 nev = 48 of 50 unknowns
+    zero = np.zeros((nev, 2 * g.N), dtype=np.complex128)
+    ends = []
+    for multik in (0, 1):
+        s = omx.HIPSolver()
+        s.options["multik"] = float(multik)
+        try:
+            ends.append(omx.solve_k(W0, ei, g, s, nev=nev, Hguess=zero, kguess=1.0, **KW)[0])
+        except omx.OmxError as e:
+            ends.append(e.status)
+        print(f"  multik {multik}: {ends[-1]}, {omx.solve_phases()}", flush=True)
+    assert omx.solve_phases()["redone"] == 1 and omx.solve_phases()["shared"] == 0
+    if isinstance(ends[0], int):
+        assert ends[1] == ends[0]
+    else:
+        assert np.max(np.abs(ends[1] / ends[0] - 1)) < 2e-10
+    k0 = _solve(g, ei, 3, 0)[0]
+    assert np.max(np.abs(_solve(g, ei, 3, 1, solver=s)[0] / k0 - 1)) < 2e-10
+
+
 def test_every_start_reaches_the_same_bands():
     print("multik starts", flush=True)
     g, ei = _eps(90, 64)
