@@ -1370,6 +1370,7 @@ __global__ __launch_bounds__(256) void k_mk_handover(MkGeo geo, const c32* cols,
   __shared__ c64 Cs[MK_MAXN][HQ];
   const int i = blockIdx.y, p = inst[i].x, j = inst[i].y, q0 = blockIdx.z * HQ;
   const MkState& s = st[p];
+  if (s.done != 1) return;
   const int nq = min(HQ, msz[p * MK_MAXM + j] - q0);
   if (nq <= 0) return;
   const int n = s.m + s.na + s.np;
@@ -1436,10 +1437,12 @@ bool multik_fits(const Solver& S) {
          pick_rows(S.ny, S.nx, 1 << 20, S.p32.plan.fy) > 0;
 }
 
-bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* eps6c, long eps_stride, int maxit,
-                  const std::vector<int>& msize, c64* X64, long ld, long istride, std::vector<double>& kout,
-                  std::vector<int>& iters, std::vector<int>& moves, SolveStats& stats) {
+std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* eps6c, long eps_stride,
+                               int maxit, const std::vector<int>& msize, c64* X64, long ld, long istride,
+                               std::vector<double>& kout, std::vector<int>& iters, std::vector<int>& moves,
+                               SolveStats& stats) {
   const int P = int(probs.size());
+  std::vector<char> ok(P, 0);
   hipStream_t sm = S.stream;
   MkGeo g{};
   g.nx = S.nx;
@@ -1475,7 +1478,7 @@ bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* e
   const int nmax = 3 * g.mmax, NT = (nmax + 15) / 16, pm = 16 * NT;
   const long vecs = long(P) * g.mmax;
   const int RB = pick_rows(S.nx, S.ny, vecs, g.fx), TX = pick_rows(S.ny, S.nx, vecs, g.fy);
-  if (RB == 0 || TX == 0) return false;
+  if (RB == 0 || TX == 0) return ok;
   const int nrb = (S.ny + RB - 1) / RB, ncb = (S.nx + TX - 1) / TX;
   // Gram chunks: about 128 over the problems, of whole 64-row steps, a stage of every wave or more
   const int nchunk = int(std::max<long>(1, std::min<long>((S.N + 255) / 256, std::max(8, 128 / P))));
@@ -1487,7 +1490,7 @@ bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* e
     OMX_HIP_CHECK(hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(&k_mk_dense<512, false>)));
     OMX_HIP_CHECK(hipFuncGetAttributes(&fb, reinterpret_cast<const void*>(&k_mk_dense<512, true>)));
     const size_t dyn = sizeof(c64) * 3 * size_t((nmax + 1) & ~1) * ((nmax + 1) | 1);
-    if (std::max(fa.sharedSizeBytes, fb.sharedSizeBytes) + dyn > 160 * 1024) return false;
+    if (std::max(fa.sharedSizeBytes, fb.sharedSizeBytes) + dyn > 160 * 1024) return ok;
   }
   MultiKWorkspace& W = S.multik_ws;
   const size_t colb = sizeof(c32) * size_t(P) * g.slots;
@@ -1568,7 +1571,7 @@ bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* e
   const dim3 gcomb(unsigned(std::min<long>((PLANES * g.cs / 2 + 255) / 256, std::max(1, 2048 / P))), P);
   const bool prof = S.prof.enabled;
   int cur = 0, it = 0;
-  bool fin = false, ok = true;
+  bool fin = false;
   for (; it < maxit && !fin; ++it) {
     switch (NT) {
       case 1: gram(std::integral_constant<int, 1>{}, cur); break;
@@ -1623,8 +1626,8 @@ bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* e
   }
   OMX_HIP_CHECK(hipStreamSynchronize(sm));
   OMX_HIP_CHECK(hipMemcpy(hs.data(), st, sizeof(MkState) * P, hipMemcpyDeviceToHost));
-  for (int p = 0; p < P; ++p) ok = ok && hs[p].done == 1;
-  if (!ok) return false;
+  for (int p = 0; p < P; ++p) ok[p] = hs[p].done == 1;
+  if (std::count(ok.begin(), ok.end(), 1) == 0) return ok;
   kout.clear();
   iters.clear();
   moves.clear();
@@ -1633,16 +1636,16 @@ bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* e
   for (int p = 0, i = 0; p < P; ++p)
     for (int j = 0; j < probs[p].nev; ++j, ++i) {
       kout.push_back(hs[p].k[j]);
-      iters.push_back(hs[p].its[j]);
+      iters.push_back(ok[p] ? hs[p].its[j] : 0);
       mmax = std::max(mmax, msize[i]);
-      stats.matvec += hs[p].its[j];
-      stats.precon += hs[p].its[j];
+      stats.matvec += iters.back();
+      stats.precon += iters.back();
     }
   dense(std::true_type{});
   hipLaunchKernelGGL(k_mk_handover, dim3(unsigned(std::min<long>((S.N + 255) / 256, 512)), ninst, (mmax + HQ - 1) / HQ),
                      dim3(256), 0, sm, g, cols, st, instd, mszd, cblk, X64, ld, istride);
   OMX_HIP_CHECK(hipGetLastError());
-  return true;
+  return ok;
 }
 
 }  // namespace omx

@@ -46,14 +46,16 @@ struct MkProblem {
 };
 
 // Runs the FP32 phase for the problems (all on S's grid; problem p reads the eps^-1 field
-// eps6c + p * eps_stride).  On success writes each band's block of FP64 Ritz vectors at its
-// k: band j of problem p is instance i = off + j (off: bands of the problems before), columns
-// 0 .. msize[i]-1 at X64 + i istride + c ld; kout[i] its k.  Iterations per band into iters,
-// per problem those that moved a band's k into moves.
-// Returns false, with nothing written, if a band did not converge within maxit iterations.
-bool multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* eps6c, long eps_stride, int maxit,
-                  const std::vector<int>& msize, c64* X64, long ld, long istride, std::vector<double>& kout,
-                  std::vector<int>& iters, std::vector<int>& moves, SolveStats& stats);
+// eps6c + p * eps_stride).  Returns per problem whether all its bands converged within maxit
+// iterations; the others are given up without holding those back.  Writes each band's block of
+// FP64 Ritz vectors at its k for the problems that did: band j of problem p is instance
+// i = off + j (off: bands of the problems before), columns 0 .. msize[i]-1 at X64 + i istride +
+// c ld; kout[i] its k.  Iterations per band into iters, per problem those that moved a band's k
+// into moves.  (Of a problem given up: nothing at X64, kout its last k, iters 0.)
+std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, const float* eps6c, long eps_stride,
+                               int maxit, const std::vector<int>& msize, c64* X64, long ld, long istride,
+                               std::vector<double>& kout, std::vector<int>& iters, std::vector<int>& moves,
+                               SolveStats& stats);
 
 // columns of the widest block handed over for nev bands on a grid of K unknowns: the space's
 // columns past the bands too

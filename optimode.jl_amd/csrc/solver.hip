@@ -2121,8 +2121,8 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
     }
     std::vector<double> kk;
     std::vector<int> its, moves;
-    if (!multik_solve(*this, {q}, p32.plan.eps6c, 0, multik_cap(*this, maxiter, max_eigsolves), msize_mk, b64.p(b64.X[0]), ld,
-                      b64.istride, kk, its, moves, stats)) {
+    if (!multik_solve(*this, {q}, p32.plan.eps6c, 0, multik_cap(*this, maxiter, max_eigsolves), msize_mk, b64.p(b64.X[0]),
+                      ld, b64.istride, kk, its, moves, stats)[0]) {
       ++solve_phases().redone;
       return false;
     }
@@ -2329,24 +2329,45 @@ void Solver::get_evecs(double* evecs) {
   OMX_HIP_CHECK(hipStreamSynchronize(stream));
 }
 
-namespace {
-
-// Host conversion of a (3,3,Nx,Ny) column-major field to the operator's two 6-entry layouts,
-// written to device memory at rowm / colm (2D cells).
-}  // namespace
-
 // Several solve_k problems on this grid in one batch (no reference counterpart as one call:
 // the reference sweeps run solve_k, src/solve.jl:182-196, one problem per call or process,
-// lib/ModeSweeps/src/batch.jl:256-265).  Problem p's band j is instance off_p + j; the block
-// size is the largest nev, each instance using min(nev_p, j + 1 + guard) columns.  Every
-// launch of the FP32 phase (shared first eigensolve per problem, inexact Newton), of the
-// FP64 refinement and of the phase canonicalisation covers all instances; the operator
-// reads instance i's eps^-1 through plan.eps_slot.  Per problem the results are those of
-// omx_solve_k on that problem alone, up to rounding.
+// lib/ModeSweeps/src/batch.jl:256-265).  Per problem the results are those of omx_solve_k on
+// that problem alone, up to rounding: the problems that the shared search space or the
+// refinement of its blocks does not finish, and only those, are solved again per band.
 void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
   require_2d("the batched solve_k");
+  if (probs.empty()) return;
+  const std::vector<int> again = solve_group(probs, true);
+  if (again.empty()) return;
+  solve_phases().redone += long(again.size());
+  // the first run's blocks make room for the second's
+  workspaces.clear();
+  multik_ws.release();
+  std::vector<MultiProblem> left;
+  for (int p : again) left.push_back(probs[p]);
+  try {
+    solve_group(left, false);
+  } catch (const Error& e) {  // theirs alone: the other problems have their results
+    for (auto& q : left) q.status = e.code();
+  }
+  for (size_t j = 0; j < again.size(); ++j) {
+    const double before = probs[again[j]].info.device_ms;
+    probs[again[j]].info = left[j].info;
+    probs[again[j]].info.device_ms += before;
+    probs[again[j]].status = left[j].status;
+  }
+}
+
+// One run over the problems: band j of problem p is instance off_p + j; the block size is the
+// largest nev, each instance using min(nev_p, j + 1 + guard) columns.  Every launch covers all
+// instances; the operator reads instance i's eps^-1 through plan.eps_slot.  FP32 phase: one
+// shared search space per problem (multik.hip), or with `shared` false, in FP64 throughout, or
+// where the grid does not fit it, one LOBPCG block per band (a first eigensolve per problem,
+// then inexact Newton).  Then the FP64 refinement and the phase canonicalisation.  Returns the
+// problems left without a result by the shared search space (their outputs are not written,
+// but for the run's device time).
+std::vector<int> Solver::solve_group(std::vector<MultiProblem>& probs, bool shared) {
   const int P = int(probs.size());
-  if (P == 0) return;
   int ninst = 0, M = 0, maxiter = 1, max_eigsolves = 1;
   for (auto& p : probs) {
     if (p.nev < 1 || p.nev > 16) throw Error(OMX_ERR_UNSUPPORTED, "nev must be in 1..16");
@@ -2367,6 +2388,13 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
   OMX_HIP_CHECK(hipEventCreate(&e0));
   OMX_HIP_CHECK(hipEventCreate(&e1));
   OMX_HIP_CHECK(hipEventRecord(e0, s));
+  auto finish_ms = [&] {  // the batch's device time, to every problem (e1 has passed)
+    float ms = 0;
+    OMX_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    for (auto& p : probs) p.info.device_ms = ms;
+  };
   // the problems' eps^-1, and which one each instance reads
   const size_t n6 = (size_t(6) * N + 63) / 64 * 64;  // fields start on whole lines
   multi_e32r.ensure(sizeof(float) * n6 * P);
@@ -2440,7 +2468,8 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
       kinit[i] = k0[p];
     }
   const int maxit64 = std::max(maxiter, opt.maxiter_fp64);
-  const bool use_multik = opt.multik && opt.refine && opt.fp32_newton && !opt.fp64_only && multik_fits(*this);
+  const bool use_multik =
+      shared && opt.multik && opt.refine && opt.fp32_newton && !opt.fp64_only && multik_fits(*this);
   const auto b64p = workspace<double>(*this, ninst, use_multik ? multik_block(M, K) : M, maxit64);
   Batch<double>& b64 = *b64p;
   std::vector<int> it32_inst(ninst, 0);
@@ -2490,9 +2519,8 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
   };
 
   // the FP32 phase of every problem in its own shared search space (multik.hip)
-  bool mk_done = false;
-  auto multik_phase = [&]() {
-    if (!use_multik) return false;
+  std::vector<char> mk_ok;
+  if (use_multik) {
     std::vector<MkProblem> mk(P);
     std::vector<int> msize_mk(ninst);
     for (int p = 0; p < P; ++p) {
@@ -2507,26 +2535,28 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
     }
     std::vector<double> kk;
     std::vector<int> its, moves;
-    if (!multik_solve(*this, mk, p32.plan.eps6c, p32.plan.eps_stride, multik_cap(*this, maxiter, max_eigsolves), msize_mk,
-                      b64.p(b64.X[0]), ld, b64.istride, kk, its, moves, stats)) {
-      solve_phases().redone += P;
-      return false;
+    mk_ok = multik_solve(*this, mk, p32.plan.eps6c, p32.plan.eps_stride, multik_cap(*this, maxiter, max_eigsolves),
+                         msize_mk, b64.p(b64.X[0]), ld, b64.istride, kk, its, moves, stats);
+    if (std::count(mk_ok.begin(), mk_ok.end(), 1) == 0) {
+      OMX_HIP_CHECK(hipEventRecord(e1, s));
+      OMX_HIP_CHECK(hipStreamSynchronize(s));
+      finish_ms();
+      std::vector<int> every(P);
+      for (int p = 0; p < P; ++p) every[p] = p;
+      return every;
     }
     msize = msize_mk;
-    mk_done = true;
     for (int i = 0; i < ninst; ++i) {
       hns[i].k = kk[i];
       hns[i].nsolves = 1;
       hns[i].k_tol = probs[prob_of[i]].k_tol;
+      if (!mk_ok[prob_of[i]]) hns[i].done = 2;  // no part in the refinement
       it32_inst[i] += its[i];
       stats.it32 += its[i];
     }
     OMX_HIP_CHECK(hipMemcpyAsync(b64.kd.as<void>(), kk.data(), sizeof(double) * ninst, hipMemcpyHostToDevice, s));
     ++newton_total;
     OMX_HIP_CHECK(hipStreamSynchronize(s));
-    return true;
-  };
-  if (!opt.fp64_only && multik_phase()) {
   } else if (!opt.fp64_only) {
     const auto b32p = workspace<float>(*this, ninst, M, maxiter);
     Batch<float>& b32 = *b32p;
@@ -2554,36 +2584,40 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
   const int left = std::max(1, max_eigsolves - newton_total);
   if (opt.refine && !opt.fp64_only)
     stats.it64 +=
-        refine_phase(*this, b64, hns, bands, msize, eig_tol, left, stats, newton_total, max_resid, &resid, mk_done);
+        refine_phase(*this, b64, hns, bands, msize, eig_tol, left, stats, newton_total, max_resid, &resid, use_multik);
   else
     stats.it64 += newton_phase(*this, b64, hns, bands, nchk, msize, eig_tol, maxit64, left, stats, newton_total, true);
-  if (mk_done && std::any_of(hns.begin(), hns.end(), [](const NewtonState& h) { return h.done != 1; })) {
-    solve_phases().redone += P;
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    WithoutMultiK off(*this);
-    return solve_k_multi(probs);
-  }
-  (mk_done ? solve_phases().shared : solve_phases().per_band) += P;
+  std::vector<int> again;
+  for (int p = 0; p < P && use_multik; ++p)
+    for (int j = 0; j < probs[p].nev; ++j)
+      if (hns[off[p] + j].done != 1) {
+        mk_ok[p] = 0;
+        again.push_back(p);
+        break;
+      }
+  auto left_out = [&](int p) { return use_multik && !mk_ok[p]; };
+  (use_multik ? solve_phases().shared : solve_phases().per_band) += P - long(again.size());
   // band eigenvectors of every instance, phase-canonicalised together (fields.jl:258-260)
   multi_evecs.ensure(sizeof(c64) * size_t(ninst) * ld);
-  for (int i = 0; i < ninst; ++i)
-    OMX_HIP_CHECK(hipMemcpyAsync(multi_evecs.as<c64>() + size_t(i) * ld,
-                                 b64.p(b64.X[b64.cur]) + i * b64.istride + long(bands[i]) * ld, sizeof(c64) * K,
-                                 hipMemcpyDeviceToDevice, s));
+  for (int i = 0; i < ninst; ++i) {
+    c64* ev = multi_evecs.as<c64>() + size_t(i) * ld;
+    if (left_out(prob_of[i]))
+      OMX_HIP_CHECK(hipMemsetAsync(ev, 0, sizeof(c64) * K, s));
+    else
+      OMX_HIP_CHECK(hipMemcpyAsync(ev, b64.p(b64.X[b64.cur]) + i * b64.istride + long(bands[i]) * ld, sizeof(c64) * K,
+                                   hipMemcpyDeviceToDevice, s));
+  }
   canonicalize_phase(b64.kd.as<double>(), multi_evecs.as<c64>(), ld, ld, ninst, 1);
   OMX_HIP_CHECK(hipEventRecord(e1, s));
   for (int p = 0; p < P; ++p)
-    if (probs[p].evecs)
+    if (probs[p].evecs && !left_out(p))
       for (int j = 0; j < probs[p].nev; ++j)
         OMX_HIP_CHECK(hipMemcpyAsync(probs[p].evecs + 2 * size_t(j) * K, multi_evecs.as<c64>() + size_t(off[p] + j) * ld,
                                      sizeof(c64) * K, hipMemcpyDeviceToHost, s));
   OMX_HIP_CHECK(hipStreamSynchronize(s));
-  float ms = 0;
-  OMX_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
+  finish_ms();
   for (int p = 0; p < P; ++p) {
+    if (left_out(p)) continue;
     MultiProblem& q = probs[p];
     bool ok = true;
     int newton = 0, it32 = 0;
@@ -2603,9 +2637,9 @@ void Solver::solve_k_multi(std::vector<MultiProblem>& probs) {
     q.info.n_matvec = stats.matvec;         // the batch's operator applications
     q.info.n_precon = stats.precon;
     q.info.max_residual = opt.refine && !opt.fp64_only ? rmax : 0.0;
-    q.info.device_ms = ms;                  // the batch's device time
     q.status = ok ? OMX_OK : OMX_ERR_NOT_CONVERGED;
   }
+  return again;
 }
 
 void Solver::require_2d(const char* what) const {

@@ -297,6 +297,10 @@ struct MultiKWorkspace {
   PinnedMem snap[2];
   size_t snap_bytes = 0;
   hipEvent_t ev[2] = {nullptr, nullptr};
+  void release() {
+    for (DevMem* m : {&cols, &dm, &part, &red, &cx, &cblk, &rot, &normp, &state, &ints}) m->release();
+    geom = 0;
+  }
   ~MultiKWorkspace() {
     for (hipEvent_t e : ev)
       if (e) (void)hipEventDestroy(e);
@@ -342,6 +346,7 @@ class Solver {
   // each) as one batch: every band of every problem is an instance of the same LOBPCG,
   // Newton and refinement launches (2D cells)
   void solve_k_multi(std::vector<MultiProblem>& probs);
+  std::vector<int> solve_group(std::vector<MultiProblem>& probs, bool shared);
   void hmh(double k, const double* A, const double* H, int m, double* out);
   void group_index(double omega, int nev, const double* kmags, const double* evecs, const double* deps_domega,
                    double* ng_out);

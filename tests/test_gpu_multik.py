@@ -153,3 +153,41 @@ def test_batch_on_an_odd_grid():
     for q, k0 in zip(res, refs):
         assert q["status"] == 0
         assert np.max(np.abs(q["kmags"] / k0 - 1)) < 2e-10
+
+
+def test_a_batch_redoes_only_the_problems_left_undone():
+    """A problem whose top bands do not propagate at its omega converges in no form, one that
+    asks for a residual below rounding not in the refinement: the others of their launch group
+    keep the shared search space's results, at the cost of those alone."""
+    print("multik batch with problems that fail", flush=True)
+    g, ei = _eps(64, 48)
+    good = [dict(grid=g, epsinv=ei, omega=W0 * f, nev=nev, k_tol=1e-10, eig_tol=1e-8, maxiter=300)
+            for f, nev in ((1.0, 4), (1.05, 3), (0.95, 5))]
+    refs = [omx.solve_k(q["omega"], ei, g, omx.HIPSolver(), nev=q["nev"], k_tol=1e-10, eig_tol=1e-8, maxiter=300)[0]
+            for q in good]
+    below = dict(good[0], omega=0.05, nev=8, max_eigsolves=8, maxiter=40)
+    exact = dict(good[1], eig_tol=1e-17, max_eigsolves=8)
+    for bad in ([below], [exact], [below, exact]):
+        res = omx.solve_k_batch(good[:1] + bad + good[1:])
+        took = omx.solve_phases()
+        print(f"  {len(bad)} of them: status {[q['status'] for q in res]}, {took}", flush=True)
+        assert took == dict(shared=3, per_band=len(bad), redone=len(bad))
+        assert all(q["status"] == omx._lib.OMX_ERR_NOT_CONVERGED for q in res[1:1 + len(bad)])
+        for q, k0 in zip(res[:1] + res[1 + len(bad):], refs):
+            assert q["status"] == 0 and q["info"]["converged"] == 1
+            assert np.max(np.abs(q["kmags"] / k0 - 1)) < 2e-9  # k_tol / (2 * 0.3 * 0.3), both sides
+
+
+def test_a_batch_redone_whole():
+    """One iteration an eigensolve allows the shared search space eight, too few for either
+    problem, and the per-band form one per Newton step, which it makes do with."""
+    print("multik batch redone", flush=True)
+    g, ei = _eps(64, 48)
+    probs = [dict(grid=g, epsinv=ei, omega=W0 * f, nev=nev, k_tol=1e-10, eig_tol=1e-8, maxiter=1, max_eigsolves=60)
+             for f, nev in ((1.0, 4), (1.05, 3))]
+    res = omx.solve_k_batch(probs)
+    assert omx.solve_phases() == dict(shared=0, per_band=2, redone=2)
+    for p, q in zip(probs, res):
+        k0 = omx.solve_k(p["omega"], ei, g, omx.HIPSolver(), nev=p["nev"], k_tol=1e-10, eig_tol=1e-8, maxiter=300)[0]
+        assert q["status"] == 0
+        assert np.max(np.abs(q["kmags"] / k0 - 1)) < 2e-9
