@@ -179,11 +179,11 @@ def test_a_batch_redoes_only_the_problems_left_undone():
 
 
 def test_a_batch_redone_whole():
-    """One iteration an eigensolve allows the shared search space eight, too few for either
-    problem, and the per-band form one per Newton step, which it makes do with."""
+    """Two iterations an eigensolve allow the shared search space sixteen, too few for either
+    problem, and the per-band form two per Newton step, which it makes do with."""
     print("multik batch redone", flush=True)
     g, ei = _eps(64, 48)
-    probs = [dict(grid=g, epsinv=ei, omega=W0 * f, nev=nev, k_tol=1e-10, eig_tol=1e-8, maxiter=1, max_eigsolves=60)
+    probs = [dict(grid=g, epsinv=ei, omega=W0 * f, nev=nev, k_tol=1e-10, eig_tol=1e-8, maxiter=2, max_eigsolves=60)
              for f, nev in ((1.0, 4), (1.05, 3))]
     res = omx.solve_k_batch(probs)
     assert omx.solve_phases() == dict(shared=0, per_band=2, redone=2)
