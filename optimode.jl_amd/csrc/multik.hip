@@ -1494,12 +1494,15 @@ std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, c
   }
   MultiKWorkspace& W = S.multik_ws;
   const size_t colb = sizeof(c32) * size_t(P) * g.slots;
-  if (W.cols.size() < colb || W.geom != g.cs * 64 + g.mmax) {
+  // The pads past N of every plane are read as zeros.  The block update runs over them, so
+  // coefficients that are not finite leave NaN there: they count as clear only after a call that
+  // ended without.
+  const long geom = g.cs * 64 + g.mmax;
+  if (W.cols.size() < colb || W.geom != geom) {
     W.cols.ensure(colb);
-    // the pads past N of every plane are read as zeros
     OMX_HIP_CHECK(hipMemsetAsync(W.cols.as<void>(), 0, W.cols.size(), sm));
-    W.geom = g.cs * 64 + g.mmax;
   }
+  W.geom = 0;
   W.dm.ensure(sizeof(c32) * size_t(vecs) * 3 * g.cs);
   W.part.ensure(sizeof(c32) * size_t(P) * nch * NGRAM * pm * pm);
   W.red.ensure(sizeof(c64) * size_t(P) * NGRAM * pm * pm);
@@ -1626,7 +1629,12 @@ std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, c
   }
   OMX_HIP_CHECK(hipStreamSynchronize(sm));
   OMX_HIP_CHECK(hipMemcpy(hs.data(), st, sizeof(MkState) * P, hipMemcpyDeviceToHost));
-  for (int p = 0; p < P; ++p) ok[p] = hs[p].done == 1;
+  bool finite = true;
+  for (int p = 0; p < P; ++p) {
+    ok[p] = hs[p].done == 1;
+    finite = finite && hs[p].done != 2;
+  }
+  if (finite) W.geom = geom;
   if (std::count(ok.begin(), ok.end(), 1) == 0) return ok;
   kout.clear();
   iters.clear();

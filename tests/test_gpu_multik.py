@@ -191,3 +191,24 @@ def test_a_batch_redone_whole():
         k0 = omx.solve_k(p["omega"], ei, g, omx.HIPSolver(), nev=p["nev"], k_tol=1e-10, eig_tol=1e-8, maxiter=300)[0]
         assert q["status"] == 0
         assert np.max(np.abs(q["kmags"] / k0 - 1)) < 2e-9
+
+
+@pytest.mark.parametrize("nx,ny,nev", [(45, 45, 4), (27, 45, 12)])
+def test_the_shared_space_works_again_after_a_solve_that_overflowed(nx, ny, nev):
+    """Start vectors of 1e25 overflow single precision in the first iteration, the norm's
+    weight 1 / k^2 at a k of 1e-9 or so in one of the first fifty, of either parity.  Whatever
+    such a solve ends in, the handle's next one runs in the shared search space, on grids
+    whose pixel counts leave the Gram products' last loads beyond the fields (2025 = 1 and
+    1215 = 3 mod 4)."""
+    print(f"multik after an overflow {nx}x{ny} nev {nev}", flush=True)
+    g, ei = _eps(nx, ny)
+    s = omx.HIPSolver()
+    k0, ev, _ = _solve(g, ei, nev, 1, solver=s)
+    H = np.stack(ev)
+    for kw in [dict(Hguess=1e25 * H)] + [dict(Hguess=H, kguess=10.0 ** (0.05 * e)) for e in range(-181, -174)]:
+        try:
+            omx.solve_k(W0, ei, g, s, nev=nev, **{**KW, "maxiter": 20, **kw})
+        except omx.OmxError:
+            pass
+        print(f"  kguess {kw.get('kguess')}: {omx.solve_phases()}", flush=True)
+        assert np.max(np.abs(_solve(g, ei, nev, 1, solver=s)[0] / k0 - 1)) < 2e-10
