@@ -78,17 +78,6 @@ __device__ __forceinline__ int space_slot(const MkGeo& g, const MkState& s, int 
   return slot_p(g, b, s.pslot[q - s.m - s.na]);
 }
 
-// Chebyshev node t over the columns' k range (widened to 2% where it is narrower)
-__device__ __forceinline__ double mk_node(const double* k, int m, int t) {
-  double lo = k[0], hi = k[0];
-  for (int j = 1; j < m; ++j) {
-    lo = fmin(lo, k[j]);
-    hi = fmax(hi, k[j]);
-  }
-  const double c = 0.5 * (lo + hi), h = fmax(0.5 * (hi - lo), 0.01 * fabs(c));
-  return c + h * cospi((t + 0.5) / MK_NODES);
-}
-
 // in-plane part of a plane wave: n = z x w / rho (y at rho = 0)
 struct Wave {
   float n0, n1, rho2, rho;
@@ -350,8 +339,7 @@ __global__ __launch_bounds__(64 * GW) void k_mk_gram(MkGeo geo, const c32* cols,
     cp[threadIdx.x] =
         int(threadIdx.x) < n ? cols + p * geo.slots + col_off(geo, space_slot(geo, s, buf, threadIdx.x)) : nullptr;
   if (threadIdx.x < MK_NODES) {
-    const double node = mk_node(s.k, s.m, threadIdx.x);
-    kap2[threadIdx.x] = float(node * node);
+    kap2[threadIdx.x] = float(exp(2.0 * mk_node(mk_range(s.k, s.m), threadIdx.x)));
   }
   __syncthreads();
   if (kind == 0)
@@ -760,21 +748,10 @@ __global__ __launch_bounds__(DT) void k_mk_dense(MkGeo geo, MkState* st, const c
     kk /= double(b - a + 1);
     kk_s = kk;
   }
-  if (threadIdx.x < MK_NODES) node[threadIdx.x] = mk_node(FINAL ? s.kold : s.k, s.m, threadIdx.x);
+  if (threadIdx.x < MK_NODES) node[threadIdx.x] = mk_node(mk_range(FINAL ? s.kold : s.k, s.m), threadIdx.x);
   __syncthreads();
   const double kk = kk_s;
-  if (threadIdx.x < MK_NODES) {  // Lagrange weights at kk and their k-derivatives
-    const int t = threadIdx.x;
-    double w = 1, dw = 0;
-    for (int u = 0; u < MK_NODES; ++u) {
-      if (u == t) continue;
-      const double q = 1.0 / (node[t] - node[u]);
-      dw = dw * (kk - node[u]) * q + w * q;
-      w *= (kk - node[u]) * q;
-    }
-    lw[t] = w;
-    dlw[t] = dw;
-  }
+  if (threadIdx.x < MK_NODES) mk_weight(node, threadIdx.x, kk, lw[threadIdx.x], dlw[threadIdx.x]);
   __syncthreads();
   const long esz = long(pm) * pm;
   const c64* G = red + long(p) * NGRAM * esz;
@@ -1209,6 +1186,14 @@ __global__ __launch_bounds__(256) void k_mk_control(MkGeo geo, MkState* st, cons
     s.rnorm[c] = rn;
     s.kold[c] = s.k[c];
     s.k[c] = s.knew[c];
+  }
+  {  // the guard columns' k no further than a fifth below the bands' range
+    double lo = s.k[0], hi = lo;
+    for (int c = 1; c < s.nev; ++c) {
+      lo = fmin(lo, s.k[c]);
+      hi = fmax(hi, s.k[c]);
+    }
+    for (int c = s.nev; c < s.m; ++c) s.k[c] = fmin(fmax(s.k[c], 0.8 * lo), hi);
   }
   s.iter += 1;
   s.moves += moved;

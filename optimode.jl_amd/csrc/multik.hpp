@@ -9,15 +9,19 @@
 //   <h, M(k) h> = <F0 + k F1, eps^-1 (F0 + k F1)>,  F0 = fft(D0), F1 = fft(D1)
 //   <h, h>      = sum |g1|^2 / (rho^2 + k^2) + |g2|^2
 // so three Gram matrices of the transformed columns give S^H M(k) S for every k, and the
-// norm's Gram matrix is interpolated in k from MK_NODES Chebyshev nodes (its entries are
-// analytic in k with the nearest pole at distance k: eight nodes over the bands' k range
-// leave about 1e-9).  Per iteration each band solves its small pencil at its own k_j on its own
-// workgroup, moves k_j by a Newton step of its Ritz value, and contributes one residual, one
-// preconditioned direction W and one previous direction P.
+// norm's Gram matrix is interpolated in ln k from MK_NODES Chebyshev nodes over the columns' k
+// range (multik_math.hpp, with the error by the range's width).  Per iteration each band
+// solves its small pencil at its own k_j on its own workgroup, moves k_j by a Newton step of its
+// Ritz value, and contributes one residual, one preconditioned direction W and one previous
+// direction P.  The guard columns are there for the bands below them: their k stays at most a
+// fifth below the bands' range (left to themselves, those that do not propagate at omega shrink
+// their k without end and widen the interpolation's range with it: ten bands with such guards
+// took 82 ms on 40 x 45, by way of the per-band form, and take 7).
 #pragma once
 #include <algorithm>
 #include <vector>
 
+#include "multik_math.hpp"
 #include "omx_common.hpp"
 
 namespace omx {
@@ -28,7 +32,6 @@ struct SolveStats;
 
 constexpr int MK_MAXM = 18;     // columns per problem: nev (16) + guard (2)
 constexpr int MK_MAXN = 54;     // search space [X W P]
-constexpr int MK_NODES = 8;     // interpolation nodes of the norm's Gram matrix
 constexpr int MK_GUARD = 2;
 
 struct MkProblem {

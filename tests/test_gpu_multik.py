@@ -212,3 +212,25 @@ def test_the_shared_space_works_again_after_a_solve_that_overflowed(nx, ny, nev)
             pass
         print(f"  kguess {kw.get('kguess')}: {omx.solve_phases()}", flush=True)
         assert np.max(np.abs(_solve(g, ei, nev, 1, solver=s)[0] / k0 - 1)) < 2e-10
+
+
+def _box(d, nx=40, ny=45):
+    """A guide that fills most of its cell: past the lowest pair the bands are near cut-off, the
+    eleventh and twelfth below it."""
+    x, y = -d / 2 + d / nx * np.arange(nx), 0.98 * (-d / 2 + d / ny * np.arange(ny))
+    eps = 2.1 + 2.1 * np.exp(-(x[:, None] / 0.4) ** 2 - (y[None, :] / 0.3) ** 2)
+    return omx.Grid(d, 0.98 * d, nx, ny), np.ascontiguousarray(np.eye(3)[:, :, None, None] / eps)
+
+
+@pytest.mark.parametrize("d,nev", [(1.1, 10), (1.3, 10), (1.1, 8), (0.95, 4)])
+def test_bands_near_cut_off(d, nev):
+    """The guard columns of ten bands do not propagate at this omega, and the bands' own k
+    spread over a factor of two and more: both must stay in the shared search space, in no
+    more iterations than the same solve without such guards needs."""
+    print(f"multik near cut-off {d} nev {nev}", flush=True)
+    g, ei = _box(d)
+    k0, _, _ = _solve(g, ei, nev, 0)
+    k1, _, info = _solve(g, ei, nev, 1)
+    print(f"  k {k1[0]:.4f} .. {k1[-1]:.4f}, {info['lobpcg_iters_fp32']} iterations over the bands", flush=True)
+    assert np.max(np.abs(k1 / k0 - 1)) < 1e-11 / (2 * 0.1 * 0.1)
+    assert info["lobpcg_iters_fp32"] <= 15 * nev

@@ -13,6 +13,16 @@ pytestmark = pytest.mark.skipif(CXX is None, reason="no host C++ compiler")
 
 SOURCE = """
 #include "multik_math.hpp"
+extern "C" void interpolation(const double* k, int n, double at, double* nodes, double* w, double* dw) {
+  const omx::MkRange r = omx::mk_range(k, n);
+  double x[omx::MK_NODES];
+  for (int t = 0; t < omx::MK_NODES; ++t) {
+    x[t] = omx::mk_node(r, t);
+    nodes[t] = exp(x[t]);
+  }
+  for (int t = 0; t < omx::MK_NODES; ++t) omx::mk_weight(x, t, at, w[t], dw[t]);
+}
+extern "C" int nodes() { return omx::MK_NODES; }
 extern "C" int position(const double* d, int n, int a) { return omx::mk_position(d, n, a); }
 """
 
@@ -40,3 +50,41 @@ def test_positions_are_a_permutation(lib, d):
     order = np.empty(len(a), dtype=int)
     order[pos] = np.arange(len(a))
     assert list(order) == list(np.argsort(a, kind="stable"))  # numpy sorts NaN last too
+
+
+def _interpolation(lib, ks, at):
+    n = lib.nodes()
+    out = [np.zeros(n) for _ in range(3)]
+    p = ctypes.POINTER(ctypes.c_double)
+    k = np.array(ks)
+    lib.interpolation(k.ctypes.data_as(p), len(k), ctypes.c_double(at), *(a.ctypes.data_as(p) for a in out))
+    return out
+
+
+def test_norm_weights_by_the_width_of_the_k_range(lib):
+    """1 / (rho^2 + k^2) and its k-derivative from the nodes, against the stated worst relative
+    errors (half a digit of slack for their rounding and the sampling here).  A derivative of the
+    interpolant loses up to the square of its degree over the half-width of the range."""
+    for ratio, bound in ((1.01, 1e-14), (1.2, 2e-12), (1.5, 1e-9), (2.0, 9e-8), (3.0, 5e-6), (5.0, 1.3e-4)):
+        for base in (0.02, 0.4, 1.3):
+            lo, hi = base, base * ratio
+            err = der = 0.0
+            for at in np.geomspace(lo, hi, 33):
+                nodes, w, dw = _interpolation(lib, [hi, lo, 0.5 * (lo + hi)], at)
+                for rho in np.r_[0.0, lo * np.geomspace(0.03, 100, 25)]:
+                    f = 1 / (rho ** 2 + nodes ** 2)
+                    exact, slope = 1 / (rho ** 2 + at ** 2), -2 * at / (rho ** 2 + at ** 2) ** 2
+                    err = max(err, abs(w @ f / exact - 1))
+                    der = max(der, abs(dw @ f - slope) / (exact / at))
+            assert err < 1.5 * bound
+            assert der < 1.5 * bound * 49 / max(np.log(ratio) / 2, 0.01) + 1e-11
+
+
+def test_norm_weights_at_a_node_and_for_negative_k(lib):
+    nodes, _, _ = _interpolation(lib, [0.9, 1.2], 1.0)
+    for t, at in enumerate(nodes):
+        _, w, _ = _interpolation(lib, [0.9, 1.2], at)
+        assert np.allclose(w, np.arange(len(nodes)) == t, atol=1e-12)
+    _, w, dw = _interpolation(lib, [0.9, 1.2], 1.1)
+    _, wn, dwn = _interpolation(lib, [-0.9, -1.2], -1.1)
+    assert np.allclose(w, wn) and np.allclose(dw, -dwn)
