@@ -36,13 +36,22 @@ namespace {
 
 constexpr int PLANES = 7;
 constexpr double MK_CLUSTER = 3e-5;  // bands whose k agree to this take their vectors at one k
+// A problem is left to the per-band form when nothing has come nearer to its thresholds for
+// MK_IDLE iterations (solves that converge pause for a few), or when its bands' k spread over
+// more than MK_WIDEST, where the norm's interpolation (multik_math.hpp) is past the thresholds:
+// bands that do not propagate at omega, tolerances below single precision.
+constexpr int MK_IDLE = 40;
+constexpr double MK_WIDEST = 12;
 constexpr int FT = 512;   // threads of the transform kernels
 constexpr int NGRAM = 3 + MK_NODES + 1;  // G00, G01, G11, the nodes, the k-independent part
 
 struct MkState {
   int m, nev;              // columns, bands
   int na, np;              // W columns and P columns of the current search space
-  int iter, done, par;     // done: 1 converged, 2 failed; par: X / P buffer of the last space
+  int iter, done, par;     // done: 1 converged, 2 not finite, 3 given up; par: X / P buffer of the last space
+  int ahead;               // most bands converged at once so far
+  int idle;                // iterations since that or `worst` got better
+  double worst;            // smallest over the iterations of the largest distance from the thresholds
   int moves;               // iterations whose Newton step moved a band's k by more than ftol
   int wcol[MK_MAXM];       // column of W slot s
   int pslot[MK_MAXM];      // P slots in use
@@ -53,7 +62,14 @@ struct MkState {
   double keval[MK_MAXM];   // k the column's Ritz pair was taken at
   double knew[MK_MAXM];    // after the Newton step
   double lam[MK_MAXM], slope[MK_MAXM], rnorm[MK_MAXM];
+  double node[MK_NODES];   // interpolation nodes (in ln k) of the iteration under way
+  float kap2[MK_NODES];    // their k^2
 };
+
+OMX_HD void set_node(MkState& s, const MkRange& r, int t) {
+  s.node[t] = mk_node(r, t);
+  s.kap2[t] = float(exp(2.0 * s.node[t]));
+}
 
 struct MkGeo {
   int nx, ny, mmax;
@@ -338,9 +354,7 @@ __global__ __launch_bounds__(64 * GW) void k_mk_gram(MkGeo geo, const c32* cols,
   if (threadIdx.x < 16 * NT)
     cp[threadIdx.x] =
         int(threadIdx.x) < n ? cols + p * geo.slots + col_off(geo, space_slot(geo, s, buf, threadIdx.x)) : nullptr;
-  if (threadIdx.x < MK_NODES) {
-    kap2[threadIdx.x] = float(exp(2.0 * mk_node(mk_range(s.k, s.m), threadIdx.x)));
-  }
+  if (threadIdx.x < MK_NODES) kap2[threadIdx.x] = s.kap2[threadIdx.x];
   __syncthreads();
   if (kind == 0)
     gram_body<NT, 0, 1, S>(geo, cp, kap2, red, p, 0, nt, rpc, part);
@@ -748,7 +762,7 @@ __global__ __launch_bounds__(DT) void k_mk_dense(MkGeo geo, MkState* st, const c
     kk /= double(b - a + 1);
     kk_s = kk;
   }
-  if (threadIdx.x < MK_NODES) node[threadIdx.x] = mk_node(mk_range(FINAL ? s.kold : s.k, s.m), threadIdx.x);
+  if (threadIdx.x < MK_NODES) node[threadIdx.x] = s.node[threadIdx.x];
   __syncthreads();
   const double kk = kk_s;
   if (threadIdx.x < MK_NODES) mk_weight(node, threadIdx.x, kk, lw[threadIdx.x], dlw[threadIdx.x]);
@@ -1155,45 +1169,40 @@ __global__ __launch_bounds__(FT) void k_mk_rowR(MkGeo geo, const c32* cols, cons
   }
 }
 
-// Residual norms, convergence, the next search space.  One block per problem.
-__global__ __launch_bounds__(256) void k_mk_control(MkGeo geo, MkState* st, const double* normp, int nrb, int cur) {
-  const int p = blockIdx.x;
-  MkState& s = st[p];
-  if (s.done) return;
-  __shared__ double nr[MK_MAXM];
-  const int lane = threadIdx.x & 63;
-  for (int c = threadIdx.x >> 6; c < s.m; c += 4) {
-    double a = 0;
-    for (int b = lane; b < nrb; b += 64) a += normp[(long(p) * geo.mmax + c) * nrb + b];
-    for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
-    if (lane == 0) nr[c] = sqrt(a);
-  }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
+// A problem's next state from its residual norms (one thread): thresholds, k, the columns that go
+// on; ext: the extent of |k| over the columns
+__device__ void control_step(MkState& s, const double* nr, int cur, double* ext) {
   bool all = true, bad = false, moved = false;
+  int nconv = 0;
+  double worst = 0;
   int act[MK_MAXM];
   for (int c = 0; c < s.m; ++c) {
-    const double rn = nr[c], dk = s.knew[c] - s.k[c];
+    // w^2's distance at the column's own k (bands of a cluster are taken at a shared one)
+    const double rn = nr[c], f = fabs(s.lam[c] + s.slope[c] * (s.k[c] - s.keval[c]) - s.omega2);
     bad = bad || !isfinite(rn) || !isfinite(s.lam[c]);
     act[c] = rn > s.tol;
-    const bool still = fabs(dk * s.slope[c]) <= s.ftol, conv = !act[c] && still;
+    // by the distance itself, not the step made of it: a band that does not propagate at
+    // omega shrinks its k, and with it the limited step times the slope, at any distance
+    const bool still = f <= s.ftol, conv = !act[c] && still;
     if (c < s.nev) {
       moved = moved || !still;
       if (conv && !s.its[c]) s.its[c] = s.iter + 1;
       if (!conv) s.its[c] = 0;
       all = all && conv;
+      nconv += conv;
+      worst = fmax(worst, fmax(rn / s.tol, f / s.ftol));
     }
     s.rnorm[c] = rn;
     s.kold[c] = s.k[c];
     s.k[c] = s.knew[c];
   }
+  bool wide = false;
   {  // the guard columns' k no further than a fifth below the bands' range
-    double lo = s.k[0], hi = lo;
-    for (int c = 1; c < s.nev; ++c) {
-      lo = fmin(lo, s.k[c]);
-      hi = fmax(hi, s.k[c]);
-    }
+    double lo, hi;
+    mk_extent(s.k, s.nev, lo, hi);
+    wide = hi > MK_WIDEST * lo;
     for (int c = s.nev; c < s.m; ++c) s.k[c] = fmin(fmax(s.k[c], 0.8 * lo), hi);
+    mk_extent(s.k, s.m, ext[0], ext[1]);
   }
   s.iter += 1;
   s.moves += moved;
@@ -1216,6 +1225,17 @@ __global__ __launch_bounds__(256) void k_mk_control(MkGeo geo, MkState* st, cons
     s.done = 1;
     return;
   }
+  if (nconv > s.ahead || worst < 0.9 * s.worst) {
+    s.ahead = max(s.ahead, nconv);
+    s.worst = fmin(s.worst, worst);
+    s.idle = 0;
+  } else {
+    s.idle += 1;
+  }
+  if (wide || s.idle >= MK_IDLE) {
+    s.done = 3;
+    return;
+  }
   int np = 0;
   for (int w = 0; w < s.na; ++w)
     if (act[s.wcol[w]]) s.pslot[np++] = w;
@@ -1224,6 +1244,26 @@ __global__ __launch_bounds__(256) void k_mk_control(MkGeo geo, MkState* st, cons
   for (int c = 0; c < s.m; ++c)
     if (act[c]) s.wcol[na++] = c;
   s.na = na;
+}
+
+// Residual norms, convergence, the next search space.  One block per problem.
+__global__ __launch_bounds__(256) void k_mk_control(MkGeo geo, MkState* st, const double* normp, int nrb, int cur) {
+  const int p = blockIdx.x;
+  MkState& s = st[p];
+  if (s.done) return;
+  __shared__ double nr[MK_MAXM], ext[2];
+  const int lane = threadIdx.x & 63;
+  for (int c = threadIdx.x >> 6; c < s.m; c += 4) {
+    double a = 0;
+    for (int b = lane; b < nrb; b += 64) a += normp[(long(p) * geo.mmax + c) * nrb + b];
+    for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
+    if (lane == 0) nr[c] = sqrt(a);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) control_step(s, nr, cur, ext);
+  __syncthreads();
+  // the next iteration's nodes; those of the last one made stay for the handover
+  if (!s.done && threadIdx.x < MK_NODES) set_node(s, mk_range(ext[0], ext[1]), threadIdx.x);
 }
 
 // FFT along y, eps_ave, FFT back, for the columns that go on
@@ -1455,7 +1495,11 @@ std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, c
     s.omega2 = q.omega * q.omega;
     s.tol = q.tol;
     s.ftol = q.ftol;
+    s.worst = 1e300;
     for (int j = 0; j < s.m; ++j) s.k[j] = s.knew[j] = s.keval[j] = q.k[std::min<size_t>(j, q.k.size() - 1)];
+    double lo, hi;
+    mk_extent(s.k, s.m, lo, hi);
+    for (int t = 0; t < MK_NODES; ++t) set_node(s, mk_range(lo, hi), t);
     g.mmax = std::max(g.mmax, s.m);
     ninst += q.nev;
   }

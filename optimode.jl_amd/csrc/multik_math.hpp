@@ -38,18 +38,20 @@ constexpr int MK_NODES = 8;  // interpolation nodes of the norm's Gram matrix
 struct MkRange {
   double c, h;  // centre and half-width in x
 };
-OMX_HD MkRange mk_range(const double* k, int n) {
-  double lo = fabs(k[0]), hi = lo;
+OMX_HD MkRange mk_range(double lo, double hi) {  // of |k|
+  const double a = log(lo), b = log(hi);
+  return MkRange{0.5 * (a + b), fmax(0.5 * (b - a), 0.01)};
+}
+OMX_HD void mk_extent(const double* k, int n, double& lo, double& hi) {
+  lo = hi = fabs(k[0]);
   for (int j = 1; j < n; ++j) {
     const double a = fabs(k[j]);
     lo = fmin(lo, a);
     hi = fmax(hi, a);
   }
-  const double a = log(lo), b = log(hi);
-  return MkRange{0.5 * (a + b), fmax(0.5 * (b - a), 0.01)};
 }
 OMX_HD double mk_node(const MkRange& r, int t) {  // in x
-  return r.c + r.h * cos(M_PI * (t + 0.5) / MK_NODES);
+  return r.c + r.h * cos(M_PI / MK_NODES * (t + 0.5));
 }
 // Lagrange weight of node t at k and its k-derivative
 OMX_HD void mk_weight(const double* node, int t, double k, double& w, double& dw) {

@@ -234,3 +234,39 @@ def test_bands_near_cut_off(d, nev):
     print(f"  k {k1[0]:.4f} .. {k1[-1]:.4f}, {info['lobpcg_iters_fp32']} iterations over the bands", flush=True)
     assert np.max(np.abs(k1 / k0 - 1)) < 1e-11 / (2 * 0.1 * 0.1)
     assert info["lobpcg_iters_fp32"] <= 15 * nev
+
+
+@pytest.mark.parametrize("why", ["evanescent bands", "below single precision"])
+def test_a_hopeless_phase_ends_early(why, monkeypatch, capfd):
+    """Bands with no k at this omega, and a threshold the phase's single precision cannot meet:
+    the shared search space stops trying well before its cap of 200 iterations."""
+    print(f"multik hopeless: {why}", flush=True)
+    monkeypatch.setenv("OMX_TRACE", "1")
+    g, ei = _eps(64, 48)
+    s = omx.HIPSolver(fp32_tol=1e-9) if "below" in why else omx.HIPSolver()
+    capfd.readouterr()
+    try:
+        k, _ = omx.solve_k(0.05 if "evan" in why else W0, ei, g, s, nev=8 if "evan" in why else 4, k_tol=1e-10,
+                           eig_tol=1e-10, maxiter=40, max_eigsolves=8)
+    except omx.OmxError as e:
+        assert e.status == omx._lib.OMX_ERR_NOT_CONVERGED
+    its = capfd.readouterr().err.count("[omx] multik it")
+    print(f"  {its} iterations, {omx.solve_phases()}", flush=True)
+    assert omx.solve_phases()["redone"] == 1
+    assert its < 80
+
+
+@pytest.mark.parametrize("sep", [1.2, 1.5, 1.8, 2.1, 2.4])
+def test_close_bands(sep):
+    """Two equal guides sep on either side of the middle: pairs of bands whose k differ by 1e-3
+    down to rounding.  Pairs closer than 3e-5 take their vectors at one k, and each must still
+    settle at its own."""
+    print(f"multik pair at {sep}", flush=True)
+    g = omx.Grid(10.0, 4.0, 100, 48)
+    x, y = np.arange(100)[:, None] * 0.1 - 5.0, np.arange(48)[None, :] / 12 - 2.0
+    eps = 2.1 + 2.0 * np.exp(-(y / 0.4) ** 2) * (np.exp(-((x - sep) / 0.5) ** 2) + np.exp(-((x + sep) / 0.5) ** 2))
+    ei = np.ascontiguousarray(np.eye(3)[:, :, None, None] / eps)
+    k0, _, _ = _solve(g, ei, 4, 0)
+    k1, _, _ = _solve(g, ei, 4, 1)
+    print(f"  k {k1}, splits {k1[0] / k1[1] - 1:.1e} {k1[2] / k1[3] - 1:.1e}", flush=True)
+    assert np.max(np.abs(k1 / k0 - 1)) < 2e-10

@@ -14,7 +14,9 @@ pytestmark = pytest.mark.skipif(CXX is None, reason="no host C++ compiler")
 SOURCE = """
 #include "multik_math.hpp"
 extern "C" void interpolation(const double* k, int n, double at, double* nodes, double* w, double* dw) {
-  const omx::MkRange r = omx::mk_range(k, n);
+  double lo, hi;
+  omx::mk_extent(k, n, lo, hi);
+  const omx::MkRange r = omx::mk_range(lo, hi);
   double x[omx::MK_NODES];
   for (int t = 0; t < omx::MK_NODES; ++t) {
     x[t] = omx::mk_node(r, t);
