@@ -1717,6 +1717,11 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
   // each band's residual at its last Newton update (the first step's is only the looser
   // jd_first_tol one); their maximum is the solve's final residual
   std::vector<double> last_rn(ninst, 0.0);
+  // loose_blocks: an instance whose k has settled and whose residual has not halved for three
+  // steps (a tolerance below rounding) ends as not done; the per-band form, which runs after it,
+  // spends the caller's whole step limit on it
+  std::vector<double> best_rn(ninst, 1e300);
+  std::vector<int> idle(ninst, 0);
   for (int step = 0; step < max_steps; ++step) {
     bool any = false;
     for (int i = 0; i < ninst; ++i) {
@@ -1897,10 +1902,16 @@ int refine_phase(Solver& S, Batch<double>& b, std::vector<NewtonState>& hns, con
         ns.slope = slope;
         ns.nsolves += 1;
         last_rn[i] = rn[i];
+        if (rn[i] < 0.5 * best_rn[i]) {
+          best_rn[i] = rn[i];
+          idle[i] = 0;
+        } else if (std::fabs(ns.f) <= ns.k_tol) {
+          ++idle[i];
+        }
         if (resid_inst) (*resid_inst)[i] = rn[i];
         if (rn[i] <= tols[i] && std::fabs(ns.f) <= ns.k_tol) {
           ns.done = 1;
-        } else if (ns.nsolves >= ns.max_solves) {
+        } else if (ns.nsolves >= ns.max_solves || (loose_blocks && idle[i] >= 3)) {
           ns.done = 2;
         } else {
           const double kn = ns.k - ns.f / slope;

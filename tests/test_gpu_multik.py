@@ -270,3 +270,22 @@ def test_close_bands(sep):
     k1, _, _ = _solve(g, ei, 4, 1)
     print(f"  k {k1}, splits {k1[0] / k1[1] - 1:.1e} {k1[2] / k1[3] - 1:.1e}", flush=True)
     assert np.max(np.abs(k1 / k0 - 1)) < 2e-10
+
+
+def test_a_tolerance_below_rounding_costs_one_solve(monkeypatch, capfd):
+    """A residual of 1e-17 is out of reach of either form.  The refinement of the shared
+    space's blocks sees that it makes no progress; only the per-band form after it goes to the
+    caller's limit of eigensolves."""
+    print("multik tolerance below rounding", flush=True)
+    monkeypatch.setenv("OMX_TRACE", "1")
+    g, ei = _eps(64, 48)
+    capfd.readouterr()
+    with pytest.raises(omx.OmxError) as e:
+        omx.solve_k(W0, ei, g, omx.HIPSolver(), nev=3, k_tol=1e-10, eig_tol=1e-17, maxiter=100, max_eigsolves=24)
+    assert e.value.status == omx._lib.OMX_ERR_NOT_CONVERGED
+    log = capfd.readouterr().err
+    first, second = log.split("[omx] fp32 lobpcg run", 1)
+    steps = [t.count("[omx] fp64 refine step") - t.count(", correction ") for t in (first, second)]
+    print(f"  refinement steps {steps}, {omx.solve_phases()}", flush=True)
+    assert omx.solve_phases() == REDONE
+    assert steps[0] <= 8
