@@ -1,9 +1,9 @@
 // omx_solve_k_batch: independent solve_k problems of uneven grid, omega and mode count.
 // Problems are bucketed by grid; each bucket runs on one handle and one stream, in launch
 // groups of as many problems as fit the device memory: every band of every problem in a
-// group is an instance of the same LOBPCG / Newton / refinement launches
-// (Solver::solve_k_multi), so the per-iteration launches and the small dense steps are
-// shared by all of them instead of repeated per problem.
+// group takes part in the same launches (Solver::solve_k_multi: one shared search space per
+// problem, then the refinement with an instance per band), so that launches and small dense
+// steps are shared by all of them instead of repeated per problem.
 #include <algorithm>
 #include <cstring>
 #include <map>
@@ -11,20 +11,10 @@
 #include <tuple>
 #include <vector>
 
+#include "multik_math.hpp"
 #include "solver.hpp"
 
 namespace omx {
-
-namespace {
-
-// device bytes of a launch group of `ninst` instances of block size M (both LOBPCG batches,
-// the refinement and correction-solve vectors)
-size_t group_bytes(long N, long ld, long ninst, long M) {
-  const size_t lob = size_t(ninst) * M * (11 * size_t(ld) + 3 * size_t(N));
-  return (16 + 8) * lob + size_t(ninst) * (16 * 16 * size_t(ld) + 16 * 3 * size_t(N));
-}
-
-}  // namespace
 
 void solve_k_batch(int device, int nprob, omx_problem* probs, int max_group, int fp64_only) {
   if (nprob < 0 || (nprob > 0 && !probs)) throw Error(OMX_ERR_INVALID_ARG, "bad problem list");
@@ -81,7 +71,8 @@ void solve_k_batch(int device, int nprob, omx_problem* probs, int max_group, int
       while (end < ids.size()) {
         const omx_problem& q = probs[ids[end]];
         const long n2 = ninst + q.nev, M2 = std::max<long>(M, q.nev);
-        if (end > at && (group_bytes(h->N, h->ld, n2, M2) > budget || (max_group > 0 && long(end - at) >= max_group)))
+        if (end > at && (group_bytes(h->N, h->K, h->ld, long(end - at) + 1, n2, M2) > budget ||
+                         (max_group > 0 && long(end - at) >= max_group)))
           break;
         ninst = n2;
         M = M2;

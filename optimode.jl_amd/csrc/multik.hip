@@ -34,7 +34,7 @@ namespace omx {
 
 namespace {
 
-constexpr int PLANES = 7;
+constexpr int PLANES = MK_PLANES;
 constexpr double MK_CLUSTER = 3e-5;  // bands whose k agree to this take their vectors at one k
 // A problem is left to the per-band form when nothing has come nearer to its thresholds for
 // MK_IDLE iterations (solves that converge pause for a few), or when its bands' k spread over
@@ -402,8 +402,6 @@ __global__ __launch_bounds__(256) void k_mk_reduce(const c32* part, int nchunk, 
 // ---------------------------------------------------------------------------------------
 // Dense step: one workgroup per band.
 // ---------------------------------------------------------------------------------------
-constexpr int MK_SWEEPS = 10;  // Jacobi sweeps whose rotations are kept (4 to 7 are made)
-
 struct MkRot {
   double c;
   c64 s;
@@ -1473,7 +1471,6 @@ std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, c
   g.nx = S.nx;
   g.ny = S.ny;
   g.N = S.N;
-  g.cs = (S.N + 63) / 64 * 64;
   g.invdx = 1.0 / S.Dx;
   g.invdy = 1.0 / S.Dy;
   g.fx = S.p32.plan.fx;
@@ -1503,16 +1500,14 @@ std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, c
     g.mmax = std::max(g.mmax, s.m);
     ninst += q.nev;
   }
-  g.slots = 5L * g.mmax * PLANES * g.cs;
-  const int nmax = 3 * g.mmax, NT = (nmax + 15) / 16, pm = 16 * NT;
-  const long vecs = long(P) * g.mmax;
+  const MkSizes z = multik_sizes(S.N, P, g.mmax);
+  g.cs = z.cs;
+  g.slots = z.slots;
+  const int nmax = 3 * g.mmax, NT = z.NT, pm = z.pm, nch = z.nch;
+  const long vecs = z.vecs, rpc = z.rpc, rotn = z.rotn;
   const int RB = pick_rows(S.nx, S.ny, vecs, g.fx), TX = pick_rows(S.ny, S.nx, vecs, g.fy);
   if (RB == 0 || TX == 0) return ok;
   const int nrb = (S.ny + RB - 1) / RB, ncb = (S.nx + TX - 1) / TX;
-  // Gram chunks: about 128 over the problems, of whole 64-row steps, a stage of every wave or more
-  const int nchunk = int(std::max<long>(1, std::min<long>((S.N + 255) / 256, std::max(8, 128 / P))));
-  const long rpc = ((S.N + nchunk - 1) / nchunk + 63) / 64 * 64;
-  const int nch = int((S.N + rpc - 1) / rpc);
   // the widest space's three matrices and the kernel's own arrays share a CU's 160 KB
   {
     hipFuncAttributes fa{}, fb{};
@@ -1522,23 +1517,22 @@ std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, c
     if (std::max(fa.sharedSizeBytes, fb.sharedSizeBytes) + dyn > 160 * 1024) return ok;
   }
   MultiKWorkspace& W = S.multik_ws;
-  const size_t colb = sizeof(c32) * size_t(P) * g.slots;
   // The pads past N of every plane are read as zeros.  The block update runs over them, so
   // coefficients that are not finite leave NaN there: they count as clear only after a call that
   // ended without.
   const long geom = g.cs * 64 + g.mmax;
-  if (W.cols.size() < colb || W.geom != geom) {
-    W.cols.ensure(colb);
+  if (W.cols.size() < z.cols || W.geom != geom) {
+    W.cols.ensure(z.cols);
     OMX_HIP_CHECK(hipMemsetAsync(W.cols.as<void>(), 0, W.cols.size(), sm));
   }
   W.geom = 0;
-  W.dm.ensure(sizeof(c32) * size_t(vecs) * 3 * g.cs);
-  W.part.ensure(sizeof(c32) * size_t(P) * nch * NGRAM * pm * pm);
-  W.red.ensure(sizeof(c64) * size_t(P) * NGRAM * pm * pm);
+  W.dm.ensure(z.dm);
+  W.part.ensure(z.part);
+  W.red.ensure(z.red);
   W.cx.ensure(sizeof(c32) * size_t(P) * MK_MAXN * MK_MAXM);
-  W.cblk.ensure(sizeof(c64) * size_t(vecs) * MK_MAXN * MK_MAXM);
-  const long rotn = long(MK_SWEEPS) * nmax * ((nmax + 1) / 2);
-  W.rot.ensure(sizeof(MkRot) * size_t(vecs) * rotn);
+  W.cblk.ensure(z.cblk);
+  static_assert(sizeof(MkRot) == 32 && NGRAM == 3 + MK_NODES + 1, "multik_sizes");
+  W.rot.ensure(z.rot);
   W.normp.ensure(sizeof(double) * size_t(vecs) * nrb);
   W.state.ensure(sizeof(MkState) * P);
   W.ints.ensure(sizeof(int) * size_t(P) * MK_MAXM + sizeof(int2) * ninst);

@@ -30,10 +30,6 @@ class Solver;
 struct NewtonState;
 struct SolveStats;
 
-constexpr int MK_MAXM = 18;     // columns per problem: nev (16) + guard (2)
-constexpr int MK_MAXN = 54;     // search space [X W P]
-constexpr int MK_GUARD = 2;
-
 struct MkProblem {
   double omega = 0;
   int nev = 0;
@@ -59,12 +55,6 @@ std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, c
                                int maxit, const std::vector<int>& msize, c64* X64, long ld, long istride,
                                std::vector<double>& kout, std::vector<int>& iters, std::vector<int>& moves,
                                SolveStats& stats);
-
-// columns of the widest block handed over for nev bands on a grid of K unknowns: the space's
-// columns past the bands too
-inline int multik_block(int nev, long K) {
-  return int(std::max<long>(nev, std::min<long>(nev + MK_GUARD, K / 3)));
-}
 
 // whether the grid fits the phase's transforms
 bool multik_fits(const Solver& S);

@@ -1,7 +1,9 @@
 // Scalar pieces of the shared search space (multik.hip): plain functions of doubles, the same
 // on the host and on the device.
 #pragma once
+#include <algorithm>
 #include <cmath>
+#include <cstddef>
 
 #if defined(__HIPCC__)
 #define OMX_HD __host__ __device__ inline
@@ -27,6 +29,11 @@ OMX_HD int mk_position(const double* d, int n, int a) {
   return r;
 }
 
+constexpr int MK_MAXM = 18;   // columns per problem: nev (16) + guard (2)
+constexpr int MK_MAXN = 54;   // search space [X W P]
+constexpr int MK_GUARD = 2;
+constexpr int MK_PLANES = 7;  // planes of a stored column
+constexpr int MK_SWEEPS = 10;  // Jacobi sweeps whose rotations are kept (4 to 7 are made)
 constexpr int MK_NODES = 8;  // interpolation nodes of the norm's Gram matrix
 
 // The norm's entries 1 / (rho^2 + k^2) are interpolated in x = ln k, at Chebyshev nodes over the
@@ -65,6 +72,62 @@ OMX_HD void mk_weight(const double* node, int t, double k, double& w, double& dw
     w *= (x - node[u]) * q;
   }
   dw /= k;
+}
+
+// columns of the widest block handed over for nev bands on a grid of K unknowns: the space's
+// columns past the bands too
+inline int multik_block(int nev, long K) {
+  return int(std::max<long>(nev, std::min<long>(nev + MK_GUARD, K / 3)));
+}
+
+// Shapes and device bytes of the phase's large buffers, for P problems of at most mmax columns on
+// N pixels.
+struct MkSizes {
+  long cs, slots, vecs;  // plane size; complex values of a problem's columns; columns in all
+  int NT, pm;            // 16-column tiles, their columns
+  long rpc;              // rows per Gram chunk
+  int nch;               // Gram chunks
+  long rotn;             // rotations kept per column
+  size_t cols, dm, part, red, cblk, rot;
+  size_t total() const { return cols + dm + part + red + cblk + rot; }
+};
+inline MkSizes multik_sizes(long N, long P, int mmax) {
+  constexpr size_t C32 = 8, C64 = 16, ROT = 32;
+  constexpr int NGRAM = 3 + MK_NODES + 1;
+  MkSizes z;
+  z.cs = (N + 63) / 64 * 64;
+  z.slots = 5L * mmax * MK_PLANES * z.cs;
+  z.vecs = P * mmax;
+  const int nmax = 3 * mmax;
+  z.NT = (nmax + 15) / 16;
+  z.pm = 16 * z.NT;
+  // about 128 Gram chunks over the problems, of whole 64-row steps, a stage of every wave or more
+  const long nchunk = std::max<long>(1, std::min<long>((N + 255) / 256, std::max<long>(8, 128 / P)));
+  z.rpc = ((N + nchunk - 1) / nchunk + 63) / 64 * 64;
+  z.nch = int((N + z.rpc - 1) / z.rpc);
+  z.rotn = long(MK_SWEEPS) * nmax * ((nmax + 1) / 2);
+  z.cols = C32 * size_t(P) * z.slots;
+  z.dm = C32 * size_t(z.vecs) * 3 * z.cs;
+  z.part = C32 * size_t(P) * z.nch * NGRAM * z.pm * z.pm;
+  z.red = C64 * size_t(P) * NGRAM * z.pm * z.pm;
+  z.cblk = C64 * size_t(z.vecs) * MK_MAXN * MK_MAXM;
+  z.rot = ROT * size_t(z.vecs) * z.rotn;
+  return z;
+}
+
+// Device bytes of a launch group of the batched solve: P problems, ninst bands in all, at most M
+// a problem, on N pixels (vectors of K = 2 N in columns of ld).  Whichever is larger: one
+// LOBPCG block per band (both precisions' batches), or the shared search space with the FP64
+// blocks it hands over and their FP32 copy and residuals (a group of few modes a problem: its
+// spaces are three columns per band and guard wide).  With both the refinement's and the
+// correction solves' vectors and the problems' stacked fields.
+inline size_t group_bytes(long N, long K, long ld, long P, long ninst, long M) {
+  M = std::max(1L, std::min(M, 16L));  // mode counts outside are refused later
+  const size_t lob = size_t(ninst) * M * (11 * size_t(ld) + 3 * size_t(N));
+  const size_t both = size_t(ninst) * (16 * 16 * size_t(ld) + 16 * 3 * size_t(N)) + size_t(P) * 144 * size_t(N);
+  const int mb = multik_block(int(M), K);
+  const size_t blocks = size_t(ninst) * mb * (16 * (2 * size_t(ld) + 3 * size_t(N)) + 2 * 8 * size_t(ld));
+  return both + std::max((16 + 8) * lob, blocks + multik_sizes(N, P, mb).total());
 }
 
 }  // namespace omx

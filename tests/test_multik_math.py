@@ -24,6 +24,7 @@ extern "C" void interpolation(const double* k, int n, double at, double* nodes, 
   }
   for (int t = 0; t < omx::MK_NODES; ++t) omx::mk_weight(x, t, at, w[t], dw[t]);
 }
+extern "C" double bytes(long N, long ld, long P, long ninst, long M) { return double(omx::group_bytes(N, 2 * N, ld, P, ninst, M)); }
 extern "C" int nodes() { return omx::MK_NODES; }
 extern "C" int position(const double* d, int n, int a) { return omx::mk_position(d, n, a); }
 """
@@ -35,7 +36,9 @@ def lib(tmp_path_factory):
     src, out = d / "m.cpp", d / "m.so"
     src.write_text(SOURCE)
     subprocess.run([CXX, "-O1", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, str(src), "-o", str(out)], check=True)
-    return ctypes.CDLL(str(out))
+    L = ctypes.CDLL(str(out))
+    L.bytes.restype, L.bytes.argtypes = ctypes.c_double, [ctypes.c_long] * 5
+    return L
 
 
 NAN, INF = float("nan"), float("inf")
@@ -90,3 +93,26 @@ def test_norm_weights_at_a_node_and_for_negative_k(lib):
     _, w, dw = _interpolation(lib, [0.9, 1.2], 1.1)
     _, wn, dwn = _interpolation(lib, [-0.9, -1.2], -1.1)
     assert np.allclose(w, wn) and np.allclose(dw, -dwn)
+
+
+@pytest.mark.parametrize("P,nev", [(1, 1), (40, 1), (40, 2), (12, 4), (5, 16)])
+def test_launch_group_bytes_cover_both_forms(lib, P, nev):
+    """What a launch group holds at once, counted buffer by buffer: the shared search space's
+    columns (X and P twice, W; seven single-precision planes each, for nev + 2 columns a
+    problem) and transform buffer, the blocks it hands over (X, M X, three components, and
+    their single-precision copy and residuals), the refinement's seven vectors and the
+    correction solves' eight with three components; or the per-band form's eleven blocks."""
+    N = 128 * 96
+    ld, ninst, m = 2 * N, P * nev, nev + 2
+    shared = P * m * (5 * 7 + 3) * 8 * N + ninst * m * (2 * 16 * ld + 16 * 3 * N + 2 * 8 * ld)
+    vectors = ninst * (5 * 16 * ld + 3 * 8 * ld + 8 * 8 * ld + 8 * 3 * N) + P * 6 * N * 2 * (4 + 8)
+    per_band = 24 * ninst * nev * (11 * ld + 3 * N)
+    got = lib.bytes(N, ld, P, ninst, nev)
+    assert got >= vectors + shared
+    assert got >= vectors + per_band
+    assert got < 3 * (vectors + max(shared, per_band))
+
+
+def test_launch_group_bytes_of_refused_mode_counts(lib):
+    for nev in (-3, 0, 17, 2 ** 31 - 1):
+        assert 0 < lib.bytes(256, 512, 1, 1, nev) < 1e9
