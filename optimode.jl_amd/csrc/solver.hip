@@ -2297,6 +2297,17 @@ void Solver::solve_k(double omega, int nev, double k_tol, double eig_tol, int ma
   }
   if (!ok && mk_done) {
     ++solve_phases().redone;
+    // this run's device time counts too, whether the next one ends in a result or an error
+    struct AddTime {
+      omx_info* info;
+      float ms = 0;
+      ~AddTime() {
+        if (info) info->device_ms += ms;
+      }
+    } before{info};
+    OMX_HIP_CHECK(hipEventRecord(e1, stream));
+    OMX_HIP_CHECK(hipStreamSynchronize(stream));
+    OMX_HIP_CHECK(hipEventElapsedTime(&before.ms, e0, e1));
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     WithoutMultiK off(*this);

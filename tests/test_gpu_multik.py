@@ -4,6 +4,9 @@ column blocks), the smallest and the widest blocks, every kind of start, and bat
 
 Both forms end in the same FP64 refinement with |change of w^2| <= k_tol = 1e-11, so k agrees
 to k_tol / (slope k) <= 1e-11 / (2 * 0.3 * 0.3) < 6e-11; 2e-10 allows for both sides."""
+import ctypes
+import time
+
 import numpy as np
 import pytest
 
@@ -289,3 +292,24 @@ def test_a_tolerance_below_rounding_costs_one_solve(monkeypatch, capfd):
     print(f"  refinement steps {steps}, {omx.solve_phases()}", flush=True)
     assert omx.solve_phases() == REDONE
     assert steps[0] <= 8
+
+
+def test_device_time_of_a_solve_done_twice():
+    """device_ms is the call's: of a solve whose first run ends undone, both runs'.  On a warm
+    handle the device works for all but the host's share of the wall time (a tenth of such a
+    solve; the first run takes three quarters of this one)."""
+    print("multik device time", flush=True)
+    g, ei = _eps(128, 96)
+    L, P = omx._lib.lib(), omx._lib
+    h = omx.HIPSolver().handle(g, ei)
+    km = np.empty(4)
+    share = []
+    for _ in range(4):
+        info = omx.OmxInfo()
+        t = time.perf_counter()
+        st = L.omx_solve_k(h.h, W0, 4, 1e-10, 1e-17, 4, 100, None, None, 0, P.dptr(km), None, ctypes.byref(info))
+        t = time.perf_counter() - t
+        assert st == P.OMX_ERR_NOT_CONVERGED and omx.solve_phases() == REDONE
+        share.append(1e-3 * info.device_ms / t)
+    print(f"  device time over wall time {share}", flush=True)
+    assert max(share[1:]) > 0.8
