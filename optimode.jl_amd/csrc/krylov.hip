@@ -834,7 +834,9 @@ template <typename F> void with_qm(int n, const F& f) {
   }
 }
 
+// the Schur form's kernels are compiled for the FP32 correction solves, the only ones that use it
 template <typename T> void VecOpsT<T>::set_schur(const C* Rb, const double* weights) {
+  if (sizeof(T) != 4) throw Error(OMX_ERR_INTERNAL, "the Schur complement is for FP32 vectors");
   if (!Q) throw Error(OMX_ERR_INTERNAL, "the Schur complement needs the block projection");
   R = Rb;
   rg = weights;
@@ -842,10 +844,11 @@ template <typename T> void VecOpsT<T>::set_schur(const C* Rb, const double* weig
 
 // partials of Q^H x and R^H x (past the real partials) and of Re <d, x> (out)
 template <typename T> void VecOpsT<T>::dots_schur(const C* x, const int* act, const C* d, double* out) {
-  with_qm(qmax, [&](auto QMc) {
-    hipLaunchKernelGGL((k_qdot<T, decltype(QMc)::value, true>), dim3(qblk, nb, 2), dim3(AB), 0, s, Q, R, ld, qistride,
-                       qn, x, d, ld, K, act, part.template as<c64>() + size_t(nb) * nblk, out);
-  });
+  if constexpr (sizeof(T) == 4)
+    with_qm(qmax, [&](auto QMc) {
+      hipLaunchKernelGGL((k_qdot<T, decltype(QMc)::value, true>), dim3(qblk, nb, 2), dim3(AB), 0, s, Q, R, ld, qistride,
+                         qn, x, d, ld, K, act, part.template as<c64>() + size_t(nb) * nblk, out);
+    });
 }
 
 template <typename T> void VecOpsT<T>::project_dot_to(C* x, const int* act, const C* dot_with, double* out) {
@@ -967,10 +970,12 @@ int minres_complement_t(Solver& S, VecOpsT<T>& V, const std::vector<double>& shi
                          wx ? coef + 4 * nb : nullptr, V.Q, V.R, V.qistride, V.qn, qrc);
     };
     auto y1q = [&](auto WXc) {
-      if (!V.R)
-        y1(WXc, std::integral_constant<int, 0>{});
-      else
-        with_qm(V.qmax, [&](auto q) { y1(WXc, q); });
+      if constexpr (sizeof(T) == 4)
+        if (V.R) {
+          with_qm(V.qmax, [&](auto q) { y1(WXc, q); });
+          return;
+        }
+      y1(WXc, std::integral_constant<int, 0>{});
     };
     if (fuse)
       y1q(std::true_type{});
