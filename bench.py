@@ -27,13 +27,13 @@ HBM_PEAK_GBS = 8000.0
 OMEGA = 1 / 1.55
 NEV = 8
 REL_TOL = 1e-8
-# HBM bytes per algorithmic byte of the FP32 operator application on this workload, from
-# rocprofv3 FETCH_SIZE + WRITE_SIZE of the k_rpass1/2/3<float, OP_M> launches of the
-# refinement's correction solves (8 vectors, all active, so their algorithmic bytes are
-# exact), FETCH scaled by 2.0 and WRITE by 1.0 (the factors `bench.py --workload copy`, a
-# 256 MiB device copy, reads back on the same box); the measurement is kept in
-# profiles/solve_k_tfln256_pmc_traffic.md.  Update when the kernels change.
-OP_TRAFFIC_RATIO = 3.78
+# HBM bytes per algorithmic byte of the shared search space's transforms on this workload (one
+# interval of omx_get_kernel_stats: k_mk_colE .. k_mk_colF of an iteration), from rocprofv3
+# FETCH_SIZE + WRITE_SIZE of those kernels over a solve, FETCH scaled by 2.0 and WRITE by 1.0
+# (the factors `bench.py --workload copy`, a 256 MiB device copy, reads back on the same
+# box), against the algorithmic bytes the same solve counts; kept in
+# profiles/shared_space_pmc.md.  Update when the kernels change.
+OP_TRAFFIC_RATIO = 7.03
 
 
 def cpu_baseline(seconds_cap=60.0):
@@ -495,7 +495,8 @@ def main():
         roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": round(achieved / HBM_PEAK_GBS, 4),
                     "traffic": round(OP_TRAFFIC_RATIO * op_bytes / op_n),
-                    "kernel": "FP32 Helmholtz operator application (3 fused passes)",
+                    "kernel": "FP32 search-space transforms of an iteration (operator, residual, preconditioner, "
+                              "directions: 5 kernels and the control step)",
                     "launches": op_n, "avg_us": round(1e3 * op_ms / op_n, 2),
                     "avg_alg_bytes": round(op_bytes / op_n)}
 
@@ -526,7 +527,8 @@ def main():
             "fp64_rr_steps_per_step": float(np.mean([i["lobpcg_iters_fp64"] for i in infos])),
             "newton_steps_per_step": float(np.mean([i["n_newton"] for i in infos])),
             "matvecs_per_step": float(np.mean([i["n_matvec"] for i in infos])),
-            "parallelism": "single GPU; bands batched as independent Newton instances",
+            "parallelism": "single GPU; FP32 phase in one search space for all bands, FP64 refinement with an "
+                           "instance per band",
             "autotuned": tuned,
             "start": "learned (omx/data/warmnet_tfln256.npz, guess inside the timed region)" if st is not None
                      else "plain (k_guess, random vectors)",

@@ -1444,7 +1444,9 @@ bool fits(int nb, const FFTFactors& f, int vpt) {
 constexpr size_t MK_LDS = 64 * 1024;
 
 // sequences of length L per block for three planes: at most 16, within MK_LDS and the bound of
-// 16 values per thread; fewer while the launch would leave CUs idle
+// 16 values per thread; fewer while the launch would leave CUs idle.  The line at 512 blocks, two
+// per CU: at 256^2 with 10 columns an iteration's transforms take 149 us with 4 sequences a
+// block and 172 us with 8 (a line at 256); a line at 1024 changes nothing from 128^2 to 512 x 256.
 int pick_rows(int L, int other, long vecs, const FFTFactors& f) {
   int r = 16;
   while (r > 1 && (sizeof(c32) * (L + 3 * size_t(r) * (L + 1)) > MK_LDS || !fits(3 * r, f, 16))) r /= 2;
@@ -1582,6 +1584,12 @@ std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, c
     transforms(v8{}, std::true_type{});
   else
     transforms(v16{}, std::true_type{});
+  // Rows per stage and lane, and norm matrices per block, by column tiles (us a launch, rows 2 /
+  // 4 at the chosen matrices, then matrices 1 / 2 / 3 at the chosen rows): 18 columns at 128^2
+  // 34.4 / 32.2, 32.5 / 28.6 / 32.2; 30 at 256^2 109 / 103, 106 / 95 / 103; 42 at 384^2 383 / 356,
+  // 424 / 383 / 783; 54 at 512 x 256 591 / 753, 591 / 961 / 2459.  Above two tiles more of either
+  // spills the accumulators; at two tiles 2 matrices and at three 4 rows are up to 8% faster than
+  // what is launched.
   auto gram = [&](auto T, int buf) {
     constexpr int nt = decltype(T)::value;
     constexpr int S_ = nt <= 2 ? 4 : 2, NB = nt <= 2 ? 3 : (nt == 3 ? 2 : 1);
@@ -1596,6 +1604,19 @@ std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, c
   };
   const dim3 gcomb(unsigned(std::min<long>((PLANES * g.cs / 2 + 255) / 256, std::max(1, 2048 / P))), P);
   const bool prof = S.prof.enabled;
+  // operator intervals (omx_get_kernel_stats): M x of every column of the problems that still
+  // ran, P r of those that went on; counted once the iteration's state is known
+  hipEvent_t mark[2][2] = {};
+  auto count = [&](int at, const MkState* h) {
+    double b = 0;
+    for (int p = 0; p < P; ++p)
+      if (h[p].iter == at + 1)
+        b += 32.0 * S.N * h[p].m + 24.0 * S.N + (h[p].done ? 0.0 : 32.0 * S.N * h[p].na + 24.0 * S.N);
+    if (b > 0)
+      S.prof.commit(mark[at & 1][0], mark[at & 1][1], &S.prof.op32, b);
+    else
+      S.prof.recycle(mark[at & 1][0], mark[at & 1][1]);
+  };
   int cur = 0, it = 0;
   bool fin = false;
   for (; it < maxit && !fin; ++it) {
@@ -1629,7 +1650,10 @@ std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, c
     else
       chain(v16{});
     OMX_HIP_CHECK(hipGetLastError());
-    if (prof) S.prof.commit(ea, S.prof.begin(sm), &S.prof.op32, 2.0 * (32.0 * S.N * vecs + 24.0 * S.N * P));
+    if (prof) {
+      mark[it & 1][0] = ea;
+      mark[it & 1][1] = S.prof.begin(sm);
+    }
     OMX_HIP_CHECK(hipMemcpyAsync(W.snap[it & 1].as<void>(), st, sizeof(MkState) * P, hipMemcpyDeviceToHost, sm));
     OMX_HIP_CHECK(hipEventRecord(W.ev[it & 1], sm));
     cur ^= 1;
@@ -1637,6 +1661,7 @@ std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, c
     // the state after the iteration before (an iteration enqueued after the end does nothing)
     OMX_HIP_CHECK(hipEventSynchronize(W.ev[(it - 1) & 1]));
     const MkState* h = W.snap[(it - 1) & 1].as<MkState>();
+    if (prof) count(it - 1, h);
     fin = true;
     for (int p = 0; p < P; ++p) fin = fin && h[p].done;
     if (S.trace) {
@@ -1652,6 +1677,7 @@ std::vector<char> multik_solve(Solver& S, const std::vector<MkProblem>& probs, c
   }
   OMX_HIP_CHECK(hipStreamSynchronize(sm));
   OMX_HIP_CHECK(hipMemcpy(hs.data(), st, sizeof(MkState) * P, hipMemcpyDeviceToHost));
+  if (prof && it > 0) count(it - 1, hs.data());
   bool finite = true;
   for (int p = 0; p < P; ++p) {
     ok[p] = hs[p].done == 1;

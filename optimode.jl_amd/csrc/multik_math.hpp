@@ -102,6 +102,8 @@ inline MkSizes multik_sizes(long N, long P, int mmax) {
   z.NT = (nmax + 15) / 16;
   z.pm = 16 * z.NT;
   // about 128 Gram chunks over the problems, of whole 64-row steps, a stage of every wave or more
+  // (32 / 64 / 128 / 256 chunks, us a launch: 128 / 111 / 103 / 103 at 256^2 and 30 columns, 554 /
+  // 406 / 383 / 383 at 384^2 and 42, 1022 / 601 / 591 / 608 at 512 x 256 and 54)
   const long nchunk = std::max<long>(1, std::min<long>((N + 255) / 256, std::max<long>(8, 128 / P)));
   z.rpc = ((N + nchunk - 1) / nchunk + 63) / 64 * 64;
   z.nch = int((N + z.rpc - 1) / z.rpc);

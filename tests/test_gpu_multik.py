@@ -316,3 +316,19 @@ def test_device_time_of_a_solve_done_twice():
         share.append(1e-3 * info.device_ms / t)
     print(f"  device time over wall time {share}", flush=True)
     assert max(share[1:]) > 0.8
+
+
+def test_kernel_stats_count_the_columns_that_ran():
+    """The profile's bytes of the shared space: the operator on all m columns of every iteration
+    made, the preconditioner on those that went on (all in the first, none in the last)."""
+    print("multik kernel stats", flush=True)
+    g, ei = _eps(64, 48)
+    nev, m = 4, 6
+    s = omx.HIPSolver(profile=True)
+    _, _, info = _solve(g, ei, nev, 1, solver=s)
+    ms, n, b = omx.kernel_stats(s, "op_fp32")
+    one, per = 32.0 * g.N, 24.0 * g.N
+    print(f"  {n} intervals, {ms:.3f} ms, {b / (one + per):.1f} columns", flush=True)
+    assert info["lobpcg_iters_fp32"] / nev <= n <= info["lobpcg_iters_fp32"]
+    assert ms > 0
+    assert n * (one * m + per) + one * m + per <= b < (2 * n - 1) * (one * m + per)
