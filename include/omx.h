@@ -102,17 +102,22 @@ const char* omx_last_error(const omx_solver* h);
    band) with its iteration cap "multik_maxit" (200; a solve that reaches it is done per band;
    the batch has the default); "guess_lowres" = hw > 0 (even, <= Nx, Ny):
    omx_solve_k's Hguess vectors hold only their hw x hw lowest plane waves, 2 hw^2 complex
-   each at c + 2(gx + hw gy) in FFT order, and are scattered into the start block on the GPU */
+   each at c + 2(gx + hw gy) in FFT order, and are scattered into the start block on the GPU.
+   With "multik" at 1, "fp32_switch", "streams2", "gram_blocks" and "combine_blocks" act on 2D
+   cells only where a solve runs per band (the default batch and solve_k otherwise do not use what
+   they set), and the FP32 operator's options on the refinement's correction solves. */
 int omx_set_option(omx_solver* h, const char* key, double value);
 
 /* Autotuner (the reference's counterpart is FFTW's PATIENT planning when a ModeSolver is built,
    lib/MaxwellEigenmodes/src/maxwell.jl:940-943): timed trials on this handle's grid of the
-   kernels of an nev-mode omx_solve_k, with the shapes its FP32 phase launches them with --
+   kernels of an nev-mode omx_solve_k, with the shapes its per-band FP32 phase launches them with --
    the operator path (register FFT, with its rows per block of passes 1/3 and threads of pass
    2, or LDS Stockham), the Stockham FFT radix variant and tile shape (rows / columns per
    block), on 3D cells the yz-slab or five-pass form, and the Gram and block-update row
    partitions.  A candidate plan is used only if its output equals the default plan's to 1e-5.
-   The fastest of each becomes the handle's option; the same choice can be applied to another
+   The block partitions are those of the per-band FP32 phase (3D cells, option "multik" = 0,
+   omx_solve_omega2); the search space of the default 2D omx_solve_k takes the FFT radix variant
+   alone, its own kernels have no trials.  The fastest of each becomes the handle's option; the same choice can be applied to another
    handle of the grid with omx_set_option ("reg_ops", "fft_variant32", "tile_rows32",
    "tile_cols32", "gram_blocks", "combine_blocks", "slab3d", "reg_rows32", "reg_nt2").
    choice_out: NULL or 9 ints in that order; us_out: NULL or 3 doubles, microseconds per launch
@@ -173,8 +178,10 @@ int omx_ng_gvd(omx_solver* h, double omega, int nev, const double* kmags, const 
    lib/ModeSweeps/src/batch.jl:256-265).  Problems may differ in grid, eps^-1, ω, nev and
    tolerances.  They are bucketed by grid; a bucket runs on one handle and one HIP stream in
    launch groups of as many problems as fit half the free device memory (at most max_group
-   problems when max_group > 0): every band of every problem of a group is an instance of the
-   same LOBPCG, Newton, refinement and phase launches.  Per-problem results and status go into
+   problems when max_group > 0): the problems of a group share the launches of the FP32 search
+   (one search space per problem, or one LOBPCG block per band), the refinement (one instance per
+   band) and the phase step.  A problem that its search space does not finish is solved again
+   per band, with the others left undone.  Per-problem results and status go into
    probs (info.lobpcg_iters_fp32 and converged are the problem's own; the FP64 step count,
    matvecs and device_ms are its launch group's); the call returns OMX_OK when every problem
    succeeded, else the first failing status.  fp64_only != 0 runs every solve in FP64. */
@@ -333,7 +340,11 @@ int omx_solve_k_learned(omx_solver* h, omx_warmnet* net, double omega, int nev, 
    measurement).  With omx_set_option(h, "profile", 1) every operator application inside
    a solve is bracketed by HIP events on the handle's stream; `family` is "op_fp32" or
    "op_fp64".  Returns total milliseconds, launches and algorithmic bytes
-   (32 N m + 24 N per FP32 application of m vectors, twice that in FP64). */
+   (32 N m + 24 N per FP32 application of m vectors, twice that in FP64).  In the search space
+   all bands share (option "multik") an interval of "op_fp32" is one iteration's transforms:
+   the operator on every column, the residuals and their norms, the convergence control, and the
+   preconditioner and the new directions' fields of the columns that go on; it counts the
+   bytes of those two applications.  The refinement's applications are not bracketed. */
 int omx_get_kernel_stats(omx_solver* h, const char* family, double* total_ms, int64_t* launches, double* bytes);
 
 /* Which form the FP32 phases of the calling thread's last omx_solve_k, omx_solve_k_learned or

@@ -99,10 +99,10 @@ class Profiler {
 };
 
 struct Options {
-  double fp32_tol_rel = 2e-3;   // solve_k: FP32 LOBPCG locking threshold of the Newton phase, relative
-                                // to omega^2 (the FP64 refinement takes the vectors from there)
+  double fp32_tol_rel = 2e-3;   // solve_k: residual threshold of the FP32 phase, relative to
+                                // omega^2 (the FP64 refinement takes the vectors from there)
   double fp32_tol_omega2 = 1e-5;  // solve_omega2: FP32 locking threshold before its FP64 LOBPCG
-  double fp32_switch = 1e-6;    // |Δω²|/ω² below which Newton moves to the FP64 phase
+  double fp32_switch = 1e-6;    // |Δω²|/ω² below which the per-band Newton moves to the FP64 phase
   double seed_tol = 0;          // locking threshold / omega^2 of the shared first eigensolve
                                 // (0: 1e-1 on 2D cells in the two-stream FP32 phase of a single
                                 // solve, 5e-2 in batches and the other paths, 3e-3 on 3D cells,
@@ -240,8 +240,7 @@ class Solver {
                const double* kguess, const double* Hguess, int nguess, double* kmags, double* evecs, omx_info* info);
   void get_evecs(double* evecs);
   // solve_k for several problems on this handle's grid (own eps^-1, omega, nev and tolerances
-  // each) as one batch: every band of every problem is an instance of the same LOBPCG,
-  // Newton and refinement launches (2D cells)
+  // each) as one batch that shares its launches (2D cells); solve_group is one run over them
   void solve_k_multi(std::vector<MultiProblem>& probs);
   std::vector<int> solve_group(std::vector<MultiProblem>& probs, bool shared);
   void hmh(double k, const double* A, const double* H, int m, double* out);

@@ -127,9 +127,9 @@ class HIPSolver:
 
     ``precision`` is the policy of the iterative phase: ``"mixed"`` (default: FP32
     operator applications, then an FP64 refinement phase) or ``"fp64"``.  Tolerance
-    knobs of the FP32 phase are relative to ω²: ``fp32_tol`` (``solve_k``'s LOBPCG locking
+    knobs of the FP32 phase are relative to ω²: ``fp32_tol`` (``solve_k``'s residual
     threshold, 2e-3: the FP64 refinement finishes the vectors) and ``fp32_switch``
-    (|Δω²|/ω² at which Newton moves to FP64).  ``reg_ops=False`` keeps
+    (|Δω²|/ω² at which the per-band form's Newton moves to FP64).  ``reg_ops=False`` keeps
     the FP32 operator on the LDS Stockham FFT even where the register-FFT kernels apply
     (power-of-two grids 64 to 512).  ``plain=True`` runs the reference's algorithm on the same
     kernels, as the baseline the optimised path is measured against: FP64 throughout, an
@@ -358,8 +358,9 @@ def solve_k_batch(problems, precision="mixed", device=0, fetch_evecs=False, max_
     is a dict with ``grid``, ``epsinv``, ``omega``, ``nev`` and optionally ``k_tol``,
     ``eig_tol`` (1e-8), ``max_eigsolves`` (60), ``maxiter`` (100).  Problems may differ in
     grid, ε⁻¹, ω and nev.  Problems on one grid run as launch groups (``max_group`` problems at
-    most when positive, else as many as fit half the free device memory): every band of
-    every problem of a group is an instance of the same kernel launches.  Returns one dict
+    most when positive, else as many as fit half the free device memory) that
+    share every kernel launch; a problem that does not finish leaves the others' results as they
+    are.  Returns one dict
     per problem: ``kmags``, ``evecs`` (when ``fetch_evecs``), ``info`` and ``status``
     (0 = OMX_OK)."""
     n = len(problems)
