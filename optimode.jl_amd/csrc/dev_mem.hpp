@@ -26,11 +26,11 @@ class DevCache {
     static thread_local DevCache* c = nullptr;
     return c;
   }
-  // A kept block serves a request of at least an eighth of it, blocks up to 64 MiB any smaller
+  // A kept block serves a request of at least an eighth of it, blocks up to 256 MiB any smaller
   // one too: a small buffer never sits on a large block that the next large one then has to
   // be allocated beside, and which dropping the kept blocks would not free.
   static bool serves(size_t cap, size_t bytes) {
-    return cap >= bytes && (cap <= (size_t(64) << 20) || cap / 8 <= bytes);
+    return cap >= bytes && (cap <= (size_t(256) << 20) || cap / 8 <= bytes);
   }
   // the smallest kept block that serves `bytes` (its size into cap), or nullptr
   void* take(size_t bytes, size_t& cap) {

@@ -65,9 +65,9 @@ int main() {
   DevMem plain(5);
   { DevMem other(std::move(plain)); CHECK(other.size() == 5 && plain.size() == 0); }
   CHECK(used == 0);
-  for (size_t cap : {size_t(1), 64 * MB, 64 * MB + 1, 1000 * MB})
+  for (size_t cap : {size_t(1), 256 * MB, 256 * MB + 1, 1000 * MB})
     for (size_t n : {size_t(1), size_t(1000), 16 * MB, 64 * MB, 250 * MB, 1000 * MB})
-      CHECK(DevCache::serves(cap, n) == (cap >= n && (cap <= 64 * MB || cap < 8 * n + 8)));
+      CHECK(DevCache::serves(cap, n) == (cap >= n && (cap <= 256 * MB || cap < 8 * n + 8)));
   return 0;
 }
 """
