@@ -199,6 +199,28 @@ def test_a_batch_redone_whole():
         assert np.max(np.abs(q["kmags"] / k0 - 1)) < 2e-9
 
 
+def test_a_batch_with_both_kinds_of_results():
+    """Sixteen iterations are enough for the lowest mode of a smooth guide, not for the ridges:
+    one problem's result comes from the shared search space, its neighbours' from the run per
+    band after it.  k and vectors of all of them against solves of their own."""
+    print("multik batch of both kinds", flush=True)
+    g, ridge = _eps(64, 48)
+    x, y = np.arange(64)[:, None] * 6 / 64 - 3, np.arange(48)[None, :] / 12 - 2
+    eps = 2.1 + 2.1 * np.exp(-x ** 2 - (y / 0.6) ** 2)
+    smooth = np.ascontiguousarray(np.eye(3)[:, :, None, None] / eps)
+    tol = dict(k_tol=1e-11, eig_tol=1e-9)
+    probs = [dict(grid=g, epsinv=e, omega=W0 * f, nev=n, maxiter=2, max_eigsolves=60, **tol)
+             for e, f, n in ((ridge, 1.0, 4), (smooth, 1.0, 1), (ridge, 1.05, 3))]
+    res = omx.solve_k_batch(probs, fetch_evecs=True)
+    assert omx.solve_phases() == dict(shared=1, per_band=2, redone=2)
+    for p, q in zip(probs, res):
+        assert q["status"] == 0 and q["info"]["converged"] == 1 and q["info"]["max_residual"] <= 1e-9
+        k0, ev0 = omx.solve_k(p["omega"], p["epsinv"], g, omx.HIPSolver(), nev=p["nev"], maxiter=300, **tol)
+        assert np.max(np.abs(q["kmags"] / k0 - 1)) < 2e-10
+        for a, b in zip(q["evecs"], ev0):
+            assert abs(abs(np.vdot(a, b)) - 1) < 1e-9
+
+
 @pytest.mark.parametrize("nx,ny,nev", [(45, 45, 4), (27, 45, 12)])
 def test_the_shared_space_works_again_after_a_solve_that_overflowed(nx, ny, nev):
     """Start vectors of 1e25 overflow single precision in the first iteration, the norm's
