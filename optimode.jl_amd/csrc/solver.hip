@@ -2569,10 +2569,13 @@ std::vector<int> Solver::solve_group(std::vector<MultiProblem>& probs, bool shar
     }
     msize = msize_mk;
     for (int i = 0; i < ninst; ++i) {
+      if (!mk_ok[prob_of[i]]) {  // no part in the refinement (and a k that may not be finite)
+        hns[i].done = 2;
+        kk[i] = kinit[i];
+      }
       hns[i].k = kk[i];
       hns[i].nsolves = 1;
       hns[i].k_tol = probs[prob_of[i]].k_tol;
-      if (!mk_ok[prob_of[i]]) hns[i].done = 2;  // no part in the refinement
       it32_inst[i] += its[i];
       stats.it32 += its[i];
     }
